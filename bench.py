@@ -65,14 +65,12 @@ def shape_of(t):
 
 
 def kernel_name(t):
-    """The device kernel a launch shape runs on the 45^3 octant (a grid the
-    pool kernel takes), as rocprofv3 names it."""
+    """The device kernels of a large sweep of the 45^3 octant (a grid the
+    pool takes) at a launch shape, as rocprofv3 names them."""
     from mocassin_amd._capi import KERNELS
-    k = t.get("kernel", 0)
-    if k == KERNELS["auto"]:
-        k = KERNELS["spare"] if t["blocks_per_cu"] <= 3 else KERNELS["pool"]
-    return {KERNELS["one"]: "mcd::transport_kernel<false>", KERNELS["spare"]: "mcd::transport_kernel<true>",
-            KERNELS["pool"]: "mcd::pool_kernel<8, 32>"}[k]
+    if t.get("kernel", 0) == KERNELS["one"]:
+        return "mcd::transport_kernel<false>"
+    return "mcd::log_kernel<8> + mcl::sort_kernel + mcl::plan_kernel + mcl::reduce_kernel"
 
 
 def lanes_per_pass(c):
@@ -381,8 +379,8 @@ def main():
     log("%.3e packets/s, kernel %.1f ms/launch, %.3g seg/packet, %.3g abs/packet"
         % (value, kms, c0["n_seg"] / npk, c0["n_abs"] / npk))
     # HBM bytes per launch: calibrated rocprofv3 FETCH_SIZE + WRITE_SIZE per
-    # packet of this workload times this launch, when the profile's launch
-    # shape is the one measured now
+    # packet of this workload times this launch, when the profile's kernels
+    # and launch shape are the ones measured now
     traffic, traffic_note = None, "no calibrated counter profile of this workload"
     valu = None
     tp = os.path.join(ROOT, "profiles", "transport_c2_traffic.json")
@@ -390,7 +388,7 @@ def main():
         try:
             tj = json.load(open(tp))
             shape = shape_of(tuning)
-            if tj.get("tuning") == shape and tj.get("tables") == "iterated":
+            if tj.get("kernel") == kernel_name(tuning) and tj.get("tuning") == shape and tj.get("tables") == "iterated":
                 traffic = tj["hbm_bytes_per_packet"] * npk
                 traffic_note = "profiles/transport_c2_traffic.json (%s)" % tj.get("tuning")
                 # the walk's instruction issue: wave64 VALU instructions of
@@ -403,10 +401,10 @@ def main():
                         "frac": insts / (kms * 1e-3) / peak, "instructions": insts,
                         "source": "profiles/transport_c2_traffic.json (SQ_INSTS_VALU, %s)" % tj.get("tuning")}
             else:
-                traffic_note = "profile of another launch shape or tables (%s, %s): not used" % (
-                    tj.get("tuning"), tj.get("tables"))
-                log("traffic profile is of %s/%s, the run is %s/iterated: traffic not reported"
-                    % (tj.get("tuning"), tj.get("tables"), shape))
+                traffic_note = "profile of other kernels, launch shape or tables (%s, %s, %s): not used" % (
+                    tj.get("kernel"), tj.get("tuning"), tj.get("tables"))
+                log("traffic profile is of %s/%s/%s, the run is %s/%s/iterated: traffic not reported"
+                    % (tj.get("kernel"), tj.get("tuning"), tj.get("tables"), kernel_name(tuning), shape))
         except (OSError, ValueError, KeyError):
             pass
     out = {

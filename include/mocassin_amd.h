@@ -101,21 +101,21 @@ typedef struct {
  *   threads        workgroup size, a multiple of 64 (64..256)
  *   emit_min       an emission pass runs when at least this many lanes of a
  *                  wavefront wait for one (1..64), or half the live lanes do
- *                  (the pool kernels: when at least this many lanes do not
+ *                  (with a packet pool: when at least this many lanes do not
  *                  walk, or none does)
  *   walk_steps     walk passes between two emission checks (1..64)
- *   kernel         MC_KERNEL_AUTO: two packets per lane when blocks_per_cu
- *                  is at most 3, else the pool kernel where the grid allows
- *                  it, else one packet per lane;
- *                  MC_KERNEL_ONE: one packet per lane;
- *                  MC_KERNEL_SPARE: two packets per lane (a lane whose
- *                  flight ends walks its spare while the next emission pass
- *                  waits; 3 wavefronts per SIMD at most);
- *                  MC_KERNEL_POOL: one packet per lane and a pool of 32
- *                  packets per wavefront in LDS (a lane whose flight ends
- *                  takes a walking packet from the pool; emission passes run
- *                  on nearly full wavefronts); needs a grid of at most
- *                  2047 x 2047 x 1023 cells and 65535 bins (MC_EUNSUP).
+ *   kernel         MC_KERNEL_ONE: one packet per lane, deposits with FP64
+ *                  atomics; every other value: one packet per lane and a pool
+ *                  of 32 packets per wavefront in LDS (a lane whose flight
+ *                  ends takes a walking packet from the pool; emission passes
+ *                  run on nearly full wavefronts) where the grid allows it
+ *                  (at most 2047 x 2047 x 1023 cells and 65535 bins; beyond
+ *                  that MC_KERNEL_POOL is MC_EUNSUP and the others run one
+ *                  packet per lane).  The pool's sweeps log their deposits
+ *                  and sum them by range of the estimators (up to 4 GiB of
+ *                  log per device, shared by its contexts and freed with the
+ *                  last); small sweeps, crossing counts and devices without
+ *                  the memory use atomics.
  * Results do not depend on these values (each packet has its own stream).
  * A new context starts with 4, 256, 16, 16, MC_KERNEL_AUTO. */
 #define MC_KERNEL_AUTO 0
@@ -219,7 +219,8 @@ int mc_fetch_crossings(mc_ctx *ctx, uint32_t *crossings);
  *   waves_per_cu  resident one-wavefront workgroups requested per compute
  *                 unit (1..32)
  *   emit_min, walk_steps  as in mc_tuning
- *   chunk         packets handed to a wavefront at a time (64..2^24)
+ *   chunk         64..2^24; sets the noalloc call's limit below.  Wavefronts
+ *                 take packets from a counter per model, whatever its value.
  * Results do not depend on these values. */
 typedef struct {
     int32_t waves_per_cu;
@@ -243,8 +244,7 @@ int mc_transport_batch(mc_ctx *const *ctx, int32_t n, const int32_t *istar, cons
 /* mc_transport_batch without any device allocation: no counterpart in the
  * reference; for callers that cannot allocate device memory (serving loops,
  * code under graph capture).  Same arguments and results.  The launch's
- * working block (the models' grids, run arguments and counters, the chunk
- * table) lives in a fixed 8 MiB device array that each GPU the library runs
+ * working block (the models' grids, run arguments and counters) lives in a fixed 8 MiB device array that each GPU the library runs
  * on holds until the process ends; a launch that needs more (at most 256
  * models; 16 bytes per chunk of `chunk` packets) is refused with MC_EINVAL
  * before anything runs.  Every call on a GPU reuses that array: calls that

@@ -3,12 +3,12 @@
 The transport kernel has five free parameters (mc_tuning in
 include/mocassin_amd.h): resident workgroups per CU, workgroup size, the
 number of waiting lanes that triggers a batched emission pass, the number
-of walk passes between emission checks, and the kernel (auto: at most 3
-workgroups of 256 per CU select the kernel with two packets per lane; pool:
-one packet per lane and a pool of packets per wavefront in LDS).  The
-default candidates are the auto grid and a pool grid.  The batched kernel
-(mc_batch_tuning) has resident wavefronts per CU, the same two scheduling
-parameters, and the packet-batch size handed to a wavefront at a time.
+of walk passes between emission checks, and the kernel (auto and pool: one
+packet per lane and a pool of packets per wavefront in LDS where the grid
+allows it; one: one packet per lane).  The default candidates are the auto
+grid and a pool grid.  The batched kernel (mc_batch_tuning) has resident
+wavefronts per CU and the same two scheduling parameters; its fourth field,
+chunk, sets a limit of mc_transport_batch_noalloc and nothing else.
 Results do not depend on any of them (every packet draws from its own
 counter-based stream), so the tuner only times: it runs a short transport
 of the real problem for each candidate and keeps the fastest by device time.

@@ -14,6 +14,7 @@
 
 #include "../../include/mocassin_amd.h"
 #include "mc_balance.h"
+#include "mc_deposit.h"
 #include "mc_device.h"
 #include "mc_dust.h"
 #include "mc_emission.h"
@@ -47,15 +48,17 @@ struct mc_ctx {
     int nStars = 0;
     std::vector<float> starPos, deltaE;
     std::vector<int> starIdx;
-    bool tables = false;
+    bool tables = false, counted = false;    // counted: among its device's contexts (the deposit log's users)
+    double seg_per_packet = 0.0;             // of the last sweep
     int cus = 256;
-    mc_tuning tune = { 4, 256, 16, 16, MC_KERNEL_AUTO };   // the pool kernel where the grid allows    // the autotuner's best on the octant; within 1.3% on the dust and clumpy grids
+    mc_tuning tune = { 4, 256, 16, 16, MC_KERNEL_AUTO };   // the pool where the grid allows it
     // device allocations
     float *d_axis = nullptr, *d_mid = nullptr, *d_dfac = nullptr;
     int *d_active = nullptr;
     float *d_opac3 = nullptr, *d_sca3 = nullptr, *d_recCDF = nullptr;
     unsigned short *d_recGuide = nullptr;
     float *d_totalLines = nullptr, *d_specCDF = nullptr, *d_nuArray = nullptr, *d_gSca = nullptr;
+    unsigned short *d_specGuide = nullptr;
     double *d_J3 = nullptr, *d_J = nullptr, *d_esc = nullptr;
     mcd::View *d_view = nullptr;            // viewing-angle bins (null: escapes in plane 0 only)
     int esc_planes = 1;                      // nAngleBins + 1
@@ -146,10 +149,20 @@ static int fail(mc_ctx *c, int code, const char *fmt, ...)
                         #call, hipGetErrorString(e_));                                    \
     } while (0)
 
+static void log_give_back(int device);
+
 template <class T>
 static hipError_t dalloc(T **p, size_t n)
 {
-    return hipMalloc((void **)p, n * sizeof(T) ? n * sizeof(T) : sizeof(T));
+    const size_t bytes = n * sizeof(T) ? n * sizeof(T) : sizeof(T);
+    const hipError_t e = hipMalloc((void **)p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    // once more without the device's deposit log
+    int device = -1;
+    (void)hipGetLastError();
+    if (hipGetDevice(&device) != hipSuccess) return e;
+    log_give_back(device);
+    return hipMalloc((void **)p, bytes);
 }
 
 // Every copy and fill of a context goes on its stream, in order with its
@@ -169,6 +182,8 @@ static hipError_t fill_on(hipStream_t s, void *dst, int value, size_t bytes)
 
 static int ctx_init(mc_ctx *c, const mc_desc *d);
 static int noalloc_scratch_init(mc_ctx *c);
+static void log_join(mc_ctx *c);
+static void log_leave(mc_ctx *c);
 
 extern "C" int mc_ctx_create(const mc_desc *d, mc_ctx **out)
 {
@@ -210,6 +225,7 @@ static int ctx_init(mc_ctx *c, const mc_desc *d)
         const int rs = noalloc_scratch_init(c);
         if (rs) return rs;
     }
+    log_join(c);
     HIPCHK(c, hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     HIPCHK(c, hipEventCreate(&c->ev0));
     HIPCHK(c, hipEventCreate(&c->ev1));
@@ -283,7 +299,13 @@ static int ctx_init(mc_ctx *c, const mc_desc *d)
     G.nx = nx; G.ny = ny; G.nz = nz; G.nCells = nc; G.nbins = nb; G.flags = d->flags;
     G.nStars = d->nStars;
     G.R_out = d->R_out;
-    G.geoCorrX = d->geoCorr[0]; G.geoCorrY = d->geoCorr[1]; G.geoCorrZ = d->geoCorr[2];
+    for (int a = 0; a < 3; ++a) {
+        const float first = ax[a][0], last = ax[a][n3[a] - 1];
+        G.edge[a] = first;
+        G.out_hi[a] = last + d->geoCorr[a];
+        G.out_lo[a] = first - d->geoCorr[a];
+        if (!(std::fabs(first) <= 1.e27f && std::fabs(last) <= 1.e27f)) G.flags |= mcd::F_FAR;
+    }
     G.ionEdge1 = d->ionEdge1;
     G.axis = c->d_axis; G.mid = c->d_mid; G.dfac = c->d_dfac; G.active = c->d_active;
     G.nuArray = c->d_nuArray;
@@ -377,6 +399,8 @@ extern "C" int mc_upload_tables(mc_ctx *c, const float *opacity, const float *sc
     (void)rc;
     if (!c->d_specCDF) HIPCHK(c, dalloc(&c->d_specCDF, (size_t)nb * c->nStars));
     HIPCHK(c, copy_on(c->stream, c->d_specCDF, specCDF, (size_t)nb * c->nStars * sizeof(float), hipMemcpyHostToDevice));
+    if (!c->d_specGuide) HIPCHK(c, dalloc(&c->d_specGuide, (size_t)c->nStars * (mcd::kGuide + 1)));
+    HIPCHK(c, mcd_guides(c->d_specCDF, c->nStars, nb, c->d_specGuide, c->stream));
     if (rec_host) {
         if (!c->d_recCDF) HIPCHK(c, dalloc(&c->d_recCDF, nt));
         if (!c->d_recGuide) HIPCHK(c, dalloc(&c->d_recGuide, (size_t)(nc + 1) * (mcd::kGuide + 1)));
@@ -390,7 +414,7 @@ extern "C" int mc_upload_tables(mc_ctx *c, const float *opacity, const float *sc
         if (!c->d_gSca) HIPCHK(c, dalloc(&c->d_gSca, nb));
         HIPCHK(c, copy_on(c->stream, c->d_gSca, gSca, nb * sizeof(float), hipMemcpyHostToDevice));
     }
-    G.opac3 = c->d_opac3; G.sca3 = c->d_sca3; G.specCDF = c->d_specCDF;
+    G.opac3 = c->d_opac3; G.sca3 = c->d_sca3; G.specCDF = c->d_specCDF; G.specGuide = c->d_specGuide;
     G.recCDF = c->d_recCDF; G.recGuide = c->d_recGuide; G.totalLines = c->d_totalLines;
     G.gSca = c->d_gSca;
     c->tables = true;
@@ -418,6 +442,7 @@ extern "C" int mc_count_crossings(mc_ctx *c, int32_t enable)
         HIPCHK(c, fill_on(c->stream, c->d_cross, 0, mcd::j3_points(c->G.js) * sizeof(unsigned)));
     }
     c->G.cross = enable ? c->d_cross : nullptr;
+    c->G.flags = enable ? c->G.flags | mcd::F_CROSS : c->G.flags & ~mcd::F_CROSS;
     return MC_OK;
 }
 
@@ -525,8 +550,10 @@ extern "C" int mc_set_view_angles(mc_ctx *c, const mc_view_angles *v)
         if (!c->d_view) HIPCHK(c, hipMalloc((void **)&c->d_view, sizeof(mcd::View)));
         HIPCHK(c, copy_on(c->stream, c->d_view, &h, sizeof h, hipMemcpyHostToDevice));
         c->G.view = c->d_view;
+        c->G.flags |= mcd::F_VIEW;
     } else {
         c->G.view = nullptr;
+        c->G.flags &= ~mcd::F_VIEW;
     }
     return MC_OK;
 }
@@ -1819,23 +1846,17 @@ extern "C" int mc_mlp_train(mc_ctx *c, const float *X, const float *T, const flo
     return MC_OK;
 }
 
-// Grids the pool kernel takes (its packed cell indices and bins).
+// Lattices whose launch shapes may ask for the pool kernel.
 static bool pool_fits(const mcd::Grid &G)
 {
     return G.nx <= 2047 && G.ny <= 2047 && G.nz <= 1023 && G.nbins <= 65535;
 }
 
-// The kernel a launch shape runs (MC_KERNEL_AUTO: two packets per lane at
-// most 3 workgroups of 256 per CU, else the pool kernel where the grid
-// allows it, else one packet per lane).
-static int transport_kernel_of(const mc_tuning &t, const mcd::Grid &G)
+// The kernel a launch shape runs: the pool kernel where the grid allows it
+// (the launcher's rule), except where one packet per lane is asked for.
+static int transport_kernel_of(const mc_tuning &t)
 {
-    switch (t.kernel) {
-    case MC_KERNEL_ONE: return MCD_KERNEL_ONE;
-    case MC_KERNEL_SPARE: return MCD_KERNEL_SPARE;
-    case MC_KERNEL_POOL: return MCD_KERNEL_POOL;
-    default: return t.blocks_per_cu <= 3 ? MCD_KERNEL_SPARE : pool_fits(G) ? MCD_KERNEL_POOL : MCD_KERNEL_ONE;
-    }
+    return t.kernel == MC_KERNEL_ONE ? MCD_KERNEL_ONE : MCD_KERNEL_POOL;
 }
 
 extern "C" int mc_set_tuning(mc_ctx *c, const mc_tuning *t)
@@ -1878,6 +1899,166 @@ static const char *packet_error_text(int code)
     }
 }
 
+// the active index of source istar's cell
+static int star_cell(const mc_ctx *c, int istar)
+{
+    const int *i = &c->starIdx[3 * (istar - 1)];
+    return c->active[(i[0] - 1) + (size_t)c->G.nx * ((i[1] - 1) + (size_t)c->G.ny * (i[2] - 1))];
+}
+
+// The deposit log of a device (mc_deposit.h), shared by its contexts: one
+// sweep uses it at a time, another that finds it taken adds with atomics.  It
+// grows to what a sweep asks for, at most kLogBytes, and is freed with the
+// device's last context or when an allocation of a context fails.
+constexpr size_t kLogBytes = (size_t)4 << 30;
+constexpr int kLogDevices = 64;
+struct LogPool {
+    std::mutex use;                      // held by the sweep that uses it
+    int contexts = 0;
+    unsigned chunks = 0;
+    size_t runs = 0, save = 0;           // their entries
+    mcd::LogEntry *entries = nullptr;
+    unsigned *count = nullptr, *state = nullptr;   // state: next, suspended, the plan
+    unsigned short *run = nullptr;
+    static constexpr size_t kState = 2 + mcl::kPlanWords;
+    uint32_t *saved = nullptr;
+
+    void release()
+    {
+        void *b[] = { entries, count, run, state, saved };
+        for (void *p : b)
+            if (p) (void)hipFree(p);
+        entries = nullptr; count = state = nullptr; run = nullptr; saved = nullptr;
+        chunks = 0;
+        runs = save = 0;
+    }
+    // room for `want` chunks with their run tables, and `words` of saved packets
+    bool reserve(unsigned want, const mcl::Shape &s, size_t words)
+    {
+        const size_t r = mcl::run_entries(std::max(want, chunks), s);
+        if (chunks >= want && runs >= r && save >= words) return true;
+        const unsigned n = std::max(want, chunks);
+        const size_t w = std::max(words, save), rr = std::max(r, runs);
+        release();
+        if (hipMalloc((void **)&entries, (size_t)n * mcd::kLogChunk * sizeof(mcd::LogEntry)) != hipSuccess ||
+            hipMalloc((void **)&count, (size_t)n * sizeof(unsigned)) != hipSuccess ||
+            hipMalloc((void **)&run, rr * sizeof(unsigned short)) != hipSuccess ||
+            hipMalloc((void **)&state, kState * sizeof(unsigned)) != hipSuccess ||
+            hipMalloc((void **)&saved, w * sizeof(uint32_t)) != hipSuccess) {
+            (void)hipGetLastError();
+            release();
+            return false;
+        }
+        chunks = n;
+        runs = rr;
+        save = w;
+        return true;
+    }
+};
+static LogPool g_log[kLogDevices];
+static std::mutex g_log_mu;              // the context counts
+
+static void log_join(mc_ctx *c)
+{
+    if (c->device < 0 || c->device >= kLogDevices) return;
+    std::lock_guard<std::mutex> lock(g_log_mu);
+    ++g_log[c->device].contexts;
+    c->counted = true;
+}
+
+static void log_leave(mc_ctx *c)
+{
+    if (!c->counted) return;
+    std::lock_guard<std::mutex> lock(g_log_mu);
+    if (--g_log[c->device].contexts > 0) return;
+    std::lock_guard<std::mutex> use(g_log[c->device].use);
+    g_log[c->device].release();
+}
+
+// Frees a device's log if no sweep uses it.
+static void log_give_back(int device)
+{
+    if (device < 0 || device >= kLogDevices) return;
+    std::unique_lock<std::mutex> use(g_log[device].use, std::try_to_lock);
+    if (use.owns_lock()) g_log[device].release();
+}
+
+// The chunks a sweep's log should have, or 0 for a sweep that adds with
+// atomics: below about 2e6 deposits the two extra kernels cost more than the
+// atomics, crossing counts go with the atomics, and the words of both
+// estimators must fit the log's ranges.  A flight's segments grow with the
+// axes; the last sweep's count is the better guess.
+static unsigned log_chunks(const mc_ctx *c, int64_t npackets, const mcl::Shape &s, int blocks, int threads)
+{
+    if (!s.bins || (c->G.flags & mcd::F_CROSS)) return 0;
+    const double per = c->seg_per_packet > 0.0 ? c->seg_per_packet : (c->G.nx + c->G.ny + c->G.nz) / 4.0;
+    const double want = 1.05 * (per + 1.0) * (double)npackets;
+    if (want < 2.e6) return 0;
+    // every wavefront holds a chunk
+    const double n = want / mcd::kLogChunk + (double)blocks * (threads / 64);
+    return (unsigned)std::min(n, (double)(kLogBytes / (mcd::kLogChunk * sizeof(mcd::LogEntry))));
+}
+
+// The workgroups of a launch: those of the launch shape, but no more than
+// leave a lane eight packets, or, up to one a CU, one packet.  A wavefront
+// that starts costs as much as several passes: 4000 packets of the 9^3 octant
+// take 0.067 ms with one a lane and 0.46 with the launch shape's 1024
+// workgroups, 1e6 of the 19^3 octant 0.78 ms with eight a lane and 0.97.
+static int launch_blocks(const mc_ctx *c, int64_t npackets)
+{
+    const int64_t most = (int64_t)c->tune.blocks_per_cu * c->cus * (256 / c->tune.threads);
+    const int64_t lanes = npackets / c->tune.threads;
+    return (int)std::min(most, std::max<int64_t>({ 1, std::min<int64_t>(lanes, c->cus), lanes / 8 }));
+}
+
+// The launches of one sweep: with the log, the walk until the log is full or
+// the packets are done, then the log is sorted and added, and so on.
+static int transport_launch(mc_ctx *c, mcd::RunArgs &RA, int blocks)
+{
+    const int threads = c->tune.threads, kernel = transport_kernel_of(c->tune);
+    // the log kernel's registers and LDS leave room for a fifth workgroup of
+    // 256 where the pool kernel's leave four: 47 against 49.5 ms (dust and gas
+    // 60^3), 23.4 against 24.5 (45^3 octant)
+    const int wide = blocks >= c->tune.blocks_per_cu * c->cus * (256 / threads) ? blocks + blocks / 4 : blocks;
+    mcl::Shape s = mcl::shape(0);
+    unsigned chunks = 0;
+    if (kernel == MCD_KERNEL_POOL && mcd_pool_fits(c->G) && c->device >= 0 && c->device < kLogDevices) {
+        const size_t je = mcd::j3_size(c->G.js, c->G.nbins);
+        s = mcl::shape(je + (size_t)(c->G.nCells + 1) * (c->G.nbins + 1) * c->esc_planes);
+        c->G.esc_word = (unsigned)je;
+        chunks = log_chunks(c, RA.npackets, s, wide, threads);
+    }
+    std::unique_lock<std::mutex> use;
+    if (chunks) {
+        use = std::unique_lock<std::mutex>(g_log[c->device].use, std::try_to_lock);
+        if (!use.owns_lock() || !g_log[c->device].reserve(chunks, s, mcd_save_words(wide, threads))) chunks = 0;
+    }
+    if (!chunks) {
+        HIPCHK(c, mcd_launch_transport(c->G, RA, blocks, threads, kernel, c->stream));
+        return MC_OK;
+    }
+    LogPool &P = g_log[c->device];
+    RA.log = P.entries;
+    RA.log_count = P.count;
+    RA.log_next = P.state;
+    RA.log_chunks = chunks;
+    RA.save = P.saved;
+    RA.suspended = reinterpret_cast<int *>(P.state + 1);
+    unsigned *plan = P.state + 2;
+    const mcl::Log L = { P.entries, P.count, P.state, chunks, P.run, reinterpret_cast<unsigned long long *>(plan),
+                         plan + 2 * mcl::kMaxBins, plan + 3 * mcl::kMaxBins,
+                         plan + 3 * mcl::kMaxBins + mcl::kMaxItems };
+    int more = 1;
+    for (RA.resume = 0; more; RA.resume = 1) {
+        HIPCHK(c, fill_on(c->stream, P.state, 0, (2 + 2 * mcl::kMaxBins) * sizeof(unsigned)));
+        HIPCHK(c, mcd_launch_transport(c->G, RA, wide, threads, MCD_KERNEL_LOG, c->stream));
+        HIPCHK(c, mcl_sort(L, s, c->cus, c->stream));
+        HIPCHK(c, mcl_reduce(L, s, c->d_J3, c->d_esc, c->G.esc_word, c->cus, c->stream));
+        HIPCHK(c, copy_on(c->stream, &more, RA.suspended, sizeof more, hipMemcpyDeviceToHost));
+    }
+    return MC_OK;
+}
+
 extern "C" int mc_transport_run(mc_ctx *c, int32_t istar, int64_t npackets, uint64_t packet_offset,
                                 double *J_out, double *esc_out, mc_counters *cnt)
 {
@@ -1889,7 +2070,7 @@ extern "C" int mc_transport_run(mc_ctx *c, int32_t istar, int64_t npackets, uint
     HIPCHK(c, hipMemsetAsync(c->d_scratch, 0, (1 + kCounts) * sizeof(unsigned long long), c->stream));
     HIPCHK(c, hipMemsetAsync(c->d_error, 0, sizeof(int), c->stream));
     HIPCHK(c, hipMemsetAsync(c->d_qphot, 0, sizeof(double), c->stream));
-    mcd::RunArgs RA;
+    mcd::RunArgs RA{};
     RA.istar = istar;
     RA.npackets = npackets;
     RA.packet_offset = packet_offset;
@@ -1902,12 +2083,15 @@ extern "C" int mc_transport_run(mc_ctx *c, int32_t istar, int64_t npackets, uint
     RA.pz = c->starPos[3 * (istar - 1) + 2];
     RA.sx = c->starIdx[3 * (istar - 1)]; RA.sy = c->starIdx[3 * (istar - 1) + 1];
     RA.sz = c->starIdx[3 * (istar - 1) + 2];
+    RA.star_cell = star_cell(c, istar);
     RA.emit_min = c->tune.emit_min;
     RA.walk_steps = c->tune.walk_steps;
-    const int blocks = c->tune.blocks_per_cu * c->cus * (256 / c->tune.threads);
+    const int blocks = launch_blocks(c, npackets);
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
-    if (npackets > 0)
-        HIPCHK(c, mcd_launch_transport(c->G, RA, blocks, c->tune.threads, transport_kernel_of(c->tune, c->G), c->stream));
+    if (npackets > 0) {
+        const int rc = transport_launch(c, RA, blocks);
+        if (rc) return rc;
+    }
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
     unsigned long long h[1 + kCounts];
     int herr = 0;
@@ -1919,6 +2103,7 @@ extern "C" int mc_transport_run(mc_ctx *c, int32_t istar, int64_t npackets, uint
     float ms = 0.f;
     HIPCHK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
     if (cnt) fill_counters(*cnt, h, q, ms);
+    if (npackets > 0) c->seg_per_packet = (double)h[1] / (double)npackets;
     if (herr) return fail(c, MC_EPACKET, "%s (code %d)", packet_error_text(herr), herr);
     if (J_out || esc_out) return mc_fetch_estimators(c, J_out, esc_out);
     return MC_OK;
@@ -1927,7 +2112,7 @@ extern "C" int mc_transport_run(mc_ctx *c, int32_t istar, int64_t npackets, uint
 // Arguments of a batched launch: the launch shape (tu), the LDS it needs and
 // its chunk count.  Failures are reported on ctx[0].
 static int batch_check(mc_ctx *const *ctx, int32_t n, const int32_t *istar, const int64_t *npackets,
-                       const mc_batch_tuning *tuning, mc_batch_tuning &tu, size_t &lds, size_t &nchunks)
+                       const mc_batch_tuning *tuning, mc_batch_tuning &tu, size_t &nchunks)
 {
     if (!ctx || n < 1 || !ctx[0]) return fail(nullptr, MC_EINVAL, "no contexts");
     mc_ctx *c0 = ctx[0];
@@ -1940,7 +2125,6 @@ static int batch_check(mc_ctx *const *ctx, int32_t n, const int32_t *istar, cons
             return fail(c0, MC_EINVAL, "batch tuning out of range");
         tu = *tuning;
     }
-    lds = 0;
     nchunks = 0;
     for (int i = 0; i < n; ++i) {
         mc_ctx *c = ctx[i];
@@ -1951,7 +2135,6 @@ static int batch_check(mc_ctx *const *ctx, int32_t n, const int32_t *istar, cons
         if (npackets[i] < 0) return fail(c0, MC_EINVAL, "context %d: negative packet count", i);
         for (int j = 0; j < i; ++j)
             if (ctx[j] == c) return fail(c0, MC_EINVAL, "context %d appears twice", i);
-        lds = std::max(lds, mcd_lds_bytes(c->G.nx, c->G.ny, c->G.nz, c->G.nbins));
         nchunks += (size_t)((npackets[i] + tu.chunk - 1) / tu.chunk);
     }
     if (nchunks > (1u << 30)) return fail(c0, MC_EINVAL, "too many chunks");
@@ -1963,14 +2146,46 @@ static void batch_run_args(const mc_ctx *c, int32_t istar, int64_t npackets, uin
                            const mc_batch_tuning &tu, mcd::RunArgs &R)
 {
     const int s = istar - 1;
+    R = mcd::RunArgs{};
     R.istar = istar;
     R.npackets = npackets;
     R.packet_offset = offset;
     R.deltaE = c->deltaE[s];
     R.px = c->starPos[3 * s]; R.py = c->starPos[3 * s + 1]; R.pz = c->starPos[3 * s + 2];
     R.sx = c->starIdx[3 * s]; R.sy = c->starIdx[3 * s + 1]; R.sz = c->starIdx[3 * s + 2];
+    R.star_cell = star_cell(c, istar);
     R.emit_min = tu.emit_min;
     R.walk_steps = tu.walk_steps;
+}
+
+// share[i] of a batched launch: the work of the models before model i, by
+// packets and lattice size (a flight's segments grow with the axes).
+static void batch_shares(mc_ctx *const *ctx, int n, const int64_t *npackets, double *share)
+{
+    share[0] = 0.0;
+    for (int i = 0; i < n; ++i)
+        share[i + 1] = share[i] + (double)npackets[i] * (ctx[i]->G.nx + ctx[i]->G.ny + ctx[i]->G.nz);
+}
+
+// The launch of a batch on context 0's stream: one launch of all models, or
+// one after another where a lattice is not for the pool kernel.
+static hipError_t batch_launch(mc_ctx *const *ctx, const mcd::BatchArgs &B, const mcd::RunArgs *RA,
+                               const mc_batch_tuning &tu, bool work)
+{
+    mc_ctx *c0 = ctx[0];
+    if (!work) return hipSuccess;
+    const int blocks = std::max(1, tu.waves_per_cu * c0->cus / 4);
+    size_t lds = 0;
+    bool fits = true;
+    for (int i = 0; i < B.models; ++i) {
+        lds = std::max(lds, mcd_pool_lds(ctx[i]->G, 256));
+        fits = fits && mcd_pool_fits(ctx[i]->G);
+    }
+    if (fits) return mcd_launch_batch(B, lds, blocks, c0->stream);
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < B.models && e == hipSuccess; ++i)
+        if (RA[i].npackets > 0) e = mcd_launch_transport(ctx[i]->G, RA[i], blocks, 256, MCD_KERNEL_POOL, c0->stream);
+    return e;
 }
 
 extern "C" int mc_transport_batch(mc_ctx *const *ctx, int32_t n, const int32_t *istar, const int64_t *npackets,
@@ -1978,8 +2193,8 @@ extern "C" int mc_transport_batch(mc_ctx *const *ctx, int32_t n, const int32_t *
                                   double *kernel_ms)
 {
     mc_batch_tuning tu;
-    size_t lds = 0, nchunks = 0;
-    int rc0 = batch_check(ctx, n, istar, npackets, tuning, tu, lds, nchunks);
+    size_t nchunks = 0;
+    int rc0 = batch_check(ctx, n, istar, npackets, tuning, tu, nchunks);
     if (rc0) return rc0;
     mc_ctx *c0 = ctx[0];
     HIPCHK(c0, hipSetDevice(c0->device));
@@ -1987,10 +2202,8 @@ extern "C" int mc_transport_batch(mc_ctx *const *ctx, int32_t n, const int32_t *
     for (int i = 0; i < n; ++i) HIPCHK(c0, hipStreamSynchronize(ctx[i]->stream));
     std::vector<mcd::Grid> G(n);
     std::vector<mcd::RunArgs> RA(n);
-    std::vector<int> cm;
-    std::vector<long long> cf;
-    std::vector<int> cc;
-    cm.reserve(nchunks); cf.reserve(nchunks); cc.reserve(nchunks);
+    std::vector<double> share(n + 1);
+    batch_shares(ctx, n, npackets, share.data());
     for (int i = 0; i < n; ++i) {
         mc_ctx *c = ctx[i];
         HIPCHK(c0, hipMemsetAsync(c->d_scratch, 0, (1 + kCounts) * sizeof(unsigned long long), c0->stream));
@@ -2003,41 +2216,25 @@ extern "C" int mc_transport_batch(mc_ctx *const *ctx, int32_t n, const int32_t *
         R.counts = c->d_scratch + 1;
         R.error = c->d_error;
         R.qphot = c->d_qphot;
-        for (long long f = 0; f < npackets[i]; f += tu.chunk) {
-            cm.push_back(i);
-            cf.push_back(f);
-            cc.push_back((int)std::min<long long>(tu.chunk, npackets[i] - f));
-        }
     }
-    // one device block: grids | run arguments | chunk table | chunk counter
+    // one device block: grids | run arguments | shares
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    const size_t oG = 0, oR = up(n * sizeof(mcd::Grid)), oM = oR + up(n * sizeof(mcd::RunArgs));
-    const size_t oF = oM + up(cm.size() * sizeof(int)), oC = oF + up(cf.size() * sizeof(long long));
-    const size_t oN = oC + up(cc.size() * sizeof(int)), tot = oN + 256;
+    const size_t oG = 0, oR = up(n * sizeof(mcd::Grid)), oS = oR + up(n * sizeof(mcd::RunArgs));
+    const size_t tot = oS + up((n + 1) * sizeof(double));
     char *buf = nullptr;
     HIPCHK(c0, dalloc(&buf, tot));
     hipError_t e = hipMemcpyAsync(buf + oG, G.data(), n * sizeof(mcd::Grid), hipMemcpyHostToDevice, c0->stream);
     if (e == hipSuccess)
         e = hipMemcpyAsync(buf + oR, RA.data(), n * sizeof(mcd::RunArgs), hipMemcpyHostToDevice, c0->stream);
-    if (e == hipSuccess && !cm.empty())
-        e = hipMemcpyAsync(buf + oM, cm.data(), cm.size() * sizeof(int), hipMemcpyHostToDevice, c0->stream);
-    if (e == hipSuccess && !cf.empty())
-        e = hipMemcpyAsync(buf + oF, cf.data(), cf.size() * sizeof(long long), hipMemcpyHostToDevice, c0->stream);
-    if (e == hipSuccess && !cc.empty())
-        e = hipMemcpyAsync(buf + oC, cc.data(), cc.size() * sizeof(int), hipMemcpyHostToDevice, c0->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(buf + oN, 0, sizeof(unsigned), c0->stream);
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(buf + oS, share.data(), (n + 1) * sizeof(double), hipMemcpyHostToDevice, c0->stream);
     mcd::BatchArgs B;
     B.G = reinterpret_cast<const mcd::Grid *>(buf + oG);
     B.RA = reinterpret_cast<const mcd::RunArgs *>(buf + oR);
-    B.chunk_model = reinterpret_cast<const int *>(buf + oM);
-    B.chunk_first = reinterpret_cast<const long long *>(buf + oF);
-    B.chunk_count = reinterpret_cast<const int *>(buf + oC);
-    B.nchunks = (int)cm.size();
-    B.next_chunk = reinterpret_cast<unsigned *>(buf + oN);
-    B.emit_min = tu.emit_min;
-    B.walk_steps = tu.walk_steps;
+    B.share = reinterpret_cast<const double *>(buf + oS);
+    B.models = n;
     if (e == hipSuccess) e = hipEventRecord(c0->ev0, c0->stream);
-    if (e == hipSuccess && B.nchunks > 0) e = mcd_launch_batch(B, lds, tu.waves_per_cu * c0->cus, c0->stream);
+    if (e == hipSuccess) e = batch_launch(ctx, B, RA.data(), tu, nchunks > 0);
     if (e == hipSuccess) e = hipEventRecord(c0->ev1, c0->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c0->stream);
     float ms = 0.f;
@@ -2101,26 +2298,6 @@ static int noalloc_scratch_init(mc_ctx *c)
 
 namespace {
 
-// chunk k of a batched launch: its model (the last i with cstart[i] <= k),
-// first packet and count, from the models' chunk prefix sums
-__global__ void noalloc_chunks_kernel(int n, const long long *cstart, const long long *npk, long long chunk,
-                                      int *cm, long long *cf, int *cc, long long nchunks)
-{
-    const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= nchunks) return;
-    int lo = 0, hi = n;
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (cstart[mid] <= k) lo = mid;
-        else hi = mid;
-    }
-    const long long f = (k - cstart[lo]) * chunk;
-    const long long left = npk[lo] - f;
-    cm[k] = lo;
-    cf[k] = f;
-    cc[k] = (int)(left < chunk ? left : chunk);
-}
-
 __global__ void noalloc_clear_kernel(unsigned long long *w, long long nwords)
 {
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < nwords;
@@ -2135,8 +2312,8 @@ extern "C" int mc_transport_batch_noalloc(mc_ctx *const *ctx, int32_t n, const i
                                           const mc_batch_tuning *tuning, mc_counters *cnt, double *kernel_ms)
 {
     mc_batch_tuning tu;
-    size_t lds = 0, nchunks = 0;
-    int rc0 = batch_check(ctx, n, istar, npackets, tuning, tu, lds, nchunks);
+    size_t nchunks = 0;
+    int rc0 = batch_check(ctx, n, istar, npackets, tuning, tu, nchunks);
     if (rc0) return rc0;
     mc_ctx *c0 = ctx[0];
     if (n > kNoAllocModels)
@@ -2150,26 +2327,27 @@ extern "C" int mc_transport_batch_noalloc(mc_ctx *const *ctx, int32_t n, const i
         base = g_scratch_ptr[c0->device];
     }
     if (!base) return fail(c0, MC_ESTATE, "no scratch address for device %d", c0->device);
-    // layout: grids | run arguments | chunk prefix | packets | counters | chunk counter | chunk table
+    // layout: grids | run arguments | shares | counters
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const size_t oG = 0, oR = up(n * sizeof(mcd::Grid)), oS = oR + up(n * sizeof(mcd::RunArgs));
-    const size_t oP = oS + up((n + 1) * sizeof(long long)), oK = oP + up(n * sizeof(long long));
-    const size_t oN = oK + up((size_t)n * kCounterWords * sizeof(unsigned long long));
-    const size_t oM = oN + 256, oF = oM + up(nchunks * sizeof(int)), oC = oF + up(nchunks * sizeof(long long));
-    const size_t tot = oC + up(nchunks * sizeof(int));
-    if (tot > kNoAllocBytes)
+    const size_t oK = oS + up((n + 1) * sizeof(double));
+    const size_t tot = oK + up((size_t)n * kCounterWords * sizeof(unsigned long long));
+    static_assert(kNoAllocModels * (sizeof(mcd::Grid) + sizeof(mcd::RunArgs) + kCounterWords * 8 + 8) + 4096 <
+                      kNoAllocBytes, "scratch too small for the most models");
+    // the scratch's contract counts 16 bytes per chunk of packets
+    if (tot + 16 * nchunks > kNoAllocBytes)
         return fail(c0, MC_EINVAL, "the launch needs %zu bytes of scratch (%zu chunks of %lld packets); the "
-                    "allocation-free launch holds %zu: use larger chunks", tot, nchunks, (long long)tu.chunk,
-                    kNoAllocBytes);
+                    "allocation-free launch holds %zu: use larger chunks", tot + 16 * nchunks, nchunks,
+                    (long long)tu.chunk, kNoAllocBytes);
     HIPCHK(c0, hipSetDevice(c0->device));
     for (int i = 0; i < n; ++i) HIPCHK(c0, hipStreamSynchronize(ctx[i]->stream));
     // host staging in thread-local arrays (no heap)
     static thread_local mcd::Grid tG[kNoAllocModels];
     static thread_local mcd::RunArgs tR[kNoAllocModels];
-    static thread_local long long tS[kNoAllocModels + 1], tP[kNoAllocModels];
+    static thread_local double tS[kNoAllocModels + 1];
     static thread_local unsigned long long tK[kNoAllocModels * kCounterWords];
     unsigned long long *dK = reinterpret_cast<unsigned long long *>(base + oK);
-    tS[0] = 0;
+    batch_shares(ctx, n, npackets, tS);
     for (int i = 0; i < n; ++i) {
         mc_ctx *c = ctx[i];
         tG[i] = c->G;
@@ -2180,41 +2358,23 @@ extern "C" int mc_transport_batch_noalloc(mc_ctx *const *ctx, int32_t n, const i
         R.counts = k + 1;
         R.error = reinterpret_cast<int *>(k + 1 + kCounts);
         R.qphot = reinterpret_cast<double *>(k + 2 + kCounts);
-        tP[i] = npackets[i];
-        tS[i + 1] = tS[i] + (npackets[i] + tu.chunk - 1) / tu.chunk;
     }
     hipStream_t st = c0->stream;
     HIPCHK(c0, hipMemcpyAsync(base + oG, tG, n * sizeof(mcd::Grid), hipMemcpyHostToDevice, st));
     HIPCHK(c0, hipMemcpyAsync(base + oR, tR, n * sizeof(mcd::RunArgs), hipMemcpyHostToDevice, st));
-    HIPCHK(c0, hipMemcpyAsync(base + oS, tS, (n + 1) * sizeof(long long), hipMemcpyHostToDevice, st));
-    HIPCHK(c0, hipMemcpyAsync(base + oP, tP, n * sizeof(long long), hipMemcpyHostToDevice, st));
-    // counters and the chunk counter start at zero (a kernel, not a memset)
-    const long long nclear = (long long)(oM - oK) / (long long)sizeof(unsigned long long);
+    HIPCHK(c0, hipMemcpyAsync(base + oS, tS, (n + 1) * sizeof(double), hipMemcpyHostToDevice, st));
+    // counters start at zero (a kernel, not a memset)
+    const long long nclear = (long long)(tot - oK) / (long long)sizeof(unsigned long long);
     hipLaunchKernelGGL(noalloc_clear_kernel, dim3(64), dim3(256), 0, st,
                        reinterpret_cast<unsigned long long *>(base + oK), nclear);
     HIPCHK(c0, hipGetLastError());
-    int *cm = reinterpret_cast<int *>(base + oM);
-    long long *cf = reinterpret_cast<long long *>(base + oF);
-    int *cc = reinterpret_cast<int *>(base + oC);
-    if (nchunks > 0) {
-        const unsigned blocks = (unsigned)((nchunks + 255) / 256);
-        hipLaunchKernelGGL(noalloc_chunks_kernel, dim3(blocks), dim3(256), 0, st, (int)n,
-                           reinterpret_cast<const long long *>(base + oS), reinterpret_cast<const long long *>(base + oP),
-                           (long long)tu.chunk, cm, cf, cc, (long long)nchunks);
-        HIPCHK(c0, hipGetLastError());
-    }
     mcd::BatchArgs B;
     B.G = reinterpret_cast<const mcd::Grid *>(base + oG);
     B.RA = reinterpret_cast<const mcd::RunArgs *>(base + oR);
-    B.chunk_model = cm;
-    B.chunk_first = cf;
-    B.chunk_count = cc;
-    B.nchunks = (int)nchunks;
-    B.next_chunk = reinterpret_cast<unsigned *>(base + oN);
-    B.emit_min = tu.emit_min;
-    B.walk_steps = tu.walk_steps;
+    B.share = reinterpret_cast<const double *>(base + oS);
+    B.models = n;
     HIPCHK(c0, hipEventRecord(c0->ev0, st));
-    if (B.nchunks > 0) HIPCHK(c0, mcd_launch_batch(B, lds, tu.waves_per_cu * c0->cus, st));
+    HIPCHK(c0, batch_launch(ctx, B, tR, tu, nchunks > 0));
     HIPCHK(c0, hipEventRecord(c0->ev1, st));
     HIPCHK(c0, hipMemcpyAsync(tK, dK, (size_t)n * kCounterWords * sizeof(unsigned long long),
                               hipMemcpyDeviceToHost, st));
@@ -2300,7 +2460,7 @@ extern "C" void mc_ctx_destroy(mc_ctx *c)
     if (!c) return;
     (void)hipSetDevice(c->device);
     void *bufs[] = { c->d_axis, c->d_mid, c->d_dfac, c->d_active, c->d_opac3, c->d_sca3,
-                     c->d_recCDF, c->d_recGuide, c->d_totalLines, c->d_specCDF, c->d_nuArray,
+                     c->d_recCDF, c->d_recGuide, c->d_totalLines, c->d_specCDF, c->d_specGuide, c->d_nuArray,
                      c->d_gSca, c->d_J3, c->d_J, c->d_esc, c->d_view, c->d_scratch, c->d_error, c->d_qphot,
                      c->d_cell_xyz, c->d_atomic, c->d_bal_tab, c->d_Hden, c->d_Te, c->d_Ne,
                      c->d_ion, c->d_flags, c->d_nIter, c->d_cold, c->d_mlp, c->d_mlpW, c->d_mX,
@@ -2315,5 +2475,6 @@ extern "C" void mc_ctx_destroy(mc_ctx *c)
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->stream) (void)hipStreamDestroy(c->stream);
+    log_leave(c);
     delete c;
 }

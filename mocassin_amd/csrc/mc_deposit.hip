@@ -1,0 +1,345 @@
+// mc_deposit.hip - sort and reduce of the deposit log (mc_deposit.h).
+#include "mc_deposit.h"
+
+namespace mcl {
+
+constexpr int kThreads = 1024;
+constexpr int kWaves = kThreads / 64;
+constexpr int kPer = kBlock / kThreads;                       // entries a thread
+constexpr int kBinsPer = (kMaxBins + kThreads - 1) / kThreads; // bins a thread
+
+// In LDS: a block's entries in sorted order, the bins' counts (then starts),
+// and the wavefront sums of the scan.
+constexpr size_t kSortLds = sizeof(mcd::LogEntry) * kBlock + sizeof(unsigned) * (kMaxBins + kWaves);
+static_assert(kSortLds <= 160 * 1024, "sort: one workgroup fills a CU's LDS");
+
+__device__ __forceinline__ unsigned chunks_used(const Log &L) { return min(*L.next, L.chunks); }
+__device__ __forceinline__ unsigned blocks_of(unsigned chunks) { return (chunks + kBlockChunks - 1) / kBlockChunks; }
+
+// One workgroup sorts a block of 16384 entries by bin, in place: a counting
+// sort whose ranks come from LDS atomics with a result.  HBM bound: 8 bytes
+// read and written per entry.  Workgroup i runs on XCD i mod 8; the 16 blocks
+// of a group go to 16 workgroups of one XCD at the same time, so that their
+// run tables, 32 bytes a bin, meet in its L2.
+__global__ void __launch_bounds__(kThreads) sort_kernel(Log L, Shape s)
+{
+    extern __shared__ __align__(16) unsigned char dyn[];
+    mcd::LogEntry *sorted = reinterpret_cast<mcd::LogEntry *>(dyn);
+    unsigned *hist = reinterpret_cast<unsigned *>(sorted + kBlock), *wsum = hist + kMaxBins;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const unsigned used = chunks_used(L), blocks = blocks_of(used), groups = (blocks + kGroup - 1) / kGroup;
+    const unsigned x = blockIdx.x % 8, j = blockIdx.x / 8, teams = gridDim.x / (8 * kGroup);
+    unsigned mine[kBinsPer] = {};                   // entries of this thread's bins in the workgroup's blocks
+    const int b0 = t * kBinsPer;
+    const unsigned k = j % kGroup;
+    // the entries of block b, 0xffffffff in place of those its chunks lack
+    mcd::LogEntry e[kPer];
+    const auto load = [&](unsigned b) {
+        const mcd::LogEntry *at = L.entries + (size_t)b * kBlock;
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            constexpr int rows = mcd::kLogChunk / kThreads;            // thread rows of a chunk
+            const unsigned c = b * kBlockChunks + i / rows, at_c = (unsigned)(i % rows) * kThreads + t;
+            const unsigned n = c < used ? L.count[c] : 0;
+            e[i].w = 0xffffffffu;
+            if (at_c < n) e[i] = at[i * kThreads + t];
+        }
+    };
+    const unsigned g0 = (j / kGroup) * 8 + x;
+    load(g0 * kGroup + k);
+    for (unsigned g = g0; g < groups; g += teams * 8) {
+        const unsigned b = g * kGroup + k;
+        mcd::LogEntry *at = L.entries + (size_t)b * kBlock;
+        unsigned short *run = L.runs + (size_t)g * (s.bins + 1) * kGroup + k;
+        if (b >= blocks) {                          // the last group's missing blocks: empty runs
+            for (int i = t; i <= s.bins; i += kThreads) run[(size_t)i * kGroup] = 0;
+            continue;
+        }
+        for (int i = t; i < kMaxBins; i += kThreads) hist[i] = 0;
+        __syncthreads();
+        unsigned rank[kPer];
+#pragma unroll
+        for (int i = 0; i < kPer; ++i)
+            if (e[i].w != 0xffffffffu) rank[i] = atomicAdd(&hist[e[i].w >> s.shift], 1u);
+        __syncthreads();
+        // exclusive scan of the counts, kBinsPer bins a thread
+        unsigned n[kBinsPer], sum = 0;
+#pragma unroll
+        for (int i = 0; i < kBinsPer; ++i) {
+            n[i] = b0 + i < kMaxBins ? hist[b0 + i] : 0;
+            mine[i] += n[i];
+            sum += n[i];
+        }
+        const unsigned own = sum;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const unsigned v = __shfl_up(sum, o);
+            if (lane >= o) sum += v;
+        }
+        if (lane == 63) wsum[wave] = sum;
+        __syncthreads();
+        unsigned before = sum - own, total = 0;
+        for (int w = 0; w < kWaves; ++w) {
+            const unsigned v = wsum[w];
+            before += w < wave ? v : 0;
+            total += v;
+        }
+#pragma unroll
+        for (int i = 0; i < kBinsPer; ++i) {
+            if (b0 + i < kMaxBins) hist[b0 + i] = before;
+            before += n[i];
+        }
+        __syncthreads();
+        for (int i = t; i <= s.bins; i += kThreads)
+            run[(size_t)i * kGroup] = (unsigned short)(i < s.bins ? hist[i] : total);
+#pragma unroll
+        for (int i = 0; i < kPer; ++i)
+            if (e[i].w != 0xffffffffu) sorted[hist[e[i].w >> s.shift] + rank[i]] = e[i];
+        load(b + teams * 8 * kGroup);               // while this block is written
+        __syncthreads();
+        for (unsigned i = t; i < total; i += kThreads) at[i] = sorted[i];
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < kBinsPer; ++i)
+        if (mine[i]) atomicAdd(&L.total[b0 + i], (unsigned long long)mine[i]);
+}
+
+// Work items: a bin's ranges, each in slices of at most 1/kParts of the log,
+// so that the bins next to the source, which a large part of all segments
+// falls in, do not hold up the end.
+__global__ void __launch_bounds__(kThreads) plan_kernel(Log L, Shape s)
+{
+    __shared__ unsigned long long all;
+    __shared__ unsigned scan[kThreads];
+    const int t = threadIdx.x;
+    const unsigned subs = 1u << (s.shift - 14);
+    static_assert(kMaxBins <= 1 << 13 && kMaxShift - 14 <= 3, "packed work items");
+    if (t == 0) all = 0;
+    __syncthreads();
+    unsigned long long n[kBinsPer], sum = 0;
+#pragma unroll
+    for (int i = 0; i < kBinsPer; ++i) {
+        n[i] = t * kBinsPer + i < s.bins ? L.total[t * kBinsPer + i] : 0;
+        sum += n[i];
+    }
+    if (sum) atomicAdd(&all, sum);
+    __syncthreads();
+    // at most kParts slices more than bins
+    const unsigned long long most = all / kParts + 1 > 16384 ? all / kParts + 1 : 16384;
+    unsigned k[kBinsPer], items = 0;
+#pragma unroll
+    for (int i = 0; i < kBinsPer; ++i) {
+        k[i] = (unsigned)((n[i] + most - 1) / most);
+        items += k[i] * subs;
+    }
+    scan[t] = items;
+    __syncthreads();
+    for (int o = 1; o < kThreads; o <<= 1) {
+        const unsigned v = t >= o ? scan[t - o] : 0;
+        __syncthreads();
+        scan[t] += v;
+        __syncthreads();
+    }
+    unsigned at = scan[t] - items;
+    if (t == kThreads - 1) *L.n_items = scan[t];
+#pragma unroll
+    for (int i = 0; i < kBinsPer; ++i) {
+        const unsigned bin = t * kBinsPer + i;
+        if (bin >= (unsigned)s.bins) continue;
+        L.slices[bin] = k[i];
+        for (unsigned q = 0; q < k[i]; ++q)
+            for (unsigned r = 0; r < subs; ++r) L.items[at++] = bin | r << 13 | q << 16;
+    }
+}
+
+// Where word w is summed: the 64 points of a tile row turned by their bin, so
+// that one cell's words of all frequencies (the source's cell has a share of
+// every packet) do not lie in one LDS bank.
+__device__ __forceinline__ unsigned place(unsigned w)
+{
+    return (w & (kRange - 64)) | ((w + (w >> 6)) & 63u);
+}
+
+// acc[w] += v of the lanes with `has`.  Lanes that share a word add one after
+// another, some 64 cycles each, so in a range with many entries up to two
+// words that four lanes or more share are summed across the lanes first.
+__device__ __forceinline__ void add(double *acc, bool has, unsigned w, double v, bool hot, int lane)
+{
+    for (int k = 0; hot && k < 2; ++k) {
+        const uint64_t m = __ballot(has);
+        if (!m) return;
+        const int leader = __ffsll((unsigned long long)m) - 1;
+        const unsigned wl = (unsigned)__builtin_amdgcn_readlane((int)w, leader);
+        const bool same = has && w == wl;
+        const uint64_t ms = __ballot(same);
+        if (__popcll(ms) < 4) break;
+        double sum = same ? v : 0.0;
+        for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o);
+        if (lane == leader) unsafeAtomicAdd(&acc[place(w)], sum);
+        has = has && !same;
+    }
+    if (has) unsafeAtomicAdd(&acc[place(w)], v);
+}
+
+// A work item is a range of kRange words and a slice of its bin (the same
+// part of every block's run): one workgroup reads the slice and adds the
+// entries of its words in LDS, then adds the sums to the estimator (atomics
+// where slices of a range meet there, 8 words to a request).  32 consecutive
+// items go to the CUs of one XCD, which read neighbouring runs out of the
+// same lines.  A run has kBlock / bins entries on average, a few, so a
+// wavefront lays the runs of 64 blocks end to end and reads them 64 entries
+// at a time (marks in LDS of where runs begin give each lane its run), kAhead
+// loads in flight.
+constexpr int kAhead = 4;
+struct Reader { unsigned mark[64 * kAhead]; int delta[64]; };
+constexpr size_t kReduceLds = sizeof(double) * kRange + sizeof(Reader) * kWaves;
+
+// set bits of m below this lane
+__device__ __forceinline__ int rank_below(uint64_t m)
+{
+    return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+}
+
+// orders a wavefront's LDS accesses (the LDS serves them in order)
+__device__ __forceinline__ void wave_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+__global__ void __launch_bounds__(kThreads) reduce_kernel(Log L, Shape s, double *J, double *esc, unsigned j_words)
+{
+    extern __shared__ __align__(16) double acc[];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    static_assert(kRange == 1 << 14, "a range is 2^14 words");
+    Reader &R = reinterpret_cast<Reader *>(acc + kRange)[wave];
+    unsigned *mark = R.mark;
+    int *delta = R.delta;
+    const unsigned blocks = blocks_of(chunks_used(L)), groups = (blocks + kGroup - 1) / kGroup;
+    const unsigned items = *L.n_items;
+    const unsigned x = blockIdx.x % 8, per = gridDim.x / 8;
+    // with fewer than 64 blocks a wavefront, several share them, a part each
+    const unsigned stripes = (groups + 3) / 4;
+    const unsigned parts = stripes >= (unsigned)kWaves ? 1 : kWaves / (stripes ? stripes : 1);
+    const unsigned part = (unsigned)wave % parts, first = (unsigned)wave / parts, step = kWaves / parts;
+    for (int i = t; i < kRange; i += kThreads) acc[i] = 0.0;
+    __syncthreads();
+    for (unsigned y = blockIdx.x / 8; (y / per * 8 + x) * per < items; y += per) {
+        const unsigned item = (y / per * 8 + x) * per + y % per;
+        if (item >= items) continue;
+        const unsigned what = L.items[item];
+        const unsigned bin = what & 0x1fffu, sub = what >> 13 & 7u, slices = L.slices[bin];
+        const size_t w0 = ((size_t)bin << s.shift) + (size_t)sub * kRange;
+        if (w0 >= s.words) continue;
+        const unsigned range = (unsigned)(w0 >> 14);
+        const bool hot = slices > 1;
+        const unsigned cut = (what >> 16) * parts + part, cuts = slices * parts;
+        // start | end << 16 of this item's part of the run in this lane's block
+        const auto descriptor = [&](unsigned g) -> unsigned {
+            if (g >= groups) return 0;
+            const unsigned short *r = L.runs + ((size_t)g * (s.bins + 1) + bin) * kGroup + (lane & 15);
+            const unsigned a = r[0], n = r[kGroup] - a;
+            return cuts == 1 ? a | (a + n) << 16 : (a + n * cut / cuts) | (a + n * (cut + 1) / cuts) << 16;
+        };
+        unsigned d = descriptor(4 * first + (lane >> 4));
+        for (unsigned g0 = 4 * first; g0 < groups && first < stripes; g0 += 4 * step) {
+            const unsigned now = d;
+            d = descriptor(g0 + 4 * step + (lane >> 4));
+            if (!__any((now & 0xffffu) != now >> 16)) continue;
+            // the runs end to end: run r begins at position p
+            const int n = (int)(now >> 16) - (int)(now & 0xffffu);
+            int p = n;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int v = __shfl_up(p, o);
+                if (lane >= o) p += v;
+            }
+            const int all = __builtin_amdgcn_readlane(p, 63);
+            p -= n;
+            const uint64_t some = __ballot(n > 0);
+            // of the non-empty runs in order: entry index less position
+            if (n > 0) delta[rank_below(some)] = (int)(lane * kBlock + (now & 0xffffu)) - p;
+            const mcd::LogEntry *from = L.entries + (size_t)g0 * kGroup * kBlock;
+            int begun = 0;                             // runs that begin before this batch of positions
+            for (int f0 = 0; f0 < all; f0 += 64 * kAhead) {
+#pragma unroll
+                for (int j = 0; j < kAhead; ++j) mark[64 * j + lane] = 0;
+                wave_order();
+                if (n > 0 && p >= f0 && p < f0 + 64 * kAhead) mark[p - f0] = 1;
+                wave_order();
+                mcd::LogEntry e[kAhead];
+#pragma unroll
+                for (int j = 0; j < kAhead; ++j) {
+                    const unsigned own = mark[64 * j + lane];
+                    const uint64_t m = __ballot(own != 0);
+                    const int r = begun + rank_below(m) + (int)own - 1;
+                    begun += __popcll(m);
+                    const int f = f0 + 64 * j + lane;
+                    e[j].w = 0xffffffffu;
+                    if (f < all) e[j] = from[delta[r] + f];
+                }
+#pragma unroll
+                for (int j = 0; j < kAhead; ++j) add(acc, e[j].w >> 14 == range, e[j].w, (double)e[j].val, hot, lane);
+                wave_order();
+            }
+        }
+        __syncthreads();
+        for (int i = t; i < kRange; i += kThreads) {
+            const size_t w = w0 + i;
+            const unsigned at = place((unsigned)w);
+            const double v = acc[at];
+            acc[at] = 0.0;
+            if (v == 0.0) continue;
+            double *to = w < j_words ? &J[w] : &esc[w - j_words];
+            if (slices > 1) unsafeAtomicAdd(to, v);
+            else *to += v;
+        }
+        __syncthreads();
+    }
+}
+
+Shape shape(size_t words)
+{
+    Shape s = { 0, 14, 0 };
+    if (words == 0 || words > (size_t)kMaxBins << kMaxShift) return s;
+    while (((words - 1) >> s.shift) + 1 > (size_t)kMaxBins) ++s.shift;
+    s.words = (unsigned)words;
+    s.bins = (int)(((words - 1) >> s.shift) + 1);
+    return s;
+}
+
+size_t run_entries(unsigned chunks, const Shape &s)
+{
+    const size_t blocks = (chunks + kBlockChunks - 1) / kBlockChunks;
+    return (blocks + kGroup - 1) / kGroup * kGroup * (size_t)(s.bins + 1);
+}
+
+}  // namespace mcl
+
+static hipError_t lds_of(const void *f, size_t bytes)
+{
+    return hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+}
+
+// a workgroup a CU, whole teams of an XCD
+static unsigned grid_of(int cus, int per) { return (unsigned)((cus + per - 1) / per * per); }
+
+hipError_t mcl_sort(const mcl::Log &L, const mcl::Shape &s, int cus, hipStream_t st)
+{
+    const hipError_t e = lds_of((const void *)mcl::sort_kernel, mcl::kSortLds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(mcl::sort_kernel, dim3(grid_of(cus, 8 * mcl::kGroup)), dim3(mcl::kThreads), mcl::kSortLds, st, L, s);
+    return hipGetLastError();
+}
+
+hipError_t mcl_reduce(const mcl::Log &L, const mcl::Shape &s, double *J, double *esc, unsigned j_words, int cus,
+                      hipStream_t st)
+{
+    const size_t lds = mcl::kReduceLds;
+    const hipError_t e = lds_of((const void *)mcl::reduce_kernel, lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(mcl::plan_kernel, dim3(1), dim3(mcl::kThreads), 0, st, L, s);
+    hipLaunchKernelGGL(mcl::reduce_kernel, dim3(grid_of(cus, 8)), dim3(mcl::kThreads), lds, st, L, s, J, esc, j_words);
+    return hipGetLastError();
+}

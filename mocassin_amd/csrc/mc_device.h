@@ -19,7 +19,10 @@ namespace mcd {
 constexpr int kSafeLimit = 500000;      // photon_mod.f90:1187-1192
 constexpr int kRecursionLimit = 5000;   // constants_mod.f90:56
 
-enum Flags { F_SYM = 1, F_DUST = 2, F_GAS = 4, F_ISO = 8, F_MULTI = 16 };
+// The last three are the library's own: crossing counts and viewing angles
+// on, and a lattice beyond 1e27 cm, whose wall distances could overflow on
+// the way (wall_quotient).
+enum Flags { F_SYM = 1, F_DUST = 2, F_GAS = 4, F_ISO = 8, F_MULTI = 16, F_CROSS = 1 << 28, F_VIEW = 1 << 29, F_FAR = 1 << 30 };
 
 // Per-problem constants and device tables.
 // Viewing-angle bins of the escapes as initCartesianGrid sets them
@@ -96,7 +99,9 @@ __host__ __device__ __forceinline__ size_t j3_index(int nb, int nu0, unsigned p)
 
 struct Grid {
     int nx, ny, nz, nCells, nbins, flags, nStars;
-    float R_out, geoCorrX, geoCorrY, geoCorrZ, ionEdge1;
+    float R_out, ionEdge1;
+    float edge[3];           // first values of the axes
+    float out_hi[3], out_lo[3];   // last value + geoCorr and first value - geoCorr, per axis
     const float *axis;       // x(1:nx), y(1:ny), z(1:nz) concatenated
     const float *mid;        // (a(i)+a(i+1))/2, i=1..n-1 per axis, concatenated
     const float *dfac;       // per-axis cell widths /1e15 (getVolume factors)
@@ -108,12 +113,14 @@ struct Grid {
     const unsigned short *recGuide;  // [cell][kGuide+1] guide table of recCDF rows
     const float *totalLines; // [cell]
     const float *specCDF;    // [star][nu]
+    const unsigned short *specGuide; // [star][kGuide+1] guide table of specCDF rows
     const float *nuArray;    // [nu]
     const float *gSca;       // [nu] or null
     double *J3;              // FP64 path-length estimator, tiled: see j3_index
     J3Shape js;              // its tiling
     double *esc;             // [plane 0..nAngle][nu 0..nbins][cell]
     const View *view;        // viewing-angle bins, or null (plane 0 only)
+    unsigned esc_word;       // the word of esc[0] in the deposit log: the words of J3
     unsigned *cross;         // [J3 point] segments walked in each cell, or null
     uint32_t seed_lo, seed_hi;
 };
@@ -124,18 +131,24 @@ struct Grid {
 // search restricted to that range returns exactly the full binary search.
 constexpr int kGuide = 32;
 
-// LDS copy of the small per-axis arrays (axis, midpoints, volume factors).
+// Per-axis tables of the walk, staged in LDS; cells are 0-based here.
+//   wall[2 i], wall[2 i + 1]  the walls a packet in cell i meets moving down
+//                             and up: the midpoints to its neighbours, the
+//                             outer edge in the first and last cell
+//   part[i]                   getVolume's factor of cell i and what its index
+//                             adds to the packet's word of the tables
+// A step reads one wall and one part per axis.
+struct AxisPart { float d; uint32_t o; };
 struct Axes {
-    const float *x, *y, *z;      // 1-based through the accessors below
-    const float *mx, *my, *mz;
-    const float *dx, *dy, *dz;
+    const float *wx, *wy, *wz;
+    const AxisPart *px, *py, *pz;
 };
-
-__device__ __forceinline__ float AX(const float *a, int i) { return a[i - 1]; }
 
 // --------------------------------------------------------------- RNG
 // Philox4x32-10 (Salmon et al., SC'11).  Counter = (draw/4, packet lo,
 // packet hi, stream), key = seed; uniform = (word >> 8) * 2^-24 in [0,1).
+// The words of the current block live only while a pass draws: a packet
+// keeps its id and the number of its draws (k).
 struct Rng {
     uint32_t plo, phi, stream, k, blk;
     uint32_t w0, w1, w2, w3;
@@ -157,10 +170,13 @@ __device__ __forceinline__ void philox(uint32_t c0, uint32_t c1, uint32_t c2, ui
     o0 = c0; o1 = c1; o2 = c2; o3 = c3;
 }
 
-__device__ __forceinline__ void rng_start(Rng &R, uint64_t packet, uint32_t stream)
+__device__ __forceinline__ Rng rng_at(uint32_t plo, uint32_t phi, uint32_t stream, uint32_t k)
 {
-    R.plo = (uint32_t)packet; R.phi = (uint32_t)(packet >> 32);
-    R.stream = stream; R.k = 0; R.blk = 0xffffffffu;
+    Rng R;
+    R.plo = plo; R.phi = phi; R.stream = stream; R.k = k;
+    R.blk = 0xffffffffu;
+    R.w0 = R.w1 = R.w2 = R.w3 = 0;
+    return R;
 }
 
 __device__ __forceinline__ float draw(Rng &R, const Grid &G)
@@ -289,37 +305,108 @@ enum StepResult { ST_CONTINUE = 0, ST_ESCAPED = 1, ST_LOST = 2, ST_ABSORBED = 3,
 struct Walker {
     float rx, ry, rz;      // rVec
     float vx, vy, vz;      // vHat
-    int xP, yP, zP;
+    float qx, qy, qz;      // 1 / vHat, correctly rounded; NaN where wall_quotient does not hold
+    int x, y, z;           // cell, 0-based
     float absTau, passProb;
-    // outputs of the last step
-    float seg;             // dS or dlLoc of the segment just walked
-    unsigned segPt;        // J3 lattice point of its cell (j3_point)
-    int segX, segY, segZ;  // its cell indices (1-based)
 };
 
-__device__ __forceinline__ int act(const Grid &G, int x, int y, int z)
+// What the walk accumulated for the segment just walked.
+struct Segment {
+    float len, dV;         // dS or dlLoc, and the cell's volume
+    unsigned w;            // the packet's word: see Word
+};
+
+// A packet's word of the J3-layout tables (its cell and frequency bin).  The
+// axis parts of narrow tables (fewer than 2^32 words) add up to
+// j3_index(nb, 0, point), so the word is their sum plus 64 nu0; the parts of
+// wide tables add up to the point, and the 64-bit index is formed where it
+// is used.
+template <bool WIDE>
+struct Word {
+    static __device__ __forceinline__ unsigned of(const AxisPart &a, const AxisPart &b, const AxisPart &c, unsigned nu0)
+    {
+        return WIDE ? a.o + b.o + c.o : a.o + b.o + c.o + nu0 * kJTile;
+    }
+    static __device__ __forceinline__ size_t index(const Grid &G, unsigned w, unsigned nu0)
+    {
+        return WIDE ? j3_index(G.nbins, (int)nu0, w) : (size_t)w;
+    }
+};
+
+// What cell i of an axis adds to the word: k = 0, 1, 2 for x, y, z.
+template <bool WIDE>
+__device__ __forceinline__ unsigned axis_word(const Grid &G, int k, int i)
 {
-    return G.active[(x - 1) + G.nx * ((y - 1) + G.ny * (z - 1))];
+    const unsigned p = j3_point(G.js, k == 0 ? i : 0, k == 1 ? i : 0, k == 2 ? i : 0);
+    return WIDE ? p : (unsigned)j3_index(G.nbins, 0, p);
+}
+
+__device__ __forceinline__ int act(const Grid &G, const Walker &W)
+{
+    return G.active[W.x + G.nx * (W.y + G.ny * W.z)];
+}
+
+// (wall - r) / v for the q of flight_reciprocals, correctly rounded in three
+// operations (a division by `/` takes eleven): with q = RN(1/v) the product
+// and its remainder give RN(a/v) for every pair of FP32 significands
+// (checked over all 2^46 of them), as long as nothing overflows or
+// underflows on the way.  |v| > 1e-10 and lattices within 1e27 cm keep the
+// product finite; a quotient whose remainder could underflow is below 1e-20
+// and goes to the general path of walk_step.
+__device__ __forceinline__ float wall_quotient(float a, float v, float q)
+{
+    const float t = a * q;
+    return __builtin_fmaf(__builtin_fmaf(-v, t, a), q, t);
+}
+
+__device__ __forceinline__ float flight_reciprocal(const Grid &G, float v)
+{
+    return (fabsf(v) > 1.e-10f && !(G.flags & F_FAR)) ? 1.f / v : __builtin_nanf("");
+}
+
+__device__ __forceinline__ void flight_reciprocals(const Grid &G, Walker &W)
+{
+    W.qx = flight_reciprocal(G, W.vx);
+    W.qy = flight_reciprocal(G, W.vy);
+    W.qz = flight_reciprocal(G, W.vz);
+}
+
+// The mirror of a symmetric octant along one axis (photon_mod.f90:1248-1261):
+// a packet at or below the first axis value is put on it, moving up.
+__device__ __forceinline__ void mirror(bool c, float edge, float &r, float &v, float &q)
+{
+    r = c ? edge : r;
+    v = c ? fabsf(v) : v;
+    q = c ? fabsf(q) : q;
+}
+
+// pathSegment's entry mirror.  It can act at the start of a flight only: a
+// segment that ends at or below the first axis value mirrors there.
+__device__ __forceinline__ void mirror_start(const Grid &G, Walker &W)
+{
+    if (!(G.flags & F_SYM)) return;
+    mirror(W.rx <= G.edge[0], G.edge[0], W.rx, W.vx, W.qx);
+    mirror(W.ry <= G.edge[1], G.edge[1], W.ry, W.vy, W.qy);
+    mirror(W.rz <= G.edge[2], G.edge[2], W.rz, W.vz, W.qz);
 }
 
 // Distance to the next wall along one axis (photon_mod.f90:1263-1298 for
 // x; y and z alike).  Moving up (v > 1e-10) the wall is the midpoint above
-// cell P, or the outer edge ax(n) in the last cell; moving down it is the
-// midpoint below, or ax(1) in the first cell; otherwise 1e35.  A packet
-// within 1e-10 of an inner wall steps over it (r = wall, P +- 1); at the
-// outer edge moving up it is lost (lost = true, r = the edge); at ax(1)
-// moving down it is put on the edge.  1 <= P <= n on entry.
-__device__ __forceinline__ float wall_distance(const float *ax, const float *mid, int n, float v, float &r,
-                                               int &P, bool &lost)
+// cell i, or the outer edge in the last cell; moving down it is the
+// midpoint below, or the first axis value in the first cell; otherwise
+// 1e35.  A packet within 1e-10 of an inner wall steps over it (r = wall,
+// i +- 1); at the outer edge moving up it is lost (lost = true, r = the
+// edge); at the first axis value moving down it is put on it.
+__device__ __forceinline__ float wall_distance(const float *wall, int n, float v, float &r, int &i, bool &lost)
 {
     const bool pos = v > 1.e-10f, neg = v < -1.e-10f;
-    const bool inner = pos ? (P < n) : (P > 1);
-    const float m = inner ? mid[pos ? P - 1 : P - 2] : ax[pos ? n - 1 : 0];
+    const bool inner = pos ? (i < n - 1) : (i > 0);
+    const float m = wall[2 * i + (pos ? 1 : 0)];
     const float d = (m - r) / v;
     lost = false;
     if (!(pos || neg)) return 1.e35f;
     if (fabsf(d) < 1.e-10f) {
-        if (inner) { r = m; P += pos ? 1 : -1; }
+        if (inner) { r = m; i += pos ? 1 : -1; }
         else if (pos) { r = m; lost = true; }
         else r = m;
     }
@@ -327,127 +414,103 @@ __device__ __forceinline__ float wall_distance(const float *ax, const float *mid
 }
 
 // One iteration of pathSegment's "do i" loop (photon_mod.f90:1194-2836) on
-// the mother grid.  ZERO_OPACITY replays geometry only.  kappa is looked up
-// here; on ST_ABSORBED the interaction point is in rVec and (xP,yP,zP).
-// err receives the fail-stop code of the reference's "insanity" stops.
-template <bool ZERO_OPACITY>
-__device__ __forceinline__ int walk_step(const Grid &G, const Axes &A, Walker &W, int nuP,
-                                         float &kappa_out, float &dV_out, int &err)
+// the mother grid.  ZERO_OPACITY replays geometry only.  On ST_ABSORBED the
+// interaction point is in rVec and the cell is the one it lies in.  err
+// receives the fail-stop code of the reference's "insanity" stops.
+//
+// A walk pass of the transport kernels is this function, and its
+// instructions bound them: the wall distances are three reciprocal products,
+// and what a segment almost never does (a packet within 1e-10 of a wall, a
+// direction along an axis plane, a NaN) is left to one branch with the
+// reference's general form.  Absorbed and free segments share the move.
+//
+// The cell stays inside the lattice: it starts there, a step moves one index
+// by one, and a packet whose index leaves is mirrored back or has escaped.
+template <bool ZERO_OPACITY, bool WIDE>
+__device__ __forceinline__ int walk_step(const Grid &G, const Axes &A, Walker &W, unsigned nu0, Segment &S, int &err)
 {
-    const int nx = G.nx, ny = G.ny, nz = G.nz;
     const bool sym = (G.flags & F_SYM) != 0;
-    float dSx, dSy, dSz, dS;
-    int xP = W.xP, yP = W.yP, zP = W.zP;
-    float rx = W.rx, ry = W.ry, rz = W.rz, vx = W.vx, vy = W.vy, vz = W.vz;
-
-    if (xP > nx || xP < 1 || yP > ny || yP < 1 || zP > nz || zP < 1) { err = 32; return ST_ERROR; }
-    // the cell's opacity, issued first so that its gather overlaps the wall
-    // distances (the indices were just checked); a packet on a wall is
-    // stepped into the next cell there, and then the gather is repeated
-    const unsigned p0 = j3_point(G.js, xP - 1, yP - 1, zP - 1);
+    AxisPart ax = A.px[W.x], ay = A.py[W.y], az = A.pz[W.z];
+    S.w = Word<WIDE>::of(ax, ay, az, nu0);
     float kappa = 0.f;
-    if (!ZERO_OPACITY) kappa = G.opac3[j3_index(G.nbins, nuP - 1, p0)];
+    if (!ZERO_OPACITY) kappa = G.opac3[Word<WIDE>::index(G, S.w, nu0)];
 
-    if (sym) {                                                   // 1248-1261
-        if (rx <= AX(A.x, 1)) { if (vx < 0.f) vx = -vx; rx = AX(A.x, 1); }
-        if (ry <= AX(A.y, 1)) { if (vy < 0.f) vy = -vy; ry = AX(A.y, 1); }
-        if (rz <= AX(A.z, 1)) { if (vz < 0.f) vz = -vz; rz = AX(A.z, 1); }
+    // wall distances (1263-1379); the wall of a component by its sign
+    const float mx = A.wx[2 * W.x + (W.vx > 0.f ? 1 : 0)];
+    const float my = A.wy[2 * W.y + (W.vy > 0.f ? 1 : 0)];
+    const float mz = A.wz[2 * W.z + (W.vz > 0.f ? 1 : 0)];
+    float dSx = fabsf(wall_quotient(mx - W.rx, W.vx, W.qx));
+    float dSy = fabsf(wall_quotient(my - W.ry, W.vy, W.qy));
+    float dSz = fabsf(wall_quotient(mz - W.rz, W.vz, W.qz));
+    float dS = fminf(fminf(dSx, dSy), dSz);
+    if (!((dSx >= 1.e-10f) & (dSy >= 1.e-10f) & (dSz >= 1.e-10f))) {
+        // the general form, in the reference's order
+        const unsigned w0 = S.w;
+        bool lostX, lostY, lostZ;
+        dSx = wall_distance(A.wx, G.nx, W.vx, W.rx, W.x, lostX);
+        dSy = wall_distance(A.wy, G.ny, W.vy, W.ry, W.y, lostY);
+        dSz = wall_distance(A.wz, G.nz, W.vz, W.rz, W.z, lostZ);
+        if (lostX) return ST_LOST;
+        if (isnan(dSx)) { err = 34; return ST_ERROR; }
+        if (lostY) return ST_LOST;
+        if (isnan(dSy)) { err = 34; return ST_ERROR; }
+        if (lostZ) return ST_LOST;
+        if (isnan(dSz)) { err = 34; return ST_ERROR; }
+        // cells on the cell wall, 1382-1384
+        if (fabsf(dSx) < 1.e-10f) dSx = A.wx[2 * G.nx - 1];
+        if (fabsf(dSy) < 1.e-10f) dSy = A.wy[2 * G.ny - 1];
+        if (fabsf(dSz) < 1.e-10f) dSz = A.wz[2 * G.nz - 1];
+        dSx = fabsf(dSx); dSy = fabsf(dSy); dSz = fabsf(dSz);
+        if (dSx <= 0.f) dS = fminf(dSy, dSz);
+        else if (dSy <= 0.f) dS = fminf(dSx, dSz);
+        else if (dSz <= 0.f) dS = fminf(dSx, dSy);
+        else { dS = fminf(dSx, dSy); dS = fminf(dS, dSz); }
+        if (dS <= 0.f) { err = 36; return ST_ERROR; }
+        ax = A.px[W.x]; ay = A.py[W.y]; az = A.pz[W.z];
+        S.w = Word<WIDE>::of(ax, ay, az, nu0);
+        if (!ZERO_OPACITY && S.w != w0) kappa = G.opac3[Word<WIDE>::index(G, S.w, nu0)];
     }
-
-    // wall distances, 1263-1379: one division per axis whatever the signs
-    // of the wavefront's directions (the reference's branches select the
-    // wall; they are evaluated here as selects, in the same order)
-    bool lostX, lostY, lostZ;
-    dSx = wall_distance(A.x, A.mx, nx, vx, rx, xP, lostX);
-    dSy = wall_distance(A.y, A.my, ny, vy, ry, yP, lostY);
-    dSz = wall_distance(A.z, A.mz, nz, vz, rz, zP, lostZ);
-    if (lostX) { W.rx = rx; return ST_LOST; }
-    if (isnan(dSx)) { err = 34; return ST_ERROR; }
-    if (lostY) { W.ry = ry; return ST_LOST; }
-    if (isnan(dSy)) { err = 34; return ST_ERROR; }
-    if (lostZ) { W.rz = rz; return ST_LOST; }
-    if (isnan(dSz)) { err = 34; return ST_ERROR; }
-
-    // cells on the cell wall, 1382-1384
-    if (fabsf(dSx) < 1.e-10f) dSx = AX(A.x, nx);
-    if (fabsf(dSy) < 1.e-10f) dSy = AX(A.y, ny);
-    if (fabsf(dSz) < 1.e-10f) dSz = AX(A.z, nz);
-    dSx = fabsf(dSx); dSy = fabsf(dSy); dSz = fabsf(dSz);
-    if (dSx <= 0.f) dS = fminf(dSy, dSz);
-    else if (dSy <= 0.f) dS = fminf(dSx, dSz);
-    else if (dSz <= 0.f) dS = fminf(dSx, dSy);
-    else { dS = fminf(dSx, dSy); dS = fminf(dS, dSz); }
-    if (dS <= 0.f) { err = 36; return ST_ERROR; }
 
     // dense opacity: inactive cells hold row 0 (= 0), so "active > 0" of the
     // interaction test (1517) holds whenever tau can exceed passProb
-    const unsigned p = j3_point(G.js, xP - 1, yP - 1, zP - 1);
-    if (!ZERO_OPACITY && p != p0) kappa = G.opac3[j3_index(G.nbins, nuP - 1, p)];
     const float tauCell = dS * kappa;
-    const float dV = AX(A.dx, xP) * AX(A.dy, yP) * AX(A.dz, zP);  // 1442-1514
-    kappa_out = kappa;
-    dV_out = dV;
-    W.segPt = p;
-    W.segX = xP; W.segY = yP; W.segZ = zP;
-
-    if (!ZERO_OPACITY && (W.absTau + tauCell > W.passProb)) {
-        // interaction, 1517-1580
-        float dlLoc = (W.passProb - W.absTau) / kappa;
-        rx = rx + dlLoc * vx;
-        ry = ry + dlLoc * vy;
-        rz = rz + dlLoc * vz;
-        if (isnan(rx) || isnan(ry) || isnan(rz)) { err = 37; return ST_ERROR; }
-        if (sym) {
-            if (rx <= AX(A.x, 1)) { if (vx < 0.f) vx = -vx; rx = AX(A.x, 1); }
-            if (ry <= AX(A.y, 1)) { if (vy < 0.f) vy = -vy; ry = AX(A.y, 1); }
-            if (rz <= AX(A.z, 1)) { if (vz < 0.f) vz = -vz; rz = AX(A.z, 1); }
+    S.dV = ax.d * ay.d * az.d;                                   // 1442-1514
+    S.len = dS;
+    const float tau = W.absTau + tauCell;
+    const bool hit = !ZERO_OPACITY && tau > W.passProb;
+    if (hit) S.len = (W.passProb - W.absTau) / kappa;            // interaction, 1517-1580
+    else W.absTau = tau;                                         // free flight to the wall, 1818-1976
+    W.rx = W.rx + S.len * W.vx;
+    W.ry = W.ry + S.len * W.vy;
+    W.rz = W.rz + S.len * W.vz;
+    if (hit) {
+        if (isnan(W.rx) || isnan(W.ry) || isnan(W.rz)) { err = 37; return ST_ERROR; }
+    } else {
+        if (dS == dSx && fabsf(W.vx) > 0.f) W.x += W.vx > 0.f ? 1 : -1;
+        else if (dS == dSy && fabsf(W.vy) > 0.f) W.y += W.vy > 0.f ? 1 : -1;
+        else if (dS == dSz && fabsf(W.vz) > 0.f) W.z += W.vz > 0.f ? 1 : -1;
+        // 1986-2554, 2728: past the outer edges; on a full grid also past the
+        // first axis values
+        bool out = W.rx >= G.out_hi[0] || W.ry >= G.out_hi[1] || W.rz >= G.out_hi[2] || W.x >= G.nx ||
+                   W.y >= G.ny || W.z >= G.nz;
+        if (!sym)
+            out = out || W.rx <= G.out_lo[0] || W.ry <= G.out_lo[1] || W.rz <= G.out_lo[2] || W.x < 0 || W.y < 0 ||
+                  W.z < 0;
+        if (out) return ST_ESCAPED;
+    }
+    if (sym) {                                                   // 1519-1575, 2674-2699
+        const bool cx = W.rx <= G.edge[0] || W.x < 0, cy = W.ry <= G.edge[1] || W.y < 0,
+                   cz = W.rz <= G.edge[2] || W.z < 0;
+        mirror(cx, G.edge[0], W.rx, W.vx, W.qx);
+        mirror(cy, G.edge[1], W.ry, W.vy, W.qy);
+        mirror(cz, G.edge[2], W.rz, W.vz, W.qz);
+        if (!hit) {
+            W.x = cx ? 0 : W.x;
+            W.y = cy ? 0 : W.y;
+            W.z = cz ? 0 : W.z;
         }
-        W.seg = dlLoc;
-        W.rx = rx; W.ry = ry; W.rz = rz; W.vx = vx; W.vy = vy; W.vz = vz;
-        W.xP = xP; W.yP = yP; W.zP = zP;
-        return ST_ABSORBED;   // caller: J, R_out escape test, scatter/absorb decision
     }
-
-    // free flight to the wall, 1818-1976
-    W.seg = dS;
-    W.absTau = W.absTau + tauCell;
-    rx = rx + dS * vx;
-    ry = ry + dS * vy;
-    rz = rz + dS * vz;
-    if (dS == dSx && vx > 0.f) xP = xP + 1;
-    else if (dS == dSx && vx < 0.f) xP = xP - 1;
-    else if (dS == dSy && vy > 0.f) yP = yP + 1;
-    else if (dS == dSy && vy < 0.f) yP = yP - 1;
-    else if (dS == dSz && vz > 0.f) zP = zP + 1;
-    else if (dS == dSz && vz < 0.f) zP = zP - 1;
-
-    int res = ST_CONTINUE;
-    if (!sym) {                                                  // 1986-2194
-        bool ret = false;
-        if (ry <= AX(A.y, 1) - G.geoCorrY || yP < 1) { yP = 1; ret = true; }
-        if (ry > AX(A.y, ny) + G.geoCorrY || yP > ny) { yP = ny; ret = true; }
-        if (rx <= AX(A.x, 1) - G.geoCorrX || xP < 1) { xP = 1; ret = true; }
-        if (rx >= AX(A.x, nx) + G.geoCorrX || xP > nx) { xP = nx; ret = true; }
-        if (rz <= AX(A.z, 1) - G.geoCorrZ || zP < 1) { zP = 1; ret = true; }
-        if (rz >= AX(A.z, nz) + G.geoCorrZ || zP > nz) { zP = nz; ret = true; }
-        if (ret) res = ST_ESCAPED;
-    }
-    if (res == ST_CONTINUE) {                                    // 2421-2554
-        if ((!sym && (rx <= AX(A.x, 1) - G.geoCorrX || ry <= AX(A.y, 1) - G.geoCorrY ||
-                      rz <= AX(A.z, 1) - G.geoCorrZ)) ||
-            rx >= AX(A.x, nx) + G.geoCorrX || ry >= AX(A.y, ny) + G.geoCorrY ||
-            rz >= AX(A.z, nz) + G.geoCorrZ || xP > nx || yP > ny || zP > nz)
-            res = ST_ESCAPED;
-    }
-    if (res == ST_CONTINUE && sym) {                             // 2674-2699
-        if (rx <= AX(A.x, 1) || xP < 1) { if (vx < 0.f) vx = -vx; xP = 1; rx = AX(A.x, 1); }
-        if (ry <= AX(A.y, 1) || yP < 1) { if (vy < 0.f) vy = -vy; yP = 1; ry = AX(A.y, 1); }
-        if (rz <= AX(A.z, 1) || zP < 1) { if (vz < 0.f) vz = -vz; zP = 1; rz = AX(A.z, 1); }
-    }
-    if (res == ST_CONTINUE && (xP > nx || yP > ny || zP > nz)) res = ST_ESCAPED;  // 2728
-    W.rx = rx; W.ry = ry; W.rz = rz; W.vx = vx; W.vy = vy; W.vz = vz;
-    W.xP = xP; W.yP = yP; W.zP = zP;
-    return res;
+    return hit ? ST_ABSORBED : ST_CONTINUE;
 }
 
 }  // namespace mcd

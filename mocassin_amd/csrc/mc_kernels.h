@@ -8,6 +8,10 @@ namespace mcd {
 struct Grid;
 struct J3Shape;
 
+// A deposit: `val` to be added to word w of an estimator (J3, then esc).
+struct alignas(8) LogEntry { unsigned w; float val; };
+constexpr int kLogChunk = 2048;
+
 // Per-launch arguments of the transport kernel.
 struct RunArgs {
     int istar;                          // 1-based source index (random stream id)
@@ -20,31 +24,44 @@ struct RunArgs {
     float deltaE;
     float px, py, pz;                   // source position [cm]
     int sx, sy, sz;                     // source cell (1-based)
+    int star_cell;                      // its active index
     int emit_min;                       // emission pass when >= this many lanes wait
     int walk_steps;                     // walk passes between emission checks
+    // the deposit log (log_kernel): chunks of kLogChunk entries, taken by
+    // wavefronts from *log_next; when they run out a wavefront saves its
+    // packets in `save` and ends, to go on in a launch with `resume` set
+    LogEntry *log;
+    unsigned *log_count;                // [log_chunks] entries of each chunk
+    unsigned *log_next;
+    unsigned log_chunks;
+    uint32_t *save;                     // kSaveWords per wavefront
+    int *suspended;
+    int resume;
 };
 
-// Chunk table and per-model arguments of a batched launch (device memory)
+// Per-model arguments of a batched launch (device memory).  share[i] is the
+// work of the models before model i (share[models]: of all).
 struct BatchArgs {
     const Grid *G;                      // [models]
-    const RunArgs *RA;                  // [models] (istar, packet_offset, source, counters)
-    const int *chunk_model;             // [nchunks], non-decreasing
-    const long long *chunk_first;       // [nchunks] first packet index within the model
-    const int *chunk_count;             // [nchunks]
-    int nchunks;
-    unsigned *next_chunk;               // zeroed per launch
-    int emit_min, walk_steps;
+    const RunArgs *RA;                  // [models]
+    const double *share;                // [models + 1]
+    int models;
 };
 
 }  // namespace mcd
 
 hipError_t mcd_launch_batch(const mcd::BatchArgs &B, size_t lds_bytes, int blocks, hipStream_t s);
-size_t mcd_lds_bytes(int nx, int ny, int nz, int nbins);
-// The transport kernels: one packet per lane; two (at most 3 wavefronts
-// per SIMD, which that kernel's registers allow); one per lane with a pool
-// of 32 packets per wavefront in LDS.  The pool kernel needs grids of at
-// most 2047 x 2047 x 1023 cells and 65535 bins.
-enum { MCD_KERNEL_ONE = 1, MCD_KERNEL_SPARE = 2, MCD_KERNEL_POOL = 3 };
+// The transport kernels: one packet per lane, and one per lane with a pool of
+// 32 packets per wavefront in LDS.  The pool kernel packs a packet's cell and
+// bin and keeps 32-bit indices of the tables: it takes grids of at most 2047 x
+// 2047 x 1023 cells, 65535 bins and 2^32 - 1 table words; other grids run the
+// first whatever kernel is asked for.
+// The log kernel is the pool kernel with the deposits written to the log of
+// its RunArgs instead of added to the estimators.
+enum { MCD_KERNEL_ONE = 1, MCD_KERNEL_POOL = 3, MCD_KERNEL_LOG = 4 };
+size_t mcd_save_words(int blocks, int threads);
+bool mcd_pool_fits(const mcd::Grid &G);
+size_t mcd_pool_lds(const mcd::Grid &G, int threads);
 hipError_t mcd_launch_transport(const mcd::Grid &G, const mcd::RunArgs &RA, int blocks, int threads, int kernel,
                                 hipStream_t s);
 hipError_t mcd_densify(const float *compact, const int *active, const mcd::J3Shape &js, int nc1, int nbins,

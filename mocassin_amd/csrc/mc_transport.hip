@@ -1,24 +1,33 @@
 // mc_transport.hip - persistent packet-transport kernels and geometry replay
 // kernel for MI355X (gfx950).
 //
-// Transport: lanes refill from a global packet counter with one atomic per
-// wavefront.  Packet events are split in two classes and scheduled per
-// wavefront so that SIMD lanes stay coherent:
-//   walk      one cell segment of pathSegment (a few FP32 divisions, one
-//             opacity gather, one J update): the common event;
+// Transport: wavefronts take packets from a counter in stocks.  Packet
+// events are split in two classes and scheduled per wavefront so that SIMD
+// lanes stay coherent:
+//   walk      one cell segment of pathSegment (three reciprocal products, one
+//             opacity gather, one deposit): the common event;
 //   emission  creation of a stellar packet or re-emission of an absorbed one
 //             (Philox draws, CDF search, direction, optical-depth draw):
 //             about ten times the instructions of a walk step.
-// Three kernels share that code and differ in how a wavefront keeps its
-// lanes busy between emission passes: one packet per lane
-// (transport_kernel<false>), a spare packet per lane in registers
-// (transport_kernel<true>), and a pool of packets per wavefront in LDS
-// (pool_kernel).  The per-axis arrays, the source CDF and its guide table
-// live in LDS.  J_nu and the opacity tables are stored in 2x2x2 bricks of
-// 4x4x4 tiles (mc_device.h); each lane queues its J updates in a ring in
-// LDS, and a full ring flushes every lane's ring with FP64 atomics, one
-// packet's consecutive updates to an instruction, so that adds sharing a
-// 64-byte line travel as one request.
+// Four kernels share that code.  log_kernel runs large sweeps: a pool of
+// packets per wavefront in LDS keeps the lanes walking, and deposits go to a
+// log that mc_deposit.hip sums by range.  pool_kernel is the same with FP64
+// atomics (small sweeps, crossing counts); transport_kernel keeps one packet
+// per lane (any lattice); batch_kernel is the pool over several models.  The
+// axes' walls and word offsets live in LDS.  J_nu and the opacity tables are
+// stored in 2x2x2 bricks of 4x4x4 tiles (mc_device.h).  Where deposits are
+// atomics each lane queues them in a ring in LDS, and a full ring flushes
+// every lane's ring, one packet's consecutive updates to an instruction, so
+// that adds sharing a 64-byte line travel as one request.
+//
+// What bounds them: an FP64 atomic add goes to the memory side as one 64-byte
+// request, 2e10 of them a second, which was 2/3 of a sweep's time; a logged
+// deposit is 8 bytes written and read three times.  The walk itself is bound
+// by its instructions at 16 and more wavefronts a CU.  One sweep of 1e8
+// packets on a 45^3 octant of 800 bins (1.8e9 deposits): 45.7 ms before (the
+// pool with atomics and divisions), 23.4 now (walk and log 14, sort 6, sums
+// 3.5); 4e7 packets in dust and gas 60^3: 67.4 ms before, 46.7 now; 8 models
+// of 15^3 cells in one launch: 60 ms before, 22 now.
 #include "mc_device.h"
 #include "mc_kernels.h"
 
@@ -26,534 +35,52 @@
 
 namespace mcd {
 
-// LDS layout: axes | mids | dV factors | source CDF | source guide (ushort)
-__device__ __forceinline__ void stage_axes(const Grid &G, float *lds, Axes &A, int extra_nu,
-                                           const float *extra_src, float **extra_dst)
+// LDS of a staged grid: walls | parts.  The tables of an axis follow those
+// of the one before.
+template <bool WIDE>
+__device__ __forceinline__ void stage_axes(const Grid &G, float *lds, Axes &A)
 {
-    const int nx = G.nx, ny = G.ny, nz = G.nz;
-    const int na = nx + ny + nz;
-    const int nm = (nx - 1) + (ny - 1) + (nz - 1);
-    float *ax = lds, *mi = lds + na, *df = lds + na + nm;
-    for (int i = threadIdx.x; i < na; i += blockDim.x) { ax[i] = G.axis[i]; df[i] = G.dfac[i]; }
-    for (int i = threadIdx.x; i < nm; i += blockDim.x) mi[i] = G.mid[i];
-    float *ex = lds + 2 * na + nm;
-    for (int i = threadIdx.x; i < extra_nu; i += blockDim.x) ex[i] = extra_src[i];
+    const int n3[3] = { G.nx, G.ny, G.nz };
+    const int na = G.nx + G.ny + G.nz;
+    AxisPart *parts = reinterpret_cast<AxisPart *>(lds + 2 * na);
+    for (int k = 0, o = 0; k < 3; o += n3[k], ++k) {
+        const float *ax = G.axis + o, *mid = G.mid + o - k;
+        for (int i = threadIdx.x; i < n3[k]; i += blockDim.x) {
+            lds[2 * (o + i)] = i > 0 ? mid[i - 1] : ax[0];
+            lds[2 * (o + i) + 1] = i < n3[k] - 1 ? mid[i] : ax[i];
+            parts[o + i] = AxisPart{ G.dfac[o + i], axis_word<WIDE>(G, k, i) };
+        }
+    }
     __syncthreads();
-    A.x = ax; A.y = ax + nx; A.z = ax + nx + ny;
-    A.mx = mi; A.my = mi + (nx - 1); A.mz = mi + (nx - 1) + (ny - 1);
-    A.dx = df; A.dy = df + nx; A.dz = df + nx + ny;
-    if (extra_dst) *extra_dst = ex;
+    A.wx = lds; A.wy = lds + 2 * G.nx; A.wz = lds + 2 * (G.nx + G.ny);
+    A.px = parts; A.py = parts + G.nx; A.pz = parts + G.nx + G.ny;
 }
 
-__host__ __device__ inline size_t lds_floats(int nx, int ny, int nz, int nbins)
+__host__ __device__ inline size_t lds_floats(int nx, int ny, int nz)
 {
-    return (size_t)(2 * (nx + ny + nz) + (nx + ny + nz - 3) + nbins) + (kGuide + 2) / 2 + 1;
+    return (size_t)4 * (nx + ny + nz);
 }
 
-// ------------------------------------------------ J update queue (per wave)
-// Each lane keeps its last D updates (J3 point, bin - 1, value) in a ring of
-// its own at the start of the wavefront's dynamic LDS: point u32 [64 x
-// (D + 1)] | value f32 [...] | bin u16 [...], entry k of lane L at
-// L * (D + 1) + k (rows padded by one word against bank conflicts).  When a
-// lane's ring is full the wavefront flushes every ring, lane-major: atomic
-// instruction j carries the rings of lanes (64 / D) j .. (64 / D)(j + 1) - 1.
-// Adds of one instruction that fall in one 64-byte line travel to memory as
-// one request, and with J3's 2x2x2 bricks a packet's next segment stays in
-// the line after half of its steps, so keeping a packet's updates in one
-// instruction turns those pairs into single requests.  The single-model
-// kernel keeps 8 per lane; the batched kernel, whose one-wavefront
-// workgroups each hold a model's tables too, keeps 4 so that 16 fit a CU.
-template <int D>
-struct JRing {
-    static_assert(D == 4 || D == 8, "rings of 4 or 8 updates");
-    static constexpr int kRow = D + 1;
-    static constexpr int kEntries = 64 * kRow;
-    static constexpr int kFloats = kEntries * 2 + kEntries / 2;
-};
-constexpr int kJDepth = 8;                            // single-model kernel
-constexpr int kJDepthBatch = 4;                       // batched kernel
-
-struct JQ {
-    unsigned *pt;
-    float *val;
-    unsigned short *nu;
-    int n;                // this lane's queued updates
+// A launch's grid and run arguments in memory, at wavefront-uniform
+// addresses of the constant address space (scalar loads; they do not change
+// in a launch).  The walk keeps the few fields it needs in scalar registers;
+// everything else is loaded by the pass that uses it: kept in registers over
+// the whole launch the arguments spilled.
+struct Args {
+    uint64_t g, r;          // addresses of the Grid and the RunArgs
 };
 
-template <int D>
-__device__ __forceinline__ JQ jq_at(float *lds, int wave)
+template <class T>
+__device__ __forceinline__ T scalar_copy(uint64_t at)
 {
-    float *b = lds + (size_t)wave * JRing<D>::kFloats;
-    JQ Q;
-    Q.pt = reinterpret_cast<unsigned *>(b);
-    Q.val = b + JRing<D>::kEntries;
-    Q.nu = reinterpret_cast<unsigned short *>(b + 2 * JRing<D>::kEntries);
-    Q.n = 0;
-    return Q;
-}
-
-// every queued update: instruction j takes entry lane % D of lane
-// (64 / D) j + lane / D's ring
-template <int D>
-__device__ __forceinline__ void jq_flush(const Grid &G, JQ &Q, int lane)
-{
-    constexpr int per = 64 / D;                       // rings per instruction
-    __builtin_amdgcn_wave_barrier();
-    const int k = lane % D;
-    for (int j = 0; j < D; ++j) {
-        const int owner = per * j + lane / D;
-        const int cnt = __shfl(Q.n, owner);
-        const bool act = k < cnt;
-        if (!__any(act)) continue;
-        if (act) {
-            const int slot = owner * JRing<D>::kRow + k;
-            const unsigned pt = Q.pt[slot];
-            unsafeAtomicAdd(&G.J3[j3_index(G.nbins, (int)Q.nu[slot], pt)], (double)Q.val[slot]);
-            if (G.cross) atomicAdd(&G.cross[pt], 1u);
-        }
-    }
-    __builtin_amdgcn_wave_barrier();
-    Q.n = 0;
-}
-
-// the J update of each lane with `has` (path length times deltaE over dV,
-// photon_mod.f90:1563-1574, 1822-1833), flushed when a lane's ring is full
-template <int D>
-__device__ __forceinline__ void jq_push(const Grid &G, JQ &Q, bool has, unsigned pt, int nuP, float v, int lane)
-{
-    if (has) {
-        const int slot = lane * JRing<D>::kRow + Q.n;
-        Q.pt[slot] = pt;
-        Q.val[slot] = v;
-        Q.nu[slot] = (unsigned short)(nuP - 1);
-        Q.n += 1;
-    }
-    if (__any(Q.n == D)) jq_flush<D>(G, Q, lane);
-}
-
-// ------------------------------------------------------------ replay kernel
-__global__ void __launch_bounds__(256) walk_replay_kernel(Grid G, int n, const float *pos,
-                                                          const float *dir, const int *cell,
-                                                          int *cell_seq, float *ds_seq, int *seq_len,
-                                                          int *status, int max_len)
-{
-    extern __shared__ float lds[];
-    Axes A;
-    stage_axes(G, lds, A, 0, nullptr, nullptr);
-    int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n) return;
-    Walker W;
-    W.rx = pos[3 * p]; W.ry = pos[3 * p + 1]; W.rz = pos[3 * p + 2];
-    W.vx = dir[3 * p]; W.vy = dir[3 * p + 1]; W.vz = dir[3 * p + 2];
-    W.xP = cell[3 * p]; W.yP = cell[3 * p + 1]; W.zP = cell[3 * p + 2];
-    W.absTau = 0.f; W.passProb = 0.f;
-    int len = 0, st = 3;
-    for (int i = 1; i <= kSafeLimit; ++i) {
-        float kappa, dV;
-        int err = 0;
-        int r = walk_step<true>(G, A, W, 1, kappa, dV, err);
-        if (r == ST_ERROR) { st = -err; break; }
-        if (r == ST_LOST) { st = 2; break; }
-        if (len < max_len) {
-            size_t o = (size_t)p * max_len + len;
-            cell_seq[3 * o] = W.segX; cell_seq[3 * o + 1] = W.segY; cell_seq[3 * o + 2] = W.segZ;
-            ds_seq[o] = W.seg;
-        }
-        ++len;
-        if (r == ST_ESCAPED) { st = 1; break; }
-    }
-    seq_len[p] = len;
-    status[p] = st;
-}
-
-// ----------------------------------------------------------- transport kernel
-enum Phase { PH_IDLE = 0, PH_EMIT_STELLAR = 1, PH_EMIT_DIFFUSE = 2, PH_WALK = 3 };
-
-struct Lane {
-    Rng R;
-    Walker W;
-    float d0x, d0y, d0z;   // enPacket%direction (start of flight / last scatter)
-    int nuP, origin;
-    int steps, runs, phase;
-};
-
-// wave-uniform event counters (scalar registers)
-struct WaveCounts {
-    unsigned long long seg, abs, sca, esc, lost, line, trapped, flights;
-    unsigned long long wpass, wlanes, epass, elanes;    // passes and the lanes in them
-};
-
-__device__ __forceinline__ unsigned long long wcount(bool p)
-{
-    return (unsigned long long)__popcll(__ballot(p));
-}
-
-__device__ __forceinline__ void esc_plane(const Grid &G, int a, int origin, int nuP, float dE)
-{
-    const size_t i = ((size_t)a * (size_t)(G.nbins + 1) + (size_t)nuP) * (size_t)(G.nCells + 1) + origin;
-    unsafeAtomicAdd(&G.esc[i], (double)dE);
-}
-
-// An escape of a packet whose flight direction (enPacket%direction) is d:
-// its theta and phi bins, then the viewing-angle planes they feed, as every
-// escape site of pathSegment and energyPacketRun does
-// (photon_mod.f90:1582-1666, 370-465).  err 60/61: the reference's stops on
-// a bin out of range.  The bin tables were range-checked on the host.
-__device__ __forceinline__ void esc_add(const Grid &G, int origin, int nuP, float dE, float dx, float dy,
-                                        float dz, int &err)
-{
-    const View *V = G.view;
-    if (!V) { esc_plane(G, 0, origin, nuP, dE); return; }
-    const bool sym = (G.flags & F_SYM) != 0;
-    const float q = mcf_acosf(sym ? fabsf(dz) : dz) / V->dTheta;
-    if (isnan(q)) { err = 60; return; }
-    int it = (int)q + 1;
-    if (it > V->totT) it = V->totT;
-    if (it < 1) { err = 60; return; }
-    int ip;
-    if (fabsf(dx) < 1.e-35f) ip = 0;
-    else if (sym) ip = (int)(mcf_atanf(fabsf(dy) / fabsf(dx)) / V->dPhi);
-    else ip = (int)(mcf_atanf(dy / dx) / V->dPhi);
-    if (ip < 0) ip = V->totP + ip;
-    ip = ip + 1;
-    if (ip > V->totP) ip = V->totP;
-    if (ip < 1) { err = 61; return; }
-    const int t = V->Pt[it], ph = V->Pp[ip];
-    if (t > 0 && V->vph[t] < 0.f) {
-        esc_plane(G, t, origin, nuP, dE);
-        esc_plane(G, 0, origin, nuP, dE);
-    } else if (t == ph || V->vth[ph] == V->vth[t] || V->vph[t] == V->vph[ph]) {
-        esc_plane(G, t, origin, nuP, dE);
-        if (t != 0) esc_plane(G, 0, origin, nuP, dE);
-    } else {
-        esc_plane(G, 0, origin, nuP, dE);
-    }
-}
-
-// newPhotonPacket + initPhotonPacket + the start of pathSegment
-// (photon_mod.f90:768-1059, 491-684, 1176-1184) for stellar packets
-// (PH_EMIT_STELLAR) and re-emissions at an absorption point (PH_EMIT_DIFFUSE).
-__device__ __forceinline__ void emit(Lane &L, const Grid &G, const RunArgs &RA, const float *spec,
-                                     const unsigned short *spec_guide, bool fold, bool dust,
-                                     bool gas, int star_cell, double &qphot, bool &line_end,
-                                     bool &esc_end, bool &flight, int &err)
-{
-    const bool stellar = (L.phase == PH_EMIT_STELLAR);
-    const float *cdf;
-    const unsigned short *guide;
-    int a;
-    if (stellar) {
-        L.runs = 1;
-        L.W.xP = RA.sx; L.W.yP = RA.sy; L.W.zP = RA.sz;
-        L.W.rx = RA.px; L.W.ry = RA.py; L.W.rz = RA.pz;
-        a = star_cell;
-        cdf = spec;
-        guide = spec_guide;
-    } else {
-        L.runs++;
-        a = act(G, L.W.xP, L.W.yP, L.W.zP);
-        if (!gas) { err = 13; return; }
-        if (a <= 0) { err = 14; return; }
-        float random = 1.f - draw(L.R, G);
-        if (random <= G.totalLines[a]) {                 // line packet (923-956)
-            line_end = true;
-            L.phase = PH_IDLE;
-            return;
-        }
-        cdf = G.recCDF + (size_t)a * G.nbins;
-        guide = G.recGuide + (size_t)a * (kGuide + 1);
-    }
-    int nuP = getnu2(L.R, G, cdf, guide, G.nbins, err);
-    if (err) return;
-    if (nuP < 1 || nuP >= G.nbins) { err = stellar ? 11 : 15; return; }
-    L.nuP = nuP;
-    new_direction(L.R, G, stellar && fold, L.d0x, L.d0y, L.d0z);
-    L.origin = a;
-    const float nu = G.nuArray[nuP - 1];
-    if (stellar && nu > 1.f) qphot += (double)(RA.deltaE / (2.1799153e-11f * nu));
-    if (!dust && nu < G.ionEdge1) {                      // escapes at birth (370-465)
-        esc_add(G, a, nuP, RA.deltaE, L.d0x, L.d0y, L.d0z, err);
-        esc_end = true;
-        L.phase = PH_IDLE;
-        return;
-    }
-    L.W.vx = L.d0x; L.W.vy = L.d0y; L.W.vz = L.d0z;
-    L.W.absTau = 0.f;
-    float random = draw(L.R, G);
-    L.W.passProb = -mcf_logf(1.f - random);
-    L.steps = 0;
-    flight = true;
-    L.phase = PH_WALK;
-}
-
-// Model-wide constants of one grid and source, read by the wavefront loop.
-struct Model {
-    bool fold, dust, gas, iso;
-    float dE;
-    int star_cell;
-};
-
-__device__ __forceinline__ Model model_of(const Grid &G, const RunArgs &RA)
-{
-    Model M;
-    const bool sym = (G.flags & F_SYM) != 0;
-    M.dust = (G.flags & F_DUST) != 0;
-    M.gas = (G.flags & F_GAS) != 0;
-    M.iso = (G.flags & F_ISO) != 0;
-    M.fold = sym && !(G.flags & F_MULTI);
-    M.dE = RA.deltaE;
-    M.star_cell = act(G, RA.sx, RA.sy, RA.sz);
-    return M;
-}
-
-// Stage the grid's axes, the source CDF and its guide table in LDS.
-__device__ __forceinline__ void stage_model(const Grid &G, const RunArgs &RA, float *lds, Axes &A,
-                                            float *&spec, unsigned short *&spec_guide)
-{
-    stage_axes(G, lds, A, G.nbins, G.specCDF + (size_t)(RA.istar - 1) * G.nbins, &spec);
-    spec_guide = (unsigned short *)(spec + G.nbins);
-    for (int j = threadIdx.x; j <= kGuide; j += blockDim.x) spec_guide[j] = guide_entry(spec, G.nbins, j);
-    __syncthreads();
-}
-
-// An emission pass of the wavefront: every lane whose packet E waits for an
-// emission runs it together.  Counts events into C.
-__device__ __forceinline__ void emission_pass(Lane &E, const Grid &G, const RunArgs &RA, const Model &M,
-                                              const float *spec, const unsigned short *spec_guide, WaveCounts &C,
-                                              double &qphot, int &err)
-{
-    const bool pend = (E.phase == PH_EMIT_STELLAR || E.phase == PH_EMIT_DIFFUSE);
-    bool line_end = false, esc_end = false, flight = false;
-    if (pend) {
-        emit(E, G, RA, spec, spec_guide, M.fold, M.dust, M.gas, M.star_cell, qphot, line_end, esc_end, flight,
-             err);
-        if (err) E.phase = PH_IDLE;
-    }
-    C.epass += 1;
-    C.elanes += wcount(pend);
-    C.line += wcount(line_end);
-    C.esc += wcount(esc_end);
-    C.flights += wcount(flight);
-    // energyPacketDriver counts the packet whose last run is the
-    // recursionLimit-th as trapped (photon_mod.f90:126)
-    C.trapped += wcount(!err && (line_end || esc_end) && E.runs >= kRecursionLimit);
-}
-
-// One walk pass of the wavefront: every lane whose packet L walks takes one
-// step of pathSegment.  Counts events into C, queues the J updates.
-template <int D>
-__device__ __forceinline__ void walk_pass(Lane &L, const Grid &G, const Axes &A, const Model &M, WaveCounts &C,
-                                          int &err, JQ &Q, int lane)
-{
-    bool seg = false, escaped = false, lost = false, absorbed = false, scattered = false,
-         trapped = false;
-    float jv = 0.f;
-    unsigned jpt = 0;
-    int jnu = 1;
-    C.wpass += 1;
-    C.wlanes += wcount(L.phase == PH_WALK);
-    if (L.phase == PH_WALK) {
-        L.steps++;
-        float kappa, dV;
-        int r = walk_step<false>(G, A, L.W, L.nuP, kappa, dV, err);
-        if (r == ST_CONTINUE || r == ST_ESCAPED) {
-            jv = L.W.seg * M.dE / dV;
-            jpt = L.W.segPt;
-            jnu = L.nuP;
-            seg = true;
-            if (r == ST_ESCAPED) {
-                esc_add(G, L.origin, L.nuP, M.dE, L.d0x, L.d0y, L.d0z, err);
-                escaped = true;
-                L.phase = PH_IDLE;
-            }
-        } else if (r == ST_LOST) {
-            lost = true;
-            L.phase = PH_IDLE;
-        } else if (r == ST_ABSORBED) {
-            jv = L.W.seg * M.dE / dV;
-            jpt = L.W.segPt;
-            jnu = L.nuP;
-            seg = true;
-            float rx = L.W.rx / 1.e10f, ry = L.W.ry / 1.e10f, rz = L.W.rz / 1.e10f;
-            if (sqrtf(rx * rx + ry * ry + rz * rz) * 1.e10f >= G.R_out && G.R_out > 0.f) {
-                esc_add(G, L.origin, L.nuP, M.dE, L.d0x, L.d0y, L.d0z, err);   // 1577-1669
-                escaped = true;
-                L.phase = PH_IDLE;
-            } else if (M.dust) {
-                float probSca = G.sca3[j3_index(G.nbins, L.nuP - 1, L.W.segPt)] / kappa;
-                float u = 1.f - draw(L.R, G);
-                if (u > probSca) {
-                    absorbed = true;
-                    if (M.gas) L.phase = PH_EMIT_DIFFUSE;
-                    else err = 41;                        // dustEmi needs dust PDFs
-                } else if (u <= probSca) {
-                    scattered = true;                     // 1720-1797
-                    L.origin = act(G, L.W.xP, L.W.yP, L.W.zP);
-                    if (M.iso) {
-                        new_direction(L.R, G, false, L.d0x, L.d0y, L.d0z);
-                    } else {
-                        for (int ihg = 1; ihg <= 10; ++ihg)
-                            if (hg(L.R, G, L.nuP, L.d0x, L.d0y, L.d0z) == 0) break;
-                    }
-                    L.W.vx = L.d0x; L.W.vy = L.d0y; L.W.vz = L.d0z;
-                    L.W.absTau = 0.f;
-                    float r2 = draw(L.R, G);
-                    L.W.passProb = -mcf_logf(1.f - r2);
-                } else {
-                    err = 39;
-                }
-            } else {
-                absorbed = true;
-                L.phase = PH_EMIT_DIFFUSE;
-            }
-        } else {
-            if (!err) err = 50;
-        }
-        if (!err) {
-            // safeLimit (2838-2846); recursionLimit (120-126)
-            if ((L.phase == PH_WALK || L.phase == PH_EMIT_DIFFUSE) && L.steps >= kSafeLimit) {
-                lost = true;
-                L.phase = PH_IDLE;
-            }
-            if (L.phase == PH_EMIT_DIFFUSE && L.runs >= kRecursionLimit) L.phase = PH_IDLE;
-            trapped = (L.phase == PH_IDLE) && L.runs >= kRecursionLimit;
-        } else {
-            L.phase = PH_IDLE;
-        }
-    }
-    jq_push<D>(G, Q, seg, jpt, jnu, jv, lane);
-    C.seg += wcount(seg);
-    C.esc += wcount(escaped);
-    C.lost += wcount(lost);
-    C.abs += wcount(absorbed);
-    C.sca += wcount(scattered);
-    C.trapped += wcount(trapped);
-}
-
-// One scheduling round of a wavefront (the batched kernel): an emission pass
-// when at least emit_min lanes (or as many as are walking) wait for one, then
-// walk_steps walk passes.  A fail-stop code goes to RA.error.
-template <int D>
-__device__ __forceinline__ void advance(Lane &L, const Grid &G, const Axes &A, const RunArgs &RA,
-                                        const Model &M, const float *spec,
-                                        const unsigned short *spec_guide, int emit_min, int walk_steps,
-                                        int npend, int nwalk, WaveCounts &C, double &qphot, int &err, JQ &Q,
-                                        int lane)
-{
-    if (npend >= emit_min || npend >= nwalk) emission_pass(L, G, RA, M, spec, spec_guide, C, qphot, err);
-    for (int s = 0; s < walk_steps; ++s) walk_pass<D>(L, G, A, M, C, err, Q, lane);
-    if (err) {
-        atomicMax(RA.error, err);
-        err = 0;
-    }
-}
-
-__device__ __forceinline__ bool pending(const Lane &L)
-{
-    return L.phase == PH_EMIT_STELLAR || L.phase == PH_EMIT_DIFFUSE;
-}
-
-// Exchange the packets of the lanes where c holds (a wavefront-wide vote
-// first: nothing to do costs one instruction).
-__device__ __forceinline__ void swap_where(bool c, Lane &a, Lane &b)
-{
-    if (!__any(c)) return;
-#define MC_SWAP(f) { const auto t_ = a.f; a.f = c ? b.f : a.f; b.f = c ? t_ : b.f; }
-    MC_SWAP(R.plo) MC_SWAP(R.phi) MC_SWAP(R.stream) MC_SWAP(R.k) MC_SWAP(R.blk)
-    MC_SWAP(R.w0) MC_SWAP(R.w1) MC_SWAP(R.w2) MC_SWAP(R.w3)
-    MC_SWAP(W.rx) MC_SWAP(W.ry) MC_SWAP(W.rz) MC_SWAP(W.vx) MC_SWAP(W.vy) MC_SWAP(W.vz)
-    MC_SWAP(W.xP) MC_SWAP(W.yP) MC_SWAP(W.zP) MC_SWAP(W.absTau) MC_SWAP(W.passProb)
-    MC_SWAP(d0x) MC_SWAP(d0y) MC_SWAP(d0z) MC_SWAP(nuP) MC_SWAP(origin) MC_SWAP(steps) MC_SWAP(runs)
-    MC_SWAP(phase)
-#undef MC_SWAP
-}
-
-// One scheduling round of a wavefront with two packets per lane (the
-// single-model kernel): L walks, S is the spare the emission pass serves.
-// A packet that waits for an emission moves to S first; after the emission
-// pass, and after every walk pass, a lane whose L does not walk takes S's
-// packet when that one does.  A lane then idles in a walk pass only when
-// both of its packets wait, so the walk passes stay fuller than with one
-// packet per lane; the packets and their streams are the same.
-template <int D>
-__device__ __forceinline__ void advance_spare(Lane &L, Lane &S, const Grid &G, const Axes &A, const RunArgs &RA,
-                                              const Model &M, const float *spec, const unsigned short *spec_guide,
-                                              int emit_min, int walk_steps, WaveCounts &C, double &qphot, int &err,
-                                              JQ &Q, int lane)
-{
-    swap_where(pending(L) && !pending(S), L, S);
-    const int npend = (int)wcount(pending(S));
-    const int nwalk = (int)wcount(L.phase == PH_WALK);
-    if (npend > 0 && (npend >= emit_min || npend >= nwalk))
-        emission_pass(S, G, RA, M, spec, spec_guide, C, qphot, err);
-    swap_where(L.phase != PH_WALK && S.phase == PH_WALK, L, S);
-    for (int s = 0; s < walk_steps; ++s) {
-        walk_pass<D>(L, G, A, M, C, err, Q, lane);
-        swap_where(L.phase != PH_WALK && S.phase == PH_WALK, L, S);
-    }
-    if (err) {
-        atomicMax(RA.error, err);
-        err = 0;
-    }
-}
-
-// ------------------------------------------------ packet pool (per wave, LDS)
-// A wavefront keeps a pool of P packets in LDS beside its 64 lanes: packets
-// that walk (the walker stack, slots 0 .. nw-1 from the bottom) and packets
-// that wait for a diffuse emission (the pending stack, slots P-npd .. P-1
-// from the top).  A lane whose flight ends takes a walker from the pool,
-// leaving its own packet on the pending stack if it waits for an emission;
-// an emission round moves walkers into the pool, so that the emission pass
-// runs on a full wavefront, and the walkers come back as flights end.  The
-// walk passes then stay nearly full between emissions.  Word k of slot s is
-// at pw[k * P + s]; the cell indices are packed in one word (11, 11 and 10
-// bits: the host runs this kernel on grids of at most 2047 x 2047 x 1023
-// cells) and the frequency bin, run count and phase in another (16, 14 and
-// 2 bits).  The Rng's stream is the launch's source, not stored.
-constexpr int kPoolWords = 23;
-// Slots per wavefront: with 8-deep J rings, 4 workgroups of 256 per CU keep
-// 32 slots within the CU's 160 KB of LDS (8.5 KB per wavefront, plus the
-// staged tables); 48 slots with 4-deep rings ran slower (the rings merge
-// fewer J adds per instruction).
-constexpr int kPoolSlots = 32;
-
-template <int P>
-__device__ __forceinline__ void pool_put(uint32_t *pw, int s, const Lane &L)
-{
-    uint32_t *q = pw + s;
-    q[0 * P] = L.R.plo; q[1 * P] = L.R.phi; q[2 * P] = L.R.k; q[3 * P] = L.R.blk;
-    q[4 * P] = L.R.w0; q[5 * P] = L.R.w1; q[6 * P] = L.R.w2; q[7 * P] = L.R.w3;
-    q[8 * P] = __float_as_uint(L.W.rx); q[9 * P] = __float_as_uint(L.W.ry); q[10 * P] = __float_as_uint(L.W.rz);
-    q[11 * P] = __float_as_uint(L.W.vx); q[12 * P] = __float_as_uint(L.W.vy); q[13 * P] = __float_as_uint(L.W.vz);
-    q[14 * P] = (uint32_t)L.W.xP | ((uint32_t)L.W.yP << 11) | ((uint32_t)L.W.zP << 22);
-    q[15 * P] = __float_as_uint(L.W.absTau); q[16 * P] = __float_as_uint(L.W.passProb);
-    q[17 * P] = __float_as_uint(L.d0x); q[18 * P] = __float_as_uint(L.d0y); q[19 * P] = __float_as_uint(L.d0z);
-    q[20 * P] = (uint32_t)L.nuP | ((uint32_t)L.runs << 16) | ((uint32_t)L.phase << 30);
-    q[21 * P] = (uint32_t)L.origin; q[22 * P] = (uint32_t)L.steps;
-}
-
-template <int P>
-__device__ __forceinline__ void pool_get(const uint32_t *pw, int s, Lane &L, uint32_t stream)
-{
-    const uint32_t *q = pw + s;
-    L.R.plo = q[0 * P]; L.R.phi = q[1 * P]; L.R.k = q[2 * P]; L.R.blk = q[3 * P];
-    L.R.w0 = q[4 * P]; L.R.w1 = q[5 * P]; L.R.w2 = q[6 * P]; L.R.w3 = q[7 * P];
-    L.R.stream = stream;
-    L.W.rx = __uint_as_float(q[8 * P]); L.W.ry = __uint_as_float(q[9 * P]); L.W.rz = __uint_as_float(q[10 * P]);
-    L.W.vx = __uint_as_float(q[11 * P]); L.W.vy = __uint_as_float(q[12 * P]); L.W.vz = __uint_as_float(q[13 * P]);
-    const uint32_t c = q[14 * P];
-    L.W.xP = (int)(c & 2047u); L.W.yP = (int)((c >> 11) & 2047u); L.W.zP = (int)(c >> 22);
-    L.W.absTau = __uint_as_float(q[15 * P]); L.W.passProb = __uint_as_float(q[16 * P]);
-    L.d0x = __uint_as_float(q[17 * P]); L.d0y = __uint_as_float(q[18 * P]); L.d0z = __uint_as_float(q[19 * P]);
-    const uint32_t f = q[20 * P];
-    L.nuP = (int)(f & 65535u); L.runs = (int)((f >> 16) & 16383u); L.phase = (int)(f >> 30);
-    L.origin = (int)q[21 * P]; L.steps = (int)q[22 * P];
+    asm volatile("" : "+s"(at));               // a load of its own, not one hoisted to the top of the kernel
+    return *(const T *)(const __attribute__((address_space(4))) T *)at;
 }
 
 // lanes below this one in m
-__device__ __forceinline__ int lane_rank(uint64_t m, int lane)
+__device__ __forceinline__ int lane_rank(uint64_t m, int)
 {
-    return __popcll(m & ((1ull << lane) - 1ull));
+    return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
 }
 
 // Orders the wavefront's LDS accesses on either side (the compiler may not
@@ -564,12 +91,575 @@ __device__ __forceinline__ void wave_lds_order()
     __builtin_amdgcn_wave_barrier();
 }
 
+// ------------------------------------------------ J update queue (per wave)
+// Each lane keeps its last D updates (word of J3, value) in a ring of its own
+// at the start of the wavefront's dynamic LDS, entry k of lane L at
+// L * (D + 1) + k (rows padded by one entry against bank conflicts); wide
+// tables (2^32 words or more) keep the point there and the bin in a second
+// array behind.  When a lane's ring is full the wavefront flushes every ring,
+// lane-major: atomic instruction j carries the rings of lanes (64 / D) j ..
+// (64 / D)(j + 1) - 1.  Adds of one instruction that fall in one 64-byte line
+// travel to memory as one request, and with J3's 2x2x2 bricks a packet's next
+// segment stays in the line after half of its steps, so keeping a packet's
+// updates in one instruction turns those pairs into single requests.
+struct JEntry { unsigned w; float val; };
+template <int D, bool WIDE>
+struct JRing {
+    static_assert(D == 4 || D == 8, "rings of 4 or 8 updates");
+    static constexpr int kRow = D + 1;
+    static constexpr int kEntries = 64 * kRow;
+    static constexpr int kFloats = kEntries * 2 + (WIDE ? kEntries / 2 : 0);
+};
+constexpr int kJDepth = 8;
+
+struct JQ {
+    JEntry *e;
+    unsigned short *nu;   // wide tables only
+    int n;                // this lane's queued updates
+};
+
+template <int D, bool WIDE>
+__device__ __forceinline__ JQ jq_at(float *lds, int wave)
+{
+    float *b = lds + (size_t)wave * JRing<D, WIDE>::kFloats;
+    JQ Q;
+    Q.e = reinterpret_cast<JEntry *>(b);
+    Q.nu = reinterpret_cast<unsigned short *>(b + 2 * JRing<D, WIDE>::kEntries);
+    Q.n = 0;
+    return Q;
+}
+
+// the J3 point of a word (crossing counts)
+template <bool WIDE>
+__device__ __forceinline__ unsigned point_of(const Grid &G, unsigned w)
+{
+    return WIDE ? w : w / ((unsigned)G.nbins * kJTile) * kJTile + w % kJTile;
+}
+
+// every queued update: instruction j takes entry lane % D of lane
+// (64 / D) j + lane / D's ring
+template <int D, bool WIDE>
+__device__ __forceinline__ void jq_flush(const Grid &G, JQ &Q, int lane)
+{
+    constexpr int per = 64 / D;                       // rings per instruction
+    __builtin_amdgcn_wave_barrier();
+    const int k = lane % D;
+    for (int j = 0; j < D; ++j) {
+        const int owner = per * j + lane / D;
+        const int cnt = __shfl(Q.n, owner);
+        if (k < cnt) {
+            const int slot = owner * JRing<D, WIDE>::kRow + k;
+            const JEntry e = Q.e[slot];
+            const unsigned nu0 = WIDE ? Q.nu[slot] : 0;
+            unsafeAtomicAdd(&G.J3[Word<WIDE>::index(G, e.w, nu0)], (double)e.val);
+            if (G.flags & F_CROSS) atomicAdd(&G.cross[point_of<WIDE>(G, e.w)], 1u);
+        }
+    }
+    __builtin_amdgcn_wave_barrier();
+    Q.n = 0;
+}
+
+// the J update of each lane with `has` (path length times deltaE over dV,
+// photon_mod.f90:1563-1574, 1822-1833), flushed when a lane's ring is full
+template <int D, bool WIDE>
+__device__ __forceinline__ void jq_push(const Grid &G, JQ &Q, bool has, unsigned w, unsigned nu0, float v, int lane)
+{
+    if (has) {
+        const int slot = lane * JRing<D, WIDE>::kRow + Q.n;
+        Q.e[slot] = JEntry{ w, v };
+        if (WIDE) Q.nu[slot] = (unsigned short)nu0;
+        Q.n += 1;
+    }
+    if (__any(Q.n == D)) jq_flush<D, WIDE>(G, Q, lane);
+}
+
+// ------------------------------------------------------------ replay kernel
+__global__ void __launch_bounds__(256) walk_replay_kernel(Grid G, int n, const float *pos,
+                                                          const float *dir, const int *cell,
+                                                          int *cell_seq, float *ds_seq, int *seq_len,
+                                                          int *status, int max_len)
+{
+    extern __shared__ float lds[];
+    Axes A;
+    stage_axes<true>(G, lds, A);
+    int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= n) return;
+    Walker W;
+    W.rx = pos[3 * p]; W.ry = pos[3 * p + 1]; W.rz = pos[3 * p + 2];
+    W.vx = dir[3 * p]; W.vy = dir[3 * p + 1]; W.vz = dir[3 * p + 2];
+    W.x = cell[3 * p] - 1; W.y = cell[3 * p + 1] - 1; W.z = cell[3 * p + 2] - 1;
+    W.absTau = 0.f; W.passProb = 0.f;
+    flight_reciprocals(G, W);
+    mirror_start(G, W);
+    int len = 0, st = 3;
+    for (int i = 1; i <= kSafeLimit; ++i) {
+        Segment S;
+        int err = 0;
+        int r = walk_step<true, true>(G, A, W, 0, S, err);
+        if (r == ST_ERROR) { st = -err; break; }
+        if (r == ST_LOST) { st = 2; break; }
+        if (len < max_len) {
+            size_t o = (size_t)p * max_len + len;
+            const int xyz = j3_lattice(G.js, S.w);
+            cell_seq[3 * o] = xyz % G.nx + 1;
+            cell_seq[3 * o + 1] = xyz / G.nx % G.ny + 1;
+            cell_seq[3 * o + 2] = xyz / (G.nx * G.ny) + 1;
+            ds_seq[o] = S.len;
+        }
+        ++len;
+        if (r == ST_ESCAPED) { st = 1; break; }
+    }
+    seq_len[p] = len;
+    status[p] = st;
+}
+
+// ----------------------------------------------------------- transport kernel
+// PH_INTERACT: at an interaction point, to be absorbed (then re-emitted) or
+// scattered; PH_ESCAPED: left the grid, its viewing-angle bins still to be
+// taken.  Both wait for an emission pass.
+enum Phase { PH_IDLE = 0, PH_STELLAR = 1, PH_INTERACT = 2, PH_WALK = 3, PH_ESCAPED = 4 };
+
+// A packet.  enPacket%direction (the direction at the start of the flight or
+// the last scatter) has the magnitudes of the walker's components, which the
+// octant's mirrors only turn over, so its signs (bits 0..2 of dsign) are all
+// that is kept of it.
+struct Lane {
+    Walker W;
+    uint32_t plo, phi, draws;   // packet id and draws taken from its stream
+    int nuP, origin;
+    int steps, runs, phase, dsign;
+};
+
+__device__ __forceinline__ float flight_direction(float v, int dsign, int k)
+{
+    return __uint_as_float((__float_as_uint(v) & 0x7fffffffu) | ((uint32_t)(dsign >> k) << 31));
+}
+
+// wave-uniform event counters (scalar registers; emptied into the launch's
+// 64-bit totals long before one could overflow, see kFlushLanes)
+struct WaveCounts {
+    unsigned seg, abs, sca, esc, lost, line, trapped, flights;
+    unsigned wpass, wlanes, epass, elanes;              // passes and the lanes in them
+};
+constexpr unsigned kFlushLanes = 1u << 31;
+
+__device__ __forceinline__ unsigned wcount(bool p)
+{
+    return (unsigned)__popcll(__ballot(p));
+}
+
+// An escape of a packet whose flight direction (enPacket%direction) is d:
+// its theta and phi bins, then the viewing-angle planes they feed, as every
+// escape site of pathSegment and energyPacketRun does
+// (photon_mod.f90:1582-1666, 370-465), as a bit mask.  err 60/61: the
+// reference's stops on a bin out of range.  The bin tables were
+// range-checked on the host.
+__device__ __forceinline__ unsigned esc_planes(const Grid &G, float dx, float dy, float dz, int &err)
+{
+    const View *V = G.view;
+    if (!V) return 1u;
+    const bool sym = (G.flags & F_SYM) != 0;
+    const float q = mcf_acosf(sym ? fabsf(dz) : dz) / V->dTheta;
+    if (isnan(q)) { err = 60; return 0; }
+    int it = (int)q + 1;
+    if (it > V->totT) it = V->totT;
+    if (it < 1) { err = 60; return 0; }
+    int ip;
+    if (fabsf(dx) < 1.e-35f) ip = 0;
+    else if (sym) ip = (int)(mcf_atanf(fabsf(dy) / fabsf(dx)) / V->dPhi);
+    else ip = (int)(mcf_atanf(dy / dx) / V->dPhi);
+    if (ip < 0) ip = V->totP + ip;
+    ip = ip + 1;
+    if (ip > V->totP) ip = V->totP;
+    if (ip < 1) { err = 61; return 0; }
+    const int t = V->Pt[it], ph = V->Pp[ip];
+    if (t > 0 && V->vph[t] < 0.f) return 1u | 1u << t;
+    if (t == ph || V->vth[ph] == V->vth[t] || V->vph[t] == V->vph[ph]) return 1u | 1u << t;
+    return 1u;
+}
+
+__device__ __forceinline__ unsigned esc_planes(const Grid &G, const Lane &L, int &err)
+{
+    return esc_planes(G, flight_direction(L.W.vx, L.dsign, 0), flight_direction(L.W.vy, L.dsign, 1),
+                      flight_direction(L.W.vz, L.dsign, 2), err);
+}
+
+// the word of plane a of esc for a packet
+__device__ __forceinline__ size_t esc_index(const Grid &G, int a, const Lane &L)
+{
+    return ((size_t)a * (size_t)(G.nbins + 1) + (size_t)L.nuP) * (size_t)(G.nCells + 1) + L.origin;
+}
+
+// ------------------------------------------------------------------- sinks
+// Where a wavefront's deposits go.  segment(): the J update of the lanes with
+// `has`; escape(): dE to the planes in each lane's mask.  ready(): room for
+// one more pass (at most three deposits a lane).
+
+// FP64 atomics, J's through the rings.
+template <int D, bool WIDE>
+struct AddSink {
+    JQ Q;
+    __device__ __forceinline__ bool ready(const Args &, int) { return true; }
+    __device__ __forceinline__ void segment(const Grid &G, bool has, unsigned w, unsigned nu0, float v, int lane)
+    {
+        jq_push<D, WIDE>(G, Q, has, w, nu0, v, lane);
+    }
+    __device__ __forceinline__ void escape(const Grid &G, unsigned planes, const Lane &L, float dE, int)
+    {
+        for (int a = 0; a < 3; ++a)
+            if (planes >> a & 1u) unsafeAtomicAdd(&G.esc[esc_index(G, a, L)], (double)dE);
+    }
+    __device__ __forceinline__ void close(const Grid &G, const Args &, int lane) { jq_flush<D, WIDE>(G, Q, lane); }
+};
+
+// The deposit log: 8 bytes a deposit, in the order they come.  A wavefront
+// queues them in LDS and writes kLogFlush at a time to chunks of its own: a
+// store in every pass would be waited for by the next pass's opacity gather
+// (loads and stores count down together).  45^3 octant, 1e8 packets: the walk
+// takes 14 ms with this sink, 45 with atomics (AddSink).
+constexpr int kLogQueue = 512;           // entries in LDS per wavefront
+constexpr int kLogFlush = 256;
+struct LogSink {
+    LogEntry *q;             // the queue
+    LogEntry *at;            // the chunk
+    unsigned n, chunk, used; // queued entries; the chunk's index and entries
+    bool open;
+    __device__ __forceinline__ void put(bool has, unsigned w, float v, int lane)
+    {
+        const uint64_t m = __ballot(has);
+        if (has) q[n + lane_rank(m, lane)] = LogEntry{ w, v };
+        n += (unsigned)__popcll(m);
+    }
+    // the first kLogFlush entries (or all) to the chunk; the rest move down
+    __device__ __forceinline__ void flush(unsigned count, int lane)
+    {
+        wave_lds_order();
+        for (unsigned i = lane; i < count; i += 64) at[used + i] = q[i];
+        used += count;
+        n -= count;
+        for (unsigned i = lane; i < n; i += 64) {
+            const LogEntry e = q[count + i];
+            wave_lds_order();
+            q[i] = e;
+        }
+        wave_lds_order();
+    }
+    __device__ __forceinline__ bool ready(const Args &P, int lane)
+    {
+        if (n + 3 * 64 <= (unsigned)kLogQueue) return true;
+        if (!open || used + kLogFlush > (unsigned)kLogChunk) {
+            const RunArgs RA = scalar_copy<RunArgs>(P.r);
+            unsigned c = 0;
+            if (lane == 0) {
+                if (open) RA.log_count[chunk] = used;
+                c = atomicAdd(RA.log_next, 1u);
+            }
+            chunk = (unsigned)__builtin_amdgcn_readfirstlane((int)c);
+            open = chunk < RA.log_chunks;
+            at = RA.log + (size_t)chunk * kLogChunk;
+            used = 0;
+            if (!open) return false;
+        }
+        flush(kLogFlush, lane);
+        return true;
+    }
+    __device__ __forceinline__ void segment(const Grid &, bool has, unsigned w, unsigned, float v, int lane)
+    {
+        put(has, w, v, lane);
+    }
+    __device__ __forceinline__ void escape(const Grid &G, unsigned planes, const Lane &L, float dE, int lane)
+    {
+        for (int a = 0; a < 3; ++a) {
+            const bool has = planes >> a & 1u;
+            if (a == 0 || (G.flags & F_VIEW)) put(has, G.esc_word + (unsigned)esc_index(G, a, L), dE, lane);
+        }
+    }
+    // What is queued goes to the end of the chunk, or (a wavefront whose
+    // packets are few, or that found the log full) to the estimators.
+    __device__ __forceinline__ void close(const Grid &G, const Args &P, int lane)
+    {
+        if (open && used + n <= (unsigned)kLogChunk) flush(n, lane);
+        wave_lds_order();
+        for (unsigned i = lane; i < n; i += 64) {
+            const LogEntry e = q[i];
+            double *to = e.w < G.esc_word ? G.J3 + e.w : G.esc + (e.w - G.esc_word);
+            unsafeAtomicAdd(to, (double)e.val);
+        }
+        n = 0;
+        if (open && lane == 0) scalar_copy<RunArgs>(P.r).log_count[chunk] = used;
+        open = false;
+    }
+};
+
+// What ends or continues a packet in a pass.
+struct Events {
+    bool absorbed = false, scattered = false, lost = false, escaped = false, line = false, flight = false;
+    unsigned planes = 0;     // of an escape
+};
+
+// The start of a flight in direction d: reciprocals, the octant's mirror and
+// the optical depth to the next interaction (photon_mod.f90:1176-1184).
+__device__ __forceinline__ void start_flight(Lane &L, const Grid &G, Rng &R, float dx, float dy, float dz)
+{
+    L.W.vx = dx; L.W.vy = dy; L.W.vz = dz;
+    L.dsign = (int)((__float_as_uint(dx) >> 31) | (__float_as_uint(dy) >> 31) << 1 | (__float_as_uint(dz) >> 31) << 2);
+    flight_reciprocals(G, L.W);
+    mirror_start(G, L.W);
+    L.W.absTau = 0.f;
+    const float random = draw(R, G);
+    L.W.passProb = -mcf_logf(1.f - random);
+    L.phase = PH_WALK;
+}
+
+// A packet at its interaction point (photon_mod.f90:1577-1797): beyond R_out
+// it has escaped, grains scatter or absorb it, gas absorbs it.  Returns true
+// when it is absorbed and due for its re-emission.
+template <bool WIDE>
+__device__ __forceinline__ bool interact(Lane &L, const Grid &G, const Axes &A, Rng &R, Events &E, int &err)
+{
+    const float rx = L.W.rx / 1.e10f, ry = L.W.ry / 1.e10f, rz = L.W.rz / 1.e10f;
+    if (sqrtf(rx * rx + ry * ry + rz * rz) * 1.e10f >= G.R_out && G.R_out > 0.f) {
+        E.planes = esc_planes(G, L, err);
+        E.escaped = true;
+        L.phase = PH_IDLE;
+        return false;
+    }
+    if (G.flags & F_DUST) {
+        const unsigned nu0 = (unsigned)(L.nuP - 1);
+        const size_t i = Word<WIDE>::index(G, Word<WIDE>::of(A.px[L.W.x], A.py[L.W.y], A.pz[L.W.z], nu0), nu0);
+        const float probSca = G.sca3[i] / G.opac3[i];
+        const float u = 1.f - draw(R, G);
+        if (u > probSca) {
+            E.absorbed = true;
+            if (!(G.flags & F_GAS)) { err = 41; return false; }           // dustEmi needs dust PDFs
+        } else if (u <= probSca) {
+            E.scattered = true;                               // 1720-1797
+            L.origin = act(G, L.W);
+            float dx = flight_direction(L.W.vx, L.dsign, 0), dy = flight_direction(L.W.vy, L.dsign, 1),
+                  dz = flight_direction(L.W.vz, L.dsign, 2);
+            if (G.flags & F_ISO) {
+                new_direction(R, G, false, dx, dy, dz);
+            } else {
+                for (int ihg = 1; ihg <= 10; ++ihg)
+                    if (hg(R, G, L.nuP, dx, dy, dz) == 0) break;
+            }
+            start_flight(L, G, R, dx, dy, dz);
+        } else {
+            err = 39;
+            return false;
+        }
+    } else {
+        E.absorbed = true;
+    }
+    // safeLimit (2838-2846); recursionLimit (120-126)
+    if (L.steps >= kSafeLimit) {
+        E.lost = true;
+        L.phase = PH_IDLE;
+    }
+    if (L.phase == PH_INTERACT && L.runs >= kRecursionLimit) L.phase = PH_IDLE;
+    return L.phase == PH_INTERACT;
+}
+
+// newPhotonPacket + initPhotonPacket + the start of pathSegment
+// (photon_mod.f90:768-1059, 491-684) for stellar packets and re-emissions at
+// an absorption point.
+__device__ __forceinline__ void emit(Lane &L, const Grid &G, const RunArgs &RA, Rng &R, double &qphot,
+                                     Events &E, int &err)
+{
+    const bool stellar = (L.phase == PH_STELLAR);
+    const float *cdf;
+    const unsigned short *guide;
+    int a;
+    if (stellar) {
+        L.runs = 1;
+        L.W.x = RA.sx - 1; L.W.y = RA.sy - 1; L.W.z = RA.sz - 1;
+        L.W.rx = RA.px; L.W.ry = RA.py; L.W.rz = RA.pz;
+        a = RA.star_cell;
+        cdf = G.specCDF + (size_t)(RA.istar - 1) * G.nbins;
+        guide = G.specGuide + (size_t)(RA.istar - 1) * (kGuide + 1);
+    } else {
+        L.runs++;
+        a = act(G, L.W);
+        if (!(G.flags & F_GAS)) { err = 13; return; }
+        if (a <= 0) { err = 14; return; }
+        float random = 1.f - draw(R, G);
+        if (random <= G.totalLines[a]) {                 // line packet (923-956)
+            E.line = true;
+            L.phase = PH_IDLE;
+            return;
+        }
+        cdf = G.recCDF + (size_t)a * G.nbins;
+        guide = G.recGuide + (size_t)a * (kGuide + 1);
+    }
+    int nuP = getnu2(R, G, cdf, guide, G.nbins, err);
+    if (err) return;
+    if (nuP < 1 || nuP >= G.nbins) { err = stellar ? 11 : 15; return; }
+    L.nuP = nuP;
+    float dx, dy, dz;
+    new_direction(R, G, stellar && (G.flags & (F_SYM | F_MULTI)) == F_SYM, dx, dy, dz);
+    L.origin = a;
+    const float nu = G.nuArray[nuP - 1];
+    if (stellar && nu > 1.f) qphot += (double)(RA.deltaE / (2.1799153e-11f * nu));
+    if (!(G.flags & F_DUST) && nu < G.ionEdge1) {        // escapes at birth (370-465)
+        E.planes = esc_planes(G, dx, dy, dz, err);
+        E.escaped = true;
+        L.phase = PH_IDLE;
+        return;
+    }
+    start_flight(L, G, R, dx, dy, dz);
+    L.steps = 0;
+    E.flight = true;
+}
+
+__device__ __forceinline__ bool pending(const Lane &L)
+{
+    return L.phase != PH_IDLE && L.phase != PH_WALK;
+}
+
+// An emission pass of the wavefront: every lane whose packet waits runs it
+// together.  Escapes and interactions end or turn their packets first; then
+// new and absorbed packets are emitted.  Taking the interactions here keeps
+// their divisions, square root and draws out of the walk passes, nearly all
+// of which have a lane or two that interacts.  Counts events into C.
+template <bool WIDE, class Sink>
+__device__ __forceinline__ void emission_pass(Lane &L, const Args &P, const Axes &A, WaveCounts &C, double &qphot,
+                                              int &err, Sink &K, int lane)
+{
+    const Grid G = scalar_copy<Grid>(P.g);
+    const RunArgs RA = scalar_copy<RunArgs>(P.r);
+    Events E;
+    Rng R = rng_at(L.plo, L.phi, (uint32_t)RA.istar, L.draws);
+    bool emits = L.phase == PH_STELLAR;
+    if (L.phase == PH_ESCAPED) {
+        E.planes = esc_planes(G, L, err);
+        L.phase = PH_IDLE;
+    } else if (L.phase == PH_INTERACT) {
+        emits = interact<WIDE>(L, G, A, R, E, err);
+    }
+    bool ends = E.escaped || (E.absorbed && L.phase == PH_IDLE) || E.lost;
+    if (emits) {
+        emit(L, G, RA, R, qphot, E, err);
+        ends = E.line || E.escaped;
+    }
+    if (err) L.phase = PH_IDLE;
+    L.draws = R.k;
+    if (__any(E.planes != 0)) K.escape(G, E.planes, L, RA.deltaE, lane);
+    C.epass += 1;
+    C.elanes += wcount(emits);
+    C.abs += wcount(E.absorbed);
+    C.sca += wcount(E.scattered);
+    C.lost += wcount(E.lost);
+    C.line += wcount(E.line);
+    C.esc += wcount(E.escaped);
+    C.flights += wcount(E.flight);
+    // energyPacketDriver counts the packet whose last run is the
+    // recursionLimit-th as trapped (photon_mod.f90:126)
+    C.trapped += wcount(!err && ends && L.runs >= kRecursionLimit);
+}
+
+// One walk pass of the wavefront: every lane whose packet walks takes one
+// step of pathSegment.  Counts events into C, queues the J updates.
+template <bool WIDE, class Sink>
+__device__ __forceinline__ void walk_pass(Lane &L, const Grid &G, const Axes &A, float dE, WaveCounts &C, int &err,
+                                          Sink &K, int lane)
+{
+    bool seg = false;
+    float jv = 0.f;
+    Segment S;
+    S.w = 0;
+    const unsigned nu0 = (unsigned)(L.nuP - 1);
+    bool escaped = false, lost = false;
+    C.wpass += 1;
+    C.wlanes += wcount(L.phase == PH_WALK);
+    if (L.phase == PH_WALK) {
+        L.steps++;
+        int e = 0;
+        const int r = walk_step<false, WIDE>(G, A, L.W, nu0, S, e);
+        seg = r != ST_LOST && r != ST_ERROR;
+        if (seg) jv = S.len * dE / S.dV;
+        if (r == ST_ABSORBED) L.phase = PH_INTERACT;
+        if (r == ST_ESCAPED) {
+            escaped = true;
+            L.phase = (G.flags & F_VIEW) ? PH_ESCAPED : PH_IDLE;
+        }
+        lost = r == ST_LOST || (r == ST_CONTINUE && L.steps >= kSafeLimit);   // safeLimit, 2838-2846
+        if (lost || r == ST_ERROR) L.phase = PH_IDLE;
+        if (e) err = e;
+    }
+    K.segment(G, seg, S.w, nu0, jv, lane);
+    if (!(G.flags & F_VIEW) && __any(escaped)) K.escape(G, escaped ? 1u : 0u, L, dE, lane);
+    C.seg += wcount(seg);
+    C.esc += wcount(escaped);
+    if (__any(lost)) C.lost += wcount(lost);
+    if (__any((lost || escaped) && L.runs >= kRecursionLimit))
+        C.trapped += wcount((lost || escaped) && L.runs >= kRecursionLimit);
+}
+
+// ------------------------------------------------ packet pool (per wave, LDS)
+// A wavefront keeps a pool of P packets in LDS beside its 64 lanes: packets
+// that walk (the walker stack, slots 0 .. nw-1 from the bottom) and packets
+// that wait for an emission pass (the pending stack, slots P-npd .. P-1 from
+// the top).  A lane whose flight ends takes a walker from the pool, leaving
+// its own packet on the pending stack if it waits; an emission round moves
+// walkers into the pool, so that the emission pass runs on a full wavefront,
+// and the walkers come back as flights end.  The walk passes then stay nearly
+// full between emissions.  Word k of slot s is at pw[k * P + s]; the cell
+// indices are packed in one word (11, 11 and 10 bits: the host runs this
+// kernel on lattices of at most 2048 x 2048 x 1024 points), the frequency
+// bin, run count and phase in another (16, 13 and 3 bits), steps and direction
+// signs in a third.  The stream is the launch's source, not stored, and a
+// waiting packet's optical depths and reciprocals are of no use any more.
+constexpr int kPoolWords = 18;
+// Slots per wavefront: with 8-deep J rings, 4 workgroups of 256 per CU keep
+// 32 slots within the CU's 160 KB of LDS (6.9 KB per wavefront, plus the
+// staged tables).
+constexpr int kPoolSlots = 32;
+constexpr int kLogSlots = 32;    // log_kernel
+static_assert(kSafeLimit < (1 << 20) && kRecursionLimit < (1 << 13), "packed packet words");
+
+template <int P>
+__device__ __forceinline__ void pool_put(uint32_t *pw, int s, const Lane &L)
+{
+    uint32_t *q = pw + s;
+    q[0 * P] = L.plo; q[1 * P] = L.phi; q[2 * P] = L.draws;
+    q[3 * P] = __float_as_uint(L.W.rx); q[4 * P] = __float_as_uint(L.W.ry); q[5 * P] = __float_as_uint(L.W.rz);
+    q[6 * P] = __float_as_uint(L.W.vx); q[7 * P] = __float_as_uint(L.W.vy); q[8 * P] = __float_as_uint(L.W.vz);
+    q[9 * P] = (uint32_t)L.W.x | ((uint32_t)L.W.y << 11) | ((uint32_t)L.W.z << 22);
+    q[10 * P] = (uint32_t)L.nuP | ((uint32_t)L.runs << 16) | ((uint32_t)L.phase << 29);
+    q[11 * P] = (uint32_t)L.origin;
+    q[12 * P] = (uint32_t)L.steps | ((uint32_t)L.dsign << 20);
+    if (L.phase == PH_WALK) {
+        q[13 * P] = __float_as_uint(L.W.absTau); q[14 * P] = __float_as_uint(L.W.passProb);
+        q[15 * P] = __float_as_uint(L.W.qx); q[16 * P] = __float_as_uint(L.W.qy); q[17 * P] = __float_as_uint(L.W.qz);
+    }
+}
+
+template <int P, bool WALKER>
+__device__ __forceinline__ void pool_get(const uint32_t *pw, int s, Lane &L)
+{
+    const uint32_t *q = pw + s;
+    L.plo = q[0 * P]; L.phi = q[1 * P]; L.draws = q[2 * P];
+    L.W.rx = __uint_as_float(q[3 * P]); L.W.ry = __uint_as_float(q[4 * P]); L.W.rz = __uint_as_float(q[5 * P]);
+    L.W.vx = __uint_as_float(q[6 * P]); L.W.vy = __uint_as_float(q[7 * P]); L.W.vz = __uint_as_float(q[8 * P]);
+    const uint32_t c = q[9 * P];
+    L.W.x = (int)(c & 2047u); L.W.y = (int)((c >> 11) & 2047u); L.W.z = (int)(c >> 22);
+    const uint32_t f = q[10 * P];
+    L.nuP = (int)(f & 65535u); L.runs = (int)((f >> 16) & 8191u); L.phase = WALKER ? PH_WALK : (int)(f >> 29);
+    L.origin = (int)q[11 * P];
+    const uint32_t t = q[12 * P];
+    L.steps = (int)(t & 0xfffffu); L.dsign = (int)(t >> 20);
+    if (WALKER) {
+        L.W.absTau = __uint_as_float(q[13 * P]); L.W.passProb = __uint_as_float(q[14 * P]);
+        L.W.qx = __uint_as_float(q[15 * P]); L.W.qy = __uint_as_float(q[16 * P]); L.W.qz = __uint_as_float(q[17 * P]);
+    }
+}
+
 // Lanes that do not walk take walkers from the pool (the first nw of them in
-// lane order); a taker whose packet waits for an emission leaves it on the
-// pending stack first, if the pool has a free slot for it.  The pending
+// lane order); a taker whose packet waits for an emission pass leaves it on
+// the pending stack first, if the pool has a free slot for it.  The pending
 // slots written lie in the free region, the walker slots read below it.
 template <int P>
-__device__ __forceinline__ void pool_settle(Lane &L, uint32_t *pw, int &nw, int &npd, int lane, uint32_t stream)
+__device__ __forceinline__ void pool_settle(Lane &L, uint32_t *pw, int &nw, int &npd, int lane)
 {
     if (nw == 0) return;
     const bool nonw = L.phase != PH_WALK;
@@ -588,26 +678,73 @@ __device__ __forceinline__ void pool_settle(Lane &L, uint32_t *pw, int &nw, int 
         npd += __popcll(mtp);
         wave_lds_order();
     }
-    if (take) pool_get<P>(pw, nw - 1 - re, L, stream);
+    if (take) pool_get<P, true>(pw, nw - 1 - re, L);
     nw -= __popcll(mt);
     wave_lds_order();
+}
+
+// The packets a wavefront holds: indices next .. end - 1 of the launch.  It
+// takes them from the launch's counter many at a time, 1/8 of its share of
+// what is left (64 to 2048).  Atomics with a result on one address are served
+// one every 12 ns: taking the packets of each emission round alone, the 4096
+// wavefronts of a sweep waited 49 us a round for one another.
+struct Stock {
+    unsigned long long next = 0, end = 0;
+    bool last = false;           // nothing left at the counter
+    __device__ __forceinline__ bool empty() const { return last && next >= end; }
+};
+
+// Fresh packets for the lanes with `need`.
+__device__ __forceinline__ void take_fresh(Lane &L, const Args &P, bool need, Stock &S, int lane)
+{
+    uint64_t m = __ballot(need);
+    if (!m) return;
+    const RunArgs RA = scalar_copy<RunArgs>(P.r);
+    const unsigned long long total = (unsigned long long)RA.npackets;
+    while (m) {
+        if (S.next >= S.end) {
+            if (S.last) break;
+            const unsigned long long waves = (unsigned long long)gridDim.x * (blockDim.x >> 6);
+            const unsigned long long share = (total - S.end) / (8 * waves) & ~63ull;
+            const unsigned long long n = share < 64 ? 64 : share > 2048 ? 2048 : share;
+            unsigned long long base = 0;
+            if (lane == 0) base = atomicAdd(RA.next_packet, n);
+            base = (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(base >> 32)) << 32 |
+                   (unsigned)__builtin_amdgcn_readfirstlane((int)base);
+            S.next = base < total ? base : total;
+            S.end = base + n < total ? base + n : total;
+            S.last = base + n >= total;
+            continue;
+        }
+        const unsigned long long id = S.next + (unsigned long long)lane_rank(m, lane);
+        const bool mine = ((m >> lane) & 1ull) && id < S.end;
+        if (mine) {
+            const uint64_t packet = RA.packet_offset + id;
+            L.plo = (uint32_t)packet;
+            L.phi = (uint32_t)(packet >> 32);
+            L.draws = 0;
+            L.phase = PH_STELLAR;
+        }
+        const uint64_t took = __ballot(mine);
+        S.next += (unsigned long long)__popcll(took);
+        m &= ~took;
+    }
 }
 
 // An emission round of the pool kernel: walkers move to the pool (as many
 // as the candidates for an emission exceed the lanes that do not walk, and
 // as fit), idle lanes take packets from the pending stack, then fresh
-// packets (one counter atomic per wavefront), and the emission pass runs.
-template <int P>
-__device__ __forceinline__ void pool_emission_round(Lane &L, uint32_t *pw, int &nw, int &npd, bool &exhausted,
-                                                    const Grid &G, const RunArgs &RA, const Model &M,
-                                                    const float *spec, const unsigned short *spec_guide,
-                                                    WaveCounts &C, double &qphot, int &err, int lane)
+// packets, and the emission pass runs.
+template <int P, bool WIDE, class Sink>
+__device__ __forceinline__ void pool_emission_round(Lane &L, uint32_t *pw, int &nw, int &npd, Stock &S,
+                                                    const Args &A_, const Axes &A, WaveCounts &C, double &qphot,
+                                                    int &err, Sink &K, int lane)
 {
     const bool walk = L.phase == PH_WALK;
     const uint64_t mw = __ballot(walk);
     const int nwalk = __popcll(mw);
     const int npl = (int)wcount(pending(L));
-    const int cand = npl + npd + (exhausted ? 0 : 64);
+    const int cand = npl + npd + (S.empty() ? 0 : 64);
     const int k = max(0, min(min(nwalk, P - nw - npd), cand - (64 - nwalk)));
     if (k > 0) {
         const int rw = lane_rank(mw, lane);
@@ -622,260 +759,259 @@ __device__ __forceinline__ void pool_emission_round(Lane &L, uint32_t *pw, int &
         const bool idle = L.phase == PH_IDLE;
         const uint64_t mi = __ballot(idle);
         const int ri = lane_rank(mi, lane);
-        if (idle && ri < npd) pool_get<P>(pw, P - npd + ri, L, (uint32_t)RA.istar);
+        if (idle && ri < npd) pool_get<P, false>(pw, P - npd + ri, L);
         npd -= min(__popcll(mi), npd);
         wave_lds_order();
     }
-    const bool need = (L.phase == PH_IDLE) && !exhausted;
-    const uint64_t m = __ballot(need);
-    if (m) {
-        const int leader = __ffsll((unsigned long long)m) - 1;
-        unsigned long long base = 0;
-        if (lane == leader) base = atomicAdd(RA.next_packet, (unsigned long long)__popcll(m));
-        base = __shfl(base, leader);
-        bool over = false;
-        if (need) {
-            const unsigned long long id = base + (unsigned long long)lane_rank(m, lane);
-            if (id < (unsigned long long)RA.npackets) {
-                rng_start(L.R, RA.packet_offset + id, (uint32_t)RA.istar);
-                L.phase = PH_EMIT_STELLAR;
-            } else {
-                over = true;
-            }
-        }
-        exhausted = __any(over);
-    }
-    if (__any(pending(L))) emission_pass(L, G, RA, M, spec, spec_guide, C, qphot, err);
+    if (!S.empty()) take_fresh(L, A_, L.phase == PH_IDLE, S, lane);
+    if (__any(pending(L))) emission_pass<WIDE>(L, A_, A, C, qphot, err, K, lane);
+}
+
+__device__ __forceinline__ Lane idle_lane()
+{
+    Lane L;
+    L.W.rx = L.W.ry = L.W.rz = L.W.vx = L.W.vy = L.W.vz = L.W.qx = L.W.qy = L.W.qz = 0.f;
+    L.W.x = L.W.y = L.W.z = 0;
+    L.W.absTau = L.W.passProb = 0.f;
+    L.plo = L.phi = L.draws = 0;
+    L.nuP = 1; L.origin = 0; L.steps = 0; L.runs = 0; L.phase = PH_IDLE; L.dsign = 0;
+    return L;
 }
 
 // Add a wavefront's counters to its model's totals and clear them.
-__device__ __forceinline__ void flush_counts(const RunArgs &RA, WaveCounts &C, double &qphot)
+__device__ __forceinline__ void flush_counts(const Args &P, WaveCounts &C)
 {
-    for (int o = 32; o >= 1; o >>= 1) qphot += __shfl_xor(qphot, o);
+    const RunArgs RA = scalar_copy<RunArgs>(P.r);
     if ((threadIdx.x & 63) == 0) {
-        atomicAdd(&RA.counts[0], C.seg);
-        atomicAdd(&RA.counts[1], C.abs);
-        atomicAdd(&RA.counts[2], C.sca);
-        atomicAdd(&RA.counts[3], C.esc);
-        atomicAdd(&RA.counts[4], C.lost);
-        atomicAdd(&RA.counts[5], C.line);
-        atomicAdd(&RA.counts[6], C.trapped);
-        atomicAdd(&RA.counts[7], C.flights);
-        atomicAdd(&RA.counts[8], C.wpass);
-        atomicAdd(&RA.counts[9], C.wlanes);
-        atomicAdd(&RA.counts[10], C.epass);
-        atomicAdd(&RA.counts[11], C.elanes);
-        unsafeAtomicAdd(RA.qphot, qphot);
+        const unsigned v[12] = { C.seg, C.abs, C.sca, C.esc, C.lost, C.line, C.trapped, C.flights,
+                                 C.wpass, C.wlanes, C.epass, C.elanes };
+        for (int i = 0; i < 12; ++i) atomicAdd(&RA.counts[i], (unsigned long long)v[i]);
     }
     C = WaveCounts{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    qphot = 0.0;
 }
 
-// The single-model kernel.  TWO: two packets per lane (advance_spare; 144
-// VGPRs, so at most 3 wavefronts per SIMD), else one (advance; 4 per SIMD).
-template <bool TWO>
-__global__ void __launch_bounds__(256) transport_kernel(Grid G, RunArgs RA)
+__device__ __forceinline__ void flush_qphot(const Args &P, double qphot)
 {
-    extern __shared__ float lds[];
-    Axes A;
-    float *spec = nullptr;
-    unsigned short *spec_guide = nullptr;
-    const int nwaves = (int)(blockDim.x >> 6);
-    stage_model(G, RA, lds + (size_t)nwaves * JRing<kJDepth>::kFloats, A, spec, spec_guide);
-    const int lane_id = threadIdx.x & 63;
-    JQ Q = jq_at<kJDepth>(lds, (int)(threadIdx.x >> 6));
-    const Model M = model_of(G, RA);
+    for (int o = 32; o >= 1; o >>= 1) qphot += __shfl_xor(qphot, o);
+    if ((threadIdx.x & 63) == 0) unsafeAtomicAdd(scalar_copy<RunArgs>(P.r).qphot, qphot);
+}
 
-    Lane L, S;
-    L.phase = PH_IDLE;
-    L.runs = 0; L.steps = 0; L.nuP = 1; L.origin = 0;
-    S = L;
-    bool exhausted = false;
-    WaveCounts C = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    double qphot = 0.0;
-    int err = 0;
-
-    for (;;) {
-        // ---- refill idle lanes (their spare with two packets per lane): one
-        // atomic per wavefront
-        Lane &N = TWO ? S : L;
-        bool need = (N.phase == PH_IDLE) && !exhausted;
-        uint64_t m = __ballot(need);
-        if (m) {
-            int leader = __ffsll((unsigned long long)m) - 1;
-            unsigned long long base = 0;
-            if (lane_id == leader)
-                base = atomicAdd(RA.next_packet, (unsigned long long)__popcll(m));
-            base = __shfl(base, leader);
-            if (need) {
-                unsigned long long rank = __popcll(m & ((1ull << lane_id) - 1ull));
-                unsigned long long id = base + rank;
-                if (id < (unsigned long long)RA.npackets) {
-                    rng_start(N.R, RA.packet_offset + id, (uint32_t)RA.istar);
-                    N.phase = PH_EMIT_STELLAR;
-                } else {
-                    exhausted = true;
-                }
-            }
-        }
-        if (TWO) {
-            if (wcount(L.phase != PH_IDLE || S.phase != PH_IDLE) == 0) break;
-            advance_spare<kJDepth>(L, S, G, A, RA, M, spec, spec_guide, RA.emit_min, RA.walk_steps, C, qphot, err,
-                                   Q, lane_id);
-        } else {
-            const int npend = (int)wcount(pending(L));
-            const int nwalk = (int)wcount(L.phase == PH_WALK);
-            if (npend + nwalk == 0) break;
-            advance<kJDepth>(L, G, A, RA, M, spec, spec_guide, RA.emit_min, RA.walk_steps, npend, nwalk, C, qphot,
-                             err, Q, lane_id);
-        }
+// A fail-stop code goes to the launch's error word.
+__device__ __forceinline__ void report(const Args &P, int &err)
+{
+    if (__any(err != 0)) {
+        if (err) atomicMax(scalar_copy<RunArgs>(P.r).error, err);
+        err = 0;
     }
-    jq_flush<kJDepth>(G, Q, lane_id);
-    flush_counts(RA, C, qphot);
 }
 
-// The single-model kernel with a packet pool of P slots per wavefront in
-// LDS (one packet per lane in registers, J rings of D updates).  An
-// emission round runs when at least emit_min lanes do not walk (or none
-// does); every walk pass is followed by a settle from the pool.
-template <int D, int P>
-__global__ void __launch_bounds__(256) pool_kernel(Grid G, RunArgs RA)
+// The arguments of the single-model kernels, read in place from the launch's
+// argument block.
+struct LaunchArgs { Grid G; RunArgs RA; };
+
+__device__ __forceinline__ Args kernel_args()
+{
+    const uint64_t at = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+    return Args{ at, at + offsetof(LaunchArgs, RA) };
+}
+
+// One packet per lane, for lattices the pool kernel does not take (64-bit
+// table indices).  An emission pass runs when at least emit_min lanes (or as
+// many as are walking) wait for one, then walk_steps walk passes.
+__global__ void __launch_bounds__(256) transport_kernel(LaunchArgs)
 {
     extern __shared__ float lds[];
+    const Args P = kernel_args();
+    const Grid G = scalar_copy<Grid>(P.g);
+    const RunArgs RA = scalar_copy<RunArgs>(P.r);
     Axes A;
-    float *spec = nullptr;
-    unsigned short *spec_guide = nullptr;
     const int nwaves = (int)(blockDim.x >> 6);
-    const int wave = (int)(threadIdx.x >> 6);
-    uint32_t *pools = reinterpret_cast<uint32_t *>(lds + (size_t)nwaves * JRing<D>::kFloats);
-    stage_model(G, RA, reinterpret_cast<float *>(pools + (size_t)nwaves * P * kPoolWords), A, spec, spec_guide);
-    uint32_t *pw = pools + (size_t)wave * P * kPoolWords;
+    stage_axes<true>(G, lds + (size_t)nwaves * JRing<kJDepth, true>::kFloats, A);
     const int lane_id = threadIdx.x & 63;
-    JQ Q = jq_at<D>(lds, wave);
-    const Model M = model_of(G, RA);
-    const uint32_t stream = (uint32_t)RA.istar;
+    AddSink<kJDepth, true> K{ jq_at<kJDepth, true>(lds, (int)(threadIdx.x >> 6)) };
 
-    Lane L;
-    L.phase = PH_IDLE;
-    L.runs = 0; L.steps = 0; L.nuP = 1; L.origin = 0;
-    int nw = 0, npd = 0;
-    bool exhausted = false;
+    Lane L = idle_lane();
+    Stock S;
     WaveCounts C = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     double qphot = 0.0;
     int err = 0;
 
     for (;;) {
-        pool_settle<P>(L, pw, nw, npd, lane_id, stream);
-        const int nwalk = (int)wcount(L.phase == PH_WALK);
-        if (nwalk == 0 && nw == 0 && npd == 0 && exhausted && !__any(pending(L))) break;
-        if (64 - nwalk >= RA.emit_min || nwalk == 0)
-            pool_emission_round<P>(L, pw, nw, npd, exhausted, G, RA, M, spec, spec_guide, C, qphot, err, lane_id);
-        for (int s = 0; s < RA.walk_steps; ++s) {
-            if (!__any(L.phase == PH_WALK)) break;
-            walk_pass<D>(L, G, A, M, C, err, Q, lane_id);
-            pool_settle<P>(L, pw, nw, npd, lane_id, stream);
-        }
-        if (err) {
-            atomicMax(RA.error, err);
-            err = 0;
-        }
-    }
-    jq_flush<D>(G, Q, lane_id);
-    flush_counts(RA, C, qphot);
-}
-
-// Many models in one persistent launch.  The packets of every model are cut
-// into chunks, listed model after model; a one-wavefront workgroup takes
-// chunks from a global counter, refills its lanes from the chunk it holds,
-// and takes the next chunk when that one is used up.  A chunk of another
-// model is taken only after the wavefront's packets of the current model
-// have finished: then its grid and source are staged in LDS and its
-// counters flushed.  Each packet keeps its own random stream, so results
-// equal those of the models' separate runs.  Compiled for 4 wavefronts per
-// SIMD (128 VGPRs, a few spilled to scratch): the one-wavefront workgroups
-// need the occupancy more than the registers.
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) batch_kernel(BatchArgs B)
-{
-    extern __shared__ float lds[];
-    const int lane_id = threadIdx.x;
-    JQ Q = jq_at<kJDepthBatch>(lds, 0);
-    float *tab = lds + JRing<kJDepthBatch>::kFloats;
-    Axes A;
-    float *spec = nullptr;
-    unsigned short *spec_guide = nullptr;
-    // the current model's grid and arguments are read in place (wave-uniform
-    // addresses: scalar loads), not copied into registers
-    const Grid *Gp = B.G;
-    const RunArgs *RAp = B.RA;
-    Model M;
-    int cur = -1;                       // model of the staged tables
-    long long cnext = 0, cend = 0;      // packets left in the held chunk (model cur)
-    int pending = -1;                   // chunk of another model, taken after draining
-    bool done = false;                  // no chunks left
-
-    Lane L;
-    L.phase = PH_IDLE;
-    L.runs = 0; L.steps = 0; L.nuP = 1; L.origin = 0;
-    WaveCounts C = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    double qphot = 0.0;
-    int err = 0;
-
-    for (;;) {
-        // ---- refill idle lanes from the held chunk, taking chunks of the same model
-        uint64_t m = __ballot(L.phase == PH_IDLE);
-        while (m && pending < 0 && !done) {
-            if (cnext >= cend) {
-                int c = 0;
-                if (lane_id == 0) c = (int)atomicAdd(B.next_chunk, 1u);
-                c = __builtin_amdgcn_readfirstlane(c);     // wave-uniform: scalar registers
-                if (c >= B.nchunks) { done = true; break; }
-                if (B.chunk_model[c] != cur) { pending = c; break; }
-                cnext = B.chunk_first[c];
-                cend = cnext + B.chunk_count[c];
-                continue;
-            }
-            const long long avail = cend - cnext;
-            const unsigned long long rank = __popcll(m & ((1ull << lane_id) - 1ull));
-            const bool mine = ((m >> lane_id) & 1ull) && (long long)rank < avail;
-            if (mine) {
-                rng_start(L.R, RAp->packet_offset + (unsigned long long)(cnext + (long long)rank),
-                          (uint32_t)RAp->istar);
-                L.phase = PH_EMIT_STELLAR;
-            }
-            const uint64_t took = __ballot(mine);
-            cnext += __popcll(took);
-            m &= ~took;
-        }
-        const bool pend = (L.phase == PH_EMIT_STELLAR || L.phase == PH_EMIT_DIFFUSE);
-        const int npend = (int)wcount(pend);
+        if (!S.empty()) take_fresh(L, P, L.phase == PH_IDLE, S, lane_id);
+        const int npend = (int)wcount(pending(L));
         const int nwalk = (int)wcount(L.phase == PH_WALK);
         if (npend + nwalk == 0) {
-            if (pending >= 0) {
-                // all lanes idle: switch to the pending chunk's model
-                if (cur >= 0) {
-                    jq_flush<kJDepthBatch>(*Gp, Q, lane_id);
-                    flush_counts(*RAp, C, qphot);
-                }
-                cur = __builtin_amdgcn_readfirstlane(B.chunk_model[pending]);
-                Gp = B.G + cur;
-                RAp = B.RA + cur;
-                __syncthreads();
-                stage_model(*Gp, *RAp, tab, A, spec, spec_guide);
-                M = model_of(*Gp, *RAp);
-                cnext = B.chunk_first[pending];
-                cend = cnext + B.chunk_count[pending];
-                pending = -1;
-                continue;
-            }
-            if (done) break;
+            if (S.empty()) break;
             continue;
         }
-        advance<kJDepthBatch>(L, *Gp, A, *RAp, M, spec, spec_guide, B.emit_min, B.walk_steps, npend, nwalk, C, qphot, err, Q,
-                lane_id);
+        if (npend >= RA.emit_min || npend >= nwalk) emission_pass<true>(L, P, A, C, qphot, err, K, lane_id);
+        for (int s = 0; s < RA.walk_steps; ++s) walk_pass<true>(L, G, A, RA.deltaE, C, err, K, lane_id);
+        report(P, err);
+        if (C.wlanes >= kFlushLanes) flush_counts(P, C);
     }
-    if (cur >= 0) {
-        jq_flush<kJDepthBatch>(*Gp, Q, lane_id);
-        flush_counts(*RAp, C, qphot);
+    K.close(G, P, lane_id);
+    flush_counts(P, C);
+    flush_qphot(P, qphot);
+}
+
+// A suspended wavefront's packets: its lanes (kPoolWords words each, phase
+// included), its pool's slots, nw, npd and its stock.
+template <int P>
+struct Save {
+    static constexpr int kWords = kPoolWords * (64 + P) + 64;
+    static __device__ __forceinline__ void put(uint32_t *at, const Lane &L, const uint32_t *pw, int nw, int npd,
+                                               const Stock &S, int lane)
+    {
+        pool_put<64>(at, lane, L);
+        for (int i = lane; i < kPoolWords * P; i += 64) at[kPoolWords * 64 + i] = pw[i];
+        if (lane == 0) {
+            uint32_t *t = at + kPoolWords * (64 + P);
+            t[0] = (uint32_t)nw; t[1] = (uint32_t)npd; t[2] = S.last;
+            t[3] = (uint32_t)S.next; t[4] = (uint32_t)(S.next >> 32); t[5] = (uint32_t)S.end; t[6] = (uint32_t)(S.end >> 32);
+        }
+    }
+    static __device__ __forceinline__ void get(const uint32_t *at, Lane &L, uint32_t *pw, int &nw, int &npd,
+                                               Stock &S, int lane)
+    {
+        pool_get<64, true>(at, lane, L);
+        L.phase = (int)(at[10 * 64 + lane] >> 29);
+        for (int i = lane; i < kPoolWords * P; i += 64) pw[i] = at[kPoolWords * 64 + i];
+        uint32_t t[7];
+        for (int i = 0; i < 7; ++i)
+            t[i] = (uint32_t)__builtin_amdgcn_readfirstlane((int)at[kPoolWords * (64 + P) + i]);
+        nw = (int)t[0];
+        npd = (int)t[1];
+        S.last = t[2] != 0;
+        S.next = t[3] | (unsigned long long)t[4] << 32;
+        S.end = t[5] | (unsigned long long)t[6] << 32;
+        wave_lds_order();
+    }
+};
+
+// One model's packets on one wavefront, with a packet pool of P slots in LDS
+// (one packet per lane in registers).  An emission round runs when at least
+// emit_min lanes do not walk (or none does); every walk pass is followed by a
+// settle from the pool.  A sink that runs out of room suspends the wavefront.
+template <int P, class Sink>
+__device__ __forceinline__ void pool_run(const Args &K, const Axes &A, uint32_t *pw, Sink &D, int lane_id)
+{
+    const Grid G = scalar_copy<Grid>(K.g);
+    const RunArgs RA = scalar_copy<RunArgs>(K.r);
+    Lane L = idle_lane();
+    int nw = 0, npd = 0;
+    Stock S;
+    bool room = true;
+    WaveCounts C = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    double qphot = 0.0;
+    int err = 0;
+    const size_t save = (size_t)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * Save<P>::kWords;
+    if (RA.resume) Save<P>::get(RA.save + save, L, pw, nw, npd, S, lane_id);
+    for (;;) {
+        pool_settle<P>(L, pw, nw, npd, lane_id);
+        const int nwalk = (int)wcount(L.phase == PH_WALK);
+        if (nwalk == 0 && nw == 0 && npd == 0 && S.empty() && !__any(pending(L))) break;
+        room = D.ready(K, lane_id);
+        if (!room) break;
+        if (64 - nwalk >= RA.emit_min || nwalk == 0)
+            pool_emission_round<P, false>(L, pw, nw, npd, S, K, A, C, qphot, err, D, lane_id);
+        for (int s = 0; s < RA.walk_steps; ++s) {
+            // on with the next round early when fewer than half the lanes
+            // walk and there are packets to fill an emission pass with
+            const int walking = (int)wcount(L.phase == PH_WALK);
+            if (walking == 0 || (s > 0 && walking < 32 &&
+                                 (!S.empty() || npd + (int)wcount(pending(L)) >= 16))) break;
+            room = D.ready(K, lane_id);
+            if (!room) break;
+            walk_pass<false>(L, G, A, RA.deltaE, C, err, D, lane_id);
+            pool_settle<P>(L, pw, nw, npd, lane_id);
+        }
+        report(K, err);
+        if (C.wlanes >= kFlushLanes) flush_counts(K, C);
+        if (!room) break;
+    }
+    D.close(G, K, lane_id);
+    flush_counts(K, C);
+    flush_qphot(K, qphot);
+    if (!room) {
+        const RunArgs RB = scalar_copy<RunArgs>(K.r);
+        Save<P>::put(RB.save + save, L, pw, nw, npd, S, lane_id);
+        if (lane_id == 0) *RB.suspended = 1;
+    } else if (RA.save && lane_id == 0) {
+        // done: nothing to go on with in a further launch
+        uint32_t *t = scalar_copy<RunArgs>(K.r).save + save + kPoolWords * (64 + P);
+        t[0] = 0; t[1] = 0; t[2] = 1;
+        t[3] = 0; t[4] = 0; t[5] = 0; t[6] = 0;
+    }
+    if (room && RA.save) scalar_copy<RunArgs>(K.r).save[save + 10 * 64 + lane_id] = 0;
+}
+
+// The single-model kernel with atomic deposits (small sweeps, crossing
+// counts, no memory for the log).
+__global__ void __launch_bounds__(256) pool_kernel(LaunchArgs)
+{
+    extern __shared__ float lds[];
+    const Args K = kernel_args();
+    Axes A;
+    const int nwaves = (int)(blockDim.x >> 6), wave = (int)(threadIdx.x >> 6);
+    uint32_t *pools = reinterpret_cast<uint32_t *>(lds + (size_t)nwaves * JRing<kJDepth, false>::kFloats);
+    stage_axes<false>(scalar_copy<Grid>(K.g), reinterpret_cast<float *>(pools + (size_t)nwaves * kPoolSlots * kPoolWords),
+                      A);
+    AddSink<kJDepth, false> D{ jq_at<kJDepth, false>(lds, wave) };
+    pool_run<kPoolSlots>(K, A, pools + (size_t)wave * kPoolSlots * kPoolWords, D, (int)(threadIdx.x & 63));
+}
+
+// The single-model kernel with its deposits in the log: 74 VGPRs, six
+// wavefronts a SIMD as far as its LDS (queue and pool, 6.3 KB a wavefront) allows.
+__global__ void __launch_bounds__(256) log_kernel(LaunchArgs)
+{
+    extern __shared__ float lds[];
+    const Args K = kernel_args();
+    Axes A;
+    const int nwaves = (int)(blockDim.x >> 6), wave = (int)(threadIdx.x >> 6);
+    LogEntry *queues = reinterpret_cast<LogEntry *>(lds);
+    uint32_t *pools = reinterpret_cast<uint32_t *>(queues + (size_t)nwaves * kLogQueue);
+    stage_axes<false>(scalar_copy<Grid>(K.g), reinterpret_cast<float *>(pools + (size_t)nwaves * kLogSlots * kPoolWords),
+                      A);
+    LogSink D{ queues + (size_t)wave * kLogQueue, nullptr, 0, 0, 0, false };
+    pool_run<kLogSlots>(K, A, pools + (size_t)wave * kLogSlots * kPoolWords, D, (int)(threadIdx.x & 63));
+}
+
+// Many models in one persistent launch.  A workgroup runs one model at a
+// time with the single-model kernel's pool: it starts with the model its
+// share of the launch falls to (shares by packets and lattice size, so that
+// the models run side by side and few workgroups change model), and when
+// that model has no packets left goes through the others in turn, helping
+// those that still have some.  Each packet keeps its own random stream, so
+// results equal those of the models' separate runs.  Every workgroup visits
+// every model at most once, which bounds the loop.
+__global__ void __launch_bounds__(256) batch_kernel(BatchArgs B)
+{
+    extern __shared__ float lds[];
+    __shared__ int s_left;
+    const int nwaves = (int)(blockDim.x >> 6), wave = (int)(threadIdx.x >> 6);
+    uint32_t *pools = reinterpret_cast<uint32_t *>(lds + (size_t)nwaves * JRing<kJDepth, false>::kFloats);
+    float *tab = reinterpret_cast<float *>(pools + (size_t)nwaves * kPoolSlots * kPoolWords);
+    // the last model whose share begins at or before this workgroup's
+    int first = 0;
+    {
+        const double at = ((double)blockIdx.x + 0.5) / (double)gridDim.x * B.share[B.models];
+        while (first + 1 < B.models && B.share[first + 1] <= at) ++first;
+    }
+    for (int t = 0; t < B.models; ++t) {
+        const int m = __builtin_amdgcn_readfirstlane((first + t) % B.models);
+        const Args K = { (uint64_t)(B.G + m), (uint64_t)(B.RA + m) };
+        __syncthreads();                       // the last model's tables and s_left are done with
+        if (threadIdx.x == 0) {
+            const RunArgs RA = scalar_copy<RunArgs>(K.r);
+            s_left = __hip_atomic_load(RA.next_packet, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
+                     (unsigned long long)RA.npackets;
+        }
+        __syncthreads();
+        if (!__builtin_amdgcn_readfirstlane(s_left)) continue;
+        Axes A;
+        stage_axes<false>(scalar_copy<Grid>(K.g), tab, A);
+        AddSink<kJDepth, false> D{ jq_at<kJDepth, false>(lds, wave) };
+        pool_run<kPoolSlots>(K, A, pools + (size_t)wave * kPoolSlots * kPoolWords, D, (int)(threadIdx.x & 63));
     }
 }
 
@@ -926,42 +1062,44 @@ __global__ void compact_kernel(const double *J3, const int *active, J3Shape js, 
 }  // namespace mcd
 
 // ---------------------------------------------------------------- launchers
+size_t mcd_pool_lds(const mcd::Grid &G, int threads)
+{
+    return sizeof(float) * ((size_t)(threads / 64) * (mcd::JRing<mcd::kJDepth, false>::kFloats +
+                                                      (size_t)mcd::kPoolSlots * mcd::kPoolWords) +
+                            mcd::lds_floats(G.nx, G.ny, G.nz));
+}
+
+size_t mcd_save_words(int blocks, int threads)
+{
+    return (size_t)blocks * (threads / 64) * mcd::Save<mcd::kLogSlots>::kWords;
+}
+
+bool mcd_pool_fits(const mcd::Grid &G)
+{
+    return G.nx <= 2047 && G.ny <= 2047 && G.nz <= 1023 && G.nbins <= 65535 &&
+           mcd::j3_size(G.js, G.nbins) <= 0xffffffffull;
+}
+
 hipError_t mcd_launch_batch(const mcd::BatchArgs &B, size_t lds_bytes, int blocks, hipStream_t s)
 {
-    hipLaunchKernelGGL(mcd::batch_kernel, dim3(blocks), dim3(64), lds_bytes, s, B);
+    hipLaunchKernelGGL(mcd::batch_kernel, dim3(blocks), dim3(256), lds_bytes, s, B);
     return hipGetLastError();
-}
-
-// dynamic LDS of a batch wavefront: its J queue, then the model's tables
-size_t mcd_lds_bytes(int nx, int ny, int nz, int nbins)
-{
-    return sizeof(float) * (mcd::JRing<mcd::kJDepthBatch>::kFloats + mcd::lds_floats(nx, ny, nz, nbins));
-}
-
-template <int D, int P>
-static size_t pool_lds(const mcd::Grid &G, int threads)
-{
-    return sizeof(float) * ((size_t)(threads / 64) * (mcd::JRing<D>::kFloats + (size_t)P * mcd::kPoolWords) +
-                            mcd::lds_floats(G.nx, G.ny, G.nz, G.nbins));
 }
 
 hipError_t mcd_launch_transport(const mcd::Grid &G, const mcd::RunArgs &RA, int blocks, int threads, int kernel,
                                 hipStream_t s)
 {
-    const size_t lds = sizeof(float) * ((size_t)(threads / 64) * mcd::JRing<mcd::kJDepth>::kFloats +
-                                        mcd::lds_floats(G.nx, G.ny, G.nz, G.nbins));
-    switch (kernel) {
-    case MCD_KERNEL_SPARE:
-        hipLaunchKernelGGL(mcd::transport_kernel<true>, dim3(blocks), dim3(threads), lds, s, G, RA);
-        break;
-    case MCD_KERNEL_POOL: {
-        const size_t pl = pool_lds<mcd::kJDepth, mcd::kPoolSlots>(G, threads);
-        hipLaunchKernelGGL((mcd::pool_kernel<mcd::kJDepth, mcd::kPoolSlots>), dim3(blocks), dim3(threads), pl, s,
-                           G, RA);
-        break;
-    }
-    default:
-        hipLaunchKernelGGL(mcd::transport_kernel<false>, dim3(blocks), dim3(threads), lds, s, G, RA);
+    if (kernel == MCD_KERNEL_LOG) {
+        const size_t lds = sizeof(float) * ((size_t)(threads / 64) * (mcd::kLogSlots * mcd::kPoolWords + 2 * mcd::kLogQueue) +
+                                            mcd::lds_floats(G.nx, G.ny, G.nz));
+        hipLaunchKernelGGL(mcd::log_kernel, dim3(blocks), dim3(threads), lds, s, mcd::LaunchArgs{ G, RA });
+    } else if (kernel == MCD_KERNEL_POOL && mcd_pool_fits(G)) {
+        hipLaunchKernelGGL(mcd::pool_kernel, dim3(blocks), dim3(threads), mcd_pool_lds(G, threads), s,
+                           mcd::LaunchArgs{ G, RA });
+    } else {
+        const size_t lds = sizeof(float) * ((size_t)(threads / 64) * mcd::JRing<mcd::kJDepth, true>::kFloats +
+                                            mcd::lds_floats(G.nx, G.ny, G.nz));
+        hipLaunchKernelGGL(mcd::transport_kernel, dim3(blocks), dim3(threads), lds, s, mcd::LaunchArgs{ G, RA });
     }
     return hipGetLastError();
 }
@@ -970,7 +1108,7 @@ hipError_t mcd_launch_replay(const mcd::Grid &G, int n, const float *pos, const 
                              const int *cell, int *cell_seq, float *ds_seq, int *seq_len,
                              int *status, int max_len, hipStream_t s)
 {
-    size_t lds = sizeof(float) * mcd::lds_floats(G.nx, G.ny, G.nz, 0);
+    size_t lds = sizeof(float) * mcd::lds_floats(G.nx, G.ny, G.nz);
     int threads = 256, blocks = (n + threads - 1) / threads;
     hipLaunchKernelGGL(mcd::walk_replay_kernel, dim3(blocks), dim3(threads), lds, s, G, n, pos,
                        dir, cell, cell_seq, ds_seq, seq_len, status, max_len);
