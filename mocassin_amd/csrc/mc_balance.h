@@ -42,7 +42,19 @@ struct Element {
 struct CelIon {
     int eidx, ion, nl, nt;
     double br, z, a_r[4], a_d[5];
-    int off_e, off_a, off_q, off_t, off_g;   // offsets: e, A(nl,nl), qom/y2(nt,npair), logT, g
+    int off_s, off_t;           // offsets: collision strengths [nt][pairs], logT
+};
+
+// Four model ions solved together (mc_cel.h), of similar size: the batches
+// hold the ions in descending order of levels.
+constexpr int kCelSlots = 4;
+constexpr int kMaxCelBatch = kMaxCel / kCelSlots;
+struct CelBatch {
+    int ion[kCelSlots];         // -1: none
+    int rows[kCelSlots];        // levels - 1
+    int base[kCelSlots];        // first pair of the slot within the batch
+    int most;                   // largest of rows
+    int npair, pair0;           // the batch's pairs in cel_pair, cel_de, cel_glo, cel_gup
 };
 
 struct Atomic {
@@ -55,11 +67,26 @@ struct Atomic {
     int dr_g[25];
     double ap_real[167][4];
     CelIon cel[kMaxCel];
+    int ncelb, cel_most, nterm; // batches, their largest pair count, radiating pairs
+    CelBatch celb[kMaxCelBatch];
+    int cel_place[kMaxCel];     // 4 * batch + slot of each model ion
     // device arrays
     const double *sigma;        // [nch][nbins]
     const double *nu;           // [nbins]
     const double *cR, *cH;      // [nch][nbins] rate and heating coefficients per bin
-    const double *cel_e, *cel_a, *cel_q, *cel_y2, *cel_t, *cel_g;
+    const double *cel_t;        // logT
+    const double2 *cel_s;       // per ion [nt][pairs]: collision strength, its spline curvature
+    // per pair (lower, upper) of a batch: (e(lo) - e(up)) hc/k, the
+    // statistical weights, slot + 4 * pair of the ion
+    const double *cel_de, *cel_glo, *cel_gup;
+    const int *cel_pair;
+    // per batch, as its lanes read them (lane = 16 slot + level - 2, zero
+    // where there is no such entry): A between level j and the lane's,
+    // [kMaxLev + 1][64]; A(up, lo) (e(up) - e(lo)) of the lane's upper level,
+    // [kMaxLev][64] by lower level; the number of the radiating pair (A not
+    // 0; forLines' order over all ions) or -1, likewise
+    const double *cel_at, *cel_ae;
+    const int *cel_term;
 };
 
 // Grains of one dust chemistry for the grain charge, photoelectric heating
@@ -105,6 +132,7 @@ struct CellArgs {
     // pointer, with the frequency-bin count for the launch's LDS size
     const Grains *grains;
     int grains_nb;
+    int ncel, cel_most;         // of the atomic data: the solves' LDS
     // nullable: block b balances cell order[b] (a permutation of 1..ncells),
     // else cell b + 1; results do not depend on the order
     const int *order;
@@ -127,6 +155,7 @@ struct LineArgs {
     const float *dfac;              // per-axis getVolume widths / 1e15, axes x, y, z concatenated
     double *part;
     int ldp;
+    int cel_most;                   // of the atomic data: the solves' LDS
 };
 
 // Host-built tables: `A` with its device pointers unset, and the flat arrays
@@ -134,7 +163,8 @@ struct LineArgs {
 // index e.
 struct Prepared {
     Atomic A{};
-    std::vector<double> sigma, nu, cR, cH, cel_e, cel_a, cel_q, cel_y2, cel_t, cel_g;
+    std::vector<double> sigma, nu, cR, cH, cel_s, cel_t, cel_de, cel_glo, cel_gup, cel_at, cel_ae;
+    std::vector<int> cel_pair, cel_term;
     std::vector<int> eidx_xref;
 };
 

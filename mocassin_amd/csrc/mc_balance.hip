@@ -7,9 +7,8 @@
 //     bins, wave reductions per channel (update_mod.f90:184-269, 1146-1234);
 //   * recombination fits, charge exchange, ion ratios: lanes over the
 //     (elem, ion) channels (calcAlpha, radRecFit, dielectronic, ionBalance);
-//   * CEL cooling: the model ions one after another, each n-level system
-//     built and eliminated cooperatively (rows and pivot updates across
-//     lanes; equilibrium/luSlv of emission_mod.f90:1913-2190);
+//   * CEL cooling: the n-level systems of four model ions at a time, one in
+//     each row of 16 lanes (mc_cel.h);
 //   * the bracketed false-position T iteration and the fixed-point ion
 //     iteration run uniformly on the wavefront (iterateT, ionBalance).
 // The collision-strength spline second derivatives depend only on the
@@ -33,14 +32,26 @@ constexpr int W = 64;
 struct Lds {
     double Te, Ne, Hden;
     double ion[kMaxElem][kMaxStage];
-    double nPhot[kMaxCh], heatNu[kMaxCh], alpha[kMaxCh], ratio[kMaxCh], chexv[kMaxCh];
-    double diO[kMaxStage];
-    double red[W];
-    double x[kMaxLev + 1][kMaxLev + 1];
-    double q[kMaxLev + 1][kMaxLev + 1];
-    double y[kMaxLev + 1];
-    double alev[kMaxLev + 1];
+    double nPhot[kMaxCh], heatNu[kMaxCh];
+    double red[2];
 };
+
+// What follows in dynamic LDS serves the ion fixed point first and the level
+// solves after it.
+struct IonLds {
+    double alpha[kMaxCh], ratio[kMaxCh], chexv[kMaxCh];
+    double diO[kMaxStage];
+};
+// the solves' block: records [ncel], cooling [ncel], rates [most]
+__host__ __device__ inline size_t cel_bytes(int ncel, int most)
+{
+    return ((size_t)ncel * (sizeof(CelRec) + sizeof(double)) + 15) / 16 * 16 + (size_t)most * sizeof(double2);
+}
+__host__ __device__ inline size_t shared_bytes(int ncel, int most)
+{
+    const size_t cel = cel_bytes(ncel, most);
+    return ((cel > sizeof(IonLds) ? cel : sizeof(IonLds)) + 15) / 16 * 16;
+}
 
 __device__ __forceinline__ double wave_sum(double v)
 {
@@ -84,46 +95,54 @@ __device__ double di_rec(const Atomic &A, int ndr, const int *dr, int ap, double
     return v;
 }
 
-// CEL cooling of one model ion [erg/s per H], levels 1..10 (forLines +
-// equilibrium + the cooling sum of thermBalance)
-__device__ __forceinline__ double cel_cool(const Atomic &A, const CelIon &ci, Lds &S, int lane, double Te)
-{
-    const int nl = ci.nl;
-    const double *E = A.cel_e + ci.off_e;
-    const double *Aa = A.cel_a + ci.off_a;
-    const double xi = S.ion[ci.eidx][ci.ion];
-    const double up = (ci.ion < A.nstages) ? S.ion[ci.eidx][ci.ion + 1] / xi : 0.0;
-    if (up != up) return 0.0;
-    cel_levels(A, ci, S, lane, Te, S.Ne, up);
-    double cool = 0.0;
-    if (lane == 0) {
-        double sumN = 0.0;
-        for (int i = 1; i <= nl; ++i) sumN = sumN + S.y[i];
-        const double s1 = A.el[ci.eidx].abun, s2 = xi;
-        const double kE = 1.9865e-16;
-        for (int i = 1; i <= 10 && i <= nl - 1; ++i)
-            for (int j = i + 1; j <= 10 && j <= nl; ++j) {
-                const double a = Aa[(j - 1) + nl * (i - 1)];
-                if (a != 0.0) {
-                    const double Eji = E[j - 1] - E[i - 1];
-                    cool = cool + a * Eji * (S.y[j] / sumN) * s1 * s2 * kE;
-                }
-            }
-    }
-    __syncthreads();
-    return cool;   // valid on lane 0
-}
-
 // total cooling at temperature T for the cell's current ionisation and Ne
 // (thermBalance, update_mod.f90:933-1113: H and He free-free and
-// recombination fits, H collisional excitation, CEL lines); valid on lane 0
-__device__ __forceinline__ double cooling(const Atomic &A, Lds &S, int lane, double T)
+// recombination fits, H collisional excitation, CEL lines); valid on lane 0.
+// dyn: the solves' block.
+__device__ __forceinline__ double cooling(const Atomic &A, Lds &S, void *dyn, int lane, double T)
 {
-    double cool = 0.0;
-    for (int k = 0; k < A.ncel; ++k) {
-        double cc = cel_cool(A, A.cel[k], S, lane, T);
-        cool = cool + cc;
+    CelRec *rec = static_cast<CelRec *>(dyn);
+    double *ions = reinterpret_cast<double *>(rec + A.ncel);
+    double2 *rate = reinterpret_cast<double2 *>(static_cast<char *>(dyn) + cel_bytes(A.ncel, 0));
+    const double sqrTe = sqrt(T), log10Te = log10(T);
+    for (int k = lane; k < A.ncel; k += W) {
+        const CelIon &ci = A.cel[k];
+        const double xi = S.ion[ci.eidx][ci.ion];
+        const double up = (ci.ion < A.nstages) ? S.ion[ci.eidx][ci.ion + 1] / xi : 0.0;
+        rec[A.cel_place[k]] = cel_record(A, ci, T, log10Te, up, A.el[ci.eidx].abun, xi);
     }
+    __syncthreads();
+    // CEL cooling of each model ion [erg/s per H] from its levels 1..10
+    // (forLines, equilibrium and the cooling sum of thermBalance), its terms
+    // added in the reference's order
+    for (int b = 0; b < A.ncelb; ++b) {
+        const CelBatch &B = A.celb[b];
+        const CelRec *R = rec + kCelSlots * b;
+        const CelLevels L = cel_levels(A, b, R, rate, lane, T, sqrTe, S.Ne);
+        const int g = lane >> 4, r = lane & 15, n = B.most;
+        const bool mine = r < B.rows[g];
+        const double part = L.y / L.sum, s1 = R[mine ? g : 0].ab, s2 = R[mine ? g : 0].x;
+        const double kE = 1.9865e-16;
+        const double *ae = A.cel_ae + (size_t)b * kMaxLev * 64 + lane;
+        const int *term = A.cel_term + (size_t)b * kMaxLev * 64 + lane;
+        double cool = 0.0;
+        static_for<0, 9>([&](auto Lo) {
+            constexpr int lo = decltype(Lo)::value;          // lower level lo + 1, upper r + 2 <= 10
+            if (lo < n) {
+                const double f = ae[64 * lo] * part * s1 * s2 * kE;
+                const double t = term[64 * lo] >= 0 ? f : 0.0;
+                static_for<lo, 9>([&](auto Up) {
+                    constexpr int up = decltype(Up)::value;
+                    cool = cool + row_lane<up>(t);
+                });
+            }
+        });
+        if (r == 0 && mine) ions[B.ion[g]] = R[g].skip ? 0.0 : cool;
+    }
+    __syncthreads();
+    double cool = 0.0;
+    for (int k = 0; k < A.ncel; ++k) cool = cool + ions[k];
+    __syncthreads();
     if (lane != 0) return 0.0;
     const double Ne = S.Ne, kB = 1.380658e-16, hcRyd = 2.1799153e-11;
     const double lg = log10(T), Te4 = T / 1.e4;
@@ -347,11 +366,16 @@ __device__ void grain_terms(const Atomic &A, const Grains &G, const double *pf, 
     __syncthreads();
 }
 
+// Registers for three wavefronts a SIMD without grains (6.5 ms against 7.6
+// for four on the 45^3 octant: the level solves' rows spill), for four with
+// grains (38 against 42 ms, dust and gas 60^3: the grain loops want the
+// wavefronts).
 template <bool PE>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) balance_kernel(const Atomic *__restrict__ Ap, CellArgs a)
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PE ? 4 : 3))) balance_kernel(const Atomic *__restrict__ Ap, CellArgs a)
 {
     __shared__ Lds S;
-    extern __shared__ double dyn[];           // grain variant: photon flux per bin, then GrainLds
+    // ion fixed point or level solves; grain variant: photon flux per bin, GrainLds
+    extern __shared__ __align__(16) double dyn[];
     const Atomic &A = *Ap;
     const int lane = threadIdx.x;
     const int cell = a.order ? a.order[blockIdx.x] : (int)blockIdx.x + 1;
@@ -375,8 +399,9 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) ba
         S.nPhot[k] = 1.e-20 + a.Rint[(size_t)cell * nch + k];
         S.heatNu[k] = a.Hint[(size_t)cell * nch + k];
     }
-    double *pf = dyn;
-    GrainLds &GL = *reinterpret_cast<GrainLds *>(dyn + A.nbins);
+    IonLds &F = *reinterpret_cast<IonLds *>(dyn);
+    double *pf = reinterpret_cast<double *>(reinterpret_cast<char *>(dyn) + shared_bytes(A.ncel, A.cel_most));
+    GrainLds &GL = *reinterpret_cast<GrainLds *>(pf + A.nbins);
     if (PE) {
         // the cell's photon flux J/(h c Ryd nu) (getGrainEmission, setPhotoelHeatCool)
         const Grains &G = *a.grains;
@@ -401,23 +426,23 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) ba
             const double Te = S.Te;
             // calcAlpha: radiative + dielectronic (oxygen rows fill empty entries)
             for (int i = 1 + lane; i < ns; i += W)
-                S.diO[i] = di_rec(A, A.odr_n[i], A.odr[i], A.oap[i], Te);
+                F.diO[i] = di_rec(A, A.odr_n[i], A.odr[i], A.oap[i], Te);
             __syncthreads();
             for (int k = lane; k < nch; k += W) {
                 const Channel &c = A.ch[k];
                 double al = rad_rec(c, Te);
                 if (c.elem >= 3) {
                     double d = di_rec(A, c.ndr, c.dr, c.ap, Te);
-                    if (d == 0.0) d = S.diO[c.ion];
+                    if (d == 0.0) d = F.diO[c.ion];
                     al = al + d;
                 }
-                S.alpha[k] = al;
+                F.alpha[k] = al;
                 // charge-exchange rate coefficient (ionBalance, 1448-1455)
                 const double t4 = Te / 10000.;
                 double cx = c.chex[0] * pow(t4, c.chex[1]) * (1. + c.chex[2] * exp(c.chex[3] * t4));
                 if (cx < 0.) cx = 0.;
                 if (Te < 6000. || Te > 5.e4) cx = 0.;
-                S.chexv[k] = cx;
+                F.chexv[k] = cx;
             }
             __syncthreads();
             // ionBalance fixed point (1320-1622)
@@ -435,16 +460,16 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) ba
                     }
                     double revRate = 0.0;
                     if (c.dEk > 1.0)
-                        revRate = S.chexv[k] * (1. - xH0) * S.Hden * 2. * exp(-c.dEk / Te) / c.g0g1;
-                    S.ratio[k] = (S.nPhot[k] + collIon + revRate) /
-                                 (S.Ne * S.alpha[k] + S.chexv[k] * S.Hden * xH0);
+                        revRate = F.chexv[k] * (1. - xH0) * S.Hden * 2. * exp(-c.dEk / Te) / c.g0g1;
+                    F.ratio[k] = (S.nPhot[k] + collIon + revRate) /
+                                 (S.Ne * F.alpha[k] + F.chexv[k] * S.Hden * xH0);
                 }
                 __syncthreads();
                 if (lane < nE) {
                     const Element &e = A.el[lane];
                     double prod[kMaxStage];
                     double den = 1.0, p = 1.0;
-                    for (int i = 0; i < e.nch; ++i) { p = 1.0; for (int q = 0; q <= i; ++q) p = p * S.ratio[e.ch0 + q]; prod[i] = p; }
+                    for (int i = 0; i < e.nch; ++i) { p = 1.0; for (int q = 0; q <= i; ++q) p = p * F.ratio[e.ch0 + q]; prod[i] = p; }
                     for (int i = 0; i < e.nch; ++i) den = den + prod[i];
                     for (int st = 1; st <= e.nst; ++st) {
                         double v = (st == 1) ? 1.0 / den : prod[st - 2] / den;
@@ -474,7 +499,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) ba
             }
             if (PE) grain_terms(A, *a.grains, pf, GL, S, lane, cell);
             // thermBalance (933-1258)
-            double cool = cooling(A, S, lane, S.Te), heat = 0.0;
+            double cool = cooling(A, S, dyn, lane, S.Te), heat = 0.0;
             if (lane == 0) {
                 for (int k = 0; k < nch; ++k) {
                     const Channel &c = A.ch[k];
@@ -729,20 +754,14 @@ __global__ void warm_kernel(const Atomic *__restrict__ Ap, CellArgs a, const flo
 }
 
 // ---- analytic line luminosities (outputGas, output_mod.f90:302-520) -----
-// One wavefront per block of consecutive cells.  Per model ion (outer loop,
-// so that a lane's accumulators stay in registers): every cell's level
-// populations (cel_levels), then lanes over the 17 x 17 (upper, lower)
-// entries add forLines' emissivity times Hden * getVolume.  Each block writes
-// its sums to its own row of `part`; lines_reduce_kernel adds the rows in
-// block order, so the result does not depend on scheduling.
-struct LineLds {
-    double x[kMaxLev + 1][kMaxLev + 1];
-    double q[kMaxLev + 1][kMaxLev + 1];
-    double y[kMaxLev + 1];
-    double alev[kMaxLev + 1];
-};
-
-constexpr int kLineR = (kLineEnt + W - 1) / W;       // entries per lane
+// One wavefront per block of consecutive cells.  Per batch of four model
+// ions (outer loop, so that a lane's sums stay in registers: its upper level,
+// 16 lower ones): every cell's level populations (mc_cel.h), then forLines'
+// emissivity times Hden * getVolume.  The records of kLineCells cells are made
+// together, one lane each.  Each block writes its sums to its own row of
+// `part`; lines_reduce_kernel adds the rows in block order, so the result
+// does not depend on scheduling.
+constexpr int kLineCells = W / kCelSlots;
 
 __device__ __forceinline__ float line_volume(const LineArgs &a, int cell)
 {
@@ -755,7 +774,10 @@ __device__ __forceinline__ float line_volume(const LineArgs &a, int cell)
 
 __global__ void __launch_bounds__(64) lines_kernel(const Atomic *__restrict__ Ap, LineArgs a)
 {
-    __shared__ LineLds S;
+    __shared__ CelRec recs[W];                   // [cell][slot]
+    __shared__ float hds[kLineCells], dvs[kLineCells], tes[kLineCells], nes[kLineCells];
+    __shared__ double hsum;
+    extern __shared__ __align__(16) double2 rate[];
     const Atomic &A = *Ap;
     const int lane = threadIdx.x;
     const int nE = A.nE, ns = A.nstages;
@@ -764,46 +786,66 @@ __global__ void __launch_bounds__(64) lines_kernel(const Atomic *__restrict__ Ap
     double *out = a.part + (size_t)blockIdx.x * a.ldp;
     // forLines' 1.9865e9 is a REAL literal
     const double kL = (double)1.9865e9f;
-    for (int k = 0; k < A.ncel; ++k) {
-        const CelIon &ci = A.cel[k];
-        const int nl = ci.nl;
-        const double *E = A.cel_e + ci.off_e;
-        const double *Aa = A.cel_a + ci.off_a;
-        const double abun = (double)(float)A.el[ci.eidx].abun;
-        double acc[kLineR];
-        for (int r = 0; r < kLineR; ++r) acc[r] = 0.0;
-        for (int cell = c0; cell <= c1; ++cell) {
-            if (a.black && (a.black[cell] & a.black_mask)) continue;
-            // the state as the host grid stores it (REAL)
-            const float te = (float)a.Te[cell], ne = (float)a.Ne[cell], hd = (float)a.Hden[cell];
-            const double *ion = a.ion + ((size_t)cell * nE + ci.eidx) * (ns + 1);
-            const float x = (float)ion[ci.ion];
-            const float up = (ci.ion < ns) ? (float)ion[ci.ion + 1] / x : 0.f;
-            if (up != up) continue;               // equilibrium's NaN test: no emission
-            const float dv = line_volume(a, cell);
-            cel_levels(A, ci, S, lane, (double)te, (double)ne, (double)up);
-            double sumN = 0.0;
-            for (int i = 1; i <= nl; ++i) sumN = sumN + S.y[i];
-            for (int r = 0; r < kLineR; ++r) {
-                const int e = lane + W * r;
-                const int hi = e / kMaxLev + 1, lo = e % kMaxLev + 1;
-                if (e < kLineEnt && lo < hi && hi <= nl) {
-                    const double av = Aa[(hi - 1) + nl * (lo - 1)];
-                    if (av != 0.0) {
-                        const double Eji = E[hi - 1] - E[lo - 1];
-                        double f = av * Eji * (S.y[hi] / sumN);
-                        f = f * abun * (double)x;
-                        f = f * kL;
-                        acc[r] = acc[r] + f * (double)hd * (double)dv;
+    const int g = lane >> 4, r = lane & 15;
+    for (int b = 0; b < A.ncelb; ++b) {
+        const CelBatch &B = A.celb[b];
+        const bool mine = r < B.rows[g];
+        const double *ae = A.cel_ae + (size_t)b * kMaxLev * 64 + lane;
+        const int *term = A.cel_term + (size_t)b * kMaxLev * 64 + lane;
+        double acc[16];
+        for (int l = 0; l < 16; ++l) acc[l] = 0.0;
+        for (int cc = c0; cc <= c1; cc += kLineCells) {
+            __syncthreads();
+            {
+                const int cell = cc + lane / kCelSlots, k = B.ion[lane % kCelSlots];
+                if (cell <= c1) {
+                    // the state as the host grid stores it (REAL)
+                    const float te = (float)a.Te[cell];
+                    if (k >= 0) {
+                        const CelIon &ci = A.cel[k];
+                        const double *ion = a.ion + ((size_t)cell * nE + ci.eidx) * (ns + 1);
+                        const float x = (float)ion[ci.ion];
+                        const float up = (ci.ion < ns) ? (float)ion[ci.ion + 1] / x : 0.f;
+                        recs[lane] = cel_record(A, ci, (double)te, log10((double)te), (double)up,
+                                                (double)(float)A.el[ci.eidx].abun, (double)x);
+                    }
+                    if (lane % kCelSlots == 0) {
+                        const int u = lane / kCelSlots;
+                        tes[u] = te;
+                        nes[u] = (float)a.Ne[cell];
+                        hds[u] = (float)a.Hden[cell];
+                        dvs[u] = line_volume(a, cell);
                     }
                 }
             }
-            __syncthreads();                      // S is rewritten by the next cell
+            __syncthreads();
+            for (int cell = cc; cell <= min(c1, cc + kLineCells - 1); ++cell) {
+                if (a.black && (a.black[cell] & a.black_mask)) continue;
+                const int u = cell - cc;
+                const CelRec *R = recs + kCelSlots * u;
+                const double Te = (double)tes[u], hd = (double)hds[u], dv = (double)dvs[u];
+                const CelLevels L = cel_levels(A, b, R, rate, lane, Te, sqrt(Te), (double)nes[u]);
+                const double part = L.y / L.sum;
+                const double abun = R[mine ? g : 0].ab, x = R[mine ? g : 0].x;
+                const bool on = mine && !R[mine ? g : 0].skip;
+                static_for<0, 16>([&](auto Lo) {
+                    constexpr int lo = decltype(Lo)::value;
+                    if (lo < B.most) {
+                        double f = ae[64 * lo] * part;
+                        f = f * abun * x;
+                        f = f * kL;
+                        const double t = acc[lo] + f * hd * dv;
+                        acc[lo] = on && term[64 * lo] >= 0 ? t : acc[lo];
+                    }
+                });
+            }
         }
-        for (int r = 0; r < kLineR; ++r) {
-            const int e = lane + W * r;
-            if (e < kLineEnt) out[(size_t)k * kLineEnt + e] = acc[r];
-        }
+        for (int s = 0; s < kCelSlots; ++s)
+            for (int e = lane; e < kLineEnt; e += W)
+                if (B.ion[s] >= 0 && (e % kMaxLev >= e / kMaxLev || e / kMaxLev > B.rows[s]))
+                    out[(size_t)B.ion[s] * kLineEnt + e] = 0.0;
+        for (int lo = 0; lo < 16; ++lo)
+            if (mine && lo <= r) out[(size_t)B.ion[g] * kLineEnt + (r + 1) * kMaxLev + lo] = acc[lo];
     }
     // RecLinesEmission's Hbeta (output_mod.f90:2065-2079), HIRecLines(4,2) =
     // (fh/hb) * Hbeta = Hbeta, times Hden * dV
@@ -818,13 +860,13 @@ __global__ void __launch_bounds__(64) lines_kernel(const Atomic *__restrict__ Ap
         hb = hb + (double)h * (double)hd * (double)line_volume(a, cell);
     }
     // lanes in order: a fixed summation order
-    if (lane == 0) S.y[0] = 0.0;
+    if (lane == 0) hsum = 0.0;
     __syncthreads();
     for (int l = 0; l < W; ++l) {
-        if (lane == l) S.y[0] = S.y[0] + hb;
+        if (lane == l) hsum = hsum + hb;
         __syncthreads();
     }
-    if (lane == 0) out[(size_t)A.ncel * kLineEnt] = S.y[0];
+    if (lane == 0) out[(size_t)A.ncel * kLineEnt] = hsum;
 }
 
 // out[t] = sum over blocks b (in order) of part[b][t]; four wavefronts per
@@ -848,12 +890,13 @@ __global__ void __launch_bounds__(256) lines_reduce_kernel(const double *__restr
 hipError_t mcb_launch_balance(const mcb::Atomic *dA, const mcb::CellArgs &a, hipStream_t s)
 {
     if (a.ncells <= 0) return hipSuccess;
+    const size_t cel = mcb::shared_bytes(a.ncel, a.cel_most);
     if (a.grains) {
         // the caller passes the frequency-bin count through grains_nb
-        const size_t lds = (size_t)a.grains_nb * sizeof(double) + sizeof(mcb::GrainLds);
+        const size_t lds = cel + (size_t)a.grains_nb * sizeof(double) + sizeof(mcb::GrainLds);
         hipLaunchKernelGGL(mcb::balance_kernel<true>, dim3(a.ncells), dim3(64), lds, s, dA, a);
     } else {
-        hipLaunchKernelGGL(mcb::balance_kernel<false>, dim3(a.ncells), dim3(64), 0, s, dA, a);
+        hipLaunchKernelGGL(mcb::balance_kernel<false>, dim3(a.ncells), dim3(64), cel, s, dA, a);
     }
     return hipGetLastError();
 }
@@ -879,7 +922,7 @@ hipError_t mcb_launch_lines(const mcb::Atomic *dA, const mcb::LineArgs &a, int n
                             hipStream_t s)
 {
     if (nblk <= 0) return hipSuccess;
-    hipLaunchKernelGGL(mcb::lines_kernel, dim3(nblk), dim3(64), 0, s, dA, a);
+    hipLaunchKernelGGL(mcb::lines_kernel, dim3(nblk), dim3(64), a.cel_most * sizeof(double2), s, dA, a);
     const int n = ncel * mcb::kLineEnt + 1;
     hipLaunchKernelGGL(mcb::lines_reduce_kernel, dim3((n + 63) / 64), dim3(256), 0, s, a.part, a.ldp, nblk, n, out);
     return hipGetLastError();
@@ -977,6 +1020,57 @@ int dr_rows(const mc_atomic *in, int ns, int z, int ion, int *rows, int *ap, cha
     return nr;
 }
 
+// The batches of model ions and the tables their lanes read (mc_cel.h) from
+// each ion's levels (energies, then A(up, lo) at up + nl lo) and weights.
+void cel_batches(Prepared &P, const std::vector<const double *> &lev, const std::vector<const float *> &wgt,
+                 const std::vector<int> &term0)
+{
+    Atomic &A = P.A;
+    std::vector<int> order(A.ncel);
+    for (int k = 0; k < A.ncel; ++k) order[k] = k;
+    std::stable_sort(order.begin(), order.end(), [&](int u, int v) { return A.cel[u].nl > A.cel[v].nl; });
+    A.ncelb = (A.ncel + kCelSlots - 1) / kCelSlots;
+    A.cel_most = 0;
+    P.cel_at.assign((size_t)A.ncelb * (kMaxLev + 1) * 64, 0.0);
+    P.cel_ae.assign((size_t)A.ncelb * kMaxLev * 64, 0.0);
+    P.cel_term.assign((size_t)A.ncelb * kMaxLev * 64, -1);
+    for (int b = 0; b < A.ncelb; ++b) {
+        CelBatch &B = A.celb[b];
+        B = CelBatch{};
+        B.pair0 = (int)P.cel_pair.size();
+        double *at = P.cel_at.data() + (size_t)b * (kMaxLev + 1) * 64;
+        double *ae = P.cel_ae.data() + (size_t)b * kMaxLev * 64;
+        int *term = P.cel_term.data() + (size_t)b * kMaxLev * 64;
+        for (int s = 0; s < kCelSlots; ++s) {
+            B.ion[s] = -1;
+            if (kCelSlots * b + s >= A.ncel) continue;
+            const int k = order[kCelSlots * b + s], nl = A.cel[k].nl;
+            const double *E = lev[k], *a = E + nl;
+            A.cel_place[k] = kCelSlots * b + s;
+            B.ion[s] = k;
+            B.rows[s] = nl - 1;
+            B.base[s] = B.npair;
+            B.most = std::max(B.most, nl - 1);
+            int t = term0[k];
+            for (int lo = 0, p = 0; lo < nl - 1; ++lo)
+                for (int up = lo + 1; up < nl; ++up, ++p) {
+                    const double av = a[up + nl * lo];
+                    P.cel_pair.push_back(s + 4 * p);
+                    P.cel_de.push_back((E[lo] - E[up]) * 1.4388463);
+                    P.cel_glo.push_back((double)wgt[k][lo]);
+                    P.cel_gup.push_back((double)wgt[k][up]);
+                    // level L (from 0) of slot s is lane 16 s + L - 1
+                    at[64 * (lo + 1) + 16 * s + up - 1] = av;
+                    if (lo > 0) at[64 * (up + 1) + 16 * s + lo - 1] = av;
+                    ae[64 * lo + 16 * s + up - 1] = av * (E[up] - E[lo]);
+                    if (av != 0.0) term[64 * lo + 16 * s + up - 1] = t++;
+                }
+            B.npair += nl * (nl - 1) / 2;
+        }
+        A.cel_most = std::max(A.cel_most, B.npair);
+    }
+}
+
 }  // namespace
 
 int prepare(const mc_atomic *in, int nb, const float *nuArray, Prepared &P, char *e, size_t n)
@@ -995,6 +1089,10 @@ int prepare(const mc_atomic *in, int nb, const float *nuArray, Prepared &P, char
     A.nbins = nb;
     A.nstages = ns;
     A.XHILimit = in->XHILimit;
+    for (auto *v : { &P.sigma, &P.cR, &P.cH, &P.cel_s, &P.cel_t, &P.cel_de, &P.cel_glo, &P.cel_gup, &P.cel_at,
+                     &P.cel_ae })
+        v->clear();
+    P.cel_pair.clear();
     P.nu.assign(nuArray, nuArray + nb);
     // elements in atomic-number order, their channels ion = 1..min(z, ns-1)
     int eidx_of_z[31];
@@ -1092,6 +1190,10 @@ int prepare(const mc_atomic *in, int nb, const float *nuArray, Prepared &P, char
     if (in->ncel < 0 || in->ncel > kMaxCel) return err(e, n, MC_EUNSUP, "more than %d CEL ions", kMaxCel);
     A.ncel = in->ncel;
     size_t od = 0, of = 0;
+    std::vector<const double *> lev(in->ncel);
+    std::vector<const float *> wgt(in->ncel);
+    std::vector<int> term0(in->ncel);             // the ion's first radiating pair
+    int nterm = 0;
     for (int k = 0; k < in->ncel; ++k) {
         const int32_t *m = in->cel_meta + 6 * k;
         const int z = m[0], ion = m[1], nl = m[4], nt = m[5];
@@ -1110,32 +1212,38 @@ int prepare(const mc_atomic *in, int nb, const float *nuArray, Prepared &P, char
         ci.z = (double)gv[nl + 1];
         for (int i = 0; i < 4; ++i) ci.a_r[i] = (double)gv[nl + 2 + i];
         for (int i = 0; i < 5; ++i) ci.a_d[i] = (double)gv[nl + 6 + i];
-        ci.off_e = (int)P.cel_e.size();
-        ci.off_a = (int)P.cel_a.size();
-        ci.off_q = (int)P.cel_q.size();
+        ci.off_s = (int)(P.cel_s.size() / 2);
         ci.off_t = (int)P.cel_t.size();
-        ci.off_g = (int)P.cel_g.size();
-        P.cel_e.insert(P.cel_e.end(), ev, ev + nl);
-        P.cel_a.insert(P.cel_a.end(), av, av + (size_t)nl * nl);
+        lev[k] = ev;
+        wgt[k] = gv;
+        term0[k] = nterm;
+        for (int lo = 0; lo < nl; ++lo)
+            for (int up = lo + 1; up < nl; ++up) nterm += av[up + nl * lo] != 0.0;
         std::vector<double> xa(nt);
         for (int t = 0; t < nt; ++t) xa[t] = (double)lt[t];
         for (int t = 1; t < nt; ++t)
             if (!(xa[t] > xa[t - 1])) return err(e, n, MC_ETABLE, "CEL ion %d: log T not increasing", k);
         P.cel_t.insert(P.cel_t.end(), xa.begin(), xa.end());
-        for (int i = 0; i < nl; ++i) P.cel_g.push_back((double)gv[i]);
         // collision strengths of each pair (lo < up) and their spline curvature
         double qq[kMaxTemp], y2[kMaxTemp];
-        for (int lo = 1; lo <= nl - 1; ++lo)
-            for (int up = lo + 1; up <= nl; ++up) {
+        const int npair = nl * (nl - 1) / 2;
+        P.cel_s.resize(P.cel_s.size() + (size_t)2 * nt * npair);
+        double *s2 = P.cel_s.data() + 2 * (size_t)ci.off_s;
+        for (int lo = 1, p = 0; lo <= nl - 1; ++lo)
+            for (int up = lo + 1; up <= nl; ++up, ++p) {
                 for (int t = 0; t < nt; ++t) qq[t] = qv[t + (size_t)nt * ((lo - 1) + (size_t)nl * (up - 1))];
                 if (nt >= 3) spline_nat(xa.data(), qq, nt, y2);
                 else for (int t = 0; t < nt; ++t) y2[t] = 0.0;
-                P.cel_q.insert(P.cel_q.end(), qq, qq + nt);
-                P.cel_y2.insert(P.cel_y2.end(), y2, y2 + nt);
+                for (int t = 0; t < nt; ++t) {
+                    s2[2 * ((size_t)t * npair + p)] = qq[t];
+                    s2[2 * ((size_t)t * npair + p) + 1] = y2[t];
+                }
             }
         od += (size_t)nl + (size_t)nl * nl + (size_t)nt * nl * nl;
         of += (size_t)nt + nl + 2 + 4 + 5;
     }
+    A.nterm = nterm;
+    cel_batches(P, lev, wgt, term0);
     return MC_OK;
 }
 

@@ -589,24 +589,29 @@ extern "C" int mc_balance_setup(mc_ctx *c, const mc_atomic *at)
     if (rc) return rc;
     if (at->nElemUsed != P.A.nE) return fail(c, MC_ETABLE, "nElemUsed %d but %d elements on", at->nElemUsed, P.A.nE);
     // one device block for every table, in this order
-    const std::vector<double> *parts[] = { &P.sigma, &P.nu, &P.cel_e, &P.cel_a, &P.cel_q,
-                                           &P.cel_y2, &P.cel_t, &P.cel_g, &P.cR, &P.cH };
+    // (cel_s first: its rows are read 16 bytes at a time)
+    const std::vector<double> *parts[] = { &P.cel_s, &P.sigma, &P.nu, &P.cR, &P.cH, &P.cel_t, &P.cel_de, &P.cel_glo,
+                                           &P.cel_gup, &P.cel_at, &P.cel_ae };
+    const std::vector<int> *ints[] = { &P.cel_pair, &P.cel_term };
     size_t tot = 0;
     for (auto *v : parts) tot += v->size();
+    for (auto *v : ints) tot += (v->size() + 1) / 2;
     if (c->d_bal_tab) { (void)hipFree(c->d_bal_tab); c->d_bal_tab = nullptr; }
     HIPCHK(c, dalloc(&c->d_bal_tab, tot));
-    const double *ptr[10];
+    const double *ptr[13];
     size_t off = 0;
-    for (int k = 0; k < 10; ++k) {
+    for (int k = 0; k < 13; ++k) {
         ptr[k] = c->d_bal_tab + off;
-        if (!parts[k]->empty())
-            HIPCHK(c, copy_on(c->stream, c->d_bal_tab + off, parts[k]->data(), parts[k]->size() * sizeof(double),
-                                hipMemcpyHostToDevice));
-        off += parts[k]->size();
+        const void *from = k < 11 ? (const void *)parts[k]->data() : (const void *)ints[k - 11]->data();
+        const size_t bytes = k < 11 ? parts[k]->size() * sizeof(double) : ints[k - 11]->size() * sizeof(int);
+        if (bytes) HIPCHK(c, copy_on(c->stream, c->d_bal_tab + off, from, bytes, hipMemcpyHostToDevice));
+        off += (bytes + 7) / 8;
     }
     mcb::Atomic A = P.A;
-    A.sigma = ptr[0]; A.nu = ptr[1]; A.cel_e = ptr[2]; A.cel_a = ptr[3]; A.cel_q = ptr[4];
-    A.cel_y2 = ptr[5]; A.cel_t = ptr[6]; A.cel_g = ptr[7]; A.cR = ptr[8]; A.cH = ptr[9];
+    A.cel_s = (const double2 *)ptr[0];
+    A.sigma = ptr[1]; A.nu = ptr[2]; A.cR = ptr[3]; A.cH = ptr[4]; A.cel_t = ptr[5]; A.cel_de = ptr[6];
+    A.cel_glo = ptr[7]; A.cel_gup = ptr[8]; A.cel_at = ptr[9]; A.cel_ae = ptr[10];
+    A.cel_pair = (const int *)ptr[11]; A.cel_term = (const int *)ptr[12];
     if (!c->d_atomic) HIPCHK(c, dalloc(&c->d_atomic, 1));
     HIPCHK(c, copy_on(c->stream, c->d_atomic, &A, sizeof A, hipMemcpyHostToDevice));
     const size_t nc1 = (size_t)c->G.nCells + 1;
@@ -662,6 +667,8 @@ static mcb::CellArgs cell_args(mc_ctx *c, double jscale)
     a.solver = MC_SOLVER_REFERENCE; a.max_iter = 25; a.tol = 0.01; a.ion_tol = 0.01; a.step0 = 0.05;
     a.slope0 = 1.0;
     a.warm_iter = a.max_iter;
+    a.ncel = c->bal.A.ncel;
+    a.cel_most = c->bal.A.cel_most;
     return a;
 }
 
@@ -1274,7 +1281,7 @@ extern "C" int mc_emission_setup(mc_ctx *c, const mc_emission_tables *t)
         if (A.el[e].z == 2) eHe = e;
     }
     if (eH != 0 || eHe < 0 || A.nstages < 3) return fail(c, MC_EUNSUP, "re-emission needs H and He (3 stages)");
-    if (mce_lds_bytes(nb, true) > 48 * 1024)
+    if (mce_mesh_bytes(nb) > 48 * 1024)
         return fail(c, MC_EUNSUP, "re-emission keeps 4 x nbins partial sums in LDS: %d bins is too many", nb);
     if (!t->tkGamma || !t->logGammaHI || !t->logGammaHeI || !t->logGammaHeII || !t->HINuEdgeP || !t->HeINuEdgeP ||
         !t->HeIINuEdgeP || !t->gauntFF || !t->gauntFFHeII || !t->xSecHI || !t->xSecHeI || !t->xSecHeII ||
@@ -1431,6 +1438,7 @@ extern "C" int mc_emission_build(mc_ctx *c, const float *Hden, const float *Te, 
     HIPCHK(c, hipSetDevice(c->device));
     mce::EmArgs a = c->em;
     const mcb::Atomic &A = c->bal.A;
+    a.ncel = A.ncel; a.cel_most = A.cel_most; a.nterm = A.nterm;
     const int nE = A.nE, ns = A.nstages;
     const size_t nion = nc1 * nE * (ns + 1);
     if (host_state) {
@@ -1551,6 +1559,7 @@ extern "C" int mc_line_luminosities(mc_ctx *c, const float *Hden, const float *T
     a.cells_per_blk = std::max(1, (nc + 4095) / 4096);
     const int nblk = (nc + a.cells_per_blk - 1) / a.cells_per_blk;
     a.ldp = ncel * mcb::kLineEnt + 1;
+    a.cel_most = A.cel_most;
     a.cell_xyz = c->d_cell_xyz;
     a.nx = c->G.nx;
     a.ny = c->G.ny;

@@ -58,10 +58,13 @@ struct EmArgs {
     float *rec;                              // [nCells+1][nb]
     float *totalLines;                       // [nCells+1]
     int *err;                                // cells whose recPDF has no positive total
+    int ncel, cel_most, nterm;               // of the atomic data: the level solves' LDS
 };
 
 }  // namespace mce
 
 // One wavefront per active cell; lds = dynamic LDS bytes (mce_lds_bytes).
-size_t mce_lds_bytes(int nb, bool dust);
+size_t mce_lds_bytes(const mce::EmArgs &a);
+// the same for a mesh of nb bins with grains, without the level solves
+size_t mce_mesh_bytes(int nb);
 hipError_t mce_launch(const mcb::Atomic *dA, const mce::EmArgs &a, hipStream_t s);

@@ -25,25 +25,20 @@ constexpr float kHPlanck = 6.6262e-27f;  // constants_mod.f90:14
 constexpr float kPi = 3.141592654f;      // constants_mod.f90:32
 constexpr int kLev = mcb::kMaxLev;
 
-struct CelLds {
-    double x[kLev + 1][kLev + 1];
-    double q[kLev + 1][kLev + 1];
-    double y[kLev + 1];
-    double alev[kLev + 1];
-};
-
 // One dynamic LDS block per wavefront.  Region A serves the forbidden-line
-// solves first (CelLds and the terms of one model ion) and then the per-bin
+// solves first (records, collision rates and line terms) and then the per-bin
 // partial sums s1, s2, s3 (and the grains' sD); the log-gamma rows, the
 // recombination-line terms and a reduction slot follow it.  Sharing region
 // A keeps the block at about 12 KB on an 800-bin mesh, so that more
 // wavefronts fit on a CU.
-__host__ __device__ inline size_t region_a_bytes(int nb, bool dust)
+__host__ __device__ inline size_t region_a_bytes(const EmArgs &a)
 {
-    const size_t cel = sizeof(CelLds) + sizeof(float) * kLev * kLev;
-    const size_t sums = (size_t)(dust ? 4 : 3) * nb * sizeof(float);
+    const size_t cel = (size_t)a.cel_most * sizeof(double2) + (size_t)a.ncel * sizeof(mcb::CelRec) +
+                       (size_t)a.nterm * sizeof(float);
+    const size_t sums = (size_t)(a.dabs ? 4 : 3) * a.nb * sizeof(float);
     return ((cel > sums ? cel : sums) + 15) / 16 * 16;
 }
+constexpr size_t kRestBytes = sizeof(float) * (3 * kMaxLim + kMaxRec + 4);
 
 // hydro2phot (emission_mod.f90:553-663), REAL arithmetic
 __device__ double hydro2phot(float nu, int Z, float Te, float Ne)
@@ -134,10 +129,11 @@ __global__ void __launch_bounds__(64) emission_kernel(const mcb::Atomic *__restr
     const float *nu = a.nu;
     const bool dust = a.dabs != nullptr;
     // region A: the forbidden-line solves, then the per-bin sums
-    CelLds &S = *reinterpret_cast<CelLds *>(dyn);
-    float *fterm = reinterpret_cast<float *>(dyn + sizeof(CelLds));
+    double2 *rate = reinterpret_cast<double2 *>(dyn);
+    mcb::CelRec *rec = reinterpret_cast<mcb::CelRec *>(rate + a.cel_most);
+    float *fterm = reinterpret_cast<float *>(rec + a.ncel);
     float *s1 = reinterpret_cast<float *>(dyn), *s2 = s1 + nb, *s3 = s1 + 2 * nb, *sD = s1 + 3 * nb;
-    unsigned char *rest = dyn + region_a_bytes(nb, dust);
+    unsigned char *rest = dyn + region_a_bytes(a);
     float (*loc)[kMaxLim] = reinterpret_cast<float (*)[kMaxLim]>(rest);
     float *rterm = reinterpret_cast<float *>(rest + sizeof(float) * 3 * kMaxLim);
     float *red = rterm + kMaxRec;
@@ -158,41 +154,39 @@ __global__ void __launch_bounds__(64) emission_kernel(const mcb::Atomic *__restr
     }
 
     float normFor = 0.f;
-    // forbidden lines (forLines), each model ion's terms above 1e-35 summed
-    // lower level outer, upper inner, as setDiffusePDF does
+    // forbidden lines (forLines): the terms above 1e-35 of every model ion's
+    // radiating pairs, summed ion by ion, lower level outer, upper inner, as
+    // setDiffusePDF does
     const double kL = (double)1.9865e9f;
-    for (int k = 0; k < A.ncel; ++k) {
+    const double TeD = (double)Te, sqrTeD = sqrt(TeD), log10TeD = log10(TeD);
+    for (int k = lane; k < A.ncel; k += W) {
         const mcb::CelIon &ci = A.cel[k];
         const float x = XION(ci.eidx, ci.ion);
         const float up = (ci.ion < a.ns1 - 1) ? XION(ci.eidx, ci.ion + 1) / x : 0.f;
-        if (up != up) continue;                  // equilibrium's NaN test: no emission
-        mcb::cel_levels(A, ci, S, lane, (double)Te, (double)NeUsed, (double)up);
-        const int nl = ci.nl;
-        const double *E = A.cel_e + ci.off_e;
-        const double *Aa = A.cel_a + ci.off_a;
-        double sumN = 0.0;
-        for (int i = 1; i <= nl; ++i) sumN = sumN + S.y[i];
-        const double ab = (double)(float)A.el[ci.eidx].abun;
-        for (int p = lane; p < kLev * kLev; p += W) {
-            const int lo = p / kLev + 1, hi = p % kLev + 1;
-            float v = 0.f;
-            if (lo < hi && hi <= nl) {
-                const double av = Aa[(hi - 1) + nl * (lo - 1)];
-                if (av != 0.0) {
-                    const double Eji = E[hi - 1] - E[lo - 1];
-                    double f = av * Eji * (S.y[hi] / sumN);
-                    f = f * ab * (double)x;
-                    f = f * kL;
-                    if (f > (double)1.e-35f) v = (float)f;
-                }
-            }
-            fterm[p] = v;
-        }
-        __syncthreads();
-        if (lane == 0)
-            for (int p = 0; p < kLev * kLev; ++p) normFor = normFor + fterm[p];
-        __syncthreads();
+        rec[A.cel_place[k]] = mcb::cel_record(A, ci, TeD, log10TeD, (double)up, (double)(float)A.el[ci.eidx].abun,
+                                              (double)x);
     }
+    __syncthreads();
+    for (int b = 0; b < A.ncelb; ++b) {
+        const mcb::CelBatch &B = A.celb[b];
+        const mcb::CelRec *R = rec + mcb::kCelSlots * b;
+        const mcb::CelLevels L = mcb::cel_levels(A, b, R, rate, lane, TeD, sqrTeD, (double)NeUsed);
+        const int g = lane >> 4;
+        const bool mine = (lane & 15) < B.rows[g];
+        const double part = L.y / L.sum, ab = R[mine ? g : 0].ab, x = R[mine ? g : 0].x;
+        const bool none = R[mine ? g : 0].skip;
+        const double *ae = A.cel_ae + (size_t)b * kLev * 64 + lane;
+        const int *term = A.cel_term + (size_t)b * kLev * 64 + lane;
+        for (int lo = 0; lo < B.most; ++lo) {
+            double f = ae[64 * lo] * part;
+            f = f * ab * x;
+            f = f * kL;
+            const int t = term[64 * lo];
+            if (t >= 0) fterm[t] = !none && f > (double)1.e-35f ? (float)f : 0.f;
+        }
+    }
+    __syncthreads();
+    for (int t = 0; t < A.nterm; ++t) normFor = normFor + fterm[t];
     __syncthreads();                             // region A now holds the per-bin sums
 
     // log gamma rows at Te (fb_ff, emission_mod.f90:306-336)
@@ -452,14 +446,19 @@ __global__ void __launch_bounds__(64) emission_kernel(const mcb::Atomic *__restr
 
 }  // namespace mce
 
-size_t mce_lds_bytes(int nb, bool dust)
+size_t mce_lds_bytes(const mce::EmArgs &a)
 {
-    return mce::region_a_bytes(nb, dust) + sizeof(float) * (3 * mce::kMaxLim + mce::kMaxRec + 4);
+    return mce::region_a_bytes(a) + mce::kRestBytes;
+}
+
+size_t mce_mesh_bytes(int nb)
+{
+    return (4 * (size_t)nb * sizeof(float) + 15) / 16 * 16 + mce::kRestBytes;
 }
 
 hipError_t mce_launch(const mcb::Atomic *dA, const mce::EmArgs &a, hipStream_t s)
 {
     if (a.nc <= 0) return hipSuccess;
-    hipLaunchKernelGGL(mce::emission_kernel, dim3(a.nc), dim3(64), mce_lds_bytes(a.nb, a.dabs != nullptr), s, dA, a);
+    hipLaunchKernelGGL(mce::emission_kernel, dim3(a.nc), dim3(64), mce_lds_bytes(a), s, dA, a);
     return hipGetLastError();
 }
