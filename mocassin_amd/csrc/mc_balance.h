@@ -129,9 +129,9 @@ struct CellArgs {
     // state to restart from when the solve from Te/Ne/ion fails (nullable)
     const double *Te0, *Ne0, *ion0;
     // grains with the photoelectric effect (nullable: gas alone); device
-    // pointer, with the frequency-bin count for the launch's LDS size
+    // pointer, with the frequency bins and grain rows for the launch's LDS size
     const Grains *grains;
-    int grains_nb;
+    int grains_nb, grains_rows;
     int ncel, cel_most;         // of the atomic data: the solves' LDS
     // nullable: block b balances cell order[b] (a permutation of 1..ncells),
     // else cell b + 1; results do not depend on the order

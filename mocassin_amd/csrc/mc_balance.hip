@@ -53,12 +53,6 @@ __host__ __device__ inline size_t shared_bytes(int ncel, int most)
     return ((cel > sizeof(IonLds) ? cel : sizeof(IonLds)) + 15) / 16 * 16;
 }
 
-__device__ __forceinline__ double wave_sum(double v)
-{
-    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
-    return v;
-}
-
 __device__ double rad_rec(const Channel &c, double Te)
 {
     if (c.rr_kind == 0) {
@@ -181,106 +175,206 @@ __device__ __forceinline__ double cooling(const Atomic &A, Lds &S, void *dyn, in
 // point: every grain row's potential (setGrainPotential's secant iteration,
 // at most 100 steps), then the photoelectric heating and cooling
 // (setPhotoelHeatCool) and the collision terms (setDustGasCollHeatCool).
-// The cell's photon flux J/(h c Ryd nu) per bin is staged in LDS once per
-// cell; the bin sums run across lanes, the collision sums with one lane per
-// grain row in the reference's order of elements and stages.
+// The rows are independent, and each step of a row's iteration waits for the
+// one before: so all rows iterate at once, each on its own group of lanes
+// (64 over the next power of two of the rows), instead of one after another
+// on the whole wavefront.  The sums over frequency are linear in the
+// potential for every bin above the threshold (yield Y (1 - V/d) with d = nu
+// - vn, photoelectron energy Y (d - V^2/d) / 2), so the cell's suffix sums of
+// u, u/d and u d (u = Y sigma flux) over 16 chunks of bins are formed once,
+// and a step adds up the bins of the threshold's chunk alone.  Bound by the
+// latency of the steps: the balance kernel of the dust and gas 60^3 grid (10
+// rows, 160 bins) took 38 ms with one row at a time over all bins, 11.5 now.
 constexpr double kPiR = (double)3.141592654f;             // constants_mod.f90:32 (REAL)
 constexpr double kFourPiR = (double)(4.f * 3.141592654f);
 constexpr double kHcRyd = 2.1799153e-11, kRyd2erg = 2.1799e-11, kKB = 1.380658e-16;
 constexpr double kAmu = 1.66053e-24, kMe = 9.109382e-28;
+constexpr int kChunks = 16;              // of the frequency bins
 
 // dynamic LDS of the grain variant, after the cell's photon flux pf[nbins]
+// and before the suffix sums [3][kChunks + 1][K]
 struct GrainLds {
-    double w[kMaxElem][kMaxStage];   // n(ion) v_mean of each (element, stage >= 2)
-    double pot[kMaxGrainRows], gdc[kMaxGrainRows], peh[kMaxGrainRows];
+    double w[kMaxCh];                // n(ion) v_mean of each channel's ion
+    double nu0[kChunks];             // first bin of each chunk
+    double gdc[kMaxGrainRows], peh[kMaxGrainRows], hg[kMaxGrainRows], gg[kMaxGrainRows];
     double gdcg, pehg;
 };
+__host__ __device__ inline size_t grain_bytes(int nb, int K)
+{
+    return (size_t)nb * sizeof(double) + sizeof(GrainLds) + (size_t)3 * (kChunks + 1) * K * sizeof(double);
+}
 
 __device__ __forceinline__ double minr(double a, double b) { return a < b ? a : b; }
 __device__ __forceinline__ double maxr(double a, double b) { return a > b ? a : b; }
 
-// locate(nuArray, x) on the increasing frequency mesh (interpolation_mod.f90:
-// 48-81): nb when x > nu(nb), 0 when x < nu(1), else the last i with
-// nu(i) <= x, at least 1 (x == nu(nb) gives 1)
-__device__ int locate_nu(const double *nu, int n, double x)
+// The rows' geometry: lane `sub` of the n lanes of row `row` (the last row
+// again on lanes without one, which are not live).
+struct RowLane {
+    int n, row, sub;
+    bool live;
+};
+__device__ __forceinline__ RowLane row_lanes(int K, int lane)
 {
-    if (x > nu[n - 1]) return n;
-    if (x < nu[0]) return 0;
-    int lo = 0, hi = n;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (nu[mid] > x) hi = mid; else lo = mid + 1;
-    }
-    const int p = lo < n ? lo + 1 : 0;
-    return p - 1 > 1 ? p - 1 : 1;
+    RowLane R;
+    R.n = W;
+    while (W / R.n < K) R.n >>= 1;
+    R.row = lane / R.n;
+    R.sub = lane % R.n;
+    R.live = R.row < K;
+    if (!R.live) R.row = K - 1;
+    return R;
 }
 
-// getGrainEmission (update_mod.f90:601-651) of row k at potential Vg, on every lane
-__device__ double grain_emission(const Atomic &A, const Grains &G, const double *pf, int k, double Vg, int lane)
+// sum over a row's n lanes, on each of them (every lane active)
+__device__ __forceinline__ double row_sum(double v, int n)
 {
-    const int nb = A.nbins, s = k / G.nSizes;
-    const double vn = G.vn[s];
-    const int ip = locate_nu(A.nu, nb, maxr(vn + Vg, vn)) + 1;
-    const double *qa = G.qa + (size_t)k * nb, *yn = G.yn + (size_t)s * nb;
+    if (n > 1) v += __builtin_amdgcn_update_dpp(0.0, v, 0xB1, 0xf, 0xf, true);      // quad_perm 1 0 3 2
+    if (n > 2) v += __builtin_amdgcn_update_dpp(0.0, v, 0x4E, 0xf, 0xf, true);      // quad_perm 2 3 0 1
+    if (n > 4) v += __builtin_amdgcn_update_dpp(0.0, v, 0x141, 0xf, 0xf, true);     // row_half_mirror
+    if (n > 8) v += __builtin_amdgcn_update_dpp(0.0, v, 0x140, 0xf, 0xf, true);     // row_mirror
+    if (n > 16) v += __shfl_xor(v, 16);
+    if (n > 32) v += __shfl_xor(v, 32);
+    return v;
+}
+
+// The spectrum's part of a row: bins above x = max(vn + V, vn), which locate
+// (interpolation_mod.f90:48-81) finds on the increasing mesh; its answer 1
+// for x equal to the last bin is `whole`.
+struct Spectrum {
+    const double *nu, *pf, *yn, *ax, *qa, *sums;
+    double vn;
+    int nb, K, row, size;             // size: bins of a chunk
+    // chunk of x: the last whose first bin is at or below x, -1 before all
+    __device__ __forceinline__ int chunk(const GrainLds &L, double x) const
+    {
+        int lo = 0, hi = kChunks;     // nu0 is infinite beyond the mesh
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if (L.nu0[mid] > x) hi = mid; else lo = mid + 1;
+        }
+        return lo - 1;
+    }
+    __device__ __forceinline__ double sum(int q, int c) const { return sums[(q * (kChunks + 1) + c) * K + row]; }
+};
+
+// getGrainEmission (update_mod.f90:601-651) at potential V: this lane's part
+__device__ __forceinline__ double grain_emission(const Spectrum &P, const GrainLds &L, double perArea, double V,
+                                                 const RowLane &R)
+{
+    const double x = maxr(P.vn + V, P.vn);
+    const int c = P.chunk(L, x);
     double sum = 0.0;
-    for (int f = ip + lane; f <= nb; f += W) {
-        const double Yhat = yn[f - 1] * minr(1., maxr(0., 1. - Vg / (A.nu[f - 1] - vn)));
-        const double photFlux = pf[f - 1] * kFourPiR;
-        sum = sum + Yhat * photFlux * qa[f - 1];
+    for (int u = R.sub; u < P.size; u += R.n) {
+        const int f = c * P.size + u;
+        if (c >= 0 && f < P.nb && P.nu[f] > x) {
+            const double Yhat = P.yn[f] * minr(1., maxr(0., 1. - V / (P.nu[f] - P.vn)));
+            sum = sum + Yhat * (P.pf[f] * kFourPiR) * P.qa[f];
+        }
     }
-    return wave_sum(sum);
+    if (R.sub == 0) {
+        const double a = P.sum(0, c + 1);
+        sum = sum + (V < 0. ? a : a - V * P.sum(1, c + 1)) * perArea;
+    }
+    if (__any(x == P.nu[P.nb - 1])) {
+        double all = 0.0;
+        for (int f = 1 + R.sub; f < P.nb; f += R.n)
+            all = all + P.yn[f] * minr(1., maxr(0., 1. - V / (P.nu[f] - P.vn))) * (P.pf[f] * kFourPiR) * P.qa[f];
+        sum = x == P.nu[P.nb - 1] ? all : sum;
+    }
+    return sum;
 }
 
-// getGrainRecombination (update_mod.f90:656-733), on every lane
-__device__ double grain_recombination(const Atomic &A, const GrainLds &L, double Te, double eNe, double Vg, int lane)
+// getGrainRecombination (update_mod.f90:656-733), the ions' part of this lane
+__device__ __forceinline__ double grain_ions(const Atomic &A, const GrainLds &L, double kT, double V, const RowLane &R)
 {
-    const double kT = 6.336e-6 * Te;
-    double eta = -(Vg / kT);
-    eta = eta <= 0. ? 1. - eta : exp(-eta);
-    const double rec = eNe * eta;
     double ions = 0.0;
-    for (int i = lane; i < A.nE * kMaxStage; i += W) {
-        const int e = i / kMaxStage, st = i % kMaxStage;
-        if (st < 2 || st > A.el[e].nst) continue;
-        double et = (double)(st - 1) * Vg / kT;
+    for (int k = R.sub; k < A.nch; k += R.n) {
+        double et = (double)A.ch[k].ion * V / kT;
         et = et <= 0. ? 1. - et : exp(-et);
-        ions = ions + L.w[e][st] * et;
+        ions = ions + L.w[k] * et;
     }
-    return rec - wave_sum(ions);
+    return ions;
+}
+__device__ __forceinline__ double grain_electrons(double kT, double eNe, double V)
+{
+    double eta = -(V / kT);
+    eta = eta <= 0. ? 1. - eta : exp(-eta);
+    return eNe * eta;
+}
+
+// the suffix sums of a cell's spectrum, once per cell
+__device__ __forceinline__ void grain_sums(const Atomic &A, const Grains &G, const double *pf, GrainLds &L,
+                                           double *sums, int lane)
+{
+    const int nb = A.nbins, K = G.K, size = (nb + kChunks - 1) / kChunks;
+    if (lane < kChunks) L.nu0[lane] = lane * size < nb ? A.nu[lane * size] : __builtin_inf();
+    for (int t = lane; t < K * kChunks; t += W) {
+        const int k = t % K, c = t / K, s = k / G.nSizes;
+        const double vn = G.vn[s];
+        const double *ax = G.absx + (size_t)k * nb, *yn = G.yn + (size_t)s * nb;
+        double a = 0.0, b = 0.0, e = 0.0;
+        for (int f = c * size; f < min(nb, (c + 1) * size); ++f) {
+            const double d = A.nu[f] - vn;
+            if (!(d > 0.)) continue;
+            const double u = yn[f] * ax[f] * pf[f];
+            a = a + u;
+            b = b + u / d;
+            e = e + u * d;
+        }
+        sums[(0 * (kChunks + 1) + c) * K + k] = a;
+        sums[(1 * (kChunks + 1) + c) * K + k] = b;
+        sums[(2 * (kChunks + 1) + c) * K + k] = e;
+    }
+    __syncthreads();
+    for (int t = lane; t < 3 * K; t += W) {
+        double *p = sums + (t / K) * (kChunks + 1) * K + t % K;
+        double v = 0.0;
+        p[kChunks * K] = 0.0;
+        for (int c = kChunks - 1; c >= 0; --c) {
+            v = v + p[c * K];
+            p[c * K] = v;
+        }
+    }
+    __syncthreads();
 }
 
 // the grain block of iterateT after ionBalance (update_mod.f90:367-388) and
 // the two heat/cool terms it adds to thermBalance (1252-1255)
-__device__ void grain_terms(const Atomic &A, const Grains &G, const double *pf, GrainLds &L, Lds &S, int lane,
-                            int cell)
+__device__ void grain_terms(const Atomic &A, const Grains &G, const double *pf, const double *sums, GrainLds &L, Lds &S,
+                            int lane, int cell)
 {
-    const int nb = A.nbins, K = G.K;
+    const int nb = A.nbins, K = G.K, nch = A.nch;
     const double Te = S.Te, Ne = S.Ne, Hden = S.Hden;
     const double kT = 6.336e-6 * Te, e8 = 1.1045e-15 * Te / kPiR;
     // n(ion) v_mean of the ions; electrons ((Ne vmean) S) with S = 1
-    for (int i = lane; i < A.nE * kMaxStage; i += W) {
-        const int e = i / kMaxStage, st = i % kMaxStage;
-        if (st < 2 || st > A.el[e].nst) continue;
+    for (int k = lane; k < nch; k += W) {
+        const int e = A.ch[k].eidx, st = A.ch[k].ion + 1;
         const double cpDen = S.ion[e][st] * A.el[e].abun * Hden;
         const double vm = sqrt(e8 / (G.aweight[A.el[e].z - 1] * kAmu));
-        L.w[e][st] = cpDen * vm * 1.;
+        L.w[k] = cpDen * vm * 1.;
     }
     __syncthreads();
     const double eNe = Ne * sqrt(e8 / kMe) * 1.;
+    const RowLane R = row_lanes(K, lane);
+    const int k = R.row, s = k / G.nSizes, ai = k % G.nSizes;
+    const double vn = G.vn[s], rad = G.radius[ai];
+    const Spectrum P{ A.nu, pf, G.yn + (size_t)s * nb, G.absx + (size_t)k * nb, G.qa + (size_t)k * nb, sums, vn, nb, K,
+                      k, (nb + kChunks - 1) / kChunks };
+    const double perArea = kFourPiR / (1.e-8 * rad * rad);
     // setGrainPotential: secant on emission - recombination, from 0 V
-    for (int k = 0; k < K; ++k) {
-        const double vn = G.vn[k / G.nSizes];
-        double slope = 0., potOld = 0.;
-        double emiOld = grain_emission(A, G, pf, k, 0., lane);
-        double recOld = grain_recombination(A, L, Te, eNe, 0., lane);
-        double pot = potOld + 0.05;
-        for (int n = 1;; ++n) {
-            const double threshold = maxr(vn + pot, vn);
-            const double emi = grain_emission(A, G, pf, k, pot, lane);
-            const double rec = grain_recombination(A, L, Te, eNe, pot, lane);
-            double delta = emi - rec;
-            double delta1 = fabs(delta / (0.5 * maxr(1.e-35, emi + rec)));
-            if (delta1 < 0.005) break;
+    double slope = 0., potOld = 0.;
+    double emiOld = row_sum(grain_emission(P, L, perArea, 0., R), R.n);
+    double recOld = grain_electrons(kT, eNe, 0.) - row_sum(grain_ions(A, L, kT, 0., R), R.n);
+    double pot = potOld + 0.05;
+    bool done = !R.live;
+    for (int n = 1; n <= 100 && __any(!done); ++n) {
+        const double threshold = maxr(vn + pot, vn);
+        const double emi = row_sum(grain_emission(P, L, perArea, pot, R), R.n);
+        const double rec = grain_electrons(kT, eNe, pot) - row_sum(grain_ions(A, L, kT, pot, R), R.n);
+        double delta = emi - rec;
+        double delta1 = fabs(delta / (0.5 * maxr(1.e-35, emi + rec)));
+        done = done || delta1 < 0.005;
+        if (!done) {
             if (pot != potOld) {
                 const double fac = (emi - emiOld) - (rec - recOld);
                 if (fac != 0.) slope = fac / (pot - potOld);
@@ -292,64 +386,80 @@ __device__ void grain_terms(const Atomic &A, const Grains &G, const double *pf, 
             delta = minr(fabs(delta1), 0.05 * threshold);
             delta = signbit(delta1) ? -fabs(delta) : fabs(delta);
             pot = pot + delta;
-            if (n >= 100) break;
         }
-        if (lane == 0) L.pot[k] = pot;
     }
-    __syncthreads();
-    // setPhotoelHeatCool: lanes over bins, one row after another
-    double pehg = 0.0;
-    for (int k = 0; k < K; ++k) {
-        const int s = k / G.nSizes, ai = k % G.nSizes;
-        const double pot = L.pot[k], vn = G.vn[s];
-        int thP = locate_nu(A.nu, nb, maxr(vn + pot, vn));
-        if (thP <= 0) thP = 1;
-        const double *ax = G.absx + (size_t)k * nb, *yn = G.yn + (size_t)s * nb;
-        double hd = 0.0, hg = 0.0;
-        for (int f = thP + lane; f <= nb; f += W) {
-            const double nu = A.nu[f - 1], Yn = yn[f - 1];
-            const double Yhat = Yn * minr(1., maxr(0., 1. - pot / (nu - vn)));
-            const double d = nu - vn;
-            const double EY = Yn * 0.5 * minr(d, maxr(0., (d * d - pot * pot) / d));
-            const double q = ax[f - 1] * pf[f - 1];
-            hd = hd + q * EY * kHcRyd / kPiR;
-            hg = hg + q * (EY - Yhat * pot) * G.gabun[s] * G.weight[ai];
-        }
-        hd = wave_sum(hd);
-        hg = wave_sum(hg);
-        if (lane == 0) L.peh[k] = hd;
-        pehg = pehg + hg;
-    }
-    pehg = pehg * G.ndust[cell] * kHcRyd / Hden;
-    // setDustGasCollHeatCool: one lane per grain row, elements and stages in
-    // the reference's order; IPerg is set for ionised stages and kept for
-    // the neutral stage that follows (it starts at 0)
-    double gd = 0.0, gg = 0.0;
-    if (lane < K) {
-        const int k = lane, s = k / G.nSizes, ai = k % G.nSizes;
-        const double pot = L.pot[k], rad = G.radius[ai], ms = G.msurf[s];
-        const double Td = G.Tdust[(size_t)cell * (G.nsMax + 1) * (G.nSizes + 1) + (s + 1) + (G.nsMax + 1) * (ai + 1)];
-        const double nd = G.ndust[cell];
-        double IPerg = 0.0;
-        for (int e = 0; e < A.nE; ++e) {
-            const int z = A.el[e].z;
-            const double mcp = G.aweight[z - 1] * kAmu;
-            const double vmean = sqrt(e8 / mcp);
-            for (int st = 1; st <= A.el[e].nst; ++st) {
-                const double Z = (double)(st - 1);
-                if (st > 1) IPerg = A.nu[A.ch[A.el[e].ch0 + st - 2].ip - 1] * kRyd2erg;
-                const double S_ = st == 1 ? 2. * mcp * ms / ((mcp + ms) * (mcp + ms)) : 1.;
-                const double psi = Z * pot / kT;
-                double eta, xi;
-                if (psi <= 0.) { eta = 1. - psi; xi = 1. - psi / 2.; }
-                else { eta = exp(-psi); xi = (1. + psi / 2.) * eta; }
-                const double x = S.ion[e][st], ab = A.el[e].abun;
-                gd = gd + x * ab * Hden * kPiR * rad * rad * 1.e-8 * S_ * vmean *
-                          (2. * kT * kRyd2erg * xi - eta * (Z * pot * kRyd2erg - IPerg + 2. * kKB * Td));
-                gg = gg + x * G.weight[ai] * G.gabun[s] * nd * ab * kPiR * rad * rad * 1.e-8 * S_ * vmean *
-                          (2. * kT * kRyd2erg * xi - eta * 2. * kKB * Td);
+    // setPhotoelHeatCool.  The photoelectron energy is zero below vn + |V|,
+    // and the bin that locate returns (the last at or below the threshold,
+    // which can lie below vn) counts too.
+    {
+        const double x = maxr(vn + pot, vn), x2 = vn + fabs(pot);
+        const int c = P.chunk(L, x), c2 = P.chunk(L, x2);
+        double hE = 0.0, hY = 0.0;
+        for (int u = R.sub; u < P.size; u += R.n) {
+            const int f = c * P.size + u, f2 = c2 * P.size + u;
+            if (c >= 0 && f < nb) {
+                const double nu = A.nu[f], q = P.ax[f] * pf[f], d = nu - vn;
+                const bool last = !(nu > x) && (f == nb - 1 || A.nu[f + 1] > x);
+                if (nu > x || last) hY = hY + q * (P.yn[f] * minr(1., maxr(0., 1. - pot / d)));
+                if (last) hE = hE + q * (P.yn[f] * 0.5 * minr(d, maxr(0., (d * d - pot * pot) / d)));
+            }
+            if (c2 >= 0 && f2 < nb && A.nu[f2] > x2) {
+                const double d = A.nu[f2] - vn;
+                hE = hE + P.ax[f2] * pf[f2] * (P.yn[f2] * 0.5 * minr(d, maxr(0., (d * d - pot * pot) / d)));
             }
         }
+        if (R.sub == 0) {
+            hY = hY + (P.sum(0, c + 1) - maxr(pot, 0.) * P.sum(1, c + 1));
+            hE = hE + 0.5 * (P.sum(2, c2 + 1) - pot * pot * P.sum(1, c2 + 1));
+        }
+        // x at the last bin (locate gives the first), or a potential that is
+        // no number: bin by bin
+        const bool whole = x == A.nu[nb - 1] || pot != pot;
+        if (__any(whole)) {
+            double aE = 0.0, aY = 0.0;
+            for (int f = R.sub; f < nb; f += R.n) {
+                const double d = A.nu[f] - vn, q = P.ax[f] * pf[f];
+                aY = aY + q * (P.yn[f] * minr(1., maxr(0., 1. - pot / d)));
+                aE = aE + q * (P.yn[f] * 0.5 * minr(d, maxr(0., (d * d - pot * pot) / d)));
+            }
+            hE = whole ? aE : hE;
+            hY = whole ? aY : hY;
+        }
+        hE = row_sum(hE, R.n);
+        hY = row_sum(hY, R.n);
+        if (R.live && R.sub == 0) {
+            L.peh[k] = hE * kHcRyd / kPiR;
+            L.hg[k] = (hE - hY * pot) * G.gabun[s] * G.weight[ai];
+        }
+    }
+    // setDustGasCollHeatCool: a row's lanes over the channels, each with its
+    // ionised stage, the first of an element with the neutral one too.  The
+    // neutral stage sees the ionisation potential of the stage before it in
+    // the reference's order (0 at the start).
+    double gd = 0.0, gg = 0.0;
+    const double ms = G.msurf[s], nd = G.ndust[cell];
+    const double Td = G.Tdust[(size_t)cell * (G.nsMax + 1) * (G.nSizes + 1) + (s + 1) + (G.nsMax + 1) * (ai + 1)];
+    auto stage = [&](int e, int st, int from) {
+        const double mcp = G.aweight[A.el[e].z - 1] * kAmu;
+        const double vmean = sqrt(e8 / mcp);
+        const double Z = (double)(st - 1), IPerg = from >= 0 ? A.nu[A.ch[from].ip - 1] * kRyd2erg : 0.0;
+        const double S_ = st == 1 ? 2. * mcp * ms / ((mcp + ms) * (mcp + ms)) : 1.;
+        const double psi = Z * pot / kT;
+        double eta, xi;
+        if (psi <= 0.) { eta = 1. - psi; xi = 1. - psi / 2.; }
+        else { eta = exp(-psi); xi = (1. + psi / 2.) * eta; }
+        const double x = S.ion[e][st], ab = A.el[e].abun;
+        gd = gd + x * ab * Hden * kPiR * rad * rad * 1.e-8 * S_ * vmean *
+                      (2. * kT * kRyd2erg * xi - eta * (Z * pot * kRyd2erg - IPerg + 2. * kKB * Td));
+        gg = gg + x * G.weight[ai] * G.gabun[s] * nd * ab * kPiR * rad * rad * 1.e-8 * S_ * vmean *
+                      (2. * kT * kRyd2erg * xi - eta * 2. * kKB * Td);
+    };
+    for (int j = R.sub; j < nch; j += R.n) {
+        const Channel &ch = A.ch[j];
+        if (ch.ion == 1) stage(ch.eidx, 1, j - 1);
+        stage(ch.eidx, ch.ion + 1, j);
+    }
+    if (R.sub == 0) {
         // electrons
         const double vme = sqrt(e8 / kMe), Z = -1.;
         const double psi = Z * pot / kT;
@@ -359,19 +469,28 @@ __device__ void grain_terms(const Atomic &A, const Grains &G, const double *pf, 
         gd = gd + Ne * kPiR * rad * rad * 1.e-8 * 1. * vme * (2. * kT * kRyd2erg * xi - eta * (Z * pot * kRyd2erg));
         gg = gg + Ne * G.weight[ai] * G.gabun[s] * nd * kPiR * rad * rad * 1.e-8 * 1. * vme *
                   (2. * kT * kRyd2erg * xi) / Hden;
-        L.gdc[k] = gd / kFourPiR;
     }
-    gg = wave_sum(gg) / kFourPiR;
-    if (lane == 0) { L.gdcg = gg; L.pehg = pehg; }
+    gd = row_sum(gd, R.n);
+    gg = row_sum(gg, R.n);
+    if (R.live && R.sub == 0) {
+        L.gdc[k] = gd / kFourPiR;
+        L.gg[k] = gg;
+    }
+    __syncthreads();
+    if (lane == 0) {
+        double p = 0.0, q = 0.0;
+        for (int r = 0; r < K; ++r) { p = p + L.hg[r]; q = q + L.gg[r]; }
+        L.pehg = p * nd * kHcRyd / Hden;
+        L.gdcg = q / kFourPiR;
+    }
     __syncthreads();
 }
 
-// Registers for three wavefronts a SIMD without grains (6.5 ms against 7.6
-// for four on the 45^3 octant: the level solves' rows spill), for four with
-// grains (38 against 42 ms, dust and gas 60^3: the grain loops want the
-// wavefronts).
+// Registers for three wavefronts a SIMD: 6.7 ms on the 45^3 octant (7.6 with
+// four, where the level solves' rows spill, 8.1 with two), 11.5 ms with grains
+// on the dust and gas 60^3 grid (12.2 with four, 11.5 with two).
 template <bool PE>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PE ? 4 : 3))) balance_kernel(const Atomic *__restrict__ Ap, CellArgs a)
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) balance_kernel(const Atomic *__restrict__ Ap, CellArgs a)
 {
     __shared__ Lds S;
     // ion fixed point or level solves; grain variant: photon flux per bin, GrainLds
@@ -402,12 +521,15 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PE ? 4 
     IonLds &F = *reinterpret_cast<IonLds *>(dyn);
     double *pf = reinterpret_cast<double *>(reinterpret_cast<char *>(dyn) + shared_bytes(A.ncel, A.cel_most));
     GrainLds &GL = *reinterpret_cast<GrainLds *>(pf + A.nbins);
+    double *gsums = reinterpret_cast<double *>(&GL + 1);
     if (PE) {
         // the cell's photon flux J/(h c Ryd nu) (getGrainEmission, setPhotoelHeatCool)
         const Grains &G = *a.grains;
         const unsigned pt = mcd::j3_point_of(mcd::j3_shape(G.nx, G.ny, G.nz), G.cell_xyz[cell]);
         for (int f = lane; f < A.nbins; f += W)
             pf[f] = G.J3[mcd::j3_index(A.nbins, f, pt)] * a.jscale / (kHcRyd * A.nu[f]);
+        __syncthreads();
+        grain_sums(A, G, pf, GL, gsums, lane);
     }
     __syncthreads();
     // lgConverged compares with the caller's H0 fraction (update_mod.f90:510-515)
@@ -497,7 +619,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PE ? 4 
                 lgIBConv = !(big && nIterX == 25);
                 break;
             }
-            if (PE) grain_terms(A, *a.grains, pf, GL, S, lane, cell);
+            if (PE) grain_terms(A, *a.grains, pf, gsums, GL, S, lane, cell);
             // thermBalance (933-1258)
             double cool = cooling(A, S, dyn, lane, S.Te), heat = 0.0;
             if (lane == 0) {
@@ -892,8 +1014,8 @@ hipError_t mcb_launch_balance(const mcb::Atomic *dA, const mcb::CellArgs &a, hip
     if (a.ncells <= 0) return hipSuccess;
     const size_t cel = mcb::shared_bytes(a.ncel, a.cel_most);
     if (a.grains) {
-        // the caller passes the frequency-bin count through grains_nb
-        const size_t lds = cel + (size_t)a.grains_nb * sizeof(double) + sizeof(mcb::GrainLds);
+        // the caller passes the frequency-bin and row counts
+        const size_t lds = cel + mcb::grain_bytes(a.grains_nb, a.grains_rows);
         hipLaunchKernelGGL(mcb::balance_kernel<true>, dim3(a.ncells), dim3(64), lds, s, dA, a);
     } else {
         hipLaunchKernelGGL(mcb::balance_kernel<false>, dim3(a.ncells), dim3(64), cel, s, dA, a);

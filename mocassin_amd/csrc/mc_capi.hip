@@ -1005,6 +1005,7 @@ static int update_cells(mc_ctx *c, double jscale, const mc_balance_opts *opts, c
         if (dust && c->dust_pe) {
             a.grains = c->d_grains;
             a.grains_nb = c->G.nbins;
+            a.grains_rows = c->dust_args.nS * c->dust_args.nSizes;
         }
         HIPCHK(c, mcb_launch_balance(c->d_atomic, a, c->stream));
         c->state_dev = true;
