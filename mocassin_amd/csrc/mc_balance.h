@@ -133,6 +133,7 @@ struct CellArgs {
     const Grains *grains;
     int grains_nb, grains_rows;
     int ncel, cel_most;         // of the atomic data: the solves' LDS
+    int nch;                    // its channels: the integrals' grid
     // nullable: block b balances cell order[b] (a permutation of 1..ncells),
     // else cell b + 1; results do not depend on the order
     const int *order;

@@ -743,84 +743,118 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) ba
 // flag (104-154) and, when X is given, the warm-start network's features of
 // the cell (row cell-1 of X [nCells][72]): log10 of J summed over 64
 // contiguous groups of bins, log10 nH, log10 abundances of its seven
-// elements (-30 when absent).  Channels are accumulated eight at a time.
+// elements (-30 when absent).
+//
+// A wavefront takes kIntCh channels of one tile of 64 points; the wavefronts
+// of a tile follow each other on one XCD, so that its L2 serves the tile's J
+// to all but the first.  The coefficients of a channel are wavefront-uniform
+// and come by scalar loads, 16 bins at a time, which leaves LDS out of the
+// loop.  Bound by the FP64 products for large grids and by the chain of bins
+// for small ones.  45^3 octant, 800
+// bins, 31 channels: 1.61 ms with all channels in one wavefront, 0.23 now;
+// 21^3: 1.39, 0.15 now (two or eight channels, or eight bins: 0.30 to 0.43 and
+// 0.15 to 0.39).
+constexpr int kIntCh = 4, kIntBins = 16;
+
+struct Coeffs { double v[kIntBins]; };
+__device__ __forceinline__ Coeffs uniform_row(const double *p)
+{
+    typedef const __attribute__((address_space(4))) Coeffs *Row;
+    return *(const Coeffs *)(Row)(uint64_t)p;
+}
+
 __global__ void __launch_bounds__(64) integrals_kernel(const Atomic *__restrict__ Ap, CellArgs a,
                                                        const double *__restrict__ J3,
-                                                       const int *__restrict__ active, mcd::J3Shape js,
+                                                       const int *__restrict__ active, mcd::J3Shape js, int groups,
                                                        double *__restrict__ Rint, double *__restrict__ Hint,
                                                        int *__restrict__ hit, float *__restrict__ X)
 {
-    constexpr int G = 8, C = 64, U = 16;
-    __shared__ double cr[G][C], ch[G][C];              // coefficients of one chunk of bins
     const Atomic &A = *Ap;
     const int lane = threadIdx.x;
-    const int xyz = mcd::j3_lattice(js, blockIdx.x * 64u + (unsigned)lane);
+    const unsigned i = blockIdx.x >> 3, tile = (i / groups) * 8 + (blockIdx.x & 7);
+    const int g0 = (int)(i % groups) * kIntCh;
+    if (tile >= mcd::j3_points(js) / mcd::kJTile) return;
+    const int xyz = mcd::j3_lattice(js, tile * 64u + (unsigned)lane);
     const int cell = xyz >= 0 ? active[xyz] : 0;
     if (!__any(cell > 0)) return;
     const int nb = A.nbins, nch = A.nch;
     // this wavefront's tile of J3: [nu][64 points], contiguous
-    const double *Jp = J3 + mcd::j3_index(nb, 0, blockIdx.x * 64u) + lane;
-    float *brow = (X && cell > 0) ? X + (size_t)(cell - 1) * mcm::kIn : nullptr;
-    int any = 0;
-    for (int g0 = 0; g0 < nch || g0 == 0; g0 += G) {
-        const int ng = nch - g0 < G ? nch - g0 : G;
-        double r[G], h[G];
-        for (int k = 0; k < G; ++k) { r[k] = 0.0; h[k] = 0.0; }
-        // the first pass visits every bin (hit flag, band sums)
-        int jlo = nb + 1, jhi = 0;
-        for (int k = 0; k < ng; ++k) {
-            const Channel &c = A.ch[g0 + k];
-            jlo = c.ip < jlo ? c.ip : jlo;
-            const int hi = c.hiR > c.hiH ? c.hiR : c.hiH;
-            jhi = hi > jhi ? hi : jhi;
+    const double *Jp = J3 + mcd::j3_index(nb, 0, tile * 64u) + lane;
+    const int ng = nch - g0 < kIntCh ? nch - g0 : kIntCh;
+    double r[kIntCh], h[kIntCh];
+    for (int k = 0; k < kIntCh; ++k) { r[k] = 0.0; h[k] = 0.0; }
+    // the first group visits every bin (hit flag, band sums)
+    int jlo = nb + 1, jhi = 0;
+    for (int k = 0; k < ng; ++k) {
+        const Channel &c = A.ch[g0 + k];
+        jlo = c.ip < jlo ? c.ip : jlo;
+        const int hi = c.hiR > c.hiH ? c.hiR : c.hiH;
+        jhi = hi > jhi ? hi : jhi;
+    }
+    float *brow = nullptr;
+    if (g0 == 0) {
+        jlo = 1;
+        jhi = nb;
+        if (X && cell > 0) brow = X + (size_t)(cell - 1) * mcm::kIn;
+    }
+    double band = 0.0;
+    int any = 0, b = 0, bend = nb / mcm::kBands;
+    double next[kIntBins];
+    for (int u = 0; u < kIntBins; ++u)
+        next[u] = jlo + u <= jhi ? Jp[(size_t)(jlo + u - 1) * mcd::kJTile] : 0.0;
+    for (int j0 = jlo; j0 <= jhi; j0 += kIntBins) {
+        double J[kIntBins];
+        for (int u = 0; u < kIntBins; ++u) {
+            J[u] = next[u] * a.jscale;
+            const int j = j0 + kIntBins + u;
+            next[u] = j <= jhi ? Jp[(size_t)(j - 1) * mcd::kJTile] : 0.0;
         }
-        if (g0 == 0) { jlo = 1; jhi = nb; }
-        double band = 0.0;
-        int b = 0, bend = nb / mcm::kBands;
-        for (int c0 = jlo; c0 <= jhi; c0 += C) {
-            const int cn = jhi - c0 + 1 < C ? jhi - c0 + 1 : C;
-            __syncthreads();
-            for (int k = 0; k < ng; ++k) {
-                const size_t o = (size_t)(g0 + k) * nb + c0 - 1 + lane;
-                cr[k][lane] = lane < cn ? A.cR[o] : 0.0;
-                ch[k][lane] = lane < cn ? A.cH[o] : 0.0;
-            }
-            __syncthreads();
-            for (int u0 = 0; u0 < cn; u0 += U) {
-                double Jv[U];
+        if (j0 + kIntBins - 1 <= jhi) {
 #pragma unroll
-                for (int u = 0; u < U; ++u)
-                    Jv[u] = u0 + u < cn ? Jp[(size_t)(c0 + u0 + u - 1) * mcd::kJTile] * a.jscale : 0.0;
+            for (int k = 0; k < kIntCh; ++k)
+                if (k < ng) {
+                    const size_t o = (size_t)(g0 + k) * nb + j0 - 1;
+                    const Coeffs cr = uniform_row(A.cR + o), ch = uniform_row(A.cH + o);
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    if (u0 + u >= cn) break;
-                    const double J = Jv[u];
-                    for (int k = 0; k < ng; ++k) {
-                        r[k] = r[k] + J * cr[k][u0 + u];
-                        h[k] = h[k] + J * ch[k][u0 + u];
-                    }
-                    if (g0 == 0) {
-                        const int j = c0 + u0 + u;
-                        any |= J > 0.0;
-                        band += J;
-                        if (j == bend) {
-                            if (brow) brow[b] = (float)log10(fmax(band, 1.e-30));
-                            band = 0.0;
-                            ++b;
-                            bend = (b + 1) * nb / mcm::kBands;
-                        }
+                    for (int u = 0; u < kIntBins; ++u) {
+                        r[k] = __builtin_fma(J[u], cr.v[u], r[k]);
+                        h[k] = __builtin_fma(J[u], ch.v[u], h[k]);
                     }
                 }
-            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < kIntBins; ++u)
+                if (j0 + u <= jhi) {
+#pragma unroll
+                    for (int k = 0; k < kIntCh; ++k)
+                        if (k < ng) {
+                            const size_t o = (size_t)(g0 + k) * nb + j0 - 1 + u;
+                            r[k] = __builtin_fma(J[u], A.cR[o], r[k]);
+                            h[k] = __builtin_fma(J[u], A.cH[o], h[k]);
+                        }
+                }
         }
-        if (cell > 0)
-            for (int k = 0; k < ng; ++k) {
-                Rint[(size_t)cell * nch + g0 + k] = r[k];
-                Hint[(size_t)cell * nch + g0 + k] = h[k];
+        if (g0 == 0)
+#pragma unroll
+            for (int u = 0; u < kIntBins; ++u) {
+                any |= J[u] > 0.0;
+                band += J[u];
+                if (j0 + u == bend) {
+                    if (brow) brow[b] = (float)log10(fmax(band, 1.e-30));
+                    band = 0.0;
+                    ++b;
+                    bend = (b + 1) * nb / mcm::kBands;
+                }
             }
-        if (nch == 0) break;
     }
     if (cell <= 0) return;
+#pragma unroll
+    for (int k = 0; k < kIntCh; ++k)
+        if (k < ng) {
+            Rint[(size_t)cell * nch + g0 + k] = r[k];
+            Hint[(size_t)cell * nch + g0 + k] = h[k];
+        }
+    if (g0 != 0) return;
     hit[cell] = any;
     if (brow) {
         float *row = brow;
@@ -1027,8 +1061,10 @@ hipError_t mcb_launch_integrals(const mcb::Atomic *dA, const mcb::CellArgs &a, c
                                int nx, int ny, int nz, double *Rint, double *Hint, int *hit, float *X, hipStream_t s)
 {
     const mcd::J3Shape js = mcd::j3_shape(nx, ny, nz);
-    hipLaunchKernelGGL(mcb::integrals_kernel, dim3((unsigned)(mcd::j3_points(js) / mcd::kJTile)), dim3(64), 0, s,
-                       dA, a, J3, active, js, Rint, Hint, hit, X);
+    const unsigned tiles = (unsigned)(mcd::j3_points(js) / mcd::kJTile);
+    const int groups = a.nch > mcb::kIntCh ? (a.nch + mcb::kIntCh - 1) / mcb::kIntCh : 1;
+    hipLaunchKernelGGL(mcb::integrals_kernel, dim3((tiles + 7) / 8 * 8 * groups), dim3(64), 0, s, dA, a, J3, active, js,
+                       groups, Rint, Hint, hit, X);
     return hipGetLastError();
 }
 

@@ -669,6 +669,7 @@ static mcb::CellArgs cell_args(mc_ctx *c, double jscale)
     a.warm_iter = a.max_iter;
     a.ncel = c->bal.A.ncel;
     a.cel_most = c->bal.A.cel_most;
+    a.nch = c->bal.A.nch;
     return a;
 }
 
