@@ -999,7 +999,7 @@ static int update_cells(mc_ctx *c, double jscale, const mc_balance_opts *opts, c
         if (rc) return rc;
         if (warm) {
             HIPCHK(c, mcm_standardise(c->d_mX, nc, mlp_scale(c), c->d_mX0, c->stream));
-            HIPCHK(c, mcm_forward(c->d_mX0, nc, mlp_net(c), c->d_mY, mcm::kOutP, nullptr, 2 * c->cus, c->stream));
+            HIPCHK(c, mcm_forward(c->d_mX0, nc, mlp_net(c), c->d_mY, mcm::kOutP, 2 * c->cus, c->stream));
             HIPCHK(c, mcm_unscale(c->d_mY, nc, mcm::kOutP, mlp_scale(c), c->stream));
             HIPCHK(c, mcb_launch_warm(c->d_atomic, a, c->d_mY, mcm::kOutP, c->d_hit, c->stream));
         }
@@ -1699,13 +1699,13 @@ extern "C" int mc_mlp_features(mc_ctx *c, double jscale, const double *Hden, flo
 
 // device copies of a host data set and the batch buffers of a training call
 struct MlpBatch {
-    float *X = nullptr, *T = nullptr, *M = nullptr, *Yb = nullptr, *Tb = nullptr, *Mb = nullptr;
-    uint16_t *X0 = nullptr, *H = nullptr, *dA = nullptr, *dB = nullptr;
+    float *X = nullptr, *T = nullptr, *M = nullptr, *part = nullptr;
+    uint16_t *mem = nullptr, *WT = nullptr;
     int *idx = nullptr;
     double *sums = nullptr;
     void release()
     {
-        void *b[] = { X, T, M, Yb, Tb, Mb, X0, H, dA, dB, idx, sums };
+        void *b[] = { X, T, M, part, mem, WT, idx, sums };
         for (void *p : b)
             if (p) (void)hipFree(p);
     }
@@ -1717,13 +1717,9 @@ static hipError_t batch_alloc(MlpBatch &B, int64_t n, int batch, int64_t nidx, i
     if ((e = dalloc(&B.X, (size_t)n * mcm::kIn)) != hipSuccess) return e;
     if ((e = dalloc(&B.T, (size_t)n * mcm::kOut)) != hipSuccess) return e;
     if ((e = dalloc(&B.M, (size_t)n * mcm::kOut)) != hipSuccess) return e;
-    if ((e = dalloc(&B.Yb, (size_t)batch * mcm::kOutP)) != hipSuccess) return e;
-    if ((e = dalloc(&B.Tb, (size_t)batch * mcm::kOut)) != hipSuccess) return e;
-    if ((e = dalloc(&B.Mb, (size_t)batch * mcm::kOut)) != hipSuccess) return e;
-    if ((e = dalloc(&B.X0, (size_t)batch * mcm::kInP)) != hipSuccess) return e;
-    if ((e = dalloc(&B.H, (size_t)3 * batch * mcm::kHid)) != hipSuccess) return e;
-    if ((e = dalloc(&B.dA, (size_t)batch * mcm::kHid)) != hipSuccess) return e;
-    if ((e = dalloc(&B.dB, (size_t)batch * mcm::kHid)) != hipSuccess) return e;
+    if ((e = dalloc(&B.part, (size_t)mcm_train_slices(batch) * mcm::kParams)) != hipSuccess) return e;
+    if ((e = dalloc(&B.mem, mcm_train_elems(batch))) != hipSuccess) return e;
+    if ((e = dalloc(&B.WT, (size_t)mcm::kParams)) != hipSuccess) return e;
     if ((e = dalloc(&B.idx, (size_t)nidx)) != hipSuccess) return e;
     return dalloc(&B.sums, (size_t)nsums);
 }
@@ -1750,15 +1746,11 @@ static hipError_t upload_data(mc_ctx *c, MlpBatch &B, const float *X, const floa
     return e;
 }
 
-// forward + backward of one batch (rows idx[0..nb)); sums must be zero
+// gradient of one batch (rows idx[0..nb)) in slices; sums must be zero
 static hipError_t train_pass(mc_ctx *c, MlpBatch &B, const int *idx, int nb, double *sums)
 {
-    hipError_t e = mcm_gather(B.X, B.T, B.M, idx, nb, mlp_scale(c), B.X0, B.Tb, B.Mb, c->stream);
-    if (e == hipSuccess) e = mcm_forward(B.X0, nb, mlp_net(c), B.Yb, mcm::kOutP, B.H, 2 * c->cus, c->stream);
-    if (e == hipSuccess)
-        e = mcm_backward(B.X0, B.H, B.Yb, B.Tb, B.Mb, nb, mlp_net(c), B.dA, B.dB,
-                         c->d_mlp + mcm::kParams, sums, c->stream);
-    return e;
+    return mcm_gradient(B.X, B.T, B.M, idx, nb, mlp_scale(c), mlp_net(c), B.WT, B.mem, B.part, sums, 2 * c->cus,
+                        c->stream);
 }
 
 extern "C" int mc_mlp_predict(mc_ctx *c, const float *X, int64_t n, float *Y)
@@ -1775,7 +1767,7 @@ extern "C" int mc_mlp_predict(mc_ctx *c, const float *X, int64_t n, float *Y)
     if (e == hipSuccess)
         e = hipMemcpyAsync(dX, X, (size_t)n * mcm::kIn * sizeof(float), hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) e = mcm_standardise(dX, (int)n, mlp_scale(c), dX0, c->stream);
-    if (e == hipSuccess) e = mcm_forward(dX0, (int)n, mlp_net(c), dY, mcm::kOut, nullptr, 2 * c->cus, c->stream);
+    if (e == hipSuccess) e = mcm_forward(dX0, (int)n, mlp_net(c), dY, mcm::kOut, 2 * c->cus, c->stream);
     if (e == hipSuccess) e = mcm_unscale(dY, (int)n, mcm::kOut, mlp_scale(c), c->stream);
     if (e == hipSuccess)
         e = hipMemcpyAsync(Y, dY, (size_t)n * mcm::kOut * sizeof(float), hipMemcpyDeviceToHost, c->stream);
@@ -1802,7 +1794,9 @@ extern "C" int mc_mlp_loss_grad(mc_ctx *c, const float *X, const float *T, const
     if (e == hipSuccess) e = upload_data(c, B, X, T, M, n);
     if (e == hipSuccess) e = hipMemcpyAsync(B.idx, idx.data(), n * sizeof(int), hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) e = hipMemsetAsync(B.sums, 0, 2 * sizeof(double), c->stream);
+    if (e == hipSuccess) e = mcm_transpose(c->d_mlpW, B.WT, c->stream);
     if (e == hipSuccess) e = train_pass(c, B, B.idx, (int)n, B.sums);
+    if (e == hipSuccess) e = mcm_sum(B.part, mcm_train_slices((int)n), c->d_mlp + mcm::kParams, c->stream);
     if (e == hipSuccess)
         e = hipMemcpyAsync(grad, c->d_mlp + mcm::kParams, mcm::kParams * sizeof(float), hipMemcpyDeviceToHost,
                            c->stream);
@@ -1836,10 +1830,12 @@ extern "C" int mc_mlp_train(mc_ctx *c, const float *X, const float *T, const flo
     if (e == hipSuccess) e = hipMemcpyAsync(B.idx, order, nidx * sizeof(int), hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) e = hipMemsetAsync(B.sums, 0, 2 * steps * sizeof(double), c->stream);
     if (e == hipSuccess) e = hipEventRecord(c->ev0, c->stream);
-    float *P = c->d_mlp, *G = P + mcm::kParams, *m1 = G + mcm::kParams, *m2 = m1 + mcm::kParams;
+    if (e == hipSuccess) e = mcm_transpose(c->d_mlpW, B.WT, c->stream);
+    float *P = c->d_mlp, *m1 = P + 2 * (size_t)mcm::kParams, *m2 = m1 + mcm::kParams;
     for (int s = 0; s < steps && e == hipSuccess; ++s) {
         e = train_pass(c, B, B.idx + (size_t)s * batch, batch, B.sums + 2 * s);
-        if (e == hipSuccess) e = mcm_adam(P, G, m1, m2, B.sums + 2 * s, ++c->mlp_step, lr, c->d_mlpW, c->stream);
+        if (e == hipSuccess) e = mcm_adam(P, B.part, mcm_train_slices(batch), m1, m2, B.sums + 2 * s, ++c->mlp_step, lr, c->d_mlpW,
+                         B.WT, c->stream);
     }
     if (e == hipSuccess) e = hipEventRecord(c->ev1, c->stream);
     std::vector<double> sums(2 * (size_t)steps);

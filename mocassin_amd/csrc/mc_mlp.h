@@ -43,25 +43,47 @@ struct Scale {
     const float *xmean, *xstd, *ymean, *ystd;
 };
 
+// What a training step keeps of a batch: BF16 inputs, hidden activations and
+// back-propagated rows as [tile][feature][16 rows]; layer l of H and D at
+// l * stride.
+struct TrainBuf {
+    uint16_t *X, *H, *D, *D3;
+    size_t stride;
+};
+
 }  // namespace mcm
 
 // launchers (mc_mlp.hip); every pointer is device memory.
-// forward: X0 bf16 [n][kInP] -> Y fp32 [n][ldy] (standardised outputs);
-// H (nullable) bf16 [3][n][kHid] keeps the hidden activations for backward.
-hipError_t mcm_forward(const uint16_t *X0, int n, mcm::Net net, float *Y, int ldy, uint16_t *H,
-                       int blocks, hipStream_t s);
-// backward of L = sum M (Y - T)^2 over a batch: grad (fp32 [kParams]) gets
-// the unnormalised gradient 2 sum M (Y - T) dY/dP; sums[0] += sum M (Y-T)^2,
-// sums[1] += sum M (zero them first).  dA, dB: bf16 scratch [n][kHid].
-hipError_t mcm_backward(const uint16_t *X0, const uint16_t *H, const float *Y, const float *T,
-                        const float *M, int n, mcm::Net net, uint16_t *dA, uint16_t *dB,
-                        float *grad, double *sums, hipStream_t s);
-// Adam step t (1-based) on grad / sums[1]; refreshes the bf16 copy
-hipError_t mcm_adam(float *P, const float *grad, float *m, float *v, const double *sums, int t,
-                    float lr, uint16_t *W, hipStream_t s);
+// forward: X0 bf16 [n][kInP] -> Y fp32 [n][ldy] (standardised outputs)
+hipError_t mcm_forward(const uint16_t *X0, int n, mcm::Net net, float *Y, int ldy, int blocks, hipStream_t s);
+// A batch of n rows: an even number of 16-row tiles (zero rows fill the
+// last), and the slices its gradient is formed in (at least 8 steps of 32
+// rows each, 16 slices at most: 4096 rows and more fill the chip).
+inline int mcm_train_tiles(int n) { return (n + 31) / 32 * 2; }
+inline int mcm_train_slices(int n)
+{
+    const int s = mcm_train_tiles(n) / 16;
+    return s < 1 ? 1 : s > 16 ? 16 : s;
+}
+// its working memory in BF16 elements
+inline size_t mcm_train_elems(int n)
+{
+    return (size_t)mcm_train_tiles(n) * 16 * (mcm::kInP + 6 * mcm::kHid + mcm::kOutP);
+}
+// W (published BF16) transposed per layer: [in][out] at w_off
+hipError_t mcm_transpose(const uint16_t *W, uint16_t *WT, hipStream_t s);
+// gradient of L = sum M (Y - T)^2 over rows idx[0..n) of a raw data set:
+// part [mcm_train_slices(n)][kParams] gets the slices of the unnormalised
+// gradient 2 sum M (Y - T) dY/dP; sums[0] += sum M (Y-T)^2, sums[1] += sum M
+// (zero them first).  mem: mcm_train_elems(n).
+hipError_t mcm_gradient(const float *Xs, const float *Ts, const float *Ms, const int *idx, int n, mcm::Scale sc,
+                        mcm::Net net, const uint16_t *WT, uint16_t *mem, float *part, double *sums, int blocks,
+                        hipStream_t s);
+hipError_t mcm_sum(const float *part, int slices, float *grad, hipStream_t s);
+// Adam step t (1-based) on the sum of the slices / sums[1]; refreshes the
+// BF16 copies
+hipError_t mcm_adam(float *P, const float *part, int slices, float *m, float *v, const double *sums, int t,
+                    float lr, uint16_t *W, uint16_t *WT, hipStream_t s);
 hipError_t mcm_publish(const float *P, uint16_t *W, hipStream_t s);
-// batch rows idx[0..n) of a raw data set: standardised bf16 features, standardised targets, mask
-hipError_t mcm_gather(const float *Xs, const float *Ts, const float *Ms, const int *idx, int n,
-                      mcm::Scale sc, uint16_t *X0, float *T, float *M, hipStream_t s);
 hipError_t mcm_standardise(const float *Xraw, int n, mcm::Scale sc, uint16_t *X0, hipStream_t s);
 hipError_t mcm_unscale(float *Y, int n, int ldy, mcm::Scale sc, hipStream_t s);

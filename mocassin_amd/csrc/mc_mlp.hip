@@ -1,5 +1,5 @@
-// mc_mlp.hip - kernels of the warm-start network (see mc_mlp.h): fused
-// forward, backward GEMMs, loss, Adam, and the data movers around them.
+// mc_mlp.hip - kernels of the warm-start network (see mc_mlp.h): the fused
+// forward pass, the training step, and the data movers around them.
 //
 // Matrix products use v_mfma_f32_16x16x32_bf16 (one 64-lane wavefront
 // computes a 16x16 FP32 tile from 16x32 and 32x16 BF16 operands).  Operand
@@ -31,6 +31,14 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c)
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
+// w_off and b_off of a layer known at run time only
+__device__ __forceinline__ int w_at(int l)
+{
+    constexpr int o[kLayers + 1] = { w_off(0), w_off(1), w_off(2), w_off(3), kParams };
+    return l == 0 ? o[0] : l == 1 ? o[1] : l == 2 ? o[2] : l == 3 ? o[3] : o[4];
+}
+__device__ __forceinline__ int b_at(int l) { return w_at(l) + layer_out(l) * layer_in(l); }
+
 // ------------------------------------------------------------- forward
 // LDS: the four weight matrices (row stride in + 8 to spread banks), the
 // biases, and per wavefront two 16-row activation buffers (stride 136).
@@ -41,14 +49,18 @@ __host__ __device__ constexpr int lw_off(int l)
 {
     return l == 0 ? 0 : lw_off(l - 1) + layer_out(l - 1) * lw_stride(l - 1);
 }
+__device__ __forceinline__ int lw_at(int l)
+{
+    constexpr int o[kLayers] = { lw_off(0), lw_off(1), lw_off(2), lw_off(3) };
+    return l == 0 ? o[0] : l == 1 ? o[1] : l == 2 ? o[2] : o[3];
+}
 constexpr int kLdsW = lw_off(kLayers);                                   // bf16 elements
 constexpr int kLdsBias = kHid * 3 + kOutP;                               // floats
 constexpr int kLdsAct = 4 * 2 * 16 * kActS;                              // bf16 elements
 constexpr size_t kFwdLds = (size_t)kLdsW * 2 + (size_t)kLdsBias * 4 + (size_t)kLdsAct * 2;
 
 __global__ void __launch_bounds__(256) forward_kernel(const uint16_t *__restrict__ X0, int n, Net net,
-                                                      float *__restrict__ Y, int ldy,
-                                                      uint16_t *__restrict__ H)
+                                                      float *__restrict__ Y, int ldy)
 {
     extern __shared__ __align__(16) unsigned char lds[];
     uint16_t *Ws = reinterpret_cast<uint16_t *>(lds);
@@ -58,16 +70,16 @@ __global__ void __launch_bounds__(256) forward_kernel(const uint16_t *__restrict
     // weights and biases into LDS, 16 bytes at a time
     for (int l = 0; l < kLayers; ++l) {
         const int K = layer_in(l), N = layer_out(l), vpr = K / 8;
-        const uint16_t *src = net.W + w_off(l);
+        const uint16_t *src = net.W + w_at(l);
         for (int e = tid; e < N * vpr; e += 256) {
             const int r = e / vpr, v = e % vpr;
-            *reinterpret_cast<uint4 *>(Ws + lw_off(l) + r * lw_stride(l) + v * 8) =
+            *reinterpret_cast<uint4 *>(Ws + lw_at(l) + r * lw_stride(l) + v * 8) =
                 *reinterpret_cast<const uint4 *>(src + (size_t)r * K + v * 8);
         }
     }
     for (int e = tid; e < kLdsBias; e += 256) {
         const int l = e < 3 * kHid ? e / kHid : 3, j = e < 3 * kHid ? e % kHid : e - 3 * kHid;
-        bias[e] = net.P[b_off(l) + j];
+        bias[e] = net.P[b_at(l) + j];
     }
     uint16_t *a0 = act + (size_t)(w * 2) * 16 * kActS, *a1 = a0 + 16 * kActS;
     const int ntiles = (n + kTile - 1) / kTile;
@@ -86,7 +98,7 @@ __global__ void __launch_bounds__(256) forward_kernel(const uint16_t *__restrict
             const uint16_t *in = (l & 1) ? a1 : a0;
             uint16_t *out = (l & 1) ? a0 : a1;
             const int K = layer_in(l), N = layer_out(l);
-            const uint16_t *Wl = Ws + lw_off(l);
+            const uint16_t *Wl = Ws + lw_at(l);
             const float *bl = bias + l * kHid;
             for (int t = 0; t < N / 16; ++t) {
                 f32x4 acc = { 0.f, 0.f, 0.f, 0.f };
@@ -101,9 +113,7 @@ __global__ void __launch_bounds__(256) forward_kernel(const uint16_t *__restrict
                     float v = acc[i] + bl[col];
                     if (l < kLayers - 1) {
                         v = v > 0.f ? v : 0.f;
-                        const uint16_t h = f2bf(v);
-                        out[row * kActS + col] = h;
-                        if (H && r0 + row < n) H[((size_t)l * n + r0 + row) * kHid + col] = h;
+                        out[row * kActS + col] = f2bf(v);
                     } else if (col < kOut && r0 + row < n) {
                         Y[(size_t)(r0 + row) * ldy + col] = v;
                     }
@@ -114,113 +124,310 @@ __global__ void __launch_bounds__(256) forward_kernel(const uint16_t *__restrict
     }
 }
 
-// ---------------------------------------------------------------- GEMM
-// C[M][N] = sum_k A(m,k) B(k,n), A(m,k) = A[m*sam + k*sak],
-// B(k,n) = B[k*sbk + n*sbn], BF16 operands staged in LDS (k contiguous),
-// 64x64 tile per workgroup, K step 32.  EPI_F32_ADD splits K over
-// blockIdx.z (kc rows each) and adds into a zeroed C32.
-enum { EPI_F32_ADD = 0, EPI_RELU_MASK = 1 };
+__device__ __forceinline__ float stdz(float x, float mean, float sd) { return (x - mean) / sd; }
 
-template <int EPI>
-__global__ void __launch_bounds__(256) gemm_kernel(const uint16_t *__restrict__ A, long sam, long sak,
-                                                   const uint16_t *__restrict__ B, long sbk, long sbn,
-                                                   int M, int N, int K, int kc, float *__restrict__ C32,
-                                                   uint16_t *__restrict__ C16, int ldc,
-                                                   const uint16_t *__restrict__ Hm, int ldh)
+template <int S> struct Steps { static constexpr int value = S; };
+
+// ------------------------------------------------------------- training
+// A training step is three launches: step_kernel takes 16 rows at a time
+// through standardisation, forward pass, loss and backward pass; grad_kernel
+// forms the weight and bias gradients of slices of the batch; adam_kernel
+// adds the slices in order and updates.  The rounding points are those of
+// the layers one by one: BF16 inputs, activations and back-propagated rows,
+// FP32 sums on the matrix cores.
+//
+// The step is bound by latency (a 4096-row batch is 4 GFLOP): so a workgroup
+// loads every weight fragment it will use into registers at its start, 44 of
+// them a lane, all in flight at once, and then needs nothing but LDS between
+// its layers.  Inputs, activations and back-propagated rows go to memory as
+// [tile][feature][16 rows]: a lane's four rows of a result are 8 contiguous
+// bytes, and grad_kernel, whose inner index is the row, reads its fragments
+// 16 bytes a lane without staging.  One step of 4096 rows: 181 us of
+// kernels as 14 launches of one operation each, 28 now (18 + 6 + 4).
+constexpr int kRows = 16;                      // rows of a tile
+constexpr int kTrainS = kHid + 8;              // LDS row stride of a tile
+
+// the four wavefronts of a workgroup share a tile; wavefront w computes the
+// feature tiles 2 w and 2 w + 1 of a layer
+__global__ void __launch_bounds__(256, 1) step_kernel(const float *__restrict__ Xs, const float *__restrict__ Ts,
+                                                      const float *__restrict__ Ms, const int *__restrict__ idx,
+                                                      int n, int tiles, Scale sc, Net net,
+                                                      const uint16_t *__restrict__ WT, TrainBuf B,
+                                                      double *__restrict__ sums)
 {
-    constexpr int S = 40;
-    __shared__ __align__(16) uint16_t As[64 * S], Bs[64 * S];
+    __shared__ __align__(16) uint16_t buf[2][kRows * kTrainS];
+    __shared__ float bias[3 * kHid + kOutP], xs[2 * kIn], ys[2 * kOut];
+    __shared__ double red[2][4];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
     const int lr = lane & 15, lk = (lane >> 4) * 8, lrow = (lane >> 4) * 4;
-    f32x4 acc[4];
-    for (int t = 0; t < 4; ++t) acc[t] = f32x4{ 0.f, 0.f, 0.f, 0.f };
-    const int rr = tid >> 2, kk = (tid & 3) * 8;
-    const int kb = blockIdx.z * kc, ke = kb + kc < K ? kb + kc : K;
-    for (int k0 = kb; k0 < ke; k0 += 32) {
-        for (int i = 0; i < 8; ++i) {
-            const int k = k0 + kk + i, m = m0 + rr, nn = n0 + rr;
-            As[rr * S + kk + i] = (m < M && k < ke) ? A[(long)m * sam + (long)k * sak] : (uint16_t)0;
-            Bs[rr * S + kk + i] = (nn < N && k < ke) ? B[(long)k * sbk + (long)nn * sbn] : (uint16_t)0;
-        }
-        __syncthreads();
-        const bf16x8 a = ld8(As + (16 * w + lr) * S + lk);
-        for (int t = 0; t < 4; ++t) acc[t] = mfma(a, ld8(Bs + (16 * t + lr) * S + lk), acc[t]);
-        __syncthreads();
-    }
-    for (int t = 0; t < 4; ++t)
+    // A tile's rows of the data set, all loads of a kind in flight together:
+    // inputs, then targets and masks of the outputs this lane will see (w <
+    // 2); rows beyond the batch and padded columns load in range.  The data
+    // of the tile after, and the row numbers of the one after that, are on
+    // their way while a tile is worked on.
+    constexpr int kE = kRows * kInP / 256;
+    const int oc = 16 * w + lr;
+    int row[kE], orow[4];
+    float xn[kE], tn[4], mn[4];
+    auto load_rows = [&](int tile) {
+        const int r0 = min(tile, tiles) * kRows;
+#pragma unroll
+        for (int u = 0; u < kE; ++u) row[u] = idx[min(n - 1, r0 + (tid + 256 * u) / kInP)];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) orow[i] = idx[min(n - 1, r0 + lrow + i)];
+    };
+    auto load_data = [&] {
+#pragma unroll
+        for (int u = 0; u < kE; ++u) xn[u] = Xs[(size_t)row[u] * kIn + min(kIn - 1, (tid + 256 * u) % kInP)];
+#pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int row = m0 + 16 * w + lrow + i, col = n0 + 16 * t + lr;
-            if (row >= M || col >= N) continue;
-            if (EPI == EPI_F32_ADD) {
-                atomicAdd(&C32[(long)row * ldc + col], acc[t][i]);
-            } else {
-                const float v = bf2f(Hm[(long)row * ldh + col]) > 0.f ? acc[t][i] : 0.f;
-                C16[(long)row * ldc + col] = f2bf(v);
-            }
+            const size_t src = (size_t)orow[i] * kOut + min(kOut - 1, oc);
+            tn[i] = Ts[src];
+            mn[i] = Ms[src];
         }
-}
-
-// dY = 2 M (Y - T) as bf16 [n][kOutP] (column kOutP-1 zero); sums of M (Y-T)^2 and M
-__global__ void __launch_bounds__(256) loss_kernel(const float *__restrict__ Y, const float *__restrict__ T,
-                                                   const float *__restrict__ Mk, int n,
-                                                   uint16_t *__restrict__ dY, double *__restrict__ sums)
-{
-    __shared__ double red[2][256];
+    };
+    load_rows(blockIdx.x);
+    for (int e = tid; e < 2 * kIn; e += 256) xs[e] = e < kIn ? sc.xmean[e] : sc.xstd[e - kIn];
+    for (int e = tid; e < 2 * kOut; e += 256) ys[e] = e < kOut ? sc.ymean[e] : sc.ystd[e - kOut];
+    load_data();
+    load_rows(blockIdx.x + gridDim.x);
+    // forward fragments W_l[out 16 t + lr][in 32 s + lk ..], backward
+    // WT_l[in 16 t + lr][out 32 s + lk ..]
+    constexpr int w0 = w_off(0), w1 = w_off(1), w2 = w_off(2), w3 = w_off(3);
+    bf16x8 f0[2][3], f1[2][4], f2[2][4], f3[4], b3[2], b2[2][4], b1[2][4];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int o = 16 * (2 * w + u) + lr;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            if (s < 3) f0[u][s] = ld8(net.W + w0 + o * kInP + 32 * s + lk);
+            f1[u][s] = ld8(net.W + w1 + o * kHid + 32 * s + lk);
+            f2[u][s] = ld8(net.W + w2 + o * kHid + 32 * s + lk);
+            b2[u][s] = ld8(WT + w2 + o * kHid + 32 * s + lk);
+            b1[u][s] = ld8(WT + w1 + o * kHid + 32 * s + lk);
+        }
+        b3[u] = ld8(WT + w3 + o * kOutP + lk);
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) f3[s] = ld8(net.W + w3 + (16 * (w & 1) + lr) * kHid + 32 * s + lk);
+    for (int e = tid; e < 3 * kHid + kOutP; e += 256) {
+        const int l = e < 3 * kHid ? e / kHid : 3;
+        bias[e] = net.P[b_at(l) + e - l * kHid];
+    }
     double l2 = 0.0, mm = 0.0;
-    for (long e = (long)blockIdx.x * 256 + threadIdx.x; e < (long)n * kOutP; e += (long)gridDim.x * 256) {
-        const long r = e / kOutP;
-        const int j = (int)(e % kOutP);
-        float g = 0.f;
-        if (j < kOut) {
-            const float m = Mk[r * kOut + j], d = Y[r * kOutP + j] - T[r * kOut + j];
-            g = 2.f * m * d;
-            l2 += (double)m * (double)d * (double)d;
-            mm += (double)m;
-        }
-        dY[e] = f2bf(g);
-    }
-    red[0][threadIdx.x] = l2;
-    red[1][threadIdx.x] = mm;
     __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) {
-            red[0][threadIdx.x] += red[0][threadIdx.x + o];
-            red[1][threadIdx.x] += red[1][threadIdx.x + o];
+
+    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const int r0 = tile * kRows;
+        float xv[kE], tv[4], mv[4];
+#pragma unroll
+        for (int u = 0; u < kE; ++u) xv[u] = xn[u];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { tv[i] = tn[i]; mv[i] = mn[i]; }
+        if (tile + (int)gridDim.x < tiles) {
+            load_data();
+            load_rows(tile + 2 * (int)gridDim.x);
+        }
+#pragma unroll
+        for (int u = 0; u < kE; ++u) {
+            const int r = (tid + 256 * u) / kInP, j = (tid + 256 * u) % kInP, k = min(kIn - 1, j);
+            const uint16_t v = f2bf(stdz(xv[u], xs[k], xs[kIn + k]));
+            buf[0][r * kTrainS + j] = j < kIn && r0 + r < n ? v : (uint16_t)0;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int k = min(kOut - 1, oc);
+            const bool on = oc < kOut && r0 + lrow + i < n;
+            tv[i] = on ? stdz(tv[i], ys[k], ys[kOut + k]) : 0.f;
+            mv[i] = on ? mv[i] : 0.f;
         }
         __syncthreads();
+        if (tid < 2 * kInP) {
+            uint16_t q[8];
+            for (int i = 0; i < 8; ++i) q[i] = buf[0][((tid & 1) * 8 + i) * kTrainS + tid / 2];
+            *reinterpret_cast<uint4 *>(B.X + ((size_t)tile * kInP + tid / 2) * kRows + (tid & 1) * 8) =
+                __builtin_bit_cast(uint4, q);
+        }
+        unsigned on[3] = { 0u, 0u, 0u };        // a bit per hidden activation above zero
+        // one layer: `in` times the fragments, through `store` per feature
+        auto product = [&](const uint16_t *in, auto steps, auto frag, auto store) {
+            constexpr int S = decltype(steps)::value;
+            bf16x8 a[S];
+#pragma unroll
+            for (int s = 0; s < S; ++s) a[s] = ld8(in + lr * kTrainS + 32 * s + lk);
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                f32x4 acc = { 0.f, 0.f, 0.f, 0.f };
+#pragma unroll
+                for (int s = 0; s < S; ++s) acc = mfma(a[s], frag(u, s), acc);
+                store(u, 16 * (2 * w + u) + lr, acc);
+            }
+        };
+        // four rows of a feature to LDS and to memory
+        auto put = [&](uint16_t *out, uint16_t *mem, int col, const uint16_t *q) {
+            if (out)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) out[(lrow + i) * kTrainS + col] = q[i];
+            *reinterpret_cast<uint2 *>(mem + ((size_t)tile * kHid + col) * kRows + lrow) =
+                make_uint2(q[0] | (unsigned)q[1] << 16, q[2] | (unsigned)q[3] << 16);
+        };
+        auto hidden = [&](int l, uint16_t *out) {
+            return [&, l, out](int u, int col, const f32x4 &acc) {
+                uint16_t q[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float v = acc[i] + bias[l * kHid + col];
+                    q[i] = f2bf(v > 0.f ? v : 0.f);
+                    if (q[i]) on[l] |= 1u << (4 * u + i);
+                }
+                put(out, B.H + (size_t)l * B.stride, col, q);
+            };
+        };
+        auto back = [&](int l, uint16_t *out) {
+            return [&, l, out](int u, int col, const f32x4 &acc) {
+                uint16_t q[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) q[i] = f2bf(on[l] >> (4 * u + i) & 1u ? acc[i] : 0.f);
+                put(out, B.D + (size_t)l * B.stride, col, q);
+            };
+        };
+        product(buf[0], Steps<3>{}, [&](int u, int s) { return f0[u][s]; }, hidden(0, buf[1]));
+        __syncthreads();
+        product(buf[1], Steps<4>{}, [&](int u, int s) { return f1[u][s]; }, hidden(1, buf[0]));
+        __syncthreads();
+        product(buf[0], Steps<4>{}, [&](int u, int s) { return f2[u][s]; }, hidden(2, buf[1]));
+        __syncthreads();
+        // outputs and dY = 2 M (Y - T): feature tile w of two
+        if (w < 2) {
+            f32x4 acc = { 0.f, 0.f, 0.f, 0.f };
+#pragma unroll
+            for (int s = 0; s < 4; ++s) acc = mfma(ld8(buf[1] + lr * kTrainS + 32 * s + lk), f3[s], acc);
+            uint16_t q[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float d = acc[i] + bias[3 * kHid + oc] - tv[i], m = mv[i];
+                q[i] = f2bf(oc < kOut && r0 + lrow + i < n ? 2.f * m * d : 0.f);
+                l2 += (double)m * (double)d * (double)d;
+                mm += (double)m;
+                buf[0][(lrow + i) * kTrainS + oc] = q[i];
+            }
+            *reinterpret_cast<uint2 *>(B.D3 + ((size_t)tile * kOutP + oc) * kRows + lrow) =
+                make_uint2(q[0] | (unsigned)q[1] << 16, q[2] | (unsigned)q[3] << 16);
+        }
+        __syncthreads();
+        product(buf[0], Steps<1>{}, [&](int u, int) { return b3[u]; }, back(2, buf[1]));
+        __syncthreads();
+        product(buf[1], Steps<4>{}, [&](int u, int s) { return b2[u][s]; }, back(1, buf[0]));
+        __syncthreads();
+        product(buf[0], Steps<4>{}, [&](int u, int s) { return b1[u][s]; }, back(0, nullptr));
+        __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        atomicAdd(&sums[0], red[0][0]);
-        atomicAdd(&sums[1], red[1][0]);
+    for (int o = 32; o >= 1; o >>= 1) {
+        l2 += __shfl_xor(l2, o);
+        mm += __shfl_xor(mm, o);
     }
+    if (lane == 0) { red[0][w] = l2; red[1][w] = mm; }
+    __syncthreads();
+    if (tid < 2) atomicAdd(&sums[tid], red[tid][0] + red[tid][1]);      // wavefronts 2 and 3 see no output
 }
 
-// out[j] = sum_r dY[r][j], one workgroup per column
-__global__ void __launch_bounds__(256) colsum_kernel(const uint16_t *__restrict__ dY, int n, int ld,
-                                                     float *__restrict__ out)
+// dW_l[out][in] = sum over rows of dZ_l[out] prev_l[in], db_l = sum of dZ_l:
+// one wavefront per 32 x 32 weights and slice of `per` steps of 32 rows,
+// into part[slice][parameter].
+constexpr int kGradTiles = 4 * 3 + 4 * 4 + 4 * 4 + 1 * 4;
+__global__ void __launch_bounds__(64) grad_kernel(TrainBuf B, int steps, int per, float *__restrict__ part)
 {
-    __shared__ float red[256];
-    const int j = blockIdx.x;
-    float s = 0.f;
-    for (int r = threadIdx.x; r < n; r += 256) s += bf2f(dY[(long)r * ld + j]);
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-        __syncthreads();
+    const int lane = threadIdx.x, g = lane >> 4, lr = lane & 15, lrow = g * 4;
+    int t = blockIdx.x, l = 0;
+    if (t >= 12) { t -= 12; l = 1; }
+    if (l == 1 && t >= 16) { t -= 16; l = 2; }
+    if (l == 2 && t >= 16) { t -= 16; l = 3; }
+    const int nd = l == 3 ? kOutP : kHid, np = l == 0 ? kInP : kHid;
+    const int n0 = t / (np / 32) * 32, k0 = t % (np / 32) * 32;
+    // rows 8 g .. of 32: tile g / 2 of two, half g % 2
+    const uint16_t *dz = (l == 3 ? B.D3 : B.D + (size_t)l * B.stride) + ((size_t)(g >> 1) * nd + n0 + lr) * kRows + (g & 1) * 8;
+    const uint16_t *pv = (l == 0 ? B.X : B.H + (size_t)(l - 1) * B.stride) + ((size_t)(g >> 1) * np + k0 + lr) * kRows + (g & 1) * 8;
+    f32x4 acc[2][2];
+    float db[2] = { 0.f, 0.f };
+    for (int a = 0; a < 2; ++a)
+        for (int b = 0; b < 2; ++b) acc[a][b] = f32x4{ 0.f, 0.f, 0.f, 0.f };
+    const int s0 = blockIdx.y * per, s1 = min(steps, s0 + per);
+    // `U` steps with their loads in flight together
+    auto sum = [&](int s, auto unroll) {
+        constexpr int U = decltype(unroll)::value;
+        bf16x8 A[U][2], P[U][2];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+                A[u][a] = ld8(dz + ((size_t)(s + u) * 2 * nd + 16 * a) * kRows);
+                P[u][a] = ld8(pv + ((size_t)(s + u) * 2 * np + 16 * a) * kRows);
+            }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+#pragma unroll
+                for (int b = 0; b < 2; ++b) acc[a][b] = mfma(A[u][a], P[u][b], acc[a][b]);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) db[a] += (float)A[u][a][i];
+            }
+    };
+    int s = s0;
+    for (; s + 8 <= s1; s += 8) sum(s, Steps<8>{});
+    for (; s < s1; ++s) sum(s, Steps<1>{});
+    float *out = part + (size_t)blockIdx.y * kParams;
+    for (int a = 0; a < 2; ++a) {
+        for (int b = 0; b < 2; ++b)
+            for (int i = 0; i < 4; ++i)
+                out[w_at(l) + (n0 + 16 * a + lrow + i) * np + k0 + 16 * b + lr] = acc[a][b][i];
+        if (k0 == 0) {
+            db[a] += __shfl_xor(db[a], 16);
+            db[a] += __shfl_xor(db[a], 32);
+            if (g == 0) out[b_at(l) + n0 + 16 * a + lr] = db[a];
+        }
     }
-    if (threadIdx.x == 0) out[j] = red[0];
 }
 
-__global__ void adam_kernel(float *__restrict__ P, const float *__restrict__ G, float *__restrict__ m,
+__device__ __forceinline__ float slice_sum(const float *part, int slices, int i)
+{
+    float g = 0.f;
+#pragma unroll 8
+    for (int s = 0; s < slices; ++s) g += part[(size_t)s * kParams + i];
+    return g;
+}
+
+__global__ void sum_kernel(const float *__restrict__ part, int slices, float *__restrict__ grad)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < kParams) grad[i] = slice_sum(part, slices, i);
+}
+
+// where the transposed copy holds parameter i (biases: -1)
+__device__ __forceinline__ int transposed(int i)
+{
+    int l = 0;
+    while (l < kLayers - 1 && i >= w_at(l + 1)) ++l;
+    const int e = i - w_at(l), K = layer_in(l), N = layer_out(l);
+    return e < N * K ? w_at(l) + e % K * N + e / K : -1;
+}
+
+__global__ void transpose_kernel(const uint16_t *__restrict__ W, uint16_t *__restrict__ WT)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= kParams) return;
+    const int t = transposed(i);
+    if (t >= 0) WT[t] = W[i];
+}
+
+__global__ void adam_kernel(float *__restrict__ P, const float *__restrict__ part, int slices, float *__restrict__ m,
                             float *__restrict__ v, const double *__restrict__ sums, float c1, float c2,
-                            float lr, uint16_t *__restrict__ W)
+                            float lr, uint16_t *__restrict__ W, uint16_t *__restrict__ WT)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= kParams) return;
     const float scale = sums[1] > 0.0 ? (float)(1.0 / sums[1]) : 0.f;
-    const float g = G[i] * scale;
+    const float g = slice_sum(part, slices, i) * scale;
     const float mi = 0.9f * m[i] + 0.1f * g;
     const float vi = 0.999f * v[i] + 0.001f * g * g;
     m[i] = mi;
@@ -228,30 +435,14 @@ __global__ void adam_kernel(float *__restrict__ P, const float *__restrict__ G, 
     const float p = P[i] - lr * (mi / c1) / (sqrtf(vi / c2) + 1e-8f);
     P[i] = p;
     W[i] = f2bf(p);
+    const int t = transposed(i);
+    if (t >= 0) WT[t] = f2bf(p);
 }
 
 __global__ void publish_kernel(const float *__restrict__ P, uint16_t *__restrict__ W)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < kParams) W[i] = f2bf(P[i]);
-}
-
-__device__ __forceinline__ float stdz(float x, float mean, float sd) { return (x - mean) / sd; }
-
-__global__ void gather_kernel(const float *__restrict__ Xs, const float *__restrict__ Ts,
-                              const float *__restrict__ Ms, const int *__restrict__ idx, int n, Scale sc,
-                              uint16_t *__restrict__ X0, float *__restrict__ T, float *__restrict__ M)
-{
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= (long)n * kInP) return;
-    const long r = e / kInP;
-    const int j = (int)(e % kInP);
-    const long src = idx[r];
-    X0[e] = j < kIn ? f2bf(stdz(Xs[src * kIn + j], sc.xmean[j], sc.xstd[j])) : (uint16_t)0;
-    if (j < kOut) {
-        T[r * kOut + j] = stdz(Ts[src * kOut + j], sc.ymean[j], sc.ystd[j]);
-        M[r * kOut + j] = Ms[src * kOut + j];
-    }
 }
 
 __global__ void standardise_kernel(const float *__restrict__ X, int n, Scale sc, uint16_t *__restrict__ X0)
@@ -278,8 +469,7 @@ using namespace mcm;
 
 static unsigned grid1(long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
-hipError_t mcm_forward(const uint16_t *X0, int n, Net net, float *Y, int ldy, uint16_t *H, int blocks,
-                       hipStream_t s)
+hipError_t mcm_forward(const uint16_t *X0, int n, Net net, float *Y, int ldy, int blocks, hipStream_t s)
 {
     if (n <= 0) return hipSuccess;
     static bool attr = false;
@@ -291,73 +481,61 @@ hipError_t mcm_forward(const uint16_t *X0, int n, Net net, float *Y, int ldy, ui
     }
     const int ntiles = (n + kTile - 1) / kTile;
     const int g = ntiles < blocks ? ntiles : blocks;
-    hipLaunchKernelGGL(forward_kernel, dim3(g), dim3(256), kFwdLds, s, X0, n, net, Y, ldy, H);
+    hipLaunchKernelGGL(forward_kernel, dim3(g), dim3(256), kFwdLds, s, X0, n, net, Y, ldy);
     return hipGetLastError();
 }
 
-template <int EPI>
-static hipError_t gemm(const uint16_t *A, long sam, long sak, const uint16_t *B, long sbk, long sbn, int M,
-                       int N, int K, float *C32, uint16_t *C16, int ldc, const uint16_t *Hm, int ldh,
-                       hipStream_t s)
+TrainBuf mcm_train_buf(uint16_t *mem, int n)
 {
-    // split K in chunks of 128 rows when accumulating (the weight gradients)
-    const int kc = EPI == EPI_F32_ADD ? 128 : K;
-    hipLaunchKernelGGL(gemm_kernel<EPI>, dim3(grid1(N, 64), grid1(M, 64), grid1(K, kc)), dim3(256), 0, s, A,
-                       sam, sak, B, sbk, sbn, M, N, K, kc, C32, C16, ldc, Hm, ldh);
+    const int t = mcm_train_tiles(n);
+    TrainBuf B;
+    B.stride = (size_t)t * kHid * kRows;
+    B.X = mem;
+    B.H = B.X + (size_t)t * kInP * kRows;
+    B.D = B.H + 3 * B.stride;
+    B.D3 = B.D + 3 * B.stride;
+    return B;
+}
+
+hipError_t mcm_transpose(const uint16_t *W, uint16_t *WT, hipStream_t s)
+{
+    hipLaunchKernelGGL(transpose_kernel, dim3(grid1(kParams, 256)), dim3(256), 0, s, W, WT);
     return hipGetLastError();
 }
 
-hipError_t mcm_backward(const uint16_t *X0, const uint16_t *H, const float *Y, const float *T, const float *M,
-                        int n, Net net, uint16_t *dA, uint16_t *dB, float *grad, double *sums, hipStream_t s)
+hipError_t mcm_gradient(const float *Xs, const float *Ts, const float *Ms, const int *idx, int n, Scale sc, Net net,
+                        const uint16_t *WT, uint16_t *mem, float *part, double *sums, int blocks, hipStream_t s)
 {
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(loss_kernel, dim3(grid1((long)n * kOutP, 256) < 1024 ? grid1((long)n * kOutP, 256) : 1024),
-                       dim3(256), 0, s, Y, T, M, n, dA, sums);
+    const TrainBuf B = mcm_train_buf(mem, n);
+    const int tiles = mcm_train_tiles(n), steps = tiles / 2, slices = mcm_train_slices(n);
+    hipLaunchKernelGGL(step_kernel, dim3(tiles < blocks ? tiles : blocks), dim3(256), 0, s, Xs, Ts, Ms, idx, n, tiles,
+                       sc, net, WT, B, sums);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    if ((e = hipMemsetAsync(grad, 0, kParams * sizeof(float), s)) != hipSuccess) return e;
-    // gradient rows of layer l flow in cur (ld = its width); prev activation
-    // of layer l: H[l-1] (or X0)
-    uint16_t *cur = dA, *nxt = dB;
-    for (int l = kLayers - 1; l >= 0; --l) {
-        const int K = layer_in(l), N = layer_out(l);
-        const uint16_t *prev = l == 0 ? X0 : H + (size_t)(l - 1) * n * kHid;
-        // dW_l [N][K] = cur^T prev
-        e = gemm<EPI_F32_ADD>(cur, 1, N, prev, K, 1, N, K, n, grad + w_off(l), nullptr, K, nullptr, 0, s);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(colsum_kernel, dim3(N), dim3(256), 0, s, cur, n, N, grad + b_off(l));
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-        if (l == 0) break;
-        // d(prev) [n][K] = (cur W_l) masked by prev > 0
-        e = gemm<EPI_RELU_MASK>(cur, N, 1, net.W + w_off(l), K, 1, n, K, N, nullptr, nxt, K, prev, K, s);
-        if (e != hipSuccess) return e;
-        uint16_t *t = cur;
-        cur = nxt;
-        nxt = t;
-    }
-    return hipSuccess;
+    hipLaunchKernelGGL(grad_kernel, dim3(kGradTiles, slices), dim3(64), 0, s, B, steps, (steps + slices - 1) / slices,
+                       part);
+    return hipGetLastError();
 }
 
-hipError_t mcm_adam(float *P, const float *grad, float *m, float *v, const double *sums, int t, float lr,
-                    uint16_t *W, hipStream_t s)
+hipError_t mcm_sum(const float *part, int slices, float *grad, hipStream_t s)
+{
+    hipLaunchKernelGGL(sum_kernel, dim3(grid1(kParams, 256)), dim3(256), 0, s, part, slices, grad);
+    return hipGetLastError();
+}
+
+hipError_t mcm_adam(float *P, const float *part, int slices, float *m, float *v, const double *sums, int t, float lr,
+                    uint16_t *W, uint16_t *WT, hipStream_t s)
 {
     const float c1 = 1.f - powf(0.9f, (float)t), c2 = 1.f - powf(0.999f, (float)t);
-    hipLaunchKernelGGL(adam_kernel, dim3(grid1(kParams, 256)), dim3(256), 0, s, P, grad, m, v, sums, c1, c2, lr, W);
+    hipLaunchKernelGGL(adam_kernel, dim3(grid1(kParams, 256)), dim3(256), 0, s, P, part, slices, m, v, sums, c1, c2, lr,
+                       W, WT);
     return hipGetLastError();
 }
 
 hipError_t mcm_publish(const float *P, uint16_t *W, hipStream_t s)
 {
     hipLaunchKernelGGL(publish_kernel, dim3(grid1(kParams, 256)), dim3(256), 0, s, P, W);
-    return hipGetLastError();
-}
-
-hipError_t mcm_gather(const float *Xs, const float *Ts, const float *Ms, const int *idx, int n, Scale sc,
-                      uint16_t *X0, float *T, float *M, hipStream_t s)
-{
-    if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(gather_kernel, dim3(grid1((long)n * kInP, 256)), dim3(256), 0, s, Xs, Ts, Ms, idx, n, sc,
-                       X0, T, M);
     return hipGetLastError();
 }
 
