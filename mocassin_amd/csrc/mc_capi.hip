@@ -124,7 +124,7 @@ struct mc_ctx {
     float *d_recCDF_b = nullptr, *d_totalLines_b = nullptr;
     unsigned short *d_recGuide_b = nullptr;
     int *d_em_i = nullptr, *d_em_err = nullptr;
-    float *d_em_f = nullptr;
+    float *d_em_f = nullptr, *d_em_for = nullptr;
     double *d_em_d = nullptr, *d_em_st = nullptr, *d_em_Td = nullptr;
     mce::EmArgs em{};
     char err[512] = "";
@@ -1383,7 +1383,7 @@ extern "C" int mc_emission_setup(mc_ctx *c, const mc_emission_tables *t)
     if (c->d_em_f) { (void)hipFree(c->d_em_f); c->d_em_f = nullptr; }
     if (c->d_em_d) { (void)hipFree(c->d_em_d); c->d_em_d = nullptr; }
     HIPCHK(c, dalloc(&c->d_em_i, iv.size()));
-    HIPCHK(c, dalloc(&c->d_em_f, fv.size()));
+    HIPCHK(c, dalloc(&c->d_em_f, fv.size() + 2 * (size_t)nb));      // the two-photon shapes behind
     HIPCHK(c, dalloc(&c->d_em_d, dv.size()));
     HIPCHK(c, copy_on(c->stream, c->d_em_i, iv.data(), iv.size() * sizeof(int), hipMemcpyHostToDevice));
     HIPCHK(c, copy_on(c->stream, c->d_em_f, fv.data(), fv.size() * sizeof(float), hipMemcpyHostToDevice));
@@ -1394,6 +1394,8 @@ extern "C" int mc_emission_setup(mc_ctx *c, const mc_emission_tables *t)
     a.nE = A.nE; a.ns1 = A.nstages + 1; a.eH = eH; a.eHe = eHe;
     a.abH = (float)A.el[eH].abun; a.abHe = (float)A.el[eHe].abun;
     a.nu = c->d_nuArray; a.widFlx = c->d_em_f + fo[14];
+    a.shape = c->d_em_f + fv.size();
+    HIPCHK(c, mce_two_photon(a.nu, nb, c->d_em_f + fv.size(), c->stream));
     a.ntk = t->ntk; a.tk = c->d_em_f + fo[0];
     size_t eo = io[0];
     for (int s_ = 0; s_ < 3; ++s_) {
@@ -1497,6 +1499,8 @@ extern "C" int mc_emission_build(mc_ctx *c, const float *Hden, const float *Te, 
         HIPCHK(c, fill_on(c->stream, c->d_totalLines_b, 0, nc1 * sizeof(float)));
     }
     if (!c->d_em_err) HIPCHK(c, dalloc(&c->d_em_err, nc1));
+    if (a.ncel > 0 && !c->d_em_for) HIPCHK(c, dalloc(&c->d_em_for, nc1));
+    a.forbidden = c->d_em_for;
     a.rec = c->d_recCDF_b; a.totalLines = c->d_totalLines_b; a.err = c->d_em_err;
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
     HIPCHK(c, mce_launch(c->d_atomic, a, c->stream));
@@ -2475,7 +2479,7 @@ extern "C" void mc_ctx_destroy(mc_ctx *c)
                      c->d_dust_tab, c->d_Tdust, c->d_dust_mono, c->d_pe_tab, c->d_grains, c->d_op_dust,
                      c->d_op_i, c->d_op_f, c->d_op_st, c->d_op_Td, c->d_op_out, c->d_op_ent,
                      c->d_ln_part, c->d_ln_st, c->d_ln_out, c->d_ln_black, c->d_em_i, c->d_em_err,
-                     c->d_em_f, c->d_em_d, c->d_em_st, c->d_em_Td, c->d_recCDF_b, c->d_recGuide_b,
+                     c->d_em_f, c->d_em_for, c->d_em_d, c->d_em_st, c->d_em_Td, c->d_recCDF_b, c->d_recGuide_b,
                      c->d_totalLines_b, c->d_order, c->d_ion_host };
     for (void *b : bufs)
         if (b) (void)hipFree(b);

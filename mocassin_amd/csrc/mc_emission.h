@@ -59,12 +59,15 @@ struct EmArgs {
     float *totalLines;                       // [nCells+1]
     int *err;                                // cells whose recPDF has no positive total
     int ncel, cel_most, nterm;               // of the atomic data: the level solves' LDS
+    const float *shape;                      // [2][nb] two-photon shapes of H I and He II
+    float *forbidden;                        // [nCells+1] normFor (ncel > 0)
 };
 
 }  // namespace mce
 
-// One wavefront per active cell; lds = dynamic LDS bytes (mce_lds_bytes).
-size_t mce_lds_bytes(const mce::EmArgs &a);
-// the same for a mesh of nb bins with grains, without the level solves
+// One wavefront per active cell.
+// LDS bytes of a mesh of nb bins with grains, without the free-bound channels
 size_t mce_mesh_bytes(int nb);
+// the two-photon shapes of H I and He II per bin, [2][nb]
+hipError_t mce_two_photon(const float *nu, int nb, float *shape, hipStream_t s);
 hipError_t mce_launch(const mcb::Atomic *dA, const mce::EmArgs &a, hipStream_t s);

@@ -2,14 +2,21 @@
 // part and setDiffusePDF (emission_mod.f90:32-1311) for every active cell,
 // written into the transport's recPDF rows ([cell][nu]) and totalLines.
 //
-// One 64-lane wavefront per cell.  Lanes over frequency bins evaluate the
-// free-bound, free-free and two-photon coefficients and the cell's partial
-// sums (sumDiffuseHI/HeI/HeII and the dust term) into LDS; lanes over lines
-// evaluate the recombination and forbidden-line terms.  The sums the
-// reference forms in REAL, in a fixed order (normHI, normRec, normFor, the
-// cumulative recPDF), are then taken by lane 0 in that order, so the tables
-// follow the reference's rounding.  The level populations of the forbidden
-// lines come from the balance's n-level solve (FP64).
+// One 64-lane wavefront per cell, in two kernels: forbidden_kernel sums the
+// forbidden-line terms from the balance's n-level solve (FP64), and
+// emission_kernel does the rest without the registers of those solves.  Lanes
+// over frequency bins evaluate the free-bound, free-free and two-photon
+// coefficients and the cell's partial sums (sumDiffuseHI/HeI/HeII and the
+// dust term) into LDS; lanes over lines evaluate the recombination terms.
+// The sums the reference forms in REAL, in a fixed order (normHI, normRec,
+// normFor, the cumulative recPDF), are taken in that order, each on a lane of
+// its own, so the tables follow the reference's rounding.
+//
+// Bound by the FP64 exponentials and powers of the bins (one per bin and
+// heavy ion above its edge, three of the recombination continua, up to three
+// of the tabulated ones).  45^3 octant, 800 bins: 10.4 ms at first, 5.0 with
+// four model ions to a wavefront, 3.9 in the two kernels (1.4 + 2.5);
+// dust and gas 60^3, 160 bins: 2.6, then 3.0, now 2.0.
 #include "mc_cel.h"
 #include "mc_emission.h"
 
@@ -25,72 +32,90 @@ constexpr float kHPlanck = 6.6262e-27f;  // constants_mod.f90:14
 constexpr float kPi = 3.141592654f;      // constants_mod.f90:32
 constexpr int kLev = mcb::kMaxLev;
 
-// One dynamic LDS block per wavefront.  Region A serves the forbidden-line
-// solves first (records, collision rates and line terms) and then the per-bin
-// partial sums s1, s2, s3 (and the grains' sD); the log-gamma rows, the
-// recombination-line terms and a reduction slot follow it.  Sharing region
-// A keeps the block at about 12 KB on an 800-bin mesh, so that more
-// wavefronts fit on a CU.
-__host__ __device__ inline size_t region_a_bytes(const EmArgs &a)
+// A heavy-ion free-bound channel of the cell (fb_ff).
+struct FreeBound {
+    int first, end, off;          // bins first .. end - 1, its cross-sections
+    float edge, g, x, abun;       // nu of the first bin, g0/g1, ion fraction, elemAbun
+};
+
+// The dynamic LDS of a wavefront: the per-bin partial sums s1, s2, s3 (and
+// the grains' sD), the free-bound channels, the log-gamma rows, the
+// recombination-line terms.
+__host__ __device__ inline int padded(int nb) { return (nb + 3) / 4 * 4; }
+__host__ __device__ inline size_t sums_bytes(const EmArgs &a)
 {
-    const size_t cel = (size_t)a.cel_most * sizeof(double2) + (size_t)a.ncel * sizeof(mcb::CelRec) +
-                       (size_t)a.nterm * sizeof(float);
-    const size_t sums = (size_t)(a.dabs ? 4 : 3) * a.nb * sizeof(float);
-    return ((cel > sums ? cel : sums) + 15) / 16 * 16;
+    return (size_t)(a.dabs ? 4 : 3) * padded(a.nb) * sizeof(float);
+}
+__host__ __device__ inline size_t fb_bytes(const EmArgs &a)
+{
+    return ((size_t)a.nfb * sizeof(FreeBound) + 15) / 16 * 16;
 }
 constexpr size_t kRestBytes = sizeof(float) * (3 * kMaxLim + kMaxRec + 4);
 
-// hydro2phot (emission_mod.f90:553-663), REAL arithmetic
-__device__ double hydro2phot(float nu, int Z, float Te, float Ne)
+// The part of hydro2phot that depends on the bin alone, gNu 1e27 of H I (Z =
+// 1) or He II; the tables of every bin are made once at setup.
+__device__ float two_photon_shape(float nu, int Z)
 {
-    float nu0, y, alpha, Ay, gNu, factor;
-    if (Z == 1) {
-        nu0 = 0.7496f;
-        y = nu / nu0;
-        if (nu >= nu0) return 0.0;
-        alpha = 0.8368f * powf(Te * 1.e-4f, -0.723f);
-        Ay = 202.0f * (y * (1.f - y) * (1.f - powf(4.f * y * (1.f - y), 0.8f)) +
-                       0.88f * powf(y * (1.f - y), 1.53f) * powf(4.f * y * (1.f - y), 0.8f));
-        gNu = kHPlanck * y * Ay / 8.2249f;
-        gNu = gNu * 1e27f;
-        float Q;
-        if (Te <= 10000.f) Q = 5.31e-4f;
-        else if (Te >= 20000.f) Q = 4.71e-4f;
-        else {
-            factor = log10f(4.71e-4f / 5.31e-4f) / log10f(2.f);
-            Q = powf(10.f, log10f(5.31e-4f) + factor * log10f(Te / 10000.f));
-        }
-        return (double)(alpha * gNu / (1.f + (Ne * Q) / 8.23f));
-    }
-    nu0 = 3.00f;
-    y = nu / nu0;
-    if (nu >= nu0) return 0.0;
-    if (Te <= 5000.f) alpha = 6.161f;
-    else if (Te >= 30000.f) alpha = 2.035f;
-    else if (Te > 5000.f && Te <= 10000.f) {
-        factor = log10f(4.091f / 6.161f) / log10f(2.f);
-        alpha = powf(10.f, log10f(6.161f) + factor * log10f(Te / 5000.f));
-    } else if (Te > 10000.f && Te <= 15000.f) {
-        factor = log10f(3.189f / 4.091f) / log10f(1.5f);
-        alpha = powf(10.f, log10f(4.091f) + factor * log10f(Te / 10000.f));
-    } else {
-        factor = log10f(2.035f / 3.189f) / log10f(2.f);
-        alpha = powf(10.f, log10f(3.189f) + factor * log10f(Te / 15000.f));
-    }
     const float z6 = 64.f;
-    Ay = z6 * 0.9994667f * 202.0f *
-         (y * (1.f - y) * (1.f - powf(4.f * y * (1.f - y), 0.8f)) +
-          0.88f * powf(y * (1.f - y), 1.53f) * powf(4.f * y * (1.f - y), 0.8f));
-    const float A2qZ = 8.226f * z6;
-    gNu = kHPlanck * y * Ay / A2qZ;
-    gNu = gNu * 1e27f;
-    return (double)(alpha * gNu);
+    const float y = nu / (Z == 1 ? 0.7496f : 3.00f);
+    float gNu;
+    if (Z == 1) {
+        const float Ay = 202.0f * (y * (1.f - y) * (1.f - powf(4.f * y * (1.f - y), 0.8f)) +
+                                   0.88f * powf(y * (1.f - y), 1.53f) * powf(4.f * y * (1.f - y), 0.8f));
+        gNu = kHPlanck * y * Ay / 8.2249f;
+    } else {
+        const float Ay = z6 * 0.9994667f * 202.0f *
+                         (y * (1.f - y) * (1.f - powf(4.f * y * (1.f - y), 0.8f)) +
+                          0.88f * powf(y * (1.f - y), 1.53f) * powf(4.f * y * (1.f - y), 0.8f));
+        const float A2qZ = 8.226f * z6;
+        gNu = kHPlanck * y * Ay / A2qZ;
+    }
+    return gNu * 1e27f;
 }
 
-// ffCoeff (emission_mod.f90:726-742)
-__device__ __forceinline__ double ffcoeff(float nu, float Z, float g, float Te, float sqrTe)
+__global__ void two_photon_kernel(const float *__restrict__ nu, int nb, float *__restrict__ shape)
 {
-    const double expF = exp((double)(-nu * kHcRydK / Te));
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nb) return;
+    shape[i] = nu[i] < 0.7496f ? two_photon_shape(nu[i], 1) : 0.f;
+    shape[nb + i] = nu[i] < 3.00f ? two_photon_shape(nu[i], 2) : 0.f;
+}
+
+// The part that depends on the cell: alpha of each, and H I's collisional
+// de-excitation 1 + Ne Q / 8.23
+struct TwoPhoton { float alpha1, quench1, alpha2; };
+// hydro2phot (emission_mod.f90:553-663), REAL arithmetic
+__device__ __forceinline__ TwoPhoton two_photon(float Te, float Ne)
+{
+    TwoPhoton T;
+    float factor;
+    T.alpha1 = 0.8368f * powf(Te * 1.e-4f, -0.723f);
+    float Q;
+    if (Te <= 10000.f) Q = 5.31e-4f;
+    else if (Te >= 20000.f) Q = 4.71e-4f;
+    else {
+        factor = log10f(4.71e-4f / 5.31e-4f) / log10f(2.f);
+        Q = powf(10.f, log10f(5.31e-4f) + factor * log10f(Te / 10000.f));
+    }
+    T.quench1 = 1.f + (Ne * Q) / 8.23f;
+    if (Te <= 5000.f) T.alpha2 = 6.161f;
+    else if (Te >= 30000.f) T.alpha2 = 2.035f;
+    else if (Te > 5000.f && Te <= 10000.f) {
+        factor = log10f(4.091f / 6.161f) / log10f(2.f);
+        T.alpha2 = powf(10.f, log10f(6.161f) + factor * log10f(Te / 5000.f));
+    } else if (Te > 10000.f && Te <= 15000.f) {
+        factor = log10f(3.189f / 4.091f) / log10f(1.5f);
+        T.alpha2 = powf(10.f, log10f(4.091f) + factor * log10f(Te / 10000.f));
+    } else {
+        factor = log10f(2.035f / 3.189f) / log10f(2.f);
+        T.alpha2 = powf(10.f, log10f(3.189f) + factor * log10f(Te / 15000.f));
+    }
+    return T;
+}
+
+// ffCoeff (emission_mod.f90:726-742); expF = exp(-h nu / k Te)
+__device__ __forceinline__ double ffcoeff(float Z, float g, double expF, float sqrTe)
+{
     return (double)(4.f * kPi * 54.43f * Z * Z * g) * expF / (double)sqrTe;
 }
 
@@ -119,39 +144,25 @@ __device__ int locate_tk(const float *xa, int n, float x)
     return p - 1 > 1 ? p - 1 : 1;
 }
 
-__global__ void __launch_bounds__(64) emission_kernel(const mcb::Atomic *__restrict__ Ap, EmArgs a)
+#define XION(e, st) ((float)ionc[(e) * a.ns1 + (st)])
+
+// normFor of every cell
+__global__ void __launch_bounds__(64) forbidden_kernel(const mcb::Atomic *__restrict__ Ap, EmArgs a)
 {
     extern __shared__ __align__(16) unsigned char dyn[];
     const mcb::Atomic &A = *Ap;
     const int cell = blockIdx.x + 1;
     const int lane = threadIdx.x;
-    const int nb = a.nb;
-    const float *nu = a.nu;
-    const bool dust = a.dabs != nullptr;
-    // region A: the forbidden-line solves, then the per-bin sums
     double2 *rate = reinterpret_cast<double2 *>(dyn);
     mcb::CelRec *rec = reinterpret_cast<mcb::CelRec *>(rate + a.cel_most);
     float *fterm = reinterpret_cast<float *>(rec + a.ncel);
-    float *s1 = reinterpret_cast<float *>(dyn), *s2 = s1 + nb, *s3 = s1 + 2 * nb, *sD = s1 + 3 * nb;
-    unsigned char *rest = dyn + region_a_bytes(a);
-    float (*loc)[kMaxLim] = reinterpret_cast<float (*)[kMaxLim]>(rest);
-    float *rterm = reinterpret_cast<float *>(rest + sizeof(float) * 3 * kMaxLim);
-    float *red = rterm + kMaxRec;
 
     // the state as the host grid stores it (REAL)
     const float Te = (float)a.Te[cell], NeIn = (float)a.Ne[cell];
     const double *ionc = a.ion + (size_t)cell * a.nE * a.ns1;
-#define XION(e, st) ((float)ionc[(e) * a.ns1 + (st)])
-    float NeUsed = NeIn;
-    const float sqrTe = sqrtf(Te);
-    const float log10Te = log10f(Te);
-    if (NeUsed < 1.e-5f) NeUsed = 1.e-5f;
-    const float xHp = XION(a.eH, 2), xHe1 = XION(a.eHe, 2), xHe2 = XION(a.eHe, 3);
-    if (!(Te > 0.f) || !isfinite(Te) || !isfinite(NeIn)) {
-        // not a state the balance leaves (its floor is 1 K): refused
-        if (lane == 0) a.err[cell] = 1;
-        return;
-    }
+    const float NeUsed = NeIn < 1.e-5f ? 1.e-5f : NeIn;
+    // a state emission_kernel refuses
+    if (!(Te > 0.f) || !isfinite(Te) || !isfinite(NeIn)) return;
 
     float normFor = 0.f;
     // forbidden lines (forLines): the terms above 1e-35 of every model ion's
@@ -187,7 +198,43 @@ __global__ void __launch_bounds__(64) emission_kernel(const mcb::Atomic *__restr
     }
     __syncthreads();
     for (int t = 0; t < A.nterm; ++t) normFor = normFor + fterm[t];
-    __syncthreads();                             // region A now holds the per-bin sums
+    if (lane == 0) a.forbidden[cell] = normFor;
+}
+
+__global__ void __launch_bounds__(64) emission_kernel(EmArgs a)
+{
+    extern __shared__ __align__(16) unsigned char dyn[];
+    const int cell = blockIdx.x + 1;
+    const int lane = threadIdx.x;
+    const int nb = a.nb, ld = padded(nb);
+    const float *nu = a.nu;
+    const bool dust = a.dabs != nullptr;
+    float *s1 = reinterpret_cast<float *>(dyn), *s2 = s1 + ld, *s3 = s1 + 2 * ld, *sD = s1 + 3 * ld;
+    FreeBound *fb = reinterpret_cast<FreeBound *>(dyn + sums_bytes(a));
+    unsigned char *rest = dyn + sums_bytes(a) + fb_bytes(a);
+    float (*loc)[kMaxLim] = reinterpret_cast<float (*)[kMaxLim]>(rest);
+    float *rterm = reinterpret_cast<float *>(rest + sizeof(float) * 3 * kMaxLim);
+    float *red = rterm + kMaxRec;
+
+    // the state as the host grid stores it (REAL)
+    const float Te = (float)a.Te[cell], NeIn = (float)a.Ne[cell];
+    const double *ionc = a.ion + (size_t)cell * a.nE * a.ns1;
+    float NeUsed = NeIn;
+    const float sqrTe = sqrtf(Te);
+    const float log10Te = log10f(Te);
+    if (NeUsed < 1.e-5f) NeUsed = 1.e-5f;
+    const float xHp = XION(a.eH, 2), xHe1 = XION(a.eHe, 2), xHe2 = XION(a.eHe, 3);
+    if (!(Te > 0.f) || !isfinite(Te) || !isfinite(NeIn)) {
+        // not a state the balance leaves (its floor is 1 K): refused
+        if (lane == 0) a.err[cell] = 1;
+        return;
+    }
+
+    for (int c = lane; c < a.nfb; c += W) {
+        const int *m = a.fb_i + 4 * c;
+        fb[c] = FreeBound{ m[2], m[3], a.fb_off[c], nu[m[2] - 1], a.fb_f[2 * c], XION(m[0], m[1]), a.fb_f[2 * c + 1] };
+    }
+    const TwoPhoton tp = two_photon(Te, NeUsed);
 
     // log gamma rows at Te (fb_ff, emission_mod.f90:306-336)
     for (int s = 0; s < 3; ++s)
@@ -228,31 +275,30 @@ __global__ void __launch_bounds__(64) emission_kernel(const mcb::Atomic *__restr
             // the Milne relation above the H, He I and He II edges, plus free-free
             const double factor = (double)((nui * nui * nui) / (Te * sqrTe));
             double expF = exp((double)((-nui + nu[a.ip[0] - 1]) * kHcRydK / Te));
+            const double expFF = exp((double)(-nui * kHcRydK / Te));
             g[0] = (double)(4.f * kPi) * (double)a.sig[0][i - a.i0[0]] * (double)statW[0] * (double)kHcRyd * constant *
                    factor * expF * (double)1.e20f * (double)1.e20f;
-            g[0] = g[0] + ffcoeff(nui, 1.f, a.gff[i - 1], Te, sqrTe);
+            g[0] = g[0] + ffcoeff(1.f, a.gff[i - 1], expFF, sqrTe);
             if (i >= a.i0[1]) {
                 expF = exp((double)((-nui + nu[a.ip[1] - 1]) * kHcRydK / Te));
                 g[1] = (double)(4.f * kPi) * (double)a.sig[1][i - a.i0[1]] * (double)statW[1] * (double)kHcRyd *
                        constant * factor * expF * (double)1.e20f * (double)1.e20f;
-                g[1] = g[1] + ffcoeff(nui, 1.f, a.gff[i - 1], Te, sqrTe);
+                g[1] = g[1] + ffcoeff(1.f, a.gff[i - 1], expFF, sqrTe);
                 if (i >= a.i0[2]) {
                     expF = exp((double)((-nui + nu[a.ip[2] - 1]) * kHcRydK / Te));
                     g[2] = (double)(4.f * kPi) * (double)a.sig[2][i - a.i0[2]] * (double)statW[2] * (double)kHcRyd *
                            constant * factor * expF * (double)1.e20f * (double)1.e20f;
-                    g[2] = g[2] + ffcoeff(nui, 2.f, a.gffHeII[i - 1], Te, sqrTe);
+                    g[2] = g[2] + ffcoeff(2.f, a.gffHeII[i - 1], expFF, sqrTe);
                 }
             }
         }
         // heavy-ion free-bound emission (fb_ff, emission_mod.f90:473-528)
         double gh = 0.0;
         for (int c = 0; c < a.nfb; ++c) {
-            const int *m = a.fb_i + 4 * c;
-            const int ipc = m[2];
-            if (i >= ipc && i < m[3]) {
-                const double expF = exp((double)((-nui + nu[ipc - 1]) * kHcRydK / Te));
-                gh = gh + expF * (double)a.fb_sig[a.fb_off[c] + (i - ipc)] * (double)a.fb_f[2 * c] *
-                              (double)XION(m[0], m[1]) * (double)a.fb_f[2 * c + 1];
+            const FreeBound f = fb[c];
+            if (i >= f.first && i < f.end) {
+                const double expF = exp((double)((-nui + f.edge) * kHcRydK / Te));
+                gh = gh + expF * (double)a.fb_sig[f.off + (i - f.first)] * (double)f.g * (double)f.x * (double)f.abun;
             }
         }
         {
@@ -261,8 +307,8 @@ __global__ void __launch_bounds__(64) emission_kernel(const mcb::Atomic *__restr
                  (double)1.e20f;
         }
         // two-photon continua (twoPhoton, HeI2photSub)
-        const double tHI = hydro2phot(nui, 1, Te, NeUsed);
-        const double tHeII = hydro2phot(nui, 2, Te, NeUsed);
+        const double tHI = nui < 0.7496f ? (double)(tp.alpha1 * a.shape[i - 1] / tp.quench1) : 0.0;
+        const double tHeII = nui < 3.00f ? (double)(tp.alpha2 * a.shape[nb + i - 1]) : 0.0;
         double tHeI = 0.0;
         const int j = a.jHeI[i - 1];
         if (j > 0) {
@@ -351,19 +397,34 @@ __global__ void __launch_bounds__(64) emission_kernel(const mcb::Atomic *__restr
         }
     }
     __syncthreads();
-    float normRec = 0.f;
-    if (lane == 0)
-        for (int t = 0; t < 70 + 315 + 34; ++t) normRec = normRec + rterm[t];
-
-    // lane 0: the partial sums in bin order, the He lines able to ionise H,
-    // totalLines, and the cumulative recPDF (in s1)
-    if (lane == 0) {
-        float nHI = 0.f, nHeI = 0.f, nHeII = 0.f, nD = 0.f;
-        for (int i = 0; i < nb; ++i) {
-            nHI = nHI + s1[i];
-            nHeI = nHeI + s2[i];
-            nHeII = nHeII + s3[i];
+    // the sums in order, a lane each: bins of H I, He I, He II and grains,
+    // recombination lines
+    float sum = 0.f;
+    {
+        const float *p = lane < 4 ? s1 + (size_t)lane * ld : rterm;
+        const int n = lane < (dust ? 4 : 3) ? nb : lane == 4 ? 70 + 315 + 34 : 0;
+        for (int i = 0; i < n; i += 4) {
+            const float4 v = *reinterpret_cast<const float4 *>(p + i);
+            sum = sum + v.x;
+            if (i + 1 < n) sum = sum + v.y;
+            if (i + 2 < n) sum = sum + v.z;
+            if (i + 3 < n) sum = sum + v.w;
         }
+    }
+    float nHI = __shfl(sum, 0), nHeI = __shfl(sum, 1), nHeII = __shfl(sum, 2), nD = __shfl(sum, 3);
+    const float normRec = __shfl(sum, 4), normFor = a.ncel > 0 ? a.forbidden[cell] : 0.f;
+    __syncthreads();
+    // setDiffusePDF scales the raw grain sums by h 4 pi 1e25 cRyd Ndust /
+    // Hden; the raw total is taken in bin order here (the reference adds
+    // sizes, species, then bins)
+    if (dust) {
+        const float cst = kHPlanck * 4.f * kPi * 1.e25f * kCRyd;
+        const float nd = a.ndust[cell], hd = (float)a.Hden[cell];
+        for (int i = lane; i < nb; i += W) sD[i] = sD[i] * cst * nd / hd;
+        nD = nD * cst * nd / hd;
+    }
+    // lane 0: the He lines able to ionise H and totalLines
+    if (lane == 0) {
         const float T4 = Te * 1.e-4f;
         const float a2tS = 27.2f * powf(T4, -0.678f);
         const float corr = a2tS * NeUsed * a.abHe * xHe1 * 1.45673f * kHcRyd * 1e11f;
@@ -379,31 +440,7 @@ __global__ void __launch_bounds__(64) emission_kernel(const mcb::Atomic *__restr
             nHeII = nHeII + ly[k];
         }
         float normalize = nHI + nHeI + nHeII;
-        if (dust) {
-            // setDiffusePDF scales the raw grain sums by h 4 pi 1e25 cRyd
-            // Ndust / Hden; the raw total is taken in bin order here (the
-            // reference adds sizes, species, then bins)
-            const float cst = kHPlanck * 4.f * kPi * 1.e25f * kCRyd;
-            const float nd = a.ndust[cell], hd = (float)a.Hden[cell];
-            for (int i = 0; i < nb; ++i) {
-                nD = nD + sD[i];
-                sD[i] = sD[i] * cst * nd / hd;
-            }
-            nD = nD * cst * nd / hd;
-            normalize = normalize + nD;
-            float r = 0.f;
-            for (int i = 0; i < nb; ++i) {
-                r = i == 0 ? s1[i] + s2[i] + s3[i] + sD[i] : r + s1[i] + s2[i] + s3[i] + sD[i];
-                s1[i] = r;
-            }
-        } else {
-            float r = 0.f;
-            for (int i = 0; i < nb; ++i) {
-                const float t = s1[i] + s2[i] + s3[i];
-                r = i == 0 ? t : r + t;
-                s1[i] = r;
-            }
-        }
+        if (dust) normalize = normalize + nD;
         const float tl = normRec + normFor;
         normalize = normalize + tl;
         // the reference's fraction; at a few tens of K its fits give inf*0
@@ -413,7 +450,32 @@ __global__ void __launch_bounds__(64) emission_kernel(const mcb::Atomic *__restr
         a.err[cell] = isnan(f) ? 2 : 0;
         if (isnan(f)) f = 0.f;
         a.totalLines[cell] = f;
-        red[0] = s1[nb - 1];
+    }
+    __syncthreads();
+    // the cumulative recPDF in bin order, in s1
+    if (!dust) {
+        for (int i = lane; i < nb; i += W) s1[i] = s1[i] + s2[i] + s3[i];
+        __syncthreads();
+    }
+    if (lane == 0) {
+        float r = 0.f;
+        if (dust) {
+            for (int i = 0; i < nb; ++i) {
+                r = i == 0 ? s1[i] + s2[i] + s3[i] + sD[i] : r + s1[i] + s2[i] + s3[i] + sD[i];
+                s1[i] = r;
+            }
+        } else {
+            for (int i = 0; i < nb; i += 4) {
+                float4 v = *reinterpret_cast<const float4 *>(s1 + i);
+                r = i == 0 ? v.x : r + v.x;
+                v.x = r;
+                if (i + 1 < nb) { r = r + v.y; v.y = r; }
+                if (i + 2 < nb) { r = r + v.z; v.z = r; }
+                if (i + 3 < nb) { r = r + v.w; v.w = r; }
+                *reinterpret_cast<float4 *>(s1 + i) = v;
+            }
+        }
+        red[0] = r;
     }
     __syncthreads();
     // recPDF = cumulative / last (setDiffusePDF).  In barely lit cells the
@@ -446,19 +508,28 @@ __global__ void __launch_bounds__(64) emission_kernel(const mcb::Atomic *__restr
 
 }  // namespace mce
 
-size_t mce_lds_bytes(const mce::EmArgs &a)
-{
-    return mce::region_a_bytes(a) + mce::kRestBytes;
-}
-
 size_t mce_mesh_bytes(int nb)
 {
     return (4 * (size_t)nb * sizeof(float) + 15) / 16 * 16 + mce::kRestBytes;
 }
 
+hipError_t mce_two_photon(const float *nu, int nb, float *shape, hipStream_t s)
+{
+    hipLaunchKernelGGL(mce::two_photon_kernel, dim3((nb + 63) / 64), dim3(64), 0, s, nu, nb, shape);
+    return hipGetLastError();
+}
+
 hipError_t mce_launch(const mcb::Atomic *dA, const mce::EmArgs &a, hipStream_t s)
 {
     if (a.nc <= 0) return hipSuccess;
-    hipLaunchKernelGGL(mce::emission_kernel, dim3(a.nc), dim3(64), mce_lds_bytes(a), s, dA, a);
+    if (a.ncel > 0) {
+        const size_t lds = (size_t)a.cel_most * sizeof(double2) + (size_t)a.ncel * sizeof(mcb::CelRec) +
+                           (size_t)a.nterm * sizeof(float);
+        hipLaunchKernelGGL(mce::forbidden_kernel, dim3(a.nc), dim3(64), lds, s, dA, a);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL(mce::emission_kernel, dim3(a.nc), dim3(64),
+                       mce::sums_bytes(a) + mce::fb_bytes(a) + mce::kRestBytes, s, a);
     return hipGetLastError();
 }
