@@ -461,6 +461,14 @@ int mc_opacity_setup(mc_ctx *ctx, const mc_opacity_tables *tables);
 int mc_opacity_build(mc_ctx *ctx, const float *Hden, const float *Te, const float *Ne, const float *ionDen,
                      const float *Tdust, float *opacity, float *scaOpac, double *kernel_ms);
 
+/* A table that mc_opacity_build or mc_emission_build left on the device, row
+ * by row: rows[(nCells+1)][nbins], row 0 zero (the builds' own outputs are
+ * column-major).  No counterpart in the reference. */
+#define MC_TABLE_OPACITY 0
+#define MC_TABLE_SCATTERING 1
+#define MC_TABLE_RECPDF 2
+int mc_fetch_table_rows(mc_ctx *ctx, int32_t table, float *rows);
+
 /* The module data emissionDriver reads for the gas re-emission (set up by
  * the reference's ph_mod, hydro_mod and readData; emission_mod.f90:32-1311).
  * Bins are 1-based; (a, b) tables are column-major as the host holds them.

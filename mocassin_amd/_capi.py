@@ -23,11 +23,13 @@ EXPORTS = ("mc_ctx_create", "mc_upload_tables", "mc_zero_estimators", "mc_transp
            "mc_mlp_train", "mc_count_crossings", "mc_fetch_crossings", "mc_transport_batch",
            "mc_transport_batch_noalloc",
            "mc_dust_setup", "mc_update_cells", "mc_opacity_setup", "mc_opacity_build",
+           "mc_fetch_table_rows",
            "mc_line_luminosities", "mc_emission_setup", "mc_emission_build", "mc_write_grid", "mc_read_grid",
            "mc_set_view_angles", "mc_esc_planes", "mc_ctx_shape", "mc_probe_atomics", "mc_probe_atomic_lines",
            "mc_ctx_last_error", "mc_ctx_destroy")
 
 MC_SOLVER_REFERENCE, MC_SOLVER_SECANT = 0, 1
+MC_TABLE_OPACITY, MC_TABLE_SCATTERING, MC_TABLE_RECPDF = 0, 1, 2
 # mc_tuning.kernel
 KERNELS = {"auto": 0, "one": 1, "spare": 2, "pool": 3}
 MC_MLP_NIN, MC_MLP_NOUT, MC_MLP_NPARAMS, MC_MLP_NSCALE = 72, 31, 49568, 206
@@ -167,6 +169,7 @@ def load():
     L.mc_update_cells.argtypes = [vp, C.c_double, C.POINTER(McBalanceOpts)] + [vp] * 8
     L.mc_opacity_setup.argtypes = [vp, C.POINTER(McOpacityTables)]
     L.mc_opacity_build.argtypes = [vp] * 9
+    L.mc_fetch_table_rows.argtypes = [vp, i32, vp]
     L.mc_line_luminosities.argtypes = [vp] * 9
     L.mc_emission_setup.argtypes = [vp, C.POINTER(McEmissionTables)]
     L.mc_write_grid.argtypes = [C.POINTER(McDesc), vp, C.c_char_p, C.POINTER(McGridState)]

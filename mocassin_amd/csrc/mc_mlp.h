@@ -84,6 +84,10 @@ hipError_t mcm_sum(const float *part, int slices, float *grad, hipStream_t s);
 // BF16 copies
 hipError_t mcm_adam(float *P, const float *part, int slices, float *m, float *v, const double *sums, int t,
                     float lr, uint16_t *W, uint16_t *WT, hipStream_t s);
+// first entry of X (bad[0]) and of T or M (bad[1]) that is not finite, or
+// negative in M; all ones where there is none
+hipError_t mcm_check(const float *X, size_t nx, const float *T, const float *M, size_t nt, unsigned long long *bad,
+                     hipStream_t s);
 hipError_t mcm_publish(const float *P, uint16_t *W, hipStream_t s);
 hipError_t mcm_standardise(const float *Xraw, int n, mcm::Scale sc, uint16_t *X0, hipStream_t s);
 hipError_t mcm_unscale(float *Y, int n, int ldy, mcm::Scale sc, hipStream_t s);

@@ -439,6 +439,20 @@ __global__ void adam_kernel(float *__restrict__ P, const float *__restrict__ par
     if (t >= 0) WT[t] = f2bf(p);
 }
 
+__global__ void __launch_bounds__(256) check_kernel(const float *__restrict__ X, size_t nx, const float *__restrict__ T,
+                                                    const float *__restrict__ M, size_t nt,
+                                                    unsigned long long *__restrict__ bad)
+{
+    const size_t step = (size_t)gridDim.x * blockDim.x, i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    unsigned long long x = ~0ull, t = ~0ull;
+    for (size_t i = i0; i < nx; i += step)
+        if (!isfinite(X[i])) { x = i; break; }
+    for (size_t i = i0; i < nt; i += step)
+        if (!isfinite(T[i]) || !isfinite(M[i]) || M[i] < 0.f) { t = i; break; }
+    if (x != ~0ull) atomicMin(&bad[0], x);
+    if (t != ~0ull) atomicMin(&bad[1], t);
+}
+
 __global__ void publish_kernel(const float *__restrict__ P, uint16_t *__restrict__ W)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -530,6 +544,15 @@ hipError_t mcm_adam(float *P, const float *part, int slices, float *m, float *v,
     const float c1 = 1.f - powf(0.9f, (float)t), c2 = 1.f - powf(0.999f, (float)t);
     hipLaunchKernelGGL(adam_kernel, dim3(grid1(kParams, 256)), dim3(256), 0, s, P, part, slices, m, v, sums, c1, c2, lr,
                        W, WT);
+    return hipGetLastError();
+}
+
+hipError_t mcm_check(const float *X, size_t nx, const float *T, const float *M, size_t nt, unsigned long long *bad,
+                     hipStream_t s)
+{
+    hipError_t e = hipMemsetAsync(bad, 0xff, 2 * sizeof(unsigned long long), s);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(check_kernel, dim3(2048), dim3(256), 0, s, X, nx, T, M, nt, bad);
     return hipGetLastError();
 }
 

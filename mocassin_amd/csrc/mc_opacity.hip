@@ -247,6 +247,34 @@ __global__ void gather_kernel(const float *t3, mcd::J3Shape js, const int *cell_
 }
 }  // namespace mco
 
+namespace mco {
+// A tiled table as rows [cell][nb]: a tile's 64 points by 64 bins through
+// LDS, lanes over points on the way in and over bins on the way out.
+__global__ void __launch_bounds__(256) rows_kernel(const float *t3, mcd::J3Shape js, const int *active, int nb, float *out)
+{
+    __shared__ float v[64][65];
+    __shared__ int cell[64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nu0 = blockIdx.y * 64;
+    const unsigned p0 = blockIdx.x * 64u;
+    if (w == 0) {
+        const int xyz = mcd::j3_lattice(js, p0 + (unsigned)lane);
+        cell[lane] = xyz >= 0 ? active[xyz] : 0;
+    }
+    const float *t = t3 + mcd::j3_index(nb, 0, p0) + lane;
+    for (int q = w; q < 64 && nu0 + q < nb; q += 4) v[lane][q] = t[(size_t)(nu0 + q) * mcd::kJTile];
+    __syncthreads();
+    for (int q = w; q < 64; q += 4)
+        if (cell[q] > 0 && nu0 + lane < nb) out[(size_t)cell[q] * nb + nu0 + lane] = v[q][lane];
+}
+}  // namespace mco
+
+hipError_t mco_launch_rows(const float *t3, const mcd::J3Shape &js, const int *active, int nb, float *out, hipStream_t s)
+{
+    hipLaunchKernelGGL(mco::rows_kernel, dim3((unsigned)(mcd::j3_points(js) / 64), (unsigned)((nb + 63) / 64)), dim3(256),
+                       0, s, t3, js, active, nb, out);
+    return hipGetLastError();
+}
+
 hipError_t mco_launch_gather(const float *t3, const mcd::J3Shape &js, const int *cell_xyz, int nc, int nb,
                              float *out, hipStream_t s)
 {

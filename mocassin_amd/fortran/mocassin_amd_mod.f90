@@ -240,6 +240,12 @@ module mocassin_amd_mod
             type(c_ptr), value :: ctx, Hden, Te, Ne, ionDen, Tdust, opacity, scaOpac, kernel_ms
         end function mc_opacity_build
 
+        integer(c_int) function mc_fetch_table_rows(ctx, table, rows) bind(C, name="mc_fetch_table_rows")
+            import :: c_int, c_int32_t, c_ptr
+            type(c_ptr), value :: ctx, rows
+            integer(c_int32_t), value :: table
+        end function mc_fetch_table_rows
+
         integer(c_int) function mc_write_grid(desc, atomic, dir, state) bind(C, name="mc_write_grid")
             import :: c_int, c_char, mc_desc, mc_atomic, mc_grid_state
             type(mc_desc), intent(in) :: desc

@@ -305,17 +305,17 @@ class Transport:
         td = None if Tdust is None else np.ascontiguousarray(Tdust, np.float32).ravel()
         if td is not None and td.size != nc1 * int(np.prod(getattr(self, "_dust_shape", (0,)))):
             raise ValueError("Tdust needs (nCells+1) x (nSizes+1) x (nSpeciesMax+1) entries (dust_setup first)")
-        op = sca = None
-        if host:
-            op = np.zeros((self.nbins, nc1), np.float32)
-            sca = np.zeros((self.nbins, nc1), np.float32)
         ms = C.c_double()
         ptr = lambda a: None if a is None else a.ctypes.data
-        self._check(self._lib.mc_opacity_build(self._h, *(ptr(a) for a in st), ptr(td), ptr(op), ptr(sca),
-                                               C.byref(ms)))
-        if host:
-            op, sca = op.T.copy(), sca.T.copy()
-        return op, sca, ms.value
+        self._check(self._lib.mc_opacity_build(self._h, *(ptr(a) for a in st), ptr(td), None, None, C.byref(ms)))
+        if not host:
+            return None, None, ms.value
+        return self._rows(_capi.MC_TABLE_OPACITY), self._rows(_capi.MC_TABLE_SCATTERING), ms.value
+
+    def _rows(self, table):
+        a = np.empty((self.nCells + 1, self.nbins), np.float32)
+        self._check(self._lib.mc_fetch_table_rows(self._h, table, a.ctypes.data))
+        return a
 
     def emission_setup(self, tkGamma, logGammaHI, logGammaHeI, logGammaHeII, HINuEdgeP, HeINuEdgeP, HeIINuEdgeP,
                        gauntFF, gauntFFHeII, HIPnuP, HeIPnuP, HeIIPnuP, xSecHI, xSecHeI, xSecHeII, fb_meta,
@@ -371,17 +371,11 @@ class Transport:
                   np.ascontiguousarray(Ne, np.float32).reshape(nc1),
                   np.asfortranarray(np.asarray(ionDen, np.float32).reshape(nc1, self._nE, self._ns))]
         td = None if Tdust is None else np.ascontiguousarray(Tdust, np.float32).ravel()
-        rec = tl = None
-        if host:
-            rec = np.zeros((self.nbins, nc1), np.float32)
-            tl = np.zeros(nc1, np.float32)
+        tl = np.zeros(nc1, np.float32) if host else None
         ms = C.c_double()
         ptr = lambda a: None if a is None else a.ctypes.data
-        self._check(self._lib.mc_emission_build(self._h, *(ptr(a) for a in st), ptr(td), ptr(rec), ptr(tl),
-                                                C.byref(ms)))
-        if host:
-            rec = rec.T.copy()
-        return rec, tl, ms.value
+        self._check(self._lib.mc_emission_build(self._h, *(ptr(a) for a in st), ptr(td), None, ptr(tl), C.byref(ms)))
+        return self._rows(_capi.MC_TABLE_RECPDF) if host else None, tl, ms.value
 
     def line_luminosities(self, Hden=None, Te=None, Ne=None, ionDen=None, lgBlack=None):
         """outputGas's analytic line luminosities: (forbVol [nCel, 17, 17]
