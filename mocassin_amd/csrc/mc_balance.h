@@ -133,7 +133,8 @@ struct CellArgs {
     const Grains *grains;
     int grains_nb, grains_rows;
     int ncel, cel_most;         // of the atomic data: the solves' LDS
-    int nch;                    // its channels: the integrals' grid
+    int nch, nE, ns1;           // its channels (the integrals' grid), elements, stages + 1
+    size_t cell_lds;            // LDS of one cell (set by the launch)
     // nullable: block b balances cell order[b] (a permutation of 1..ncells),
     // else cell b + 1; results do not depend on the order
     const int *order;

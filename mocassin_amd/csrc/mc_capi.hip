@@ -675,6 +675,8 @@ static mcb::CellArgs cell_args(mc_ctx *c, double jscale)
     a.ncel = c->bal.A.ncel;
     a.cel_most = c->bal.A.cel_most;
     a.nch = c->bal.A.nch;
+    a.nE = c->bal.A.nE;
+    a.ns1 = c->bal.A.nstages + 1;
     return a;
 }
 
