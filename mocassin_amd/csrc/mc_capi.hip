@@ -1169,13 +1169,24 @@ extern "C" int mc_opacity_setup(mc_ctx *c, const mc_opacity_tables *t)
     std::vector<int> bstart(nb + 1, 0);
     std::vector<mco::Ent> ent;
     for (int i = 0; i < nb; ++i) {
-        bstart[i + 1] = bstart[i] + (int)bins[i].size();
         for (auto &p : bins[i]) ent.push_back(mco::Ent{ p.first * 2 + kind[p.first], p.second });
+        while (ent.size() % 4) ent.push_back(mco::Ent{ nslot * 2 + 1, 0.f });
+        bstart[i + 1] = (int)ent.size();
     }
     std::vector<int> iv;
     iv.insert(iv.end(), bstart.begin(), bstart.end());
     iv.insert(iv.end(), sl_e.begin(), sl_e.end());
     iv.insert(iv.end(), sl_st.begin(), sl_st.end());
+    // where the wavefronts of a tile divide the bins, for 1 to kMaxParts of
+    // them: equal shares of a cost of a few entries a bin and one an entry
+    const size_t cuts = iv.size();
+    for (int parts = 1; parts <= mco::kMaxParts; ++parts) {
+        const auto cost = [&](int i) { return (long long)mco::kBinCost * i + bstart[i]; };
+        for (int k = 0, i = 0; k <= parts; ++k) {
+            while (i < nb && cost(i) * parts < cost(nb) * k) ++i;
+            iv.push_back(k == parts ? nb : i);
+        }
+    }
     std::vector<float> fv;
     fv.insert(fv.end(), sabun.begin(), sabun.end());
     fv.insert(fv.end(), efac.begin(), efac.end());
@@ -1187,11 +1198,11 @@ extern "C" int mc_opacity_setup(mc_ctx *c, const mc_opacity_tables *t)
     if (c->d_op_st) { (void)hipFree(c->d_op_st); c->d_op_st = nullptr; }
     HIPCHK(c, dalloc(&c->d_op_i, iv.size()));
     HIPCHK(c, dalloc(&c->d_op_f, fv.size()));
+    ent.resize(ent.size() + mco::kEntPad, mco::Ent{ nslot * 2 + 1, 0.f });
     HIPCHK(c, dalloc(&c->d_op_ent, ent.size()));
     HIPCHK(c, copy_on(c->stream, c->d_op_i, iv.data(), iv.size() * sizeof(int), hipMemcpyHostToDevice));
     HIPCHK(c, copy_on(c->stream, c->d_op_f, fv.data(), fv.size() * sizeof(float), hipMemcpyHostToDevice));
-    if (!ent.empty())
-        HIPCHK(c, copy_on(c->stream, c->d_op_ent, ent.data(), ent.size() * sizeof(mco::Ent), hipMemcpyHostToDevice));
+    HIPCHK(c, copy_on(c->stream, c->d_op_ent, ent.data(), ent.size() * sizeof(mco::Ent), hipMemcpyHostToDevice));
     const size_t nc1 = (size_t)c->G.nCells + 1;
     const int ldst = 3 + nslot;
     HIPCHK(c, dalloc(&c->d_op_st, nc1 * ldst));
@@ -1203,6 +1214,7 @@ extern "C" int mc_opacity_setup(mc_ctx *c, const mc_opacity_tables *t)
     o.st = c->d_op_st; o.ldst = ldst; o.nslot = nslot;
     o.bin_start = c->d_op_i;
     o.ent = c->d_op_ent;
+    o.cuts = c->d_op_i + cuts;
     o.slot_abun = c->d_op_f;
     o.slot_efac = c->d_op_f + nslot;
     o.slot_he2 = he2;
@@ -1272,7 +1284,7 @@ extern "C" int mc_opacity_build(mc_ctx *c, const float *Hden, const float *Te, c
         const mcg::DustArgs &da = c->dust_args;
         HIPCHK(c, mco_launch_f32(c->d_Tdust, nc1 * (da.nsMax + 1) * (da.nSizes + 1), c->d_op_Td, c->stream));
     }
-    const size_t lds = (size_t)(nslot + o.ndrow) * 64 * sizeof(float);
+    const size_t lds = (size_t)(nslot + 1 + o.ndrow) * 64 * sizeof(float);
     HIPCHK(c, mco_launch_opacity(o, lds, c->stream));
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
     if (opacity || scaOpac) {

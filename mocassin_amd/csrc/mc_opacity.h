@@ -10,7 +10,9 @@ namespace mco {
 
 constexpr int kMaxSlots = 160;      // (element, ion) densities per cell
 constexpr int kMaxDustRows = 32;    // grain (species, size) rows
-constexpr int kSplit = 4;           // wavefronts per tile of 64 lattice points
+constexpr int kMaxParts = 16;       // wavefronts per tile of 64 lattice points at most
+constexpr int kBinCost = 4;         // of a bin, in entries
+constexpr int kEntPad = 128;        // entries behind the last that may be read
 
 // one cross-section entry of a bin: qk = slot * 2 + (1 for a heavy ion,
 // added only when its density is > 0)
@@ -32,9 +34,11 @@ struct OpacArgs {
                                      // (eDenSum), in eDenSum's order
     int slot_he2;                    // slot of He+ (density(2,2) of fac1), -1 if absent
     // bins: entries [bin_start[i], bin_start[i+1]) of bin i (0-based), in
-    // addOpacity's order
+    // addOpacity's order, then up to three of slot nslot marked as a heavy
+    // ion's (a density of zero): every bin has a multiple of four
     const int *bin_start;
-    const Ent *ent;
+    const int *cuts;                 // first bins of each of n parts, n + 1 numbers, n = 1 .. kMaxParts
+    const Ent *ent;                  // (kEntPad more than there are)
     float brems1, nu1, xlf1;         // free-free factor, nu(1), log10 nu(1)
     // grains (nullable): rows k = (species-1)*nSizes + size-1
     int ndrow, nSizes, nsMax;

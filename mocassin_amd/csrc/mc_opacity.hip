@@ -6,9 +6,18 @@
 // One lane per lattice point, one wavefront per 64 consecutive points, so
 // every bin's row of opac3 is written in one coalesced 256-byte store.  A
 // lane forms its cell's ion densities in its LDS column once, then walks the
-// bins; each bin's cross-section entries are the same for every lane
-// (scalar loads), in addOpacity's order, and are added in FP32 in that
-// order, so the tables equal the reference's bit for bit.  Bin 1 also
+// bins; each bin's cross-section entries are the same for every lane, in
+// addOpacity's order, and are added in FP32 in that order, so the tables
+// equal the reference's bit for bit.  The entries of successive bins follow
+// each other in memory, each bin's filled up to a multiple of four with
+// entries that never count: a wavefront loads 64 of them at a time, one a
+// lane and the next 64 ahead, and reads them out of the lanes four by four
+// (scalar loads would be waited for together with the densities' LDS reads).
+// The wavefronts of a tile share its bins by their cost: nearly all entries lie
+// in the last fourth of them, and equal ranges left one wavefront the work.
+// Bound by the instructions of the entries on large grids and by the chain of
+// bins on small ones.  45^3 octant, 800 bins: 0.78 ms with loads where a bin
+// needed them, 0.25 now; 21^3: 0.49, 0.05 now.  Bin 1 also
 // carries the free-free term: addOpacity assigns FFOpacity at i = 1 only
 // (ionization_mod.f90:369-393), with the Gaunt factor of the cell's own Te
 // (Hummer 1988, getGauntFF, 195-318).
@@ -99,18 +108,22 @@ __device__ float gaunt_ff(float z, float log10Te, float xlf)
     return g;
 }
 
-__global__ void __launch_bounds__(64) opacity_kernel(OpacArgs a)
+__global__ void __launch_bounds__(64) opacity_kernel(OpacArgs a, int parts)
 {
     extern __shared__ float lds[];               // [nslot][64] densities, then [ndrow][64] weights
     const int lane = threadIdx.x;
-    // kSplit wavefronts share a tile of 64 lattice points, each writing one
+    // `parts` wavefronts share a tile of 64 lattice points, each writing one
     // contiguous range of bins (more wavefronts in flight to hide latency)
-    const int tile = blockIdx.x / kSplit, part = blockIdx.x % kSplit;
+    const int tile = blockIdx.x / parts, part = blockIdx.x % parts;
     const int xyz = mcd::j3_lattice(a.js, (unsigned)(tile * 64 + lane));   // -1: a padding point
     const bool in = xyz >= 0;
     const int cell = in ? a.active[xyz] : 0;
-    float *dens = lds, *wr = lds + a.nslot * 64;
+    // row nslot: zero, of the entries that never count
+    float *dens = lds, *wr = lds + (a.nslot + 1) * 64;
+    dens[a.nslot * 64 + lane] = 0.f;
     float ff1 = 0.f;
+    if (cell <= 0)
+        for (int q = 0; q < a.nslot; ++q) dens[q * 64 + lane] = 0.f;
     if (cell > 0) {
         const float *s = a.st + (size_t)cell * a.ldst;
         const float T = s[0], N = s[1], H = s[2];
@@ -146,34 +159,46 @@ __global__ void __launch_bounds__(64) opacity_kernel(OpacArgs a)
             }
         }
     }
-    const int per = (a.nb + kSplit - 1) / kSplit;
-    const int i0 = part * per, i1 = min(a.nb, i0 + per);
-    const Ent *ent = a.ent;
+    const int *cut = a.cuts + (parts - 1) * (parts + 2) / 2 + part;
+    const int i0 = cut[0], i1 = cut[1];
+    if (i0 >= i1) return;
+    if (!__any(cell > 0)) {
+        for (int i = i0; i < i1; ++i) {
+            const size_t o = ((size_t)tile * a.nb + i) * 64 + lane;
+            a.opac3[o] = 0.f;
+            if (a.sca3) a.sca3[o] = 0.f;
+        }
+        return;
+    }
+    int bound = a.bin_start[min(i0 + lane, a.nb)];       // where bin i0 + lane begins
+    int e = __builtin_amdgcn_readlane(bound, 0), r = 0;
+    const int2 *E = reinterpret_cast<const int2 *>(a.ent) + lane;
+    int2 now = E[e], next = E[e + 64];
     for (int i = i0; i < i1; ++i) {
-        float acc = 0.f, sca = 0.f;
+        const int b = (i - i0 + 1) & 63;
+        if (b == 0) bound = a.bin_start[min(i + 1 + lane, a.nb)];
+        const int e1 = __builtin_amdgcn_readlane(bound, b);
+        float acc = i == 0 ? 0.f + ff1 : 0.f, sca = 0.f;
+        for (; e < e1; e += 4, r += 4) {
+            if (r == 64) {
+                now = next;
+                next = E[e + 64];
+                r = 0;
+            }
+            int qk[4];
+            float sigma[4], d[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                qk[k] = __builtin_amdgcn_readlane(now.x, r + k);
+                sigma[k] = __uint_as_float((unsigned)__builtin_amdgcn_readlane(now.y, r + k));
+                d[k] = dens[(qk[k] >> 1) * 64 + lane];
+            }
+            // a heavy ion (qk odd) counts only where its density is above zero
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (!(qk[k] & 1) || d[k] > 0.f) acc = acc + sigma[k] * d[k];
+        }
         if (cell > 0) {
-            acc = acc + (i == 0 ? ff1 : 0.f);
-            const int e1 = a.bin_start[i + 1];
-            int e = a.bin_start[i];
-            // four entries' (slot, kind, sigma) fetched ahead of the
-            // dependent FP32 sum, which stays in the reference's order
-            for (; e + 4 <= e1; e += 4) {
-                Ent en[4];
-                float d[4];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) en[k] = ent[e + k];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) d[k] = dens[(en[k].qk >> 1) * 64 + lane];
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    if (!((en[k].qk & 1) && !(d[k] > 0.f))) acc = acc + en[k].sigma * d[k];
-            }
-            for (; e < e1; ++e) {
-                const Ent en = ent[e];
-                const float d = dens[(en.qk >> 1) * 64 + lane];
-                if ((en.qk & 1) && !(d > 0.f)) continue;
-                acc = acc + en.sigma * d;
-            }
             if (a.ndrow) {
                 float ab = 0.f;
                 for (int r = 0; r < a.ndrow; ++r) {
@@ -184,6 +209,8 @@ __global__ void __launch_bounds__(64) opacity_kernel(OpacArgs a)
                 }
                 acc = acc + (sca + ab);
             }
+        } else {
+            acc = 0.f;
         }
         const size_t o = ((size_t)tile * a.nb + i) * 64 + lane;   // padding points get 0
         a.opac3[o] = acc;
@@ -216,7 +243,13 @@ __global__ void f32_kernel(const double *in, size_t n, float *out)
 hipError_t mco_launch_opacity(const mco::OpacArgs &a, size_t lds_bytes, hipStream_t s)
 {
     const unsigned tiles = (unsigned)(mcd::j3_points(a.js) / 64);
-    hipLaunchKernelGGL(mco::opacity_kernel, dim3(tiles * mco::kSplit), dim3(64), lds_bytes, s, a);
+    // wavefronts for the chip (16 a CU), at least four a tile; each lays out
+    // the tile's densities for itself, which eight a tile repeated too often
+    // (0.18 against 0.15 ms for H and He on 45^3; 0.25 against 0.31 with 80
+    // segments, at twice the cost of a bin)
+    const unsigned want = (4096 + tiles - 1) / tiles;
+    const unsigned parts = want < 4 ? 4 : want > mco::kMaxParts ? mco::kMaxParts : want;
+    hipLaunchKernelGGL(mco::opacity_kernel, dim3(tiles * parts), dim3(64), lds_bytes, s, a, (int)parts);
     return hipGetLastError();
 }
 
