@@ -21,7 +21,7 @@ constexpr int kBlock = 16384;            // entries sorted together
 constexpr int kBlockChunks = kBlock / mcd::kLogChunk;
 constexpr int kGroup = 16;               // blocks whose run tables lie together
 constexpr int kRange = 16384;            // words summed by one workgroup (128 KB of LDS)
-constexpr int kMaxBins = 7936;           // with a block's entries they fill the LDS of a CU
+constexpr int kMaxBins = 7936;           // with half a block's entries, 4 bytes each, they fill half the LDS of a CU
 constexpr int kMaxShift = 17;
 
 // `words` estimator words in at most kMaxBins bins of 2^shift; a bin is one
