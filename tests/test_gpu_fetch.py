@@ -50,6 +50,34 @@ def test_estimators_of_any_size_come_back_whole(n, nb):
         assert len(got[k]) == 5 and all(np.array_equal(g, want[k]) for g in got[k])
 
 
+# the smallest, columns of one brick, of several workgroups and on their edge (16
+# points of 4 x 4 each 512 to a workgroup), ragged bricks, bins in slices
+@pytest.mark.parametrize("shape,nb", [((2, 2, 2), 3), ((5, 3, 32), 7), ((4, 4, 33), 3), ((2, 9, 130), 31),
+                                      ((13, 6, 27), 411), ((31, 30, 29), 61)])
+def test_estimators_of_any_lattice_come_back(shape, nb):
+    """Cells numbered in any order, a third of the positions inactive."""
+    from mocassin_amd.transport import Transport
+    print("lattice", shape, nb, flush=True)
+    rng = np.random.default_rng(nb)
+    n = int(np.prod(shape))
+    nc = n - n // 3
+    act = np.zeros(n, np.int32)
+    act[rng.permutation(n)[:nc]] = rng.permutation(nc) + 1
+    ax = [np.linspace(0.0, 1.e17, k).astype(np.float32) for k in shape]
+    at = int(np.flatnonzero(act == 1)[0])
+    star = np.unravel_index(at, shape, order="F")
+    T = Transport(*ax, act.reshape(shape, order="F"), nc, nb, np.geomspace(1e-5, 25, nb).astype(np.float32), R_out=1.e17,
+                  geoCorr=(0, 0, 0), ionEdge1=1.0, starPos=[float(a[k]) for a, k in zip(ax, star)],
+                  starIdx=[int(k) + 1 for k in star], deltaE=1.0)
+    try:
+        want = rng.random((nc + 1, nb))
+        want[0] = 0.0
+        T.set_estimators(np.asfortranarray(want))
+        assert np.array_equal(T.fetch()[0], want)
+    finally:
+        T.close()
+
+
 @pytest.mark.parametrize("name", ["c2mini", "dust_pe"])
 def test_table_rows_equal_the_columns(name):
     from test_gpu_emission import _ctx as emission_ctx
