@@ -70,7 +70,7 @@ def kernel_name(t):
     from mocassin_amd._capi import KERNELS
     if t.get("kernel", 0) == KERNELS["one"]:
         return "mcd::transport_kernel<false>"
-    return "mcd::log_kernel<8> + mcl::sort_kernel + mcl::plan_kernel + mcl::reduce_kernel"
+    return "mcd::log_kernel + mcl::sort_kernel + mcl::plan_kernel + mcl::reduce_kernel"
 
 
 def lanes_per_pass(c):

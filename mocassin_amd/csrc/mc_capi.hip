@@ -2139,8 +2139,8 @@ static void log_give_back(int device)
 // The chunks a sweep's log should have, or 0 for a sweep that adds with
 // atomics: below about 2e6 deposits the two extra kernels cost more than the
 // atomics, crossing counts go with the atomics, and the words of both
-// estimators must fit the log's ranges.  A flight's segments grow with the
-// axes; the last sweep's count is the better guess.
+// estimators must fit the log's ranges (at most 5.2e8).  A flight's segments
+// grow with the axes; the last sweep's count is the better guess.
 static unsigned log_chunks(const mc_ctx *c, int64_t npackets, const mcl::Shape &s, int blocks, int threads)
 {
     if (!s.bins || (c->G.flags & mcd::F_CROSS)) return 0;
