@@ -69,7 +69,7 @@ def kernel_name(t):
     pool takes) at a launch shape, as rocprofv3 names them."""
     from mocassin_amd._capi import KERNELS
     if t.get("kernel", 0) == KERNELS["one"]:
-        return "mcd::transport_kernel<false>"
+        return "mcd::transport_kernel"
     return "mcd::log_kernel + mcl::sort_kernel + mcl::plan_kernel + mcl::reduce_kernel"
 
 

@@ -4,8 +4,9 @@
 // One 64-lane wavefront per cell (one wavefront per workgroup), or several
 // cells to a wavefront where there are no model ions; cell state in LDS.
 // Lanes share the work of each stage of the reference's schedule:
-//   * photoionisation rates and heating integrals: lanes over frequency
-//     bins, wave reductions per channel (update_mod.f90:184-269, 1146-1234);
+//   * photoionisation rates and heating integrals: a kernel of their own
+//     before the balance, lanes over lattice points (update_mod.f90:184-269,
+//     1146-1234);
 //   * recombination fits, charge exchange, ion ratios: lanes over the
 //     (elem, ion) channels (calcAlpha, radRecFit, dielectronic, ionBalance);
 //   * CEL cooling: the n-level systems of four model ions at a time, one in
@@ -207,14 +208,15 @@ __device__ __forceinline__ double cooling(const Atomic &A, const Lds &S, int lan
 // (setPhotoelHeatCool) and the collision terms (setDustGasCollHeatCool).
 // The rows are independent, and each step of a row's iteration waits for the
 // one before: so all rows iterate at once, each on its own group of lanes
-// (64 over the next power of two of the rows), instead of one after another
-// on the whole wavefront.  The sums over frequency are linear in the
+// (the cell's lanes over the next power of two of the rows), instead of one
+// after another on all of them.  The sums over frequency are linear in the
 // potential for every bin above the threshold (yield Y (1 - V/d) with d = nu
 // - vn, photoelectron energy Y (d - V^2/d) / 2), so the cell's suffix sums of
 // u, u/d and u d (u = Y sigma flux) over 16 chunks of bins are formed once,
 // and a step adds up the bins of the threshold's chunk alone.  Bound by the
 // latency of the steps: the balance kernel of the dust and gas 60^3 grid (10
-// rows, 160 bins) took 38 ms with one row at a time over all bins, 11.5 now.
+// rows, 160 bins) took 38 ms with one row at a time over all bins, 11.5 with
+// all rows at once, 6.3 with four cells to a wavefront besides.
 constexpr double kPiR = (double)3.141592654f;             // constants_mod.f90:32 (REAL)
 constexpr double kFourPiR = (double)(4.f * 3.141592654f);
 constexpr double kHcRyd = 2.1799153e-11, kRyd2erg = 2.1799e-11, kKB = 1.380658e-16;

@@ -2171,7 +2171,7 @@ static int transport_launch(mc_ctx *c, mcd::RunArgs &RA, int blocks)
     const int threads = c->tune.threads, kernel = transport_kernel_of(c->tune);
     // the log kernel's registers and LDS leave room for a fifth workgroup of
     // 256 where the pool kernel's leave four: 47 against 49.5 ms (dust and gas
-    // 60^3), 23.4 against 24.5 (45^3 octant)
+    // 60^3), 23.4 against 24.5 (45^3 octant), before the sort's second workgroup
     const int wide = blocks >= c->tune.blocks_per_cu * c->cus * (256 / threads) ? blocks + blocks / 4 : blocks;
     mcl::Shape s = mcl::shape(0);
     unsigned chunks = 0;
@@ -2417,15 +2417,14 @@ extern "C" int mc_transport_batch(mc_ctx *const *ctx, int32_t n, const int32_t *
 // ------------------------------------------ batched launch, no allocation
 // mc_transport_batch_noalloc: mc_transport_batch for callers that cannot
 // allocate device memory.  The launch's working block (the models' grids,
-// run arguments and counters, the chunk table and the chunk counter) lives
-// in the file-scope device array `scratch` (kNoAllocBytes on every GPU the
-// library runs on, held until the process ends) instead of a per-call
-// allocation.  Its device address is taken once per device when the first
+// run arguments, shares and counters) lives in the file-scope device array
+// `scratch` (kNoAllocBytes on every GPU the library runs on, held until the
+// process ends) instead of a per-call allocation.  Its device address is taken once per device when the first
 // context on that device is created (noalloc_scratch_init) and only that
 // address is handed to kernels and copies.  Every call on one GPU reuses the
-// array, which keeps the last call's contents: the counters and the chunk
-// counter are cleared by a kernel at the start of each call, and calls that
-// overlap on one GPU race.
+// array, which keeps the last call's contents: the counters are
+// cleared by a kernel at the start of each call, and calls that overlap on
+// one GPU race.
 constexpr size_t kNoAllocBytes = 8u << 20;
 constexpr int kNoAllocModels = 256;
 constexpr int kNoAllocDevices = 64;

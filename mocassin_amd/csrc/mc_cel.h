@@ -12,8 +12,8 @@
 // rows in LDS and the back substitution on one lane, 22 ions took 2.0e3
 // vector instructions each and most of the time waited for LDS.  45^3 octant
 // (46890 cells, 22 ions of 2 to 15 levels), before and now: line luminosities
-// 9.3 -> 1.7 ms, the balance's reference schedule 24.6 -> 6.5 ms, re-emission
-// tables 10.4 -> 5.0 ms.
+// 9.3 -> 1.7 ms, the balance's reference schedule 24.6 -> 5.6 ms (with the
+// shorter ion steps), re-emission tables 10.4 -> 3.8 ms (1.3 of it here).
 // What depends on the atomic data alone (level differences, A times energy,
 // which pairs radiate) is prepared once on the host, laid out as the lanes
 // read it; the ions are sorted by size, so that a batch's ions are alike.

@@ -24,10 +24,10 @@
 // request, 2e10 of them a second, which was 2/3 of a sweep's time; a logged
 // deposit is 8 bytes written and read three times.  The walk itself is bound
 // by its instructions at 16 and more wavefronts a CU.  One sweep of 1e8
-// packets on a 45^3 octant of 800 bins (1.8e9 deposits): 45.7 ms before (the
-// pool with atomics and divisions), 23.4 now (walk and log 14, sort 6, sums
-// 3.5); 4e7 packets in dust and gas 60^3: 67.4 ms before, 46.7 now; 8 models
-// of 15^3 cells in one launch: 60 ms before, 22 now.
+// packets on a 45^3 octant of 800 bins (1.8e9 deposits): 64.8 ms before (the
+// pool with atomics and divisions), 39.0 now (walk and log 22.6, sort 8.4,
+// sums 7.8); 4e7 packets in dust and gas 60^3: 67.4 ms before, 42.0 now; 8
+// models of 20^3 to 50^3 cells, 2e6 packets each, in one launch: 5.9 ms.
 #include <algorithm>
 
 #include "mc_device.h"
