@@ -111,7 +111,7 @@ struct mc_ctx {
     mco::Ent *d_op_ent = nullptr;                // cross-section entries of every bin
     float *d_hs = nullptr;              // a state given by the host, and the same in rows
     double *d_hst = nullptr;
-    size_t hs_n = 0;
+    size_t hs_n = 0, hst_n = 0, cold_n = 0, ion_host_n = 0, op_Td_n = 0, em_Td_n = 0;   // entries (room)
     float *d_op_st = nullptr, *d_op_Td = nullptr, *d_op_out = nullptr;
     mco::OpacArgs op{};
     int *op_slot_e = nullptr, *op_slot_st = nullptr;   // into d_op_i
@@ -166,6 +166,20 @@ static hipError_t dalloc(T **p, size_t n)
     if (hipGetDevice(&device) != hipSuccess) return e;
     log_give_back(device);
     return hipMalloc((void **)p, bytes);
+}
+
+// Room for n entries in a buffer that is kept between calls, `have` of them
+// so far: a later set-up's elements, stages or grains may need more.
+template <class T>
+static hipError_t room(T **p, size_t *have, size_t n)
+{
+    if (*p && *have >= n) return hipSuccess;
+    if (*p) (void)hipFree(*p);
+    *p = nullptr;
+    *have = 0;
+    const hipError_t e = dalloc(p, n);
+    if (e == hipSuccess) *have = n;
+    return e;
 }
 
 // Every copy and fill of a context goes on its stream, in order with its
@@ -924,14 +938,8 @@ static int upload_state(mc_ctx *c, const float *Hden, const float *Te, const flo
 {
     const int nE = c->bal.A.nE, ns = c->bal.A.nstages;
     const size_t nc1 = (size_t)c->G.nCells + 1, nf = nc1 * (3 + (size_t)nE * ns), nd = nc1 * (3 + (size_t)nE * (ns + 1));
-    if (c->hs_n < nd) {
-        if (c->d_hs) { (void)hipFree(c->d_hs); c->d_hs = nullptr; }
-        if (c->d_hst) { (void)hipFree(c->d_hst); c->d_hst = nullptr; }
-        c->hs_n = 0;
-        HIPCHK(c, dalloc(&c->d_hs, nf));
-        HIPCHK(c, dalloc(&c->d_hst, nd));
-        c->hs_n = nd;
-    }
+    HIPCHK(c, room(&c->d_hs, &c->hs_n, nf));
+    HIPCHK(c, room(&c->d_hst, &c->hst_n, nd));
     const float *part[3] = { Te, Ne, Hden };
     for (int k = 0; k < 3; ++k)
         HIPCHK(c, hipMemcpyAsync(c->d_hs + k * nc1, part[k], nc1 * sizeof(float), hipMemcpyHostToDevice, c->stream));
@@ -1008,7 +1016,7 @@ static int update_cells(mc_ctx *c, double jscale, const mc_balance_opts *opts, c
         // ionDen(0:nCells, xref, stage) goes up as the host holds it; a
         // kernel lays it out as [cell][element index][stage 0..ns]
         for (int ei = 0; ei < nE; ++ei) imap.xr[ei] = c->bal.eidx_xref[ei] - 1;
-        if (!c->d_ion_host) HIPCHK(c, dalloc(&c->d_ion_host, nc1 * nE * ns));
+        HIPCHK(c, room(&c->d_ion_host, &c->ion_host_n, nc1 * nE * ns));
         HIPCHK(c, hipMemcpyAsync(c->d_Hden, Hden, nc1 * sizeof(double), hipMemcpyHostToDevice, c->stream));
         HIPCHK(c, hipMemcpyAsync(c->d_Te, Te, nc1 * sizeof(double), hipMemcpyHostToDevice, c->stream));
         HIPCHK(c, hipMemcpyAsync(c->d_Ne, Ne, nc1 * sizeof(double), hipMemcpyHostToDevice, c->stream));
@@ -1022,7 +1030,7 @@ static int update_cells(mc_ctx *c, double jscale, const mc_balance_opts *opts, c
     HIPCHK(c, hipMemsetAsync(c->d_flags, 0, nc1 * sizeof(int), c->stream));
     HIPCHK(c, hipMemsetAsync(c->d_nIter, 0, nc1 * sizeof(int), c->stream));
     if (warm) {
-        if (!c->d_cold) HIPCHK(c, dalloc(&c->d_cold, 2 * nc1 + nion));
+        HIPCHK(c, room(&c->d_cold, &c->cold_n, 2 * nc1 + nion));
         int rc = mlp_rows(c);
         if (rc) return rc;
         HIPCHK(c, hipMemcpyAsync(c->d_cold, c->d_Te, nc1 * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
@@ -1261,7 +1269,7 @@ extern "C" int mc_opacity_build(mc_ctx *c, const float *Hden, const float *Te, c
     if (dust) {
         const mcg::DustArgs &da = c->dust_args;
         const size_t ntd = nc1 * (da.nsMax + 1) * (da.nSizes + 1);
-        if (!c->d_op_Td) HIPCHK(c, dalloc(&c->d_op_Td, ntd));
+        HIPCHK(c, room(&c->d_op_Td, &c->op_Td_n, ntd));
         if (Tdust) HIPCHK(c, copy_on(c->stream, c->d_op_Td, Tdust, ntd * sizeof(float), hipMemcpyHostToDevice));
         const int K = c->dust_rows;
         o.ndrow = K; o.nSizes = da.nSizes; o.nsMax = da.nsMax;
@@ -1551,7 +1559,7 @@ extern "C" int mc_emission_build(mc_ctx *c, const float *Hden, const float *Te, 
         a.dweight = a.ndust + nc1;
         a.dgabun = a.dweight + da.nSizes;
         const size_t ntd = nc1 * (da.nsMax + 1) * (da.nSizes + 1);
-        if (Tdust && !c->d_em_Td) HIPCHK(c, dalloc(&c->d_em_Td, ntd));
+        if (Tdust) HIPCHK(c, room(&c->d_em_Td, &c->em_Td_n, ntd));
         if (Tdust) {
             std::vector<double> td(ntd);
             for (size_t i = 0; i < ntd; ++i) td[i] = Tdust[i];
