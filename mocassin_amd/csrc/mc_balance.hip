@@ -1120,11 +1120,20 @@ hipError_t mcb_launch_balance(const mcb::Atomic *dA, const mcb::CellArgs &a, hip
     // schedule: 7.2 ms with a wavefront a cell, 1.1 with 4 lanes; secant from
     // the network's prediction, bound by the slowest cell's steps: 3.1 and
     // 1.7.  The same with grains, dust and gas 60^3: 11.5 and 6.3 (16 lanes).
+    // Grains on many bins or rows have a wavefront a cell again: a row's few
+    // lanes then sum long chunks one after another, and four cells' LDS lets
+    // few wavefronts on a CU (with 4096 bins and 16 rows it is more than a CU
+    // has).  Both grow alike, so the line is drawn by the LDS.  30000 cells,
+    // 16 lanes against 64, ms, by the KB of four cells: 10 rows 160 bins (25)
+    // 2.5, 3.6, 320 bins (30) 4.4, 4.3, 640 bins (40) 8.7, 6.0; 16 rows 96
+    // bins (33) 3.7, 4.0, 240 bins (37) 5.8, 4.9; 5 rows 640 bins (31) 2.9, 3.1.
     const int K = a.grains ? a.grains_rows : 0, most = std::max(a.nch, a.nE);
-    const int lanes = a.ncel > 0 || most > 16 || K > 16 ? 64 : most > 4 || K > 0 ? 16 : 4;
+    constexpr size_t kSideBySide = 32 * 1024;
     mcb::CellArgs b = a;
     b.cell_lds = (mcb::state_bytes(a.nE, a.ns1, a.nch) + mcb::shared_bytes(a.ncel, a.cel_most, a.nE, a.ns1, a.nch) +
                   (K ? mcb::grain_bytes(a.grains_nb, a.nch, K) : 0) + 7) / 8 * 8;
+    const bool wide = a.ncel > 0 || most > 16 || K > 16 || (K > 0 && 4 * b.cell_lds > kSideBySide);
+    const int lanes = wide ? 64 : most > 4 || K > 0 ? 16 : 4;
     // an odd number of words apart, the cells' equal words lie in different banks
     if (lanes < 64 && b.cell_lds % 16 == 0) b.cell_lds += 8;
     const int per = 64 / lanes;
