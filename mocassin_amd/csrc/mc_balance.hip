@@ -178,7 +178,8 @@ __device__ __forceinline__ double cooling(const Atomic &A, const Lds &S, int lan
     double bRec = 9.4255985E-11 - 4.04794384E-12 * lg - 1.0055237E-11 * lg * lg +
                   1.99266862E-12 * lg * lg * lg - 1.06681387E-13 * lg * lg * lg * lg;
     double coolRec = Np * Ne * bRec * kB * T / sqrt(T);
-    Np = S.ion[1 * S.ns1 + 3] * A.el[1].abun;
+    // (with two stages there is no He++, nor a word for it in the row)
+    Np = S.ns1 > 3 ? S.ion[1 * S.ns1 + 3] * A.el[1].abun : 0.0;
     const double ls = log10(T / 4.);
     bFF = 2. * (1.0108464E-11 + 9.7930778E-13 * ls - 6.6433144E-13 * ls * ls +
                 2.4793747E-13 * ls * ls * ls - 2.3938215E-14 * ls * ls * ls * ls);
