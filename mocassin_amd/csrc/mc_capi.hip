@@ -18,6 +18,7 @@
 #include "mc_device.h"
 #include "mc_dust.h"
 #include "mc_emission.h"
+#include "mc_hold.h"
 #include "mc_kernels.h"
 #include "mc_mlp.h"
 #include "mc_opacity.h"
@@ -2189,12 +2190,12 @@ static int transport_launch(mc_ctx *c, mcd::RunArgs &RA, int blocks)
         c->G.esc_word = (unsigned)je;
         chunks = log_chunks(c, RA.npackets, s, wide, threads);
     }
-    std::unique_lock<std::mutex> use;
-    if (chunks) {
-        use = std::unique_lock<std::mutex>(g_log[c->device].use, std::try_to_lock);
-        if (!use.owns_lock() || !g_log[c->device].reserve(chunks, s, mcd_save_words(wide, threads))) chunks = 0;
-    }
+    const auto wait = [c] { (void)hipStreamSynchronize(c->stream); };
+    mcl::Hold<decltype(wait)> use(wait);
+    if (chunks && (!use.take(g_log[c->device].use) || !g_log[c->device].reserve(chunks, s, mcd_save_words(wide, threads))))
+        chunks = 0;
     if (!chunks) {
+        use.drop();
         HIPCHK(c, mcd_launch_transport(c->G, RA, blocks, threads, kernel, c->stream));
         return MC_OK;
     }
@@ -2211,11 +2212,13 @@ static int transport_launch(mc_ctx *c, mcd::RunArgs &RA, int blocks)
                          plan + 3 * mcl::kMaxBins + mcl::kMaxItems };
     int more = 1;
     for (RA.resume = 0; more; RA.resume = 1) {
+        use.began();
         HIPCHK(c, fill_on(c->stream, P.state, 0, (2 + 2 * mcl::kMaxBins) * sizeof(unsigned)));
         HIPCHK(c, mcd_launch_transport(c->G, RA, wide, threads, MCD_KERNEL_LOG, c->stream));
         HIPCHK(c, mcl_sort(L, s, c->cus, c->stream));
         HIPCHK(c, mcl_reduce(L, s, c->d_J3, c->d_esc, c->G.esc_word, c->cus, c->stream));
         HIPCHK(c, copy_on(c->stream, &more, RA.suspended, sizeof more, hipMemcpyDeviceToHost));
+        use.ended();
     }
     return MC_OK;
 }
