@@ -319,7 +319,9 @@ static int ctx_init(mc_ctx *c, const mc_desc *d)
     HIPCHK(c, copy_on(c->stream, c->d_nuArray, d->nuArray, nb * sizeof(float), hipMemcpyHostToDevice));
 
     mcd::Grid &G = c->G;
-    G.nx = nx; G.ny = ny; G.nz = nz; G.nCells = nc; G.nbins = nb; G.flags = d->flags;
+    G.nx = nx; G.ny = ny; G.nz = nz; G.nCells = nc; G.nbins = nb;
+    // the host's flags alone: the others are the library's own (mcd::Flags)
+    G.flags = d->flags & (MC_SYMMETRIC | MC_DUST | MC_GAS | MC_ISOTROPIC | MC_MULTISTARS);
     G.nStars = d->nStars;
     G.R_out = d->R_out;
     for (int a = 0; a < 3; ++a) {
