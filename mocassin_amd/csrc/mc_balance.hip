@@ -907,12 +907,12 @@ __global__ void __launch_bounds__(64) integrals_kernel(const Atomic *__restrict_
             for (int u = 0; u < kIntBins; ++u) {
                 any |= J[u] > 0.0;
                 band += J[u];
-                // (the last step's bins beyond the mesh are no band's end)
-                if (j0 + u == bend && b < mcm::kBands) {
+                if (j0 + u == bend) {
                     if (brow) brow[b] = (float)log10(fmax(band, 1.e-30));
                     band = 0.0;
                     ++b;
-                    bend = (b + 1) * nb / mcm::kBands;
+                    // (no bin beyond the mesh ends a band)
+                    bend = b < mcm::kBands ? (b + 1) * nb / mcm::kBands : 0;
                 }
             }
     }
