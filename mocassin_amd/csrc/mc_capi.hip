@@ -2349,8 +2349,13 @@ static hipError_t batch_launch(mc_ctx *const *ctx, const mcd::BatchArgs &B, cons
     }
     if (fits) return mcd_launch_batch(B, lds, blocks, c0->stream);
     hipError_t e = hipSuccess;
-    for (int i = 0; i < B.models && e == hipSuccess; ++i)
-        if (RA[i].npackets > 0) e = mcd_launch_transport(ctx[i]->G, RA[i], blocks, 256, MCD_KERNEL_POOL, c0->stream);
+    for (int i = 0; i < B.models && e == hipSuccess; ++i) {
+        if (RA[i].npackets <= 0) continue;
+        const mcd::Grid &G = ctx[i]->G;
+        e = mcd_pool_fits(G) || mcd_transport_fits(G, 256)
+                ? mcd_launch_transport(G, RA[i], blocks, 256, MCD_KERNEL_POOL, c0->stream)
+                : mcd_launch_transport(G, RA[i], 4 * blocks, 64, MCD_KERNEL_THIN, c0->stream);
+    }
     return e;
 }
 

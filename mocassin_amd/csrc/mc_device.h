@@ -132,12 +132,13 @@ struct Grid {
 constexpr int kGuide = 32;
 
 // Per-axis tables of the walk, staged in LDS; cells are 0-based here.
-//   wall[2 i], wall[2 i + 1]  the walls a packet in cell i meets moving down
-//                             and up: the midpoints to its neighbours, the
-//                             outer edge in the first and last cell
-//   part[i]                   getVolume's factor of cell i and what its index
-//                             adds to the packet's word of the tables
-// A step reads one wall and one part per axis.
+//   wall[i], wall[i + 1]  the walls a packet in cell i meets moving down and
+//                         up: the midpoints to its neighbours, the outer edge
+//                         in the first and last cell
+//   part[i]               getVolume's factor of cell i and what its index
+//                         adds to the packet's word of the tables
+// A step reads one wall and one part per axis.  12 bytes a cell: with
+// wavefronts' rings and pools beside it this decides how long the axes may be.
 struct AxisPart { float d; uint32_t o; };
 struct Axes {
     const float *wx, *wy, *wz;
@@ -401,7 +402,7 @@ __device__ __forceinline__ float wall_distance(const float *wall, int n, float v
 {
     const bool pos = v > 1.e-10f, neg = v < -1.e-10f;
     const bool inner = pos ? (i < n - 1) : (i > 0);
-    const float m = wall[2 * i + (pos ? 1 : 0)];
+    const float m = wall[i + (pos ? 1 : 0)];
     const float d = (m - r) / v;
     lost = false;
     if (!(pos || neg)) return 1.e35f;
@@ -436,9 +437,9 @@ __device__ __forceinline__ int walk_step(const Grid &G, const Axes &A, Walker &W
     if (!ZERO_OPACITY) kappa = G.opac3[Word<WIDE>::index(G, S.w, nu0)];
 
     // wall distances (1263-1379); the wall of a component by its sign
-    const float mx = A.wx[2 * W.x + (W.vx > 0.f ? 1 : 0)];
-    const float my = A.wy[2 * W.y + (W.vy > 0.f ? 1 : 0)];
-    const float mz = A.wz[2 * W.z + (W.vz > 0.f ? 1 : 0)];
+    const float mx = A.wx[W.x + (W.vx > 0.f ? 1 : 0)];
+    const float my = A.wy[W.y + (W.vy > 0.f ? 1 : 0)];
+    const float mz = A.wz[W.z + (W.vz > 0.f ? 1 : 0)];
     float dSx = fabsf(wall_quotient(mx - W.rx, W.vx, W.qx));
     float dSy = fabsf(wall_quotient(my - W.ry, W.vy, W.qy));
     float dSz = fabsf(wall_quotient(mz - W.rz, W.vz, W.qz));
@@ -457,9 +458,9 @@ __device__ __forceinline__ int walk_step(const Grid &G, const Axes &A, Walker &W
         if (lostZ) return ST_LOST;
         if (isnan(dSz)) { err = 34; return ST_ERROR; }
         // cells on the cell wall, 1382-1384
-        if (fabsf(dSx) < 1.e-10f) dSx = A.wx[2 * G.nx - 1];
-        if (fabsf(dSy) < 1.e-10f) dSy = A.wy[2 * G.ny - 1];
-        if (fabsf(dSz) < 1.e-10f) dSz = A.wz[2 * G.nz - 1];
+        if (fabsf(dSx) < 1.e-10f) dSx = A.wx[G.nx];
+        if (fabsf(dSy) < 1.e-10f) dSy = A.wy[G.ny];
+        if (fabsf(dSz) < 1.e-10f) dSz = A.wz[G.nz];
         dSx = fabsf(dSx); dSy = fabsf(dSy); dSz = fabsf(dSz);
         if (dSx <= 0.f) dS = fminf(dSy, dSz);
         else if (dSy <= 0.f) dS = fminf(dSx, dSz);

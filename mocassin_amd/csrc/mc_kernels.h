@@ -57,8 +57,11 @@ hipError_t mcd_launch_batch(const mcd::BatchArgs &B, size_t lds_bytes, int block
 // 2047 x 1023 cells, 65535 bins and 2^32 - 1 table words; other grids run the
 // first whatever kernel is asked for.
 // The log kernel is the pool kernel with the deposits written to the log of
-// its RunArgs instead of added to the estimators.
-enum { MCD_KERNEL_ONE = 1, MCD_KERNEL_POOL = 3, MCD_KERNEL_LOG = 4 };
+// its RunArgs instead of added to the estimators.  The thin kernel is the
+// first with shorter rings, for axes that leave no room for more.
+enum { MCD_KERNEL_ONE = 1, MCD_KERNEL_POOL = 3, MCD_KERNEL_LOG = 4, MCD_KERNEL_THIN = 5 };
+// the first kernel's tables and rings fit a CU's LDS
+bool mcd_transport_fits(const mcd::Grid &G, int threads);
 size_t mcd_save_words(int blocks, int threads);
 bool mcd_pool_fits(const mcd::Grid &G);
 size_t mcd_pool_lds(const mcd::Grid &G, int threads);

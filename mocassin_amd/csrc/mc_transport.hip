@@ -37,30 +37,31 @@
 
 namespace mcd {
 
-// LDS of a staged grid: walls | parts.  The tables of an axis follow those
+// LDS of a staged grid: parts | walls.  The tables of an axis follow those
 // of the one before.
 template <bool WIDE>
 __device__ __forceinline__ void stage_axes(const Grid &G, float *lds, Axes &A)
 {
     const int n3[3] = { G.nx, G.ny, G.nz };
     const int na = G.nx + G.ny + G.nz;
-    AxisPart *parts = reinterpret_cast<AxisPart *>(lds + 2 * na);
+    AxisPart *parts = reinterpret_cast<AxisPart *>(lds);
+    float *walls = lds + 2 * na;
     for (int k = 0, o = 0; k < 3; o += n3[k], ++k) {
         const float *ax = G.axis + o, *mid = G.mid + o - k;
-        for (int i = threadIdx.x; i < n3[k]; i += blockDim.x) {
-            lds[2 * (o + i)] = i > 0 ? mid[i - 1] : ax[0];
-            lds[2 * (o + i) + 1] = i < n3[k] - 1 ? mid[i] : ax[i];
-            parts[o + i] = AxisPart{ G.dfac[o + i], axis_word<WIDE>(G, k, i) };
+        const int n = n3[k];
+        for (int i = threadIdx.x; i <= n; i += blockDim.x) {
+            walls[o + k + i] = i == 0 ? ax[0] : i < n ? mid[i - 1] : ax[n - 1];
+            if (i < n) parts[o + i] = AxisPart{ G.dfac[o + i], axis_word<WIDE>(G, k, i) };
         }
     }
     __syncthreads();
-    A.wx = lds; A.wy = lds + 2 * G.nx; A.wz = lds + 2 * (G.nx + G.ny);
+    A.wx = walls; A.wy = walls + G.nx + 1; A.wz = walls + G.nx + G.ny + 2;
     A.px = parts; A.py = parts + G.nx; A.pz = parts + G.nx + G.ny;
 }
 
 __host__ __device__ inline size_t lds_floats(int nx, int ny, int nz)
 {
-    return (size_t)4 * (nx + ny + nz);
+    return (size_t)3 * (nx + ny + nz) + 3;
 }
 
 // A launch's grid and run arguments in memory, at wavefront-uniform
@@ -819,7 +820,10 @@ __device__ __forceinline__ Args kernel_args()
 
 // One packet per lane, for lattices the pool kernel does not take (64-bit
 // table indices).  An emission pass runs when at least emit_min lanes (or as
-// many as are walking) wait for one, then walk_steps walk passes.
+// many as are walking) wait for one, then walk_steps walk passes.  Rings of
+// D: in a batch, lattices with axes too long for four wavefronts' rings of
+// eight beside their tables run one-wavefront workgroups with rings of four.
+template <int D>
 __global__ void __launch_bounds__(256) transport_kernel(LaunchArgs)
 {
     extern __shared__ float lds[];
@@ -828,9 +832,9 @@ __global__ void __launch_bounds__(256) transport_kernel(LaunchArgs)
     const RunArgs RA = scalar_copy<RunArgs>(P.r);
     Axes A;
     const int nwaves = (int)(blockDim.x >> 6);
-    stage_axes<true>(G, lds + (size_t)nwaves * JRing<kJDepth, true>::kFloats, A);
+    stage_axes<true>(G, lds + (size_t)nwaves * JRing<D, true>::kFloats, A);
     const int lane_id = threadIdx.x & 63;
-    AddSink<kJDepth, true> K{ jq_at<kJDepth, true>(lds, (int)(threadIdx.x >> 6)) };
+    AddSink<D, true> K{ jq_at<D, true>(lds, (int)(threadIdx.x >> 6)) };
 
     Lane L = idle_lane();
     Stock S;
@@ -985,8 +989,10 @@ __global__ void __launch_bounds__(256) log_kernel(LaunchArgs)
 // that model has no packets left goes through the others in turn, helping
 // those that still have some.  Each packet keeps its own random stream, so
 // results equal those of the models' separate runs.  Every workgroup visits
-// every model at most once, which bounds the loop.
-__global__ void __launch_bounds__(256) batch_kernel(BatchArgs B)
+// every model at most once, which bounds the loop.  128 VGPRs: with two more
+// three wavefronts fit a SIMD instead of four (8 models of 20^3 to 50^3 cells:
+// 6.76 ms against 6.18).
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) batch_kernel(BatchArgs B)
 {
     extern __shared__ float lds[];
     __shared__ int s_left;
@@ -1107,6 +1113,18 @@ bool mcd_pool_fits(const mcd::Grid &G)
            mcd::j3_size(G.js, G.nbins) <= 0xffffffffull;
 }
 
+// dynamic LDS of transport_kernel
+template <int D>
+static size_t transport_lds(const mcd::Grid &G, int threads)
+{
+    return sizeof(float) * ((size_t)(threads / 64) * mcd::JRing<D, true>::kFloats + mcd::lds_floats(G.nx, G.ny, G.nz));
+}
+
+bool mcd_transport_fits(const mcd::Grid &G, int threads)
+{
+    return transport_lds<mcd::kJDepth>(G, threads) <= 160 * 1024;
+}
+
 hipError_t mcd_launch_batch(const mcd::BatchArgs &B, size_t lds_bytes, int blocks, hipStream_t s)
 {
     hipLaunchKernelGGL(mcd::batch_kernel, dim3(blocks), dim3(256), lds_bytes, s, B);
@@ -1123,10 +1141,12 @@ hipError_t mcd_launch_transport(const mcd::Grid &G, const mcd::RunArgs &RA, int 
     } else if (kernel == MCD_KERNEL_POOL && mcd_pool_fits(G)) {
         hipLaunchKernelGGL(mcd::pool_kernel, dim3(blocks), dim3(threads), mcd_pool_lds(G, threads), s,
                            mcd::LaunchArgs{ G, RA });
+    } else if (kernel == MCD_KERNEL_THIN) {
+        hipLaunchKernelGGL(mcd::transport_kernel<4>, dim3(blocks), dim3(threads), transport_lds<4>(G, threads), s,
+                           mcd::LaunchArgs{ G, RA });
     } else {
-        const size_t lds = sizeof(float) * ((size_t)(threads / 64) * mcd::JRing<mcd::kJDepth, true>::kFloats +
-                                            mcd::lds_floats(G.nx, G.ny, G.nz));
-        hipLaunchKernelGGL(mcd::transport_kernel, dim3(blocks), dim3(threads), lds, s, mcd::LaunchArgs{ G, RA });
+        hipLaunchKernelGGL(mcd::transport_kernel<mcd::kJDepth>, dim3(blocks), dim3(threads),
+                           transport_lds<mcd::kJDepth>(G, threads), s, mcd::LaunchArgs{ G, RA });
     }
     return hipGetLastError();
 }
