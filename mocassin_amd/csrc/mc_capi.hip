@@ -2466,6 +2466,16 @@ static int noalloc_scratch_init(mc_ctx *c)
     return MC_OK;
 }
 
+// The bytes that the call's contract counts for n models and their chunks:
+// 456 a model, 16 a chunk, each part of it in units of 256.
+static size_t noalloc_contract(size_t n, size_t chunks)
+{
+    size_t sum = 256;
+    for (size_t b : { 216 * n, 96 * n, 8 * (n + 1), 8 * n, 128 * n, 4 * chunks, 8 * chunks, 4 * chunks })
+        sum += (b + 255) & ~(size_t)255;
+    return sum;
+}
+
 namespace {
 
 __global__ void noalloc_clear_kernel(unsigned long long *w, long long nwords)
@@ -2504,10 +2514,12 @@ extern "C" int mc_transport_batch_noalloc(mc_ctx *const *ctx, int32_t n, const i
     const size_t tot = oK + up((size_t)n * kCounterWords * sizeof(unsigned long long));
     static_assert(kNoAllocModels * (sizeof(mcd::Grid) + sizeof(mcd::RunArgs) + kCounterWords * 8 + 8) + 4096 <
                       kNoAllocBytes, "scratch too small for the most models");
-    // the scratch's contract counts 16 bytes per chunk of packets
-    if (tot + 16 * nchunks > kNoAllocBytes)
+    // the scratch's contract: what a call is refused by does not depend on
+    // what the launch keeps there now
+    const size_t need = noalloc_contract(n, nchunks);
+    if (need > kNoAllocBytes)
         return fail(c0, MC_EINVAL, "the launch needs %zu bytes of scratch (%zu chunks of %lld packets); the "
-                    "allocation-free launch holds %zu: use larger chunks", tot + 16 * nchunks, nchunks,
+                    "allocation-free launch holds %zu: use larger chunks", need, nchunks,
                     (long long)tu.chunk, kNoAllocBytes);
     HIPCHK(c0, hipSetDevice(c0->device));
     for (int i = 0; i < n; ++i) HIPCHK(c0, hipStreamSynchronize(ctx[i]->stream));
