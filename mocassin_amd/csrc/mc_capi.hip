@@ -2148,16 +2148,16 @@ static void log_give_back(int device)
 }
 
 // The chunks a sweep's log should have, or 0 for a sweep that adds with
-// atomics: below about 2e6 deposits the two extra kernels cost more than the
-// atomics, crossing counts go with the atomics, and the words of both
-// estimators must fit the log's ranges (at most 5.2e8).  A flight's segments
-// grow with the axes; the last sweep's count is the better guess.
+// atomics: few deposits for the words of both estimators (least_deposits),
+// more words than the log's ranges take, or crossing counts, which go with the
+// atomics.  A flight's segments grow with the axes; the last sweep's count is
+// the better guess.
 static unsigned log_chunks(const mc_ctx *c, int64_t npackets, const mcl::Shape &s, int blocks, int threads)
 {
     if (!s.bins || (c->G.flags & mcd::F_CROSS)) return 0;
     const double per = c->seg_per_packet > 0.0 ? c->seg_per_packet : (c->G.nx + c->G.ny + c->G.nz) / 4.0;
     const double want = 1.05 * (per + 1.0) * (double)npackets;
-    if (want < 2.e6) return 0;
+    if (want < mcl::least_deposits(s)) return 0;
     // every wavefront holds a chunk
     const double n = want / mcd::kLogChunk + (double)blocks * (threads / 64);
     return (unsigned)std::min(n, (double)(kLogBytes / (mcd::kLogChunk * sizeof(mcd::LogEntry))));

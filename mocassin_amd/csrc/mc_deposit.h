@@ -14,26 +14,13 @@
 #include <stdint.h>
 
 #include "mc_kernels.h"
+#include "mc_log_shape.h"
 
 namespace mcl {
 
 constexpr int kBlock = 16384;            // entries sorted together
 constexpr int kBlockChunks = kBlock / mcd::kLogChunk;
 constexpr int kGroup = 16;               // blocks whose run tables lie together
-constexpr int kRange = 16384;            // words summed by one workgroup (128 KB of LDS)
-constexpr int kMaxBins = 7936;           // with half a block's entries, 4 bytes each, they fill half the LDS of a CU
-constexpr int kMaxShift = 16;
-
-// `words` estimator words in at most kMaxBins bins of 2^shift; a bin is one
-// range of kRange words, or up to four, each of which reads all of it.  With
-// eight the log loses to atomics: H+He on 100^3 cells, 6e8 words, 2e8 packets,
-// 220 ms against 199; with four it gains still: 88^3, 4.1e8 words, 2e7
-// packets, 15.5 ms against 20.0; with two, 64^3, 1.6e8 words, 13.1 against 22.3.
-struct Shape {
-    unsigned words;
-    int shift, bins;
-};
-
 struct Log {
     mcd::LogEntry *entries;              // [chunks * kLogChunk]
     unsigned *count;                     // [chunks] (what the sweep left in each)
@@ -50,8 +37,6 @@ constexpr int kParts = 1024;             // a slice is at most about 1/kParts of
 constexpr int kMaxItems = (kMaxBins + kParts) << (kMaxShift - 14);
 constexpr size_t kPlanWords = 3 * kMaxBins + kMaxItems + 1;
 
-// The shape of `words` words, or bins = 0 if the log does not take that many.
-Shape shape(size_t words);
 size_t run_entries(unsigned chunks, const Shape &s);
 
 }  // namespace mcl

@@ -351,16 +351,6 @@ __global__ void __launch_bounds__(kThreads) reduce_kernel(Log L, Shape s, double
     }
 }
 
-Shape shape(size_t words)
-{
-    Shape s = { 0, 14, 0 };
-    if (words == 0 || words > (size_t)kMaxBins << kMaxShift) return s;
-    while (((words - 1) >> s.shift) + 1 > (size_t)kMaxBins) ++s.shift;
-    s.words = (unsigned)words;
-    s.bins = (int)(((words - 1) >> s.shift) + 1);
-    return s;
-}
-
 size_t run_entries(unsigned chunks, const Shape &s)
 {
     const size_t blocks = (chunks + kBlockChunks - 1) / kBlockChunks;
