@@ -30,7 +30,7 @@ DEFAULT_GRID = {
 POOL_GRID = {
     "blocks_per_cu": (4,),
     "threads": (256,),
-    "emit_min": (16, 24, 32),
+    "emit_min": (16, 24),            # (from 32 on: the auto grid)
     "walk_steps": (8, 16),
     "kernel": ("pool",),
 }
@@ -69,7 +69,7 @@ BATCH_GRID = {
     "waves_per_cu": (8, 12, 16),
     "emit_min": (32, 64),
     "walk_steps": (8, 16, 32),
-    "chunk": (1024, 4096),
+    "chunk": (4096,),
 }
 
 
