@@ -610,6 +610,11 @@ extern "C" int mc_balance_setup(mc_ctx *c, const mc_atomic *at)
     int rc = mcb::prepare(at, c->G.nbins, nu.data(), P, c->err, sizeof c->err);
     if (rc) return rc;
     if (at->nElemUsed != P.A.nE) return fail(c, MC_ETABLE, "nElemUsed %d but %d elements on", at->nElemUsed, P.A.nE);
+    // opacity and re-emission tables that were laid out for ions these rows do
+    // not hold, or for rows of another length, have to be set up again
+    for (size_t k = 0; k < c->op_sl_e.size(); ++k)
+        if (c->op_sl_e[k] >= P.A.nE || c->op_sl_st[k] > P.A.nstages) c->opac = false;
+    if (c->em.nE != P.A.nE || c->em.ns1 != P.A.nstages + 1) c->emis = false;
     // one device block for every table, in this order
     // (cel_s first: its rows are read 16 bytes at a time)
     const std::vector<double> *parts[] = { &P.cel_s, &P.sigma, &P.nu, &P.cR, &P.cH, &P.cel_t, &P.cel_de, &P.cel_glo,
