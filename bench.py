@@ -64,12 +64,20 @@ def shape_of(t):
     return s if name == "auto" else s + "," + name
 
 
-def kernel_name(t):
-    """The device kernels of a large sweep of the 45^3 octant (a grid the
-    pool takes) at a launch shape, as rocprofv3 names them."""
+def kernel_name(t, c, p):
+    """The device kernels of a sweep of the 45^3 octant p (a grid the pool
+    takes) with counters c at a launch shape, as rocprofv3 names them: with
+    enough deposits for its words the sweep is logged
+    (mcl::least_deposits)."""
     from mocassin_amd._capi import KERNELS
     if t.get("kernel", 0) == KERNELS["one"]:
-        return "mcd::transport_kernel"
+        return "mcd::transport_kernel<8>"
+    points = 1
+    for a in ("xAxis", "yAxis", "zAxis"):
+        points *= -(-len(p[a]) // 4) * 4
+    words = points * p["nbins"] + (p["nCells"] + 1) * (p["nbins"] + 1)
+    if c["n_seg"] + c["n_esc"] < 3e6 + words / 5:
+        return "mcd::pool_kernel"
     return "mcd::log_kernel + mcl::sort_kernel + mcl::plan_kernel + mcl::reduce_kernel"
 
 
@@ -388,7 +396,8 @@ def main():
         try:
             tj = json.load(open(tp))
             shape = shape_of(tuning)
-            if tj.get("kernel") == kernel_name(tuning) and tj.get("tuning") == shape and tj.get("tables") == "iterated":
+            kernel = kernel_name(tuning, c0, p)
+            if tj.get("kernel") == kernel and tj.get("tuning") == shape and tj.get("tables") == "iterated":
                 traffic = tj["hbm_bytes_per_packet"] * npk
                 traffic_note = "profiles/transport_c2_traffic.json (%s)" % tj.get("tuning")
                 # the walk's instruction issue: wave64 VALU instructions of
@@ -404,7 +413,7 @@ def main():
                 traffic_note = "profile of other kernels, launch shape or tables (%s, %s, %s): not used" % (
                     tj.get("kernel"), tj.get("tuning"), tj.get("tables"))
                 log("traffic profile is of %s/%s/%s, the run is %s/%s/iterated: traffic not reported"
-                    % (tj.get("kernel"), tj.get("tuning"), tj.get("tables"), kernel_name(tuning), shape))
+                    % (tj.get("kernel"), tj.get("tuning"), tj.get("tables"), kernel, shape))
         except (OSError, ValueError, KeyError):
             pass
     out = {
@@ -422,7 +431,7 @@ def main():
                    "segments_per_packet": c0["n_seg"] / npk, "absorptions_per_packet": c0["n_abs"] / npk},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic, "traffic_source": traffic_note,
-                     "algorithmic_bytes": byts, "kernel": kernel_name(tuning), "kernel_ms": kms,
+                     "algorithmic_bytes": byts, "kernel": kernel_name(tuning, c0, p), "kernel_ms": kms,
                      "segments": c0["n_seg"], "absorptions": c0["n_abs"], "escapes": c0["n_esc"],
                      "lanes_per_pass": lanes_per_pass(c0)},
     }

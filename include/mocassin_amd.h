@@ -114,8 +114,9 @@ typedef struct {
  *                  packet per lane).  The pool's sweeps log their deposits
  *                  and sum them by range of the estimators (up to 4 GiB of
  *                  log per device, shared by its contexts and freed with the
- *                  last); small sweeps, crossing counts and devices without
- *                  the memory use atomics.
+ *                  last); sweeps with few deposits for their estimators'
+ *                  words, crossing counts and devices without the memory use
+ *                  atomics.
  * Results do not depend on these values (each packet has its own stream).
  * A new context starts with 4, 256, 16, 16, MC_KERNEL_AUTO. */
 #define MC_KERNEL_AUTO 0
@@ -216,8 +217,8 @@ int mc_fetch_crossings(mc_ctx *ctx, uint32_t *crossings);
 
 /* Launch shape of a batched transport (chosen by the autotuner; no
  * counterpart in the reference):
- *   waves_per_cu  resident one-wavefront workgroups requested per compute
- *                 unit (1..32)
+ *   waves_per_cu  wavefronts per compute unit (1..32), launched in workgroups
+ *                 of four
  *   emit_min, walk_steps  as in mc_tuning
  *   chunk         64..2^24; sets the noalloc call's limit below.  Wavefronts
  *                 take packets from a counter per model, whatever its value.
@@ -244,10 +245,11 @@ int mc_transport_batch(mc_ctx *const *ctx, int32_t n, const int32_t *istar, cons
 /* mc_transport_batch without any device allocation: no counterpart in the
  * reference; for callers that cannot allocate device memory (serving loops,
  * code under graph capture).  Same arguments and results.  The launch's
- * working block (the models' grids, run arguments and counters) lives in a fixed 8 MiB device array that each GPU the library runs
- * on holds until the process ends; a launch that needs more (at most 256
- * models; 16 bytes per chunk of `chunk` packets) is refused with MC_EINVAL
- * before anything runs.  Every call on a GPU reuses that array: calls that
+ * working block (the models' grids, run arguments and counters) lives in a
+ * fixed 8 MiB device array that each GPU the library runs on holds until the
+ * process ends; a launch that needs more (at most 256 models; counted as some
+ * 456 bytes a model and 16 per chunk of `chunk` packets) is refused with
+ * MC_EINVAL before anything runs.  Every call on a GPU reuses that array: calls that
  * overlap on one GPU race. */
 int mc_transport_batch_noalloc(mc_ctx *const *ctx, int32_t n, const int32_t *istar, const int64_t *npackets,
                                const uint64_t *packet_offset, const mc_batch_tuning *tuning, mc_counters *c,

@@ -11,9 +11,10 @@ constexpr int kMaxShift = 16;
 
 // `words` estimator words in at most kMaxBins bins of 2^shift; a bin is one
 // range of kRange words, or up to four, each of which reads all of it.  With
-// eight the log loses to atomics: H+He on 100^3 cells, 6e8 words, 2e8 packets,
-// 220 ms against 199; with four it gains still: 88^3, 4.1e8 words, 2e7
-// packets, 15.5 ms against 20.0; with two, 64^3, 1.6e8 words, 13.1 against 22.3.
+// eight the log gains nothing any more: H+He octants on the cold start's
+// tables, 2e7 packets, logged and with atomics: 64^3 cells (1.6e8 words, two
+// ranges to a bin) 17.4, 30.0 ms, 88^3 (4.1e8, four) 31.9, 37.1, 100^3 (6e8,
+// eight) 46.0, 39.3; a full 100^3 grid 24.4, 24.9.
 struct Shape {
     unsigned words;
     int shift, bins;

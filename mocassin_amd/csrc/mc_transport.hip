@@ -27,7 +27,7 @@
 // packets on a 45^3 octant of 800 bins (1.8e9 deposits): 64.8 ms before (the
 // pool with atomics and divisions), 39.0 now (walk and log 22.6, sort 8.4,
 // sums 7.8); 4e7 packets in dust and gas 60^3: 67.4 ms before, 42.0 now; 8
-// models of 20^3 to 50^3 cells, 2e6 packets each, in one launch: 5.9 ms.
+// models of 20^3 to 50^3 cells, 2.8e5 to 2e6 packets, in one launch: 5.9-6.6 ms.
 #include <algorithm>
 
 #include "mc_device.h"
@@ -608,7 +608,8 @@ __device__ __forceinline__ void walk_pass(Lane &L, const Grid &G, const Axes &A,
 // and the walkers come back as flights end.  The walk passes then stay nearly
 // full between emissions.  Word k of slot s is at pw[k * P + s]; the cell
 // indices are packed in one word (11, 11 and 10 bits: the host runs this
-// kernel on lattices of at most 2048 x 2048 x 1024 points), the frequency
+// kernel on lattices of at most 2047 x 2047 x 1023 points: an escaped packet's
+// index is one past the last), the frequency
 // bin, run count and phase in another (16, 13 and 3 bits), steps and direction
 // signs in a third.  The stream is the launch's source, not stored, and a
 // waiting packet's optical depths and reciprocals are of no use any more.
@@ -1057,7 +1058,7 @@ __global__ void guide_kernel(const float *cdf, int rows, int nbins, unsigned sho
 // a thread takes one (x,y,z) of a column of bricks, z fastest, and goes
 // through the bins: a wavefront's stores are runs of the column's length, and
 // its workgroup reads whole rows of the bricks.  In the lattice's order (x
-// fastest) every store was a request of its own: 27^3 cells 440 -> 47 us, 19^3
+// fastest) every store was a request of its own: 27^3 cells 448 -> 21 us, 19^3
 // octant 96 -> 11.
 constexpr int kCompact = 512;
 __global__ void __launch_bounds__(kCompact)
