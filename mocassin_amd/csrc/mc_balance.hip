@@ -19,6 +19,7 @@
 #include "mc_balance.h"
 #include "mc_cel.h"
 #include "mc_device.h"
+#include "mc_grid_limit.h"
 #include "mc_mlp.h"
 
 #include <algorithm>
@@ -834,12 +835,12 @@ __device__ __forceinline__ Coeffs uniform_row(const double *p)
 __global__ void __launch_bounds__(64) integrals_kernel(const Atomic *__restrict__ Ap, CellArgs a,
                                                        const double *__restrict__ J3,
                                                        const int *__restrict__ active, mcd::J3Shape js, int groups,
-                                                       double *__restrict__ Rint, double *__restrict__ Hint,
+                                                       unsigned tile0, double *__restrict__ Rint, double *__restrict__ Hint,
                                                        int *__restrict__ hit, float *__restrict__ X)
 {
     const Atomic &A = *Ap;
     const int lane = threadIdx.x;
-    const unsigned i = blockIdx.x >> 3, tile = (i / groups) * 8 + (blockIdx.x & 7);
+    const unsigned i = blockIdx.x >> 3, tile = tile0 + (i / groups) * 8 + (blockIdx.x & 7);
     const int g0 = (int)(i % groups) * kIntCh;
     if (tile >= mcd::j3_points(js) / mcd::kJTile) return;
     const int xyz = mcd::j3_lattice(js, tile * 64u + (unsigned)lane);
@@ -1153,9 +1154,15 @@ hipError_t mcb_launch_integrals(const mcb::Atomic *dA, const mcb::CellArgs &a, c
     const mcd::J3Shape js = mcd::j3_shape(nx, ny, nz);
     const unsigned tiles = (unsigned)(mcd::j3_points(js) / mcd::kJTile);
     const int groups = a.nch > mcb::kIntCh ? (a.nch + mcb::kIntCh - 1) / mcb::kIntCh : 1;
-    hipLaunchKernelGGL(mcb::integrals_kernel, dim3((tiles + 7) / 8 * 8 * groups), dim3(64), 0, s, dA, a, J3, active, js,
-                       groups, Rint, Hint, hit, X);
-    return hipGetLastError();
+    const unsigned most = mcb::tiles_per_launch((unsigned)groups);
+    for (unsigned t = 0; t < tiles; t += most) {
+        const unsigned n = std::min(most, tiles - t);
+        hipLaunchKernelGGL(mcb::integrals_kernel, dim3((n + 7) / 8 * 8 * groups), dim3(64), 0, s, dA, a, J3, active, js,
+                           groups, t, Rint, Hint, hit, X);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 hipError_t mcb_launch_warm(const mcb::Atomic *dA, const mcb::CellArgs &a, const float *Y, int ldy, const int *hit,
