@@ -540,9 +540,9 @@ __device__ __forceinline__ void grain_terms(const Atomic &A, const Grains &G, co
 }
 
 // G lanes a cell.  Registers for three wavefronts a SIMD with model ions (5.6
-// ms on the 45^3 octant; four spill the level solves' rows, two take 6.6), for
-// two without (the chain of steps bounds it: dust and gas 60^3 6.3 ms against
-// 7.0 for three and 8.0 for four).
+// ms on the 45^3 octant; two take 6.6; for four more would spill than the 71
+// registers that do), for two without (the chain of steps bounds it: dust and
+// gas 60^3 6.3 ms against 7.0 for three and 8.0 for four).
 template <bool PE, int G>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(G == 64 ? 3 : 2))) balance_kernel(const Atomic *__restrict__ Ap, CellArgs a)
 {

@@ -55,7 +55,9 @@ hipError_t mcd_launch_batch(const mcd::BatchArgs &B, size_t lds_bytes, int block
 // 32 packets per wavefront in LDS.  The pool kernel packs a packet's cell and
 // bin and keeps 32-bit indices of the tables: it takes grids of at most 2047 x
 // 2047 x 1023 cells, 65535 bins and 2^32 - 1 table words; other grids run the
-// first whatever kernel is asked for.
+// first whatever kernel is asked for, which there is no slower (2e7 packets,
+// 240^3 octant of 320 bins, 4.4e9 words: 109 ms, and 115 with a pool of 64-bit
+// indices; 200^3 of 300, 2.4e9 words: 108, and 110 with this pool).
 // The log kernel is the pool kernel with the deposits written to the log of
 // its RunArgs instead of added to the estimators.  The thin kernel is the
 // first with shorter rings, for axes that leave no room for more.

@@ -967,7 +967,7 @@ __global__ void __launch_bounds__(256) pool_kernel(LaunchArgs)
     pool_run<kPoolSlots>(K, A, pools + (size_t)wave * kPoolSlots * kPoolWords, D, (int)(threadIdx.x & 63));
 }
 
-// The single-model kernel with its deposits in the log: 74 VGPRs, six
+// The single-model kernel with its deposits in the log: 78 VGPRs, six
 // wavefronts a SIMD as far as its LDS (queue and pool, 6.3 KB a wavefront) allows.
 __global__ void __launch_bounds__(256) log_kernel(LaunchArgs)
 {
