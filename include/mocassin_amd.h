@@ -464,7 +464,8 @@ int mc_opacity_build(mc_ctx *ctx, const float *Hden, const float *Te, const floa
                      const float *Tdust, float *opacity, float *scaOpac, double *kernel_ms);
 
 /* A table that mc_opacity_build or mc_emission_build left on the device, row
- * by row: rows[(nCells+1)][nbins], row 0 zero (the builds' own outputs are
+ * by row: rows[(nCells+1)][nbins]; row 0 is zero, and so are the opacity rows
+ * of cells that no lattice point has (the builds' own outputs are
  * column-major).  No counterpart in the reference. */
 #define MC_TABLE_OPACITY 0
 #define MC_TABLE_SCATTERING 1

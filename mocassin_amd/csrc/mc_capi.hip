@@ -1344,6 +1344,9 @@ extern "C" int mc_fetch_table_rows(mc_ctx *c, int32_t table, float *rows)
         HIPCHK(c, mco_launch_rows(table == MC_TABLE_OPACITY ? c->d_opac3 : c->d_sca3, c->G.js, c->d_active, (int)nb,
                                   c->d_op_out, c->stream));
         HIPCHK(c, fetch(c, rows, c->d_op_out, nt * sizeof(float)));
+        // rows that no lattice point wrote
+        for (size_t cell = 1; cell <= (size_t)c->G.nCells; ++cell)
+            if (c->cell_xyz[cell] < 0) std::memset(rows + cell * nb, 0, nb * sizeof(float));
         break;
     case MC_TABLE_RECPDF:
         if (!c->rec_built) return fail(c, MC_ESTATE, "mc_emission_build has not been called");
