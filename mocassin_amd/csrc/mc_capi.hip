@@ -200,7 +200,7 @@ static hipError_t fill_on(hipStream_t s, void *dst, int value, size_t bytes)
 
 // Large results come through two pinned buffers of the device (Staging
 // below): a piece is copied out of one while the next arrives in the other.
-// Returns when dst holds the data.
+// dst holds the data when the stream has been waited for.
 static hipError_t fetch(mc_ctx *c, void *dst, const void *src, size_t bytes);
 
 static int ctx_init(mc_ctx *c, const mc_desc *d);
@@ -1344,6 +1344,7 @@ extern "C" int mc_fetch_table_rows(mc_ctx *c, int32_t table, float *rows)
         HIPCHK(c, mco_launch_rows(table == MC_TABLE_OPACITY ? c->d_opac3 : c->d_sca3, c->G.js, c->d_active, (int)nb,
                                   c->d_op_out, c->stream));
         HIPCHK(c, fetch(c, rows, c->d_op_out, nt * sizeof(float)));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
         // rows that no lattice point wrote
         for (size_t cell = 1; cell <= (size_t)c->G.nCells; ++cell)
             if (c->cell_xyz[cell] < 0) std::memset(rows + cell * nb, 0, nb * sizeof(float));
@@ -1351,6 +1352,7 @@ extern "C" int mc_fetch_table_rows(mc_ctx *c, int32_t table, float *rows)
     case MC_TABLE_RECPDF:
         if (!c->rec_built) return fail(c, MC_ESTATE, "mc_emission_build has not been called");
         HIPCHK(c, fetch(c, rows, c->d_recCDF, nt * sizeof(float)));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
         break;
     default:
         return fail(c, MC_EINVAL, "unknown table %d", table);
@@ -1619,6 +1621,7 @@ extern "C" int mc_emission_build(mc_ctx *c, const float *Hden, const float *Te, 
     if (recPDF) {
         std::vector<float> rec(nt);
         HIPCHK(c, fetch(c, rec.data(), c->d_recCDF, nt * sizeof(float)));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
         // 16 cells at a time: a line of the rows and one of the columns each
         for (size_t c0 = 1; c0 < nc1; c0 += 16)
             for (int i = 0; i < nb; ++i)
@@ -2106,10 +2109,10 @@ static Staging g_stage[kLogDevices];
 static hipError_t fetch(mc_ctx *c, void *dst, const void *src, size_t bytes)
 {
     if (bytes < kStageMin || c->device < 0 || c->device >= kLogDevices)
-        return copy_on(c->stream, dst, src, bytes, hipMemcpyDeviceToHost);
+        return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream);
     Staging &S = g_stage[c->device];
     std::unique_lock<std::mutex> use(S.use, std::try_to_lock);
-    if (!use.owns_lock() || !S.ready()) return copy_on(c->stream, dst, src, bytes, hipMemcpyDeviceToHost);
+    if (!use.owns_lock() || !S.ready()) return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream);
     const size_t n = (bytes + kStage - 1) / kStage;
     auto piece = [&](size_t k) { return std::min(kStage, bytes - k * kStage); };
     hipError_t e = hipSuccess;
