@@ -112,6 +112,7 @@ struct mc_ctx {
     mco::Ent *d_op_ent = nullptr;                // cross-section entries of every bin
     float *d_hs = nullptr;              // a state given by the host, and the same in rows
     double *d_hst = nullptr;
+    std::vector<double> rows_h;         // a small one's rows on the host
     size_t hs_n = 0, hst_n = 0, cold_n = 0, ion_host_n = 0, op_Td_n = 0, em_Td_n = 0;   // entries (room)
     float *d_op_st = nullptr, *d_op_Td = nullptr, *d_op_out = nullptr;
     mco::OpacArgs op{};
@@ -202,6 +203,10 @@ static hipError_t fill_on(hipStream_t s, void *dst, int value, size_t bytes)
 // below): a piece is copied out of one while the next arrives in the other.
 // dst holds the data when the stream has been waited for.
 static hipError_t fetch(mc_ctx *c, void *dst, const void *src, size_t bytes);
+// Host arrays one after another into dst, through the same buffers.  Returns
+// when dst holds them.
+struct HostPart { const void *from; size_t bytes; };
+static hipError_t send(mc_ctx *c, void *dst, const HostPart *part, int parts);
 
 static int ctx_init(mc_ctx *c, const mc_desc *d);
 static int noalloc_scratch_init(mc_ctx *c);
@@ -940,24 +945,44 @@ __global__ void state_rows_kernel(const float *__restrict__ host, double *__rest
             st[t] = host[t];
 }
 
-// The host's state on the device, laid out there (a host pass over ionDen in
-// cell order strides through it): st gets the block of state_rows_kernel.
+// The host's state on the device as the block of state_rows_kernel, st.  A
+// small state is laid out on the host, which saves a launch; a pass over a large
+// one's ionDen in cell order strides through it, so that is laid out on the
+// device.  Line luminosities, us, laid out on the host and on the device: H and
+// He octants of 9^3 cells (60 KB of rows) 62, 70, 15^3 (270 KB) 109, 110, 24^3
+// (1.1 MB) 249, 181; seven elements 11^3 (250 KB) 239, 239, 24^3 865, 710.
+constexpr size_t kHostRows = 256 << 10;
 static int upload_state(mc_ctx *c, const float *Hden, const float *Te, const float *Ne, const float *ionDen, double **st)
 {
     const int nE = c->bal.A.nE, ns = c->bal.A.nstages;
     const size_t nc1 = (size_t)c->G.nCells + 1, nf = nc1 * (3 + (size_t)nE * ns), nd = nc1 * (3 + (size_t)nE * (ns + 1));
-    HIPCHK(c, room(&c->d_hs, &c->hs_n, nf));
     HIPCHK(c, room(&c->d_hst, &c->hst_n, nd));
-    const float *part[3] = { Te, Ne, Hden };
-    for (int k = 0; k < 3; ++k)
-        HIPCHK(c, hipMemcpyAsync(c->d_hs + k * nc1, part[k], nc1 * sizeof(float), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->d_hs + 3 * nc1, ionDen, nc1 * nE * ns * sizeof(float), hipMemcpyHostToDevice, c->stream));
+    *st = c->d_hst;
+    if (nd * sizeof(double) <= kHostRows) {
+        std::vector<double> &rows = c->rows_h;
+        rows.assign(nd, 0.0);
+        double *ion = rows.data() + 3 * nc1;
+        for (size_t cell = 0; cell < nc1; ++cell) {
+            rows[cell] = Te[cell];
+            rows[nc1 + cell] = Ne[cell];
+            rows[2 * nc1 + cell] = Hden[cell];
+            for (int e = 0; e < nE; ++e)
+                for (int k = 1; k <= ns; ++k)
+                    ion[(cell * nE + e) * (ns + 1) + k] =
+                        ionDen[cell + nc1 * ((size_t)c->bal.eidx_xref[e] - 1 + (size_t)nE * (k - 1))];
+        }
+        HIPCHK(c, copy_on(c->stream, c->d_hst, rows.data(), nd * sizeof(double), hipMemcpyHostToDevice));
+        return MC_OK;
+    }
+    HIPCHK(c, room(&c->d_hs, &c->hs_n, nf));
+    const HostPart part[4] = { { Te, nc1 * sizeof(float) }, { Ne, nc1 * sizeof(float) }, { Hden, nc1 * sizeof(float) },
+                               { ionDen, nc1 * nE * ns * sizeof(float) } };
+    HIPCHK(c, send(c, c->d_hs, part, 4));
     IonMap m{};
     for (int e = 0; e < nE; ++e) m.xr[e] = c->bal.eidx_xref[e] - 1;
     hipLaunchKernelGGL(state_rows_kernel, dim3(ion_blocks(nc1 * nE)), dim3(256), 0, c->stream, c->d_hs, c->d_hst,
                        (long long)nc1, nE, ns, m);
     HIPCHK(c, hipGetLastError());
-    *st = c->d_hst;
     return MC_OK;
 }
 
@@ -1685,10 +1710,10 @@ extern "C" int mc_line_luminosities(mc_ctx *c, const float *Hden, const float *T
             for (size_t i = 0; i < nc1; ++i) bl[i] = lgBlack[i] >= 1 ? 1 : 0;
             if (!c->d_ln_black) HIPCHK(c, dalloc(&c->d_ln_black, nc1));
             HIPCHK(c, hipMemcpyAsync(c->d_ln_black, bl.data(), nc1 * sizeof(int), hipMemcpyHostToDevice, c->stream));
+            HIPCHK(c, hipStreamSynchronize(c->stream));
             a.black = c->d_ln_black;
             a.black_mask = 1;
         }
-        HIPCHK(c, hipStreamSynchronize(c->stream));
     } else {
         a.Te = c->d_Te;
         a.Ne = c->d_Ne;
@@ -2074,11 +2099,12 @@ struct LogPool {
 static LogPool g_log[kLogDevices];
 static std::mutex g_log_mu;              // the context counts
 
-// Two pinned buffers per device for results on their way to the host, made
-// at the first large one, used by one call at a time (another copies
-// directly) and freed with the device's last context.  The 46 MB of a 19^3
-// octant's estimators take 1.07 ms against 1.37 by direct copies; the least
-// is a piece's size so that one buffer is filled while the other is emptied.
+// Two pinned buffers per device for results on their way to the host and
+// states on theirs to the device, made at the first large one, used by one
+// call at a time (another copies directly) and freed with the device's last
+// context.  The 46 MB of a 19^3 octant's estimators take 1.07 ms against 1.37
+// by direct copies; the least of results is a piece's size so that one buffer
+// is filled while the other is emptied.
 constexpr size_t kStage = (size_t)4 << 20, kStageMin = kStage;
 struct Staging {
     std::mutex use;
@@ -2129,6 +2155,40 @@ static hipError_t fetch(mc_ctx *c, void *dst, const void *src, size_t bytes)
     // nothing of this call may still be on its way into the buffers
     if (e != hipSuccess) (void)hipStreamSynchronize(c->stream);
     return e;
+}
+
+static hipError_t send(mc_ctx *c, void *dst, const HostPart *part, int parts)
+{
+    size_t bytes = 0;
+    for (int k = 0; k < parts; ++k) bytes += part[k].bytes;
+    char *to = static_cast<char *>(dst);
+    hipError_t e = hipSuccess;
+    const bool known = c->device >= 0 && c->device < kLogDevices;
+    Staging &S = g_stage[known ? c->device : 0];
+    std::unique_lock<std::mutex> use(S.use, std::defer_lock);
+    if (!known || !use.try_lock() || !S.ready()) {
+        for (int k = 0; k < parts && e == hipSuccess; to += part[k++].bytes)
+            e = hipMemcpyAsync(to, part[k].from, part[k].bytes, hipMemcpyHostToDevice, c->stream);
+    } else {
+        size_t at = 0;                       // within the part part[0]
+        for (size_t i = 0, sent = 0; sent < bytes && e == hipSuccess; ++i) {
+            if (i >= 2) e = hipEventSynchronize(S.there[i & 1]);
+            size_t n = 0;
+            while (e == hipSuccess && n < kStage && sent + n < bytes) {
+                const size_t m = std::min(kStage - n, part->bytes - at);
+                std::memcpy(S.buf[i & 1] + n, static_cast<const char *>(part->from) + at, m);
+                n += m;
+                at += m;
+                if (at == part->bytes) { at = 0; ++part; }
+            }
+            if (e == hipSuccess) e = hipMemcpyAsync(to + sent, S.buf[i & 1], n, hipMemcpyHostToDevice, c->stream);
+            if (e == hipSuccess) e = hipEventRecord(S.there[i & 1], c->stream);
+            sent += n;
+        }
+    }
+    // nothing may still be on its way out of the buffers
+    const hipError_t w = hipStreamSynchronize(c->stream);
+    return e == hipSuccess ? w : e;
 }
 
 static void log_join(mc_ctx *c)

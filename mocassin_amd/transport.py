@@ -301,7 +301,7 @@ class Transport:
         if Te is not None:
             st = [np.ascontiguousarray(Hden, np.float32).reshape(nc1), np.ascontiguousarray(Te, np.float32).reshape(nc1),
                   np.ascontiguousarray(Ne, np.float32).reshape(nc1),
-                  np.asfortranarray(np.asarray(ionDen, np.float32).reshape(nc1, self._nE, self._ns))]
+                  np.asarray(np.reshape(ionDen, (nc1, self._nE, self._ns)), np.float32, order="F")]
         td = None if Tdust is None else np.ascontiguousarray(Tdust, np.float32).ravel()
         if td is not None and td.size != nc1 * int(np.prod(getattr(self, "_dust_shape", (0,)))):
             raise ValueError("Tdust needs (nCells+1) x (nSizes+1) x (nSpeciesMax+1) entries (dust_setup first)")
@@ -369,7 +369,7 @@ class Transport:
         if Te is not None:
             st = [np.ascontiguousarray(Hden, np.float32).reshape(nc1), np.ascontiguousarray(Te, np.float32).reshape(nc1),
                   np.ascontiguousarray(Ne, np.float32).reshape(nc1),
-                  np.asfortranarray(np.asarray(ionDen, np.float32).reshape(nc1, self._nE, self._ns))]
+                  np.asarray(np.reshape(ionDen, (nc1, self._nE, self._ns)), np.float32, order="F")]
         td = None if Tdust is None else np.ascontiguousarray(Tdust, np.float32).ravel()
         tl = np.zeros(nc1, np.float32) if host else None
         ms = C.c_double()
@@ -389,7 +389,7 @@ class Transport:
         if Te is not None:
             st = [np.ascontiguousarray(Hden, np.float32).reshape(nc1), np.ascontiguousarray(Te, np.float32).reshape(nc1),
                   np.ascontiguousarray(Ne, np.float32).reshape(nc1),
-                  np.asfortranarray(np.asarray(ionDen, np.float32).reshape(nc1, self._nE, self._ns))]
+                  np.asarray(np.reshape(ionDen, (nc1, self._nE, self._ns)), np.float32, order="F")]
             if lgBlack is not None:
                 bl = np.ascontiguousarray(lgBlack, np.int32).reshape(nc1)
         forb = np.zeros((self._ncel, 17, 17), np.float64)
