@@ -59,7 +59,6 @@ struct mc_ctx {
     float *d_opac3 = nullptr, *d_sca3 = nullptr, *d_recCDF = nullptr;
     unsigned short *d_recGuide = nullptr;
     float *d_totalLines = nullptr, *d_specCDF = nullptr, *d_nuArray = nullptr, *d_gSca = nullptr;
-    unsigned short *d_specGuide = nullptr;
     double *d_J3 = nullptr, *d_J = nullptr, *d_esc = nullptr;
     mcd::View *d_view = nullptr;            // viewing-angle bins (null: escapes in plane 0 only)
     int esc_planes = 1;                      // nAngleBins + 1
@@ -406,7 +405,7 @@ extern "C" int mc_upload_tables(mc_ctx *c, const float *opacity, const float *sc
             if (opacity[(size_t)nu * (nc + 1)] != 0.f)
                 return fail(c, MC_ETABLE, "opacity row 0 (inactive cells) must be zero (bin %d)", nu + 1);
     float *tmp = nullptr;
-    HIPCHK(c, dalloc(&tmp, nt));
+    if (opacity || (dust && scaOpac)) HIPCHK(c, dalloc(&tmp, nt));
     int rc = MC_OK;
     hipError_t e = hipSuccess;
     if (opacity) {
@@ -427,10 +426,16 @@ extern "C" int mc_upload_tables(mc_ctx *c, const float *opacity, const float *sc
     if (e != hipSuccess)
         return fail(c, e == hipErrorOutOfMemory ? MC_ENOMEM : MC_ENODEV, "table upload: %s", hipGetErrorString(e));
     (void)rc;
-    if (!c->d_specCDF) HIPCHK(c, dalloc(&c->d_specCDF, (size_t)nb * c->nStars));
-    HIPCHK(c, copy_on(c->stream, c->d_specCDF, specCDF, (size_t)nb * c->nStars * sizeof(float), hipMemcpyHostToDevice));
-    if (!c->d_specGuide) HIPCHK(c, dalloc(&c->d_specGuide, (size_t)c->nStars * (mcd::kGuide + 1)));
-    HIPCHK(c, mcd_guides(c->d_specCDF, c->nStars, nb, c->d_specGuide, c->stream));
+    // the sources' rows and their guides in one copy
+    const size_t nspec = (size_t)nb * c->nStars, nguide = (size_t)c->nStars * (mcd::kGuide + 1);
+    std::vector<float> spec(nspec + (nguide + 1) / 2);
+    std::memcpy(spec.data(), specCDF, nspec * sizeof(float));
+    for (size_t i = 0; i < nguide; ++i) {
+        const unsigned short g = mcd::guide_entry(specCDF + i / (mcd::kGuide + 1) * nb, nb, (int)(i % (mcd::kGuide + 1)));
+        std::memcpy(reinterpret_cast<char *>(spec.data() + nspec) + i * sizeof g, &g, sizeof g);
+    }
+    if (!c->d_specCDF) HIPCHK(c, dalloc(&c->d_specCDF, spec.size()));
+    HIPCHK(c, copy_on(c->stream, c->d_specCDF, spec.data(), spec.size() * sizeof(float), hipMemcpyHostToDevice));
     if (rec_host) {
         if (!c->d_recCDF) HIPCHK(c, dalloc(&c->d_recCDF, nt));
         if (!c->d_recGuide) HIPCHK(c, dalloc(&c->d_recGuide, (size_t)(nc + 1) * (mcd::kGuide + 1)));
@@ -444,7 +449,8 @@ extern "C" int mc_upload_tables(mc_ctx *c, const float *opacity, const float *sc
         if (!c->d_gSca) HIPCHK(c, dalloc(&c->d_gSca, nb));
         HIPCHK(c, copy_on(c->stream, c->d_gSca, gSca, nb * sizeof(float), hipMemcpyHostToDevice));
     }
-    G.opac3 = c->d_opac3; G.sca3 = c->d_sca3; G.specCDF = c->d_specCDF; G.specGuide = c->d_specGuide;
+    G.opac3 = c->d_opac3; G.sca3 = c->d_sca3; G.specCDF = c->d_specCDF;
+    G.specGuide = reinterpret_cast<const unsigned short *>(c->d_specCDF + nspec);
     G.recCDF = c->d_recCDF; G.recGuide = c->d_recGuide; G.totalLines = c->d_totalLines;
     G.gSca = c->d_gSca;
     c->tables = true;
@@ -1644,14 +1650,17 @@ extern "C" int mc_emission_build(mc_ctx *c, const float *Hden, const float *Te, 
         *kernel_ms = ms;
     }
     if (recPDF) {
-        std::vector<float> rec(nt);
-        HIPCHK(c, fetch(c, rec.data(), c->d_recCDF, nt * sizeof(float)));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        // 16 cells at a time: a line of the rows and one of the columns each
-        for (size_t c0 = 1; c0 < nc1; c0 += 16)
-            for (int i = 0; i < nb; ++i)
-                for (size_t cell = c0; cell < std::min(nc1, c0 + 16); ++cell)
-                    recPDF[cell + nc1 * i] = rec[cell * nb + i];
+        // in the host's order, through the next build's rows (whose row 0 is
+        // zero again after it); the host's row 0 stays
+        if (!c->d_recCDF_b) HIPCHK(c, dalloc(&c->d_recCDF_b, nt));
+        HIPCHK(c, mco_launch_columns(c->d_recCDF, nc1, nb, c->d_recCDF_b, c->stream));
+        std::vector<float> row0(nb);
+        for (int i = 0; i < nb; ++i) row0[i] = recPDF[nc1 * i];
+        const hipError_t e = fetch(c, recPDF, c->d_recCDF_b, nt * sizeof(float)), w = hipStreamSynchronize(c->stream);
+        for (int i = 0; i < nb; ++i) recPDF[nc1 * i] = row0[i];
+        HIPCHK(c, e);
+        HIPCHK(c, w);
+        HIPCHK(c, fill_on(c->stream, c->d_recCDF_b, 0, (size_t)nb * sizeof(float)));
     }
     if (totalLines) {
         std::vector<float> tl(nc1);
@@ -2713,7 +2722,7 @@ extern "C" void mc_ctx_destroy(mc_ctx *c)
     if (!c) return;
     (void)hipSetDevice(c->device);
     void *bufs[] = { c->d_axis, c->d_mid, c->d_dfac, c->d_active, c->d_opac3, c->d_sca3,
-                     c->d_recCDF, c->d_recGuide, c->d_totalLines, c->d_specCDF, c->d_specGuide, c->d_nuArray,
+                     c->d_recCDF, c->d_recGuide, c->d_totalLines, c->d_specCDF, c->d_nuArray,
                      c->d_gSca, c->d_J3, c->d_J, c->d_esc, c->d_view, c->d_scratch, c->d_error, c->d_qphot,
                      c->d_cell_xyz, c->d_atomic, c->d_bal_tab, c->d_Hden, c->d_Te, c->d_Ne,
                      c->d_ion, c->d_flags, c->d_nIter, c->d_cold, c->d_mlp, c->d_mlpW, c->d_mX,

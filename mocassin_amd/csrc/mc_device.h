@@ -219,7 +219,7 @@ __device__ __forceinline__ int getnu2(Rng &R, const Grid &G, const float *cdf,
 }
 
 // g[j] = #{i : cdf[i] <= j/kGuide}, j = 0..kGuide, for a monotone row
-__device__ __forceinline__ unsigned short guide_entry(const float *cdf, int nbins, int j)
+__host__ __device__ __forceinline__ unsigned short guide_entry(const float *cdf, int nbins, int j)
 {
     const float t = (float)j / (float)kGuide;
     int lo = 0, hi = nbins;

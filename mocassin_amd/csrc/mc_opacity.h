@@ -63,6 +63,8 @@ hipError_t mco_launch_f32(const double *in, size_t n, float *out, hipStream_t s)
 // rows [cell][nb] of a J3-layout table (row 0 not written)
 hipError_t mco_launch_rows(const float *t3, const mcd::J3Shape &js, const int *active, int nb, float *out,
                            hipStream_t s);
+// (0:nc, 1:nb) column-major copy of rows [nc + 1][nb]
+hipError_t mco_launch_columns(const float *rows, size_t nc1, int nb, float *out, hipStream_t s);
 // (0:nc, 1:nb) column-major copy of a J3-layout table (row 0 zero)
 hipError_t mco_launch_gather(const float *t3, const mcd::J3Shape &js, const int *cell_xyz, int nc, int nb,
                              float *out, hipStream_t s);

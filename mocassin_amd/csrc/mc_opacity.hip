@@ -301,6 +301,31 @@ __global__ void __launch_bounds__(256) rows_kernel(const float *t3, mcd::J3Shape
 }
 }  // namespace mco
 
+namespace mco {
+// Rows [cell][nb] as the host's columns (0:nc, nb), 64 cells by 64 bins through
+// LDS.  Bound by the copy to the host that follows: the columns of a 36^3
+// octant, H and He on 400 bins (39 MB), took COLS.
+__global__ void __launch_bounds__(256) columns_kernel(const float *__restrict__ rows, size_t nc1, int nb,
+                                                      float *__restrict__ out)
+{
+    __shared__ float v[64][65];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nu0 = blockIdx.y * 64;
+    const size_t c0 = (size_t)blockIdx.x * 64;
+    for (int q = w; q < 64 && c0 + q < nc1; q += 4)
+        if (nu0 + lane < nb) v[q][lane] = rows[(c0 + q) * nb + nu0 + lane];
+    __syncthreads();
+    for (int q = w; q < 64 && nu0 + q < nb; q += 4)
+        if (c0 + lane < nc1) out[c0 + lane + nc1 * (nu0 + q)] = v[lane][q];
+}
+}  // namespace mco
+
+hipError_t mco_launch_columns(const float *rows, size_t nc1, int nb, float *out, hipStream_t s)
+{
+    hipLaunchKernelGGL(mco::columns_kernel, dim3((unsigned)((nc1 + 63) / 64), (unsigned)((nb + 63) / 64)), dim3(256), 0, s,
+                       rows, nc1, nb, out);
+    return hipGetLastError();
+}
+
 hipError_t mco_launch_rows(const float *t3, const mcd::J3Shape &js, const int *active, int nb, float *out, hipStream_t s)
 {
     hipLaunchKernelGGL(mco::rows_kernel, dim3((unsigned)(mcd::j3_points(js) / 64), (unsigned)((nb + 63) / 64)), dim3(256),
